@@ -211,7 +211,7 @@ class QuantOpts:  # src/quantizer.hpp:11-19
     want_hatW: bool = False
     feedback: int = 0          # 0: fp64 feedback (default), 1: fp32 feedback + bf16 hi/lo split MFMA
     skip_proxy: bool = False
-    ldl_device_updates: bool = True    # the LDL's trailing updates run on the GPU (same L bit for bit); False: host alone
+    ldl_device_updates: bool = True    # the LDL runs on the GPU (same L bit for bit); False: on the host
     ldlq_chains: int = 0       # independent chains of launches the tile rows are dealt to (0: the library's default: 3 where its side streams have hardware queues of their own, else 2: ldlq_default_chains())
     group_lanes: int = 0       # run_groups: groups run side by side on this many lanes (0: as many as fit the chip, 1 for large groups; 1: one after the other)
 
@@ -417,7 +417,7 @@ class Quantizer:
         hp.t_ldl = time.time() - t0
 
     def ldl_hessian_device_updates(self, hp: HessPrep, threads=16):
-        """ldl_hessian with the trailing updates of the host's panels on the GPU; hp.L equals ldl_hessian's."""
+        """ldl_hessian on the GPU; hp.L equals ldl_hessian's (threads is not used)."""
         import time
         t0 = time.time()
         hp.L = np.zeros((hp.n, hp.n), np.float32)
@@ -429,8 +429,7 @@ class Quantizer:
 
     def ldl_hessian_device_resident(self, dHRr, n, L_host, dL=None, threads=16):
         """The same with the rotated Hessian on the device (dHRr, never written), as run_groups runs it: L goes to
-        L_host (n x n fp32, page-locked when dL is given) and, column block by column block, to the device buffer
-        dL.  Returns the seconds the call took."""
+        L_host (n x n fp32) and to the device buffer dL.  Returns the seconds the call took."""
         import time
         t0 = time.time()
         _check(lib().qtip_ldl_hessian_device_updates_dev(self._h, _ptr(dHRr), n, threads, _ptr(L_host),
@@ -534,7 +533,7 @@ class Quantizer:
     def nvfp4_quantize_group(self, ws, n, H=None, scale_search=True, calibrate=True, sigma_reg=1e-2,
                              factor_on_host=False):
         """nvfp4_quantize_group, src/nvfp4_gpu.hip:174-241 -> (tensors, calibrated).  factor_on_host: the calibration's
-        Cholesky factorization on the host alone (default: its trailing updates on the GPU, same bits)."""
+        Cholesky factorization on the host alone (default: on the GPU, same bits)."""
         mats, outs, keep = self._nvfp4_marshal(ws, n)
         o = _Nvfp4OptsC(1 if scale_search else 0, 1 if calibrate else 0, sigma_reg, 1 if factor_on_host else 0)
         used = C.c_int()
@@ -603,7 +602,7 @@ class Quantizer:
         return lanes.value
 
     def nvfp4_prepare_device_updates(self, H, sigma_reg=1e-2, threads=16):
-        """nvfp4_prepare (calibrated) with the factorization's trailing updates on the GPU -> (L, dw), same bits."""
+        """nvfp4_prepare (calibrated) with the factorization on the GPU -> (L, dw), same bits."""
         H = np.ascontiguousarray(H, np.float32)
         n = H.shape[0]
         L = np.zeros((n, n), np.float32)

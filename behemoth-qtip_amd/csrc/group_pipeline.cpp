@@ -1,6 +1,6 @@
 // Several Hessian groups through one context, scheduled like the reference's run_qtip_groups
-// (src/pipeline.cpp:229-312): Hessians are rotated on the GPU ahead of use, a side thread runs the host fp64 LDL of
-// the groups in order, and the calling thread quantizes group g as soon as its factor is there, so the LDL of group
+// (src/pipeline.cpp:229-312): Hessians are rotated on the GPU ahead of use, a side thread runs the fp64 LDL of
+// the groups in order (on the GPU by default, or on the host), and the calling thread quantizes group g as soon as its factor is there, so the LDL of group
 // g+1 overlaps the GPU work of group g.  The reference rotates all Hessians of a layer up front and keeps every HRr;
 // here rotation runs two groups ahead through a ring of three page-locked (HRr, L) pairs kept by the context, so
 // host memory stays at 6 n^2 floats however many groups are queued.
@@ -42,11 +42,10 @@ void run_groups_on(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opt
   int nmax = 0;
   for (int g = 0; g < ng; ++g) nmax = std::max(nmax, groups[g].n);
   const int R = std::min(3, ng);
-  reserve_group_ring(c, nmax, R);
-  // with the LDL's updates on the device the rotated Hessian never leaves it: the factorization reads it there and so
-  // does the proxy, and the factor goes up column block by column block as it is assembled: one copy down and three up
-  // fewer per group on the quantizing stream (HRr in the host ring is then unused)
+  // with the LDL on the device neither the rotated Hessian nor the factor leaves it: the factorization and the proxy read
+  // the one, LDLQ the other, and the host ring is not used
   const bool keep_dev = opt.ldl_device_updates != 0;
+  if (!keep_dev) reserve_group_ring(c, nmax, R);
   if (keep_dev)
     for (int b = 0; b < R; ++b) {
       c->ring_dHRr[b].ensure(size_t(nmax) * nmax);
@@ -211,8 +210,7 @@ void run_groups_on(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opt
       try {
         if (opt.ldl_device_updates) {
           QTIP_HIP(hipSetDevice(c->device));  // this thread's own current device
-          ldl_hessian_assisted_impl(c, nullptr, groups[g].n, opt.ldl_threads, c->ring_L[g % R].p, c->ring_dHRr[g % R].p,
-                                    c->ring_dL[g % R].p);
+          ldl_hessian_device_impl(c, nullptr, groups[g].n, nullptr, c->ring_dHRr[g % R].p, c->ring_dL[g % R].p);
         } else {
           ldl_hessian_impl(c->ring_HRr[g % R].p, groups[g].n, opt.ldl_threads, c->ring_L[g % R].p);
         }
@@ -249,7 +247,7 @@ void run_groups_on(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opt
         T.rht = t_rot[size_t(g)];
         T.ldl_cpu = t_ldl[size_t(g)];
         quantize_group_impl(c, groups[g].nlin, dl[size_t(g)].data(), groups[g].n, groups[g].seed, su[size_t(b)].data(),
-                            creg[size_t(g)], keep_dev ? nullptr : c->ring_HRr[b].p, c->ring_L[b].p, opt, groups[g].outs, &T,
+                            creg[size_t(g)], keep_dev ? nullptr : c->ring_HRr[b].p, keep_dev ? nullptr : c->ring_L[b].p, opt, groups[g].outs, &T,
                             keep_dev ? c->ring_dHRr[b].p : nullptr, keep_dev ? c->ring_dL[b].p : nullptr);
         if (tms) tms[g] = T;
         {
@@ -276,8 +274,8 @@ void run_groups_in_line(qtip_ctx* c, int ng, const qtip_group* groups, const qti
                         double* ldl_wait) {
   int nmax = 0;
   for (int g = 0; g < ng; ++g) nmax = std::max(nmax, groups[g].n);
-  reserve_group_ring(c, nmax, 1);
   const bool keep_dev = opt.ldl_device_updates != 0;
+  if (!keep_dev) reserve_group_ring(c, nmax, 1);
   if (keep_dev) {
     c->ring_dHRr[0].ensure(size_t(nmax) * nmax);
     c->ring_dL[0].ensure(size_t(nmax) * nmax);
@@ -292,14 +290,13 @@ void run_groups_in_line(qtip_ctx* c, int ng, const qtip_group* groups, const qti
     T.rht = now_s() - t0;
     t0 = now_s();
     if (keep_dev)
-      ldl_hessian_assisted_impl(c, nullptr, groups[g].n, opt.ldl_threads, c->ring_L[0].p, c->ring_dHRr[0].p,
-                                c->ring_dL[0].p);
+      ldl_hessian_device_impl(c, nullptr, groups[g].n, nullptr, c->ring_dHRr[0].p, c->ring_dL[0].p);
     else
       ldl_hessian_impl(c->ring_HRr[0].p, groups[g].n, opt.ldl_threads, c->ring_L[0].p);
     T.ldl_cpu = now_s() - t0;
     if (ldl_wait) ldl_wait[g] = T.ldl_cpu;  // all of it: the lane's GPU work waits for its own factorization
     quantize_group_impl(c, groups[g].nlin, groups[g].lins, groups[g].n, groups[g].seed, su.data(), creg,
-                        keep_dev ? nullptr : c->ring_HRr[0].p, c->ring_L[0].p, opt, groups[g].outs, &T,
+                        keep_dev ? nullptr : c->ring_HRr[0].p, keep_dev ? nullptr : c->ring_L[0].p, opt, groups[g].outs, &T,
                         keep_dev ? c->ring_dHRr[0].p : nullptr, keep_dev ? c->ring_dL[0].p : nullptr);
     if (tms) tms[g] = T;
   }

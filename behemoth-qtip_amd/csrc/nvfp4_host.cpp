@@ -149,20 +149,22 @@ void nvfp4_prepare_host(const float* H, int n, double sigma_reg, bool calibrate,
 }
 
 // The block loop for the matrices of one group.  host_L / host_dw as nvfp4_prepare_host leaves them (host_L null:
-// no calibration; host_dw null: uniform weights for the scale search).
+// no calibration; host_dw null: uniform weights for the scale search), or as device buffers of the same contents.
 void nvfp4_quantize_prepared_impl(qtip_ctx* c, int nmat, const qtip_nvfp4_matrix* mats, int n, const float* host_L,
-                                  const float* host_dw, bool search) {
+                                  const float* host_dw, bool search, const float* dev_L, const float* dev_dw) {
   QTIP_REQUIRE(nmat >= 0 && (nmat == 0 || mats) && n > 0 && n % 16 == 0, "NVFP4 group geometry");
   hipStream_t s = c->stream;
-  const bool cal = host_L != nullptr;
-  DBuf<float> d_L, d_dw;
-  if (cal) {
-    d_L.alloc(size_t(n) * n);
-    QTIP_HIP(hipMemcpyAsync(d_L, host_L, d_L.bytes(), hipMemcpyHostToDevice, s));
+  const bool cal = host_L != nullptr || dev_L != nullptr;
+  DBuf<float> own_L, own_dw;
+  if (cal && !dev_L) {
+    own_L.alloc(size_t(n) * n);
+    QTIP_HIP(hipMemcpyAsync(own_L, host_L, own_L.bytes(), hipMemcpyHostToDevice, s));
+    dev_L = own_L.p;
   }
-  if (host_dw) {
-    d_dw.alloc(size_t(n));
-    QTIP_HIP(hipMemcpyAsync(d_dw, host_dw, d_dw.bytes(), hipMemcpyHostToDevice, s));
+  if (host_dw && !dev_dw) {
+    own_dw.alloc(size_t(n));
+    QTIP_HIP(hipMemcpyAsync(own_dw, host_dw, own_dw.bytes(), hipMemcpyHostToDevice, s));
+    dev_dw = own_dw.p;
   }
   for (int mi = 0; mi < nmat; ++mi) {
     const qtip_nvfp4_matrix& M = mats[mi];
@@ -186,12 +188,12 @@ void nvfp4_quantize_prepared_impl(qtip_ctx* c, int nmat, const qtip_nvfp4_matrix
     }
     for (long cb = top; cb >= 0; cb -= 128) {
       const long hi = std::min<long>(n, cb + 128);
-      if (cal && hi < n) launch_nvfp4_gather(FT, m, n, cb, E, d_L, s);
+      if (cal && hi < n) launch_nvfp4_gather(FT, m, n, cb, E, dev_L, s);
       for (long c0 = hi - 16; c0 >= cb; c0 -= 16) {
         float* e = cal ? E.p + size_t(c0) * m : E.p;
-        launch_nvfp4_block(WT, cal ? FT.p : nullptr, m, n, c0, cal ? d_L.p : nullptr, host_dw ? d_dw.p : nullptr, g,
+        launch_nvfp4_block(WT, cal ? FT.p : nullptr, m, n, c0, dev_L, dev_dw, g,
                            cal, search, pT, sT, e, s);
-        if (cal) launch_nvfp4_feedback(FT, m, n, c0, cb, e, d_L, s);
+        if (cal) launch_nvfp4_feedback(FT, m, n, c0, cb, e, dev_L, s);
       }
     }
     launch_transpose_u8(pT, n / 2, m, pk, s);

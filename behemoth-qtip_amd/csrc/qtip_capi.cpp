@@ -640,7 +640,13 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr, "nvfp4_prepare_device_updates: bad arguments");
     DeviceGuard g(ctx);
-    nvfp4_prepare_assisted_impl(ctx, host_H, n, sigma_reg, threads, host_L, host_dw);
+    QTIP_REQUIRE(host_H && host_L && host_dw && n > 0 && n % 16 == 0, "nvfp4_prepare (device): bad arguments (n = %d)", n);
+    const size_t nn = size_t(n) * n;
+    DBuf<float> L(nn), dw(static_cast<size_t>(n));
+    nvfp4_prepare_device_impl(ctx, host_H, n, sigma_reg, L.p, dw.p);
+    QTIP_HIP(hipMemcpyAsync(host_L, L.p, nn * 4, hipMemcpyDeviceToHost, ctx->stream));
+    QTIP_HIP(hipMemcpyAsync(host_dw, dw.p, size_t(n) * 4, hipMemcpyDeviceToHost, ctx->stream));
+    QTIP_HIP(hipStreamSynchronize(ctx->stream));
   });
 }
 int qtip_nvfp4_quantize_prepared(qtip_ctx* ctx, int nmat, qtip_nvfp4_matrix* mats, int n, const float* host_L,
@@ -660,21 +666,28 @@ int qtip_nvfp4_quantize_group(qtip_ctx* ctx, int nmat, qtip_nvfp4_matrix* mats, 
     if (opts) o = *opts;
     const bool cal = o.calibrate != 0 && host_H != nullptr;
     if (calibrated) *calibrated = cal ? 1 : 0;
-    std::vector<float> dw;
-    float* L = nullptr;
-    if (host_H) {
-      dw.resize(static_cast<size_t>(n));
-      if (cal) {
-        // the factor goes through a page-locked buffer the context keeps (the staging of qtip_run_groups): no 3.3 GB
-        // of fresh pages per call at n = 28672, and an upload at the bus's rate
-        const size_t nn = size_t(n) * n;
-        if (ctx->ring_L[0].n < nn) ctx->ring_L[0].alloc(nn);
-        L = ctx->ring_L[0].p;
-      }
-      if (cal && !o.factor_on_host) nvfp4_prepare_assisted_impl(ctx, host_H, n, o.sigma_reg, 16, L, dw.data());
-      else nvfp4_prepare_host(host_H, n, o.sigma_reg, cal, 16, L, dw.data());
+    if (!host_H) {
+      nvfp4_quantize_prepared_impl(ctx, nmat, mats, n, nullptr, nullptr, o.scale_search != 0);
+      return;
     }
-    nvfp4_quantize_prepared_impl(ctx, nmat, mats, n, L, host_H ? dw.data() : nullptr, o.scale_search != 0);
+    if (cal && !o.factor_on_host) {
+      // the factor is formed on the device and used there
+      DBuf<float> L(size_t(n) * n), dw(static_cast<size_t>(n));
+      nvfp4_prepare_device_impl(ctx, host_H, n, o.sigma_reg, L.p, dw.p);
+      nvfp4_quantize_prepared_impl(ctx, nmat, mats, n, nullptr, nullptr, o.scale_search != 0, L.p, dw.p);
+      return;
+    }
+    std::vector<float> dw(static_cast<size_t>(n));
+    float* L = nullptr;
+    if (cal) {
+      // the factor goes through a page-locked buffer the context keeps (the staging of qtip_run_groups): no 3.3 GB
+      // of fresh pages per call at n = 28672, and an upload at the bus's rate
+      const size_t nn = size_t(n) * n;
+      if (ctx->ring_L[0].n < nn) ctx->ring_L[0].alloc(nn);
+      L = ctx->ring_L[0].p;
+    }
+    nvfp4_prepare_host(host_H, n, o.sigma_reg, cal, 16, L, dw.data());
+    nvfp4_quantize_prepared_impl(ctx, nmat, mats, n, L, dw.data(), o.scale_search != 0);
   });
 }
 
@@ -849,16 +862,17 @@ int qtip_ldl_hessian_device_updates(qtip_ctx* ctx, const float* host_HRr, int n,
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr, "null context");
     DeviceGuard g(ctx);
-    ldl_hessian_assisted_impl(ctx, host_HRr, n, threads, host_L);
+    QTIP_REQUIRE(host_HRr != nullptr && host_L != nullptr, "ldl_hessian (device): bad arguments (n = %d)", n);
+    ldl_hessian_device_impl(ctx, host_HRr, n, host_L, nullptr, nullptr);
   });
 }
 
 int qtip_ldl_hessian_device_updates_dev(qtip_ctx* ctx, const float* dev_HRr, int n, int threads, float* host_L,
                                         float* dev_L) {
   return guarded([&] {
-    QTIP_REQUIRE(ctx != nullptr && dev_HRr != nullptr, "ldl_hessian (device updates): null context or Hessian");
+    QTIP_REQUIRE(ctx != nullptr && dev_HRr != nullptr && host_L != nullptr, "ldl_hessian (device): null context, Hessian or L");
     DeviceGuard g(ctx);
-    ldl_hessian_assisted_impl(ctx, nullptr, n, threads, host_L, dev_HRr, dev_L);
+    ldl_hessian_device_impl(ctx, nullptr, n, host_L, dev_HRr, dev_L);
   });
 }
 
@@ -917,7 +931,7 @@ int qtip_quantize_group_h(qtip_ctx* ctx, int nlin, const qtip_linear_in* lins, i
     auto t0 = std::chrono::steady_clock::now();
     rotate_hessian_impl(ctx, H, h_on_device != 0, n, seed, o.sigma_reg, su.data(), &creg, HRr.data());
     auto t1 = std::chrono::steady_clock::now();
-    if (o.ldl_device_updates) ldl_hessian_assisted_impl(ctx, HRr.data(), n, o.ldl_threads, L.data());
+    if (o.ldl_device_updates) ldl_hessian_device_impl(ctx, HRr.data(), n, L.data(), nullptr, nullptr);
     else ldl_hessian_impl(HRr.data(), n, o.ldl_threads, L.data());
     auto t2 = std::chrono::steady_clock::now();
     T.rht = std::chrono::duration<double>(t1 - t0).count();

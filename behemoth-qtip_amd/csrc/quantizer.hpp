@@ -36,8 +36,8 @@ struct QuantOpts {  // src/quantizer.hpp:11-19
   bool share_su = true;
   std::string dump_dir;  // if set: W (fp32) and, unless want_hatW, the reconstructed hatW (fp32) are written per linear
   bool want_hatW = false;
-  // not in the reference: the group calls hand the trailing updates of the host LDL to the GPU (the factor is the
-  // host's bit for bit); false keeps the factorization on the host alone
+  // not in the reference: the group calls factor on the GPU (the factor is the host's bit for bit); false keeps the
+  // factorization on the host
   bool ldl_device_updates = true;
   // not in the reference: run_groups runs groups that cannot fill the chip side by side (0: as many as fit, 1: one at
   // a time, as the reference schedules them); the outputs do not depend on it

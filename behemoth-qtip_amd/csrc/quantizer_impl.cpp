@@ -485,7 +485,7 @@ void group_finish(qtip_ctx* c, GroupWork& w, int nlin, const qtip_linear_in* lin
 void quantize_group_impl(qtip_ctx* c, int nlin, const qtip_linear_in* lins, int n, uint64_t seed, const float* host_su,
                          double creg, const float* host_HRr, const float* host_L, const qtip_opts& opt,
                          qtip_linear_out* outs, qtip_timing* tm, const float* dev_HRr, const float* dev_L) {
-  QTIP_REQUIRE(host_L != nullptr, "quantize_group: bad arguments");
+  QTIP_REQUIRE(host_L != nullptr || dev_L != nullptr, "quantize_group: bad arguments");
   QTIP_REQUIRE(opt.skip_proxy || host_HRr || dev_HRr, "quantize_group: HRr is needed for the proxy");
   GroupWork w;
   group_prepare(c, w, nlin, lins, n, seed, host_su, opt, outs, tm);

@@ -55,12 +55,12 @@ struct qtip_ctx {
   qtipmi::DBuf<float> up_H[kUploadSlots];
   qtipmi::DBuf<uint8_t> up_W[kUploadSlots];
   qtipmi::DBuf<float> ring_dHRr[3], ring_dL[3];  // run_groups with device-updated LDL: rotated Hessians and factors stay here
-  // LDL with the trailing updates on the device (ldl_assist.hip): own stream, fp64 work matrix, fp32 upload of HRr,
-  // solved panel rows, two page-locked panel buffers (the panels travel one ahead); allocated on first use
+  // LDL on the device (ldl_device.hip): own stream, fp64 work matrix, fp32 upload of HRr, a panel's solved rows
+  // transposed, the reciprocals and 16 x 16 inverses of its diagonal block, a flag; allocated on first use
   hipStream_t ldl_stream = nullptr;
-  qtipmi::DBuf<double> ldl_A, ldl_X, ldl_Xt, ldl_P;
+  qtipmi::DBuf<double> ldl_A, ldl_Xt, ldl_diag;
+  qtipmi::DBuf<int> ldl_bad;
   qtipmi::DBuf<float> ldl_H;
-  qtipmi::HBuf<double> ldl_panel[2];
 };
 
 namespace qtipmi {
@@ -68,10 +68,8 @@ void ensure_viterbi_workspace(qtip_ctx* c);
 void rotate_hessian_impl(qtip_ctx* c, const float* H, bool on_device, int n, uint64_t seed, double sigma_reg,
                          float* host_su, double* creg, float* host_HRr, float* dev_HRr = nullptr);
 void ldl_hessian_impl(const float* host_HRr, int n, int threads, float* host_L);
-void ldl_hessian_assisted_impl(qtip_ctx* c, const float* host_HRr, int n, int threads, float* host_L,
-                               const float* dev_HRr = nullptr, float* dev_L = nullptr);
-void nvfp4_prepare_assisted_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, int threads, float* host_L,
-                                 float* host_dw);
+void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* host_L, const float* dev_HRr, float* dev_L);
+void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw);
 void ldlq_impl(qtip_ctx* c, const float* dWT, const float* dL, long n, long m, float* d_hatWT, uint16_t* dQ,
                int feedback, double* vit_seconds, int chains);
 int ldlq_default_chains(qtip_ctx* c);  // what chains = 0 stands for in this context (decided on the first call)
@@ -113,5 +111,6 @@ void nvfp4_dequantize_host(const uint8_t* packed, const uint8_t* scales, float g
 double nvfp4_proxy_error_host(const float* w, const float* what, int m, int n, const float* H);
 void nvfp4_prepare_host(const float* H, int n, double sigma_reg, bool calibrate, int threads, float* L, float* dw);
 void nvfp4_quantize_prepared_impl(qtip_ctx* c, int nmat, const qtip_nvfp4_matrix* mats, int n, const float* host_L,
-                                  const float* host_dw, bool search);
+                                  const float* host_dw, bool search, const float* dev_L = nullptr,
+                                  const float* dev_dw = nullptr);
 }  // namespace qtipmi

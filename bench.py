@@ -325,7 +325,7 @@ def run_group(args, pkg):
              4: "config4: gate+up 2x(28672x12288) group", 5: "config5: 12288x28672 down-proj group"}
     return dict(weights=weights_per_step * args.steps, wall=wall, vit_launch_s=stats["viterbi_s"] / launches,
                 vit_launch_weights=ntr * 256 * 8 * lanes, blocks_per_launch=8, workload=names[cfg] + (" (RHT + host fp64 LDL + LDLQ + 2-pass Viterbi + pack)" if args.host_ldl else
-                                       " (RHT + fp64 LDL: host panels, GPU trailing updates + LDLQ + 2-pass Viterbi + pack)"),
+                                       " (RHT + fp64 LDL + LDLQ + 2-pass Viterbi + pack)"),
                 extra=extra, cpu_group=cpu_group, concurrent=nch * lanes,
                 ldlq_s=stats["ldlq_s"], weights_per_step=weights_per_step)
 
@@ -351,8 +351,8 @@ def run_ldl_only(args, pkg):
         q.ldl_hessian_device_updates(hp, threads=args.ldl_threads)
         dev.append(hp.t_ldl)
     L_dev = hp.L
-    # the form the group pipeline runs: rotated Hessian resident on the device, L into a page-locked buffer that exists
-    # already and, as it is assembled, into a device buffer
+    # rotated Hessian resident on the device, L into a device buffer, as the group pipeline runs it, and from there into
+    # a page-locked buffer that exists already
     dHRr = torch.from_numpy(hp.HRr).cuda()
     L_pin = torch.empty((n, n), dtype=torch.float32, pin_memory=True)
     dL = torch.empty((n, n), dtype=torch.float32, device="cuda")
@@ -413,11 +413,11 @@ def main():
     ap.add_argument("--ldl-threads", type=int, default=16, help="OpenMP team of the host LDL")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--host-ldl", action="store_true",
-                    help="keep the fp64 block LDL on the host alone, as the reference does (default: the host factors and "
-                         "solves the panels and hands the trailing updates to the GPU; the factor is the same bit for bit)")
+                    help="keep the fp64 block LDL on the host alone, as the reference does (default: on the GPU; the "
+                         "factor is the same bit for bit)")
     ap.add_argument("--ldl-only", action="store_true",
-                    help="time the block LDL of the configuration's rotated Hessian by itself, three times each: host panels "
-                         "with GPU trailing updates, and host alone (not the contract's metric; one line of JSON)")
+                    help="time the block LDL of the configuration's rotated Hessian by itself, three times each: on "
+                         "the GPU, and on the host alone (not the contract's metric; one line of JSON)")
     ap.add_argument("--rht-only", action="store_true",
                     help="time the row transform by itself on the large configurations' shapes (not the contract's "
                          "metric; one line of JSON with the HBM rate of each pass)")

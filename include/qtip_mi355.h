@@ -144,18 +144,17 @@ int qtip_ldl_hessian(const float* host_HRr, int n, int threads, float* host_L);
  * order of operations, hence its bits.  Host only.  QTIP_E_NOT_PD if the matrix is not positive definite. */
 int qtip_cholesky_inplace(double* host_A, int n, int threads);
 
-/* The same factorization with the trailing updates of the host's panels on the GPU.  No counterpart in the
- * reference (its ldl_hessian is host only, src/quantizer.cpp:154-165): the host still factors and solves every
- * panel in fp64 with its own code, the device keeps the fp64 work matrix and applies the rank-256 updates on the
- * matrix cores in the host's own order of operations, so host_L is qtip_ldl_hessian's bit for bit.  Works on a
- * stream of its own inside ctx; may run on a side thread while another thread quantizes through the same ctx. */
+/* The same factorization on the GPU.  No counterpart in the reference (its ldl_hessian is host only,
+ * src/quantizer.cpp:154-165): the device factors the diagonal blocks, solves the panels and applies the rank-256
+ * updates in fp64 in the host's own order of operations, so host_L is qtip_ldl_hessian's bit for bit; threads is not
+ * used.  Works on a stream of its own inside ctx; may run on a side thread while another thread quantizes through the
+ * same ctx. */
 int qtip_ldl_hessian_device_updates(qtip_ctx* ctx, const float* host_HRr, int n, int threads, float* host_L);
 
 /* The same with the rotated Hessian already on the device (dev_HRr, n x n fp32, read only): the form
  * qtip_run_groups uses for the groups it schedules (the schedule of run_qtip_groups, src/pipeline.cpp:229-312, where
  * the reference calls its host-only ldl_hessian).  host_L as above; dev_L (optional, may be NULL): n x n fp32 device
- * buffer that receives L as well, column block by column block while the factorization runs - host_L is the source
- * of those copies and should then be page-locked. */
+ * buffer that receives L as well. */
 int qtip_ldl_hessian_device_updates_dev(qtip_ctx* ctx, const float* dev_HRr, int n, int threads, float* host_L,
                                         float* dev_L);
 
@@ -195,8 +194,8 @@ typedef struct { /* QuantOpts, src/quantizer.hpp:11-19 */
                             1: fp32 feedback sums + bf16 hi/lo split MFMA prod cache (the reference GPU's arithmetic) */
   int skip_proxy;        /* 1: leave proxy fields 0 */
   int ldl_device_updates;/* 1 (default): qtip_run_groups and qtip_quantize_group_h factor through
-                            qtip_ldl_hessian_device_updates (panels on the host, trailing updates on the GPU, same L
-                            bit for bit); 0: block LDL on the host alone, as in the reference */
+                            qtip_ldl_hessian_device_updates (on the GPU, same L bit for bit); 0: block LDL on the
+                            host alone, as in the reference */
   int ldlq_chains;       /* LDLQ deals the tile rows of a group to this many independent chains of launches (each on
                             a stream of its own inside ctx), so that the trace-backs of one run under the forward
                             passes of the others; same codes whatever the number.  At most 3.  0 (default): 3 if the
@@ -267,8 +266,8 @@ typedef struct { /* Nvfp4Opts, src/nvfp4_gpu.hpp:21-25 */
   int scale_search; /* 1 */
   int calibrate;    /* 1 */
   double sigma_reg; /* 1e-2 */
-  int factor_on_host; /* 0 (default): the calibration's Cholesky factorization runs its trailing updates on the GPU
-                         (same L and dw bit for bit); 1: on the host alone, as qtip_nvfp4_prepare */
+  int factor_on_host; /* 0 (default): the calibration's Cholesky factorization runs on the GPU (same L and dw bit for
+                         bit); 1: on the host alone, as qtip_nvfp4_prepare */
 } qtip_nvfp4_opts;
 typedef struct { /* one matrix of a group: input and the caller-allocated outputs (Nvfp4Tensor, src/nvfp4.hpp:35-41) */
   int m;
@@ -289,14 +288,13 @@ int qtip_nvfp4_prepare(const float* host_H, int n, double sigma_reg, int calibra
                        float* host_dw);
 int qtip_nvfp4_quantize_prepared(qtip_ctx* ctx, int nmat, qtip_nvfp4_matrix* mats, int n, const float* host_L,
                                  const float* host_dw, int scale_search);
-/* qtip_nvfp4_prepare with calibration, the rank-256 trailing updates of its fp64 Cholesky factorization on the GPU
- * (the host still factors and solves every panel): the same L and dw bit for bit, 0.6 s instead of 4.3 s at
- * n = 28672.  No counterpart in the reference, which factors on the host (src/nvfp4_gpu.hip:181-207). */
+/* qtip_nvfp4_prepare with calibration, its fp64 Cholesky factorization on the GPU: the same L and dw bit for bit;
+ * threads is not used.  No counterpart in the reference, which factors on the host (src/nvfp4_gpu.hip:181-207). */
 int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n, double sigma_reg, int threads,
                                       float* host_L, float* host_dw);
 
 /* Several groups through one context with the overlap of run_qtip_groups, src/pipeline.cpp:229-312: Hessians are
- * rotated on the GPU ahead of use, a side thread runs the host fp64 LDL of the groups in order, and group g is
+ * rotated on the GPU ahead of use, a side thread runs the fp64 LDL of the groups in order, and group g is
  * quantized as soon as its factor is ready (the LDL of group g+1 overlaps the GPU work of group g).  HRr and L live
  * in page-locked staging buffers owned by the context (a ring of three pairs, 6 n^2 floats, kept between calls).
  * timings / ldl_wait_s (seconds the GPU side waited for each group's factor) may be NULL.  On an error the
@@ -363,9 +361,8 @@ long qtip_selftest_device_alloc_calls(void);
 int qtip_selftest_failed_alloc_is_retried(void);
 
 /* Host-only self test (no GPU needed, no counterpart in the reference): the block LDL through the panel hand-over
- * that qtip_ldl_hessian_device_updates uses (a panel's columns fetched, factored and solved by the host, the rows
- * handed back, L assembled from them as they pass), with the trailing matrix held and updated by plain host code
- * instead of the device.  host_L must come out as qtip_ldl_hessian's, bit for bit. */
+ * (a panel's columns fetched, factored and solved, the rows handed back, L assembled from them as they pass), with the
+ * trailing matrix held and updated by plain host code.  host_L must come out as qtip_ldl_hessian's, bit for bit. */
 int qtip_selftest_ldl_panel_handover(const float* host_HRr, int n, int threads, float* host_L);
 
 /* Host packers (pack_trellis / unpack_trellis / swizzle_for_kernel / unswizzle_for_kernel,

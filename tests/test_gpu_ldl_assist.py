@@ -1,7 +1,6 @@
-"""Block LDL with the trailing updates on the GPU (qtip_ldl_hessian_device_updates): the factor must equal the host
-factorization's bit for bit (same panel code on the host; the rank-256 updates on the fp64 matrix cores in the host
-micro-kernel's order of operations), including ragged last panels, and must fail the same way on a matrix that is not
-positive definite."""
+"""Block LDL on the GPU (qtip_ldl_hessian_device_updates): the factor must equal the host factorization's bit for bit
+(every sum in the host code's order of operations), including ragged last panels, and must fail the same way on a matrix
+that is not positive definite."""
 import numpy as np
 import pytest
 
@@ -63,6 +62,21 @@ def test_device_resident_form_equals_host_factor(qz, pkg, n):
     L2 = np.full((n, n), -1.0, np.float32)
     qz.ldl_hessian_device_resident(dH, n, L2, None, threads=16)
     assert np.array_equal(L2.view(np.uint32), a.L.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [32, 48, 256, 288])
+def test_factor_of_uneven_matrix_equals_host_factor(qz, pkg, n):
+    """Channels of very different scale, and pairs of channels that do not hang together at all (zeros in the factor)."""
+    say("case: LDL on the device, uneven matrix, n = %d" % n)
+    H = spd(n, 900 + n)
+    scale = (2.0 ** np.random.default_rng(n).integers(-12, 13, n)).astype(np.float32)
+    H = H * scale[:, None] * scale[None, :]
+    H[n // 2:, :n // 2] = 0
+    H[:n // 2, n // 2:] = 0
+    a, b = pkg.HessPrep(n=n, HRr=H.copy()), pkg.HessPrep(n=n, HRr=H.copy())
+    pkg.Quantizer.ldl_hessian(a, threads=4)
+    qz.ldl_hessian_device_updates(b)
+    assert np.array_equal(a.L.view(np.uint32), b.L.view(np.uint32))
 
 
 def test_rank_deficient_matrix_is_refused(qz, pkg):
