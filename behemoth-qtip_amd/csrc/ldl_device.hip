@@ -516,7 +516,6 @@ __global__ __launch_bounds__(64) void ldl_solve_kernel(const double* __restrict_
     }
   } else {
     bool finite = true;
-#pragma unroll 4
     for (int b = 0; b < last; ++b) {
       double4_t o = double4_t{0, 0, 0, 0};
 #pragma unroll

@@ -6,9 +6,10 @@ void launch_fp8_to_f32(const uint8_t* w, const uint16_t* scale_bf16, float* out,
 void launch_scale_rc(float* X, long rows, long cols, long ld, const float* rs, const float* cs, hipStream_t s);
 // states of one linear (m x n weights, tiles row-major) -> kernel-layout trellis words
 void launch_pack_swizzle(const uint16_t* Q, long m, long n, uint16_t* out, hipStream_t s);
-// kernel-layout trellis words of one linear -> hatWr (m x n fp32, row stride ld): lookup of every 16-bit window (decode.hip)
+// kernel-layout trellis words of one linear -> hatWr (m x n fp32, row stride ld): lookup of every 16-bit window (decode.hip);
+// transposed: hatWr^T (n x m) instead
 void launch_decode_trellis(const uint16_t* trellis, long m, long n, const float* entry_f, float* out, long ld,
-                           hipStream_t s);
+                           hipStream_t s, bool transposed = false);
 // H (n x n fp32) += X^T X for X = rows x n bf16, tiles on or below the diagonal only; then mirror + scale (hessian.hip)
 void launch_hessian_accumulate(const uint16_t* X, long rows, long n, float* H, DBuf<uint16_t>& image, hipStream_t s);
 void launch_hessian_finish(float* H, long n, float scale, hipStream_t s);

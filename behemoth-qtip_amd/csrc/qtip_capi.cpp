@@ -548,23 +548,26 @@ int qtip_dequantize_linear(qtip_ctx* ctx, const uint16_t* host_trellis, const ui
     DeviceGuard g(ctx);
     hipStream_t s = ctx->stream;
     const size_t words = size_t(m / 16) * (n / 16) * 32;
+    // the call's buffers stay in the context's arena: two hipMalloc and hipFree of 4 m n bytes per call (the frees wait
+    // for the whole device) cost more than the kernels (12288 x 12288: 33 ms a call in a
+    // row of calls, of which 4 were the kernels and the copy; now 2.4, of which the pageable copy of the words is 1.3)
+    ArenaScope memory(&ctx->arena);
     DBuf<uint16_t> tr(words);
-    DBuf<float> a(size_t(n) * m), b(size_t(m) * n), d_su(n), d_sv(m);
+    DBuf<float> a(size_t(n) * m), own(hatW_on_device ? 0 : size_t(m) * n), d_su(n), d_sv(m);
+    float* const b = hatW_on_device ? hatW : own.p;
     std::vector<float> su(n);
     for (int i = 0; i < n; ++i) su[i] = bf16_to_f32(host_su_bf16[i]);
     QTIP_HIP(hipMemcpyAsync(tr, host_trellis, words * 2, hipMemcpyHostToDevice, s));
     QTIP_HIP(hipMemcpyAsync(d_su, su.data(), size_t(n) * 4, hipMemcpyHostToDevice, s));
     QTIP_HIP(hipMemcpyAsync(d_sv, host_sv, size_t(m) * 4, hipMemcpyHostToDevice, s));
-    launch_decode_trellis(tr, m, n, ctx->d_entry_f, b, n, s);
     // same operation order as the reconstruction at the end of quantize_group (src/quantizer.cpp:321-338), starting
-    // from hatWr^T, so that both give the same bits
-    ctx->rht.transpose(b, m, n, n, a, m);
+    // from hatWr^T, so that both give the same bits: 7 passes over 4 m n bytes (the decoder writes hatWr^T, the scales
+    // ride on the last transform's stores, a device result is formed where the caller wants it) instead of 15
+    launch_decode_trellis(tr, m, n, ctx->d_entry_f, a, m, s, true);
     ctx->rht.hadamard_rows(a, n, m, m, false);
     ctx->rht.transpose(a, n, m, m, b, n);
-    ctx->rht.hadamard_rows(b, m, n, n, false);
-    ctx->rht.scale(b, m, n, n, wscale);
-    launch_scale_rc(b, m, n, n, d_sv, d_su, s);
-    QTIP_HIP(hipMemcpyAsync(hatW, b, size_t(m) * n * 4, hatW_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
+    ctx->rht.hadamard_rows(b, m, n, n, false, nullptr, nullptr, RowScale{wscale, d_sv.p, d_su.p});
+    if (!hatW_on_device) QTIP_HIP(hipMemcpyAsync(hatW, b, size_t(m) * n * 4, hipMemcpyDeviceToHost, s));
     QTIP_HIP(hipStreamSynchronize(s));
   });
 }

@@ -15,6 +15,7 @@
 #include <mutex>
 
 #include "data/qtip_tables.h"
+#include "misc.hpp"
 #include "qtip_internal.hpp"
 #include "rht.hpp"
 
@@ -108,7 +109,8 @@ __global__ __launch_bounds__(kRowThreads) void rht_rows_kernel(float* __restrict
                                                               int seg, int nseg, float scale,
                                                               const float* __restrict__ rs,
                                                               const float* __restrict__ cs,
-                                                              const uint32_t* __restrict__ neg, int mix) {
+                                                              const uint32_t* __restrict__ neg, int mix,
+                                                              RowScale after) {
   extern __shared__ float v[];
   const long row = blockIdx.x / nseg;
   const int col0 = int(blockIdx.x % nseg) * seg;
@@ -131,9 +133,20 @@ __global__ __launch_bounds__(kRowThreads) void rht_rows_kernel(float* __restrict
     __syncthreads();
   }
   if (!mix) {
-    for (int i = threadIdx.x; i < seg_len; i += kRowThreads) x[i] = v[i] * scale;
+    if (after.rows) {
+      const float rr = after.rows[row];
+      for (int i = threadIdx.x; i < seg_len; i += kRowThreads) x[i] = v[i] * scale * after.all * rr * after.cols[col0 + i];
+    } else {
+      for (int i = threadIdx.x; i < seg_len; i += kRowThreads) x[i] = v[i] * scale;
+    }
     return;
   }
+  // (the row is whole here: col0 = 0)
+  auto store = [&](int k2, int i, float s) {
+    float y = s * scale;
+    if (after.rows) y = y * after.all * after.rows[row] * after.cols[k2 * P + i];
+    x[long(k2) * P + i] = y;
+  };
   // P <= 1024 here would leave threads idle: the outputs k2 of one i are shared out over kRowThreads / P threads
   const int W = (K + 31) >> 5;
   const int per = P < kRowThreads ? kRowThreads / P : 1;
@@ -148,14 +161,14 @@ __global__ __launch_bounds__(kRowThreads) void rht_rows_kernel(float* __restrict
         float s = 0.0f;
 #pragma unroll
         for (int k = 0; k < KT; ++k) s += flip(y[k], neg_bit(bits, k));
-        x[long(k2) * P + i] = s * scale;
+        store(k2, i, s);
       }
     } else {
       for (int k2 = first; k2 < K; k2 += per) {
         const uint32_t* bits = neg + k2 * W;
         float s = 0.0f;
         for (int k = 0; k < K; ++k) s += flip(v[k * P + i], neg_bit(bits, k));
-        x[long(k2) * P + i] = s * scale;
+        store(k2, i, s);
       }
     }
   }
@@ -228,10 +241,10 @@ __device__ __forceinline__ void fwht_wave1024(float (&r)[16], int lane) {
 }
 
 // X: rows of KT * 1024 values, 16-byte aligned (ld % 4 == 0).  gridDim.x workgroups share the rows out in turn.
-template <int KT, bool kTranspose>
+template <int KT, bool kTranspose, bool kAfter>
 __global__ __launch_bounds__(kRowThreads) void rht_rows_p1024_kernel(float* __restrict__ X, long ld, long rows,
                                                                     float scale, const float* __restrict__ rs,
-                                                                    const float* __restrict__ cs) {
+                                                                    const float* __restrict__ cs, RowScale after) {
   extern __shared__ float v[];
   constexpr int kWaves = kRowThreads / 64;
   constexpr int kTurns = (KT + kWaves - 1) / kWaves;  // chunks a wave takes at most
@@ -299,7 +312,8 @@ __global__ __launch_bounds__(kRowThreads) void rht_rows_p1024_kernel(float* __re
         if ((kHad.minus[k2] >> k) & 1) s -= y[k];
         else s += y[k];
       }
-      x[k2 * 1024] = s * scale;
+      if constexpr (kAfter) x[k2 * 1024] = s * scale * after.all * after.rows[row] * after.cols[k2 * 1024 + i];
+      else x[k2 * 1024] = s * scale;
     }
   }
 }
@@ -441,7 +455,7 @@ const uint32_t* Rht::device_had(int K, bool transpose) {
 
 namespace {
 using RowKernel = void (*)(float*, long, int, int, int, int, int, float, const float*, const float*, const uint32_t*,
-                           int);
+                           int, RowScale);
 RowKernel row_kernel(int K) {
   switch (K) {
     case 12: return rht_rows_kernel<12>;
@@ -451,13 +465,19 @@ RowKernel row_kernel(int K) {
     default: return rht_rows_kernel<0>;
   }
 }
-using PipeKernel = void (*)(float*, long, long, float, const float*, const float*);
-PipeKernel pipe_kernel(int K, bool transpose) {
+using PipeKernel = void (*)(float*, long, long, float, const float*, const float*, RowScale);
+// (factors after the transform come with the inverse alone: dequantization)
+template <int K>
+PipeKernel pipe_kernel_of(bool transpose, bool after) {
+  if (transpose) return after ? nullptr : rht_rows_p1024_kernel<K, true, false>;
+  return after ? rht_rows_p1024_kernel<K, false, true> : rht_rows_p1024_kernel<K, false, false>;
+}
+PipeKernel pipe_kernel(int K, bool transpose, bool after) {
   switch (K) {
-    case 12: return transpose ? rht_rows_p1024_kernel<12, true> : rht_rows_p1024_kernel<12, false>;
-    case 20: return transpose ? rht_rows_p1024_kernel<20, true> : rht_rows_p1024_kernel<20, false>;
-    case 28: return transpose ? rht_rows_p1024_kernel<28, true> : rht_rows_p1024_kernel<28, false>;
-    case 36: return transpose ? rht_rows_p1024_kernel<36, true> : rht_rows_p1024_kernel<36, false>;
+    case 12: return pipe_kernel_of<12>(transpose, after);
+    case 20: return pipe_kernel_of<20>(transpose, after);
+    case 28: return pipe_kernel_of<28>(transpose, after);
+    case 36: return pipe_kernel_of<36>(transpose, after);
     default: return nullptr;
   }
 }
@@ -475,13 +495,16 @@ void allow_full_lds() {
                                  hipFuncAttributeMaxDynamicSharedMemorySize, kRowLdsFloats * int(sizeof(float))));
   for (int K : {12, 20, 28, 36})
     for (bool t : {false, true})
-      QTIP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(pipe_kernel(K, t)),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, kRowLdsFloats * int(sizeof(float))));
+      for (bool a : {false, true})
+        if (PipeKernel k = pipe_kernel(K, t, a))
+          QTIP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       kRowLdsFloats * int(sizeof(float))));
   configured[size_t(dev)] = true;
 }
 }  // namespace
 
-void Rht::hadamard_rows(float* X, long rows, int n, long ld, bool transpose, const float* rs, const float* cs) {
+void Rht::hadamard_rows(float* X, long rows, int n, long ld, bool transpose, const float* rs, const float* cs,
+                        RowScale after) {
   const int K = had_K(n);
   QTIP_REQUIRE(K > 0, "unsupported hadamard dim %d", n);
   const int P = n / K;
@@ -492,13 +515,15 @@ void Rht::hadamard_rows(float* X, long rows, int n, long ld, bool transpose, con
   const float sc = 1.0f / std::sqrt(float(n));
   // rows of K x 1024 values that are 16-byte aligned: the form that keeps the next row in flight
   const auto aligned16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-  if (P == 1024 && pipe_kernel(K, transpose) && n <= kRowLdsFloats && ld % 4 == 0 && aligned16(X) && aligned16(cs)) {
+  QTIP_REQUIRE((after.rows != nullptr) == (after.cols != nullptr), "hadamard: row factors without column factors");
+  const PipeKernel pipe = P == 1024 ? pipe_kernel(K, transpose, after.rows != nullptr) : nullptr;
+  if (pipe && n <= kRowLdsFloats && ld % 4 == 0 && aligned16(X) && aligned16(cs)) {
     // as many workgroups as are resident at once (a K = 12 row leaves room for two per compute unit)
     int per_cu = 1;
-    QTIP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(pipe_kernel(K, transpose)),
+    QTIP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(pipe),
                                                           kRowThreads, size_t(n) * sizeof(float)));
     const unsigned grid = unsigned(std::min<long>(rows, long(cus_) * std::max(per_cu, 1)));
-    pipe_kernel(K, transpose)<<<dim3(grid), dim3(kRowThreads), size_t(n) * sizeof(float), s_>>>(X, ld, rows, sc, rs, cs);
+    pipe<<<dim3(grid), dim3(kRowThreads), size_t(n) * sizeof(float), s_>>>(X, ld, rows, sc, rs, cs, after);
     QTIP_HIP(hipGetLastError());
     return;
   }
@@ -512,7 +537,7 @@ void Rht::hadamard_rows(float* X, long rows, int n, long ld, bool transpose, con
   const int mix = whole && K > 1;
   const float first_scale = (K == 1) ? sc : (mix ? sc : 1.0f);
   row_kernel(K)<<<dim3(unsigned(rows * nseg)), dim3(kRowThreads), size_t(seg) * sizeof(float), s_>>>(
-      X, ld, n, P, K, seg, nseg, first_scale, rs, cs, neg, mix);
+      X, ld, n, P, K, seg, nseg, first_scale, rs, cs, neg, mix, K == 1 || mix ? after : RowScale{});
   QTIP_HIP(hipGetLastError());
   if (K > 1 && !mix) {
     const long per_row = (P + kMixLanes - 1) / kMixLanes;
@@ -520,6 +545,10 @@ void Rht::hadamard_rows(float* X, long rows, int n, long ld, bool transpose, con
     had_mix_long_rows_kernel<<<dim3(unsigned(rows * per_row)), dim3(kMixLanes), size_t(K) * kMixLanes * sizeof(float),
                                s_>>>(X, ld, P, K, sc, neg);
     QTIP_HIP(hipGetLastError());
+    if (after.rows) {
+      scale(X, rows, n, ld, after.all);
+      launch_scale_rc(X, rows, n, ld, after.rows, after.cols, s_);
+    }
   }
 }
 

@@ -9,12 +9,20 @@
 
 namespace qtipmi {
 
+// Factors a transform's results are multiplied by as they are stored, one after the other: `all`, the row's, the column's.
+struct RowScale {
+  float all = 1.0f;
+  const float* rows = nullptr;  // null: no factors at all
+  const float* cols = nullptr;
+};
+
 class Rht {
  public:
   void init(int device, hipStream_t stream);
   // x <- (hadK^(T) (x) H_{n/K}) (x * rs[row] * cs[col]) / sqrt(n) on `rows` rows of length n, stride ld; rs / cs may be null
+  // after: what the result is multiplied by (the same products as scale() and launch_scale_rc() one after the other)
   void hadamard_rows(float* X, long rows, int n, long ld, bool transpose, const float* rs = nullptr,
-                     const float* cs = nullptr);
+                     const float* cs = nullptr, RowScale after = {});
   void transpose(const float* in, long rows, long cols, long ld_in, float* out, long ld_out);
   void scale(float* X, long rows, long cols, long ld, float a);
   void add_diag(float* H, long n, float a);

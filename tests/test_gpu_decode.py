@@ -118,6 +118,38 @@ def test_dequantize_equals_group_reconstruction(qz, oracle, pkg, hyb):
         assert np.array_equal(hr, _decode_expected(lo.trellis, lo.m, n, hyb.lut0, hyb.lut1))
 
 
+@pytest.mark.parametrize("m,n", [(32, 256), (96, 12288), (160, 4096), (224, 9216), (64, 57344), (4096, 32)])
+def test_dequantize_equals_its_steps(qz, pkg, m, n):
+    """dequantize_linear against decode_trellis_dev, the row transforms and the three products one after the other: every
+    form of the row transform's last pass (one chunk, K chunks in both kernels, rows too long for LDS), patches of the
+    transposed decoder with fewer than four blocks, results on the host, on the device, and at an address that is only
+    4-byte aligned.  Same bits."""
+    import torch
+    say("case: dequantize %dx%d against its steps" % (m, n))
+    qz.set_tlut(None)
+    rng = np.random.default_rng(m * 7 + n)
+    tr = rng.integers(0, 65536, (m // 16) * (n // 16) * 32, dtype=np.uint16)
+    su = np.where(rng.integers(0, 2, n), np.uint16(0xBF80), np.uint16(0x3F80))
+    sv = np.where(rng.integers(0, 2, m), np.float32(-1), np.float32(1)) * rng.random(m).astype(np.float32)
+    lo = pkg.LinearOut(name="w", m=m, n=n, wscale=0.0163, trellis=tr, su_bf16=su, sv=sv)
+    a = torch.from_numpy(_gpu_decode(qz, tr, m, n).T.copy()).cuda()
+    torch.cuda.synchronize()
+    qz.hadamard_rows_dev(a, n, m, m, False)
+    qz.synchronize()
+    b = a.T.contiguous()
+    torch.cuda.synchronize()
+    qz.hadamard_rows_dev(b, m, n, n, False)
+    qz.synchronize()
+    sign = torch.from_numpy((su.astype(np.uint32) << 16).view(np.float32)).cuda()
+    want = (b * torch.tensor(np.float32(0.0163)).cuda()) * torch.from_numpy(sv).cuda()[:, None] * sign[None, :]
+    assert np.array_equal(qz.dequantize_linear(lo), want.cpu().numpy())
+    room = torch.zeros(m * n + 1, device="cuda")
+    torch.cuda.synchronize()
+    for view in (room[:m * n].view(m, n), room[1:].view(m, n)):
+        qz.dequantize_linear(lo, view)
+        assert torch.equal(view, want)
+
+
 def test_decode_full_size_sample(qz, hyb):
     """Benchmark configuration 5 shape (12288 x 28672): random words decoded on the device, a sample of 32-row blocks
     compared with the CPU decoder, every value a codebook entry; prints the achieved HBM rate."""
