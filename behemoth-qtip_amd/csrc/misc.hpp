@@ -17,13 +17,13 @@ void launch_hessian_finish(float* H, long n, float scale, hipStream_t s);
 // fp32, from bf16 hi/lo products on the matrix cores; synchronises the stream
 double quad_trace_bf16x3(long n, long m, const float* H, const float* A, const float* B, long ld, DBuf<uint16_t>& stack,
                          DBuf<double>& scratch, hipStream_t s);
-// NVFP4 fallback quantizer (nvfp4.hip): one 16-column block of the transposed matrices, the feedback of its residual
-// into the columns before it, and a byte transposer for the outputs
-void launch_nvfp4_block(const float* WT, const float* FT, long m, long n, long c0, const float* L, const float* dw,
-                        float global, bool calibrate, bool search, uint8_t* packedT, uint8_t* scalesT, float* E,
-                        hipStream_t s);
-void launch_nvfp4_feedback(float* FT, long m, long n, long c0, long col_lo, const float* E, const float* L,
-                           hipStream_t s);
+// NVFP4 fallback quantizer (nvfp4.hip): the blocks of one 128-column buffer of the transposed matrices (of all buffers
+// without calibration), the feedback a buffer gets from the columns behind it, the largest magnitude
+// of a matrix (*top: zero before, its bits after), and a byte transposer for the outputs
+void launch_nvfp4_buffer(const float* WT, const float* FT, long m, long n, long cb, const float* L, const float* dw,
+                         float global, bool calibrate, bool search, uint8_t* packedT, uint8_t* scalesT, float* ET,
+                         hipStream_t s);
+void launch_nvfp4_largest(const float* w, long count, unsigned* top, hipStream_t s);
 void launch_nvfp4_gather(float* FT, long m, long n, long cb, const float* ET, const float* L, hipStream_t s);
 void launch_transpose_u8(const uint8_t* in, long rows, long cols, uint8_t* out, hipStream_t s);
 }  // namespace qtipmi

@@ -11,19 +11,23 @@
 namespace qtipmi {
 namespace {
 
-// one fp32 global scale per matrix: the largest magnitude lands on the largest representable product 448 * 6
-float global_scale(const float* w, size_t numel) {
-  float top = 0;
-  bool finite = true;
-  for (size_t i = 0; i < numel; ++i) {
-    const float a = std::fabs(w[i]);
-    finite = finite && a <= 3.4028234663852886e38f;  // false for infinity and NaN
-    top = a > top ? a : top;
-  }
-  QTIP_REQUIRE(finite, "NVFP4: the matrix holds a value that is not finite");
+// one fp32 global scale per matrix: the largest magnitude lands on the largest representable product 448 * 6.
+// top_bits: the largest bit pattern of the matrix's magnitudes (infinities and NaNs lie above all finite ones)
+float global_scale_of(uint32_t top_bits) {
+  QTIP_REQUIRE(top_bits < 0x7f800000u, "NVFP4: the matrix holds a value that is not finite");
+  float top;
+  std::memcpy(&top, &top_bits, sizeof top);
   const float g = top > 0 ? top / (448.f * 6) : 1.f;
   QTIP_REQUIRE(g > 0 && g <= 3.4028234663852886e38f, "NVFP4: global scale %g is not a positive finite float", double(g));
   return g;
+}
+float global_scale(const float* w, size_t numel) {
+  uint32_t top = 0;
+  for (size_t i = 0; i < numel; ++i) {
+    const uint32_t a = nvcodec::bits_of(w[i]) & 0x7fffffffu;
+    top = a > top ? a : top;
+  }
+  return global_scale_of(top);
 }
 
 // value of a scale byte as stored: NaN for the two NaN codes, negative for a set sign bit
@@ -170,31 +174,31 @@ void nvfp4_quantize_prepared_impl(qtip_ctx* c, int nmat, const qtip_nvfp4_matrix
     const qtip_nvfp4_matrix& M = mats[mi];
     QTIP_REQUIRE(M.m > 0 && M.w && M.packed && M.scales, "NVFP4 matrix %d is incomplete", mi);
     const long m = M.m;
-    const float g = global_scale(M.w, size_t(m) * n);
-    const_cast<qtip_nvfp4_matrix&>(M).global = g;
-    // E: the residuals W - q of the finished columns, transposed like W; all of them when they are fed back
-    DBuf<float> W(size_t(m) * n), WT(size_t(m) * n), FT, E(cal ? size_t(m) * n : size_t(16) * m);
+    // E: the residuals W - q of the finished columns, transposed like W, for the feedback
+    DBuf<float> W(size_t(m) * n), WT(size_t(m) * n), FT, E(cal ? size_t(m) * n : 0);
+    DBuf<unsigned> top(1);
     DBuf<uint8_t> pT(size_t(m) * n / 2), sT(size_t(m) * n / 16), pk(size_t(m) * n / 2), sc(size_t(m) * n / 16);
+    unsigned top_bits = 0;
     QTIP_HIP(hipMemcpyAsync(W, M.w, W.bytes(), hipMemcpyHostToDevice, s));
+    QTIP_HIP(hipMemcpyAsync(top, &top_bits, sizeof top_bits, hipMemcpyHostToDevice, s));
+    launch_nvfp4_largest(W, m * n, top, s);
+    QTIP_HIP(hipMemcpyAsync(&top_bits, top, sizeof top_bits, hipMemcpyDeviceToHost, s));
+    QTIP_HIP(hipStreamSynchronize(s));
+    const float g = global_scale_of(top_bits);  // refuses a matrix that is not finite before anything is quantized
+    const_cast<qtip_nvfp4_matrix&>(M).global = g;
     c->rht.transpose(W, m, n, n, WT, m);
-    W.release();
     // Columns go in buffers of 128 from the last to the first.  A buffer first gathers the feedback of every block
     // behind it in one pass; inside the buffer every block then feeds the columns of the buffer left of it.  Values
     // and order of the additions are those of the block-by-block form.
-    const long top = (long(n) - 1) / 128 * 128;
+    const long last = (long(n) - 1) / 128 * 128;
     if (cal) {
-      FT.alloc(size_t(m) * n);
-      QTIP_HIP(hipMemsetAsync(FT.p + size_t(top) * m, 0, size_t(n - top) * m * sizeof(float), s));
-    }
-    for (long cb = top; cb >= 0; cb -= 128) {
-      const long hi = std::min<long>(n, cb + 128);
-      if (cal && hi < n) launch_nvfp4_gather(FT, m, n, cb, E, dev_L, s);
-      for (long c0 = hi - 16; c0 >= cb; c0 -= 16) {
-        float* e = cal ? E.p + size_t(c0) * m : E.p;
-        launch_nvfp4_block(WT, cal ? FT.p : nullptr, m, n, c0, dev_L, dev_dw, g,
-                           cal, search, pT, sT, e, s);
-        if (cal) launch_nvfp4_feedback(FT, m, n, c0, cb, e, dev_L, s);
+      FT.alloc(size_t(128) * m);
+      for (long cb = last; cb >= 0; cb -= 128) {
+        if (cb < last) launch_nvfp4_gather(FT, m, n, cb, E, dev_L, s);
+        launch_nvfp4_buffer(WT, FT, m, n, cb, dev_L, dev_dw, g, true, search, pT, sT, E, s);
       }
+    } else {
+      launch_nvfp4_buffer(WT, nullptr, m, n, 0, nullptr, dev_dw, g, false, search, pT, sT, nullptr, s);
     }
     launch_transpose_u8(pT, n / 2, m, pk, s);
     launch_transpose_u8(sT, n / 16, m, sc, s);

@@ -665,6 +665,7 @@ int qtip_nvfp4_quantize_group(qtip_ctx* ctx, int nmat, qtip_nvfp4_matrix* mats, 
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr && n > 0 && n % 16 == 0, "nvfp4_quantize_group: bad arguments");
     DeviceGuard g(ctx);
+    ArenaScope memory(&ctx->arena);  // the call's device buffers stay with the context
     qtip_nvfp4_opts o{1, 1, 1e-2, 0};
     if (opts) o = *opts;
     const bool cal = o.calibrate != 0 && host_H != nullptr;

@@ -34,6 +34,36 @@ def test_block_loop_bytes_equal_the_cpu_restatement(qz, pkg, oracle, name):
     assert off.global_scale == plain.global_scale
 
 
+@pytest.mark.parametrize("m,n", [(1, 16), (63, 128), (65, 144), (200, 272), (64, 656)])
+def test_buffers_with_remainders_equal_the_cpu_restatement(qz, oracle, m, n):
+    """Rows that do not fill a workgroup, buffers of fewer than 128 columns, one buffer and several: byte for byte."""
+    say("case: nvfp4 buffers %dx%d" % (m, n))
+    rng = np.random.default_rng(m * 1000 + n)
+    w = rng.standard_normal((m, n)).astype(np.float32) * np.float32(0.02)
+    w[rng.random((m, n)) < 0.02] *= 8
+    w[0, :16] = 0
+    H = _hessian(oracle, n, 22)
+    L, D = oracle.nvfp4_prepare(H, 1e-2, True)
+    g = oracle.nvfp4_quantize(w)[2]
+    for (Lx, dx, search) in ((None, None, False), (None, D, True), (L, D, False), (L, D, True)):
+        t = qz.nvfp4_quantize_prepared([w], n, Lx, dx, search)[0]
+        want = oracle.nvfp4_blocks(w, Lx, dx, g, Lx is not None, search)
+        assert t.global_scale == g
+        assert np.array_equal(t.packed, want[0]) and np.array_equal(t.scales, want[1]), (Lx is not None, search)
+
+
+def test_values_that_are_not_finite_are_refused(qz, pkg):
+    say("case: nvfp4, infinities and NaN are refused, zeros and the largest value are not")
+    w = np.zeros((32, 32), np.float32)
+    assert qz.nvfp4_quantize_prepared([w], 32)[0].global_scale == 1.0
+    for v in (np.inf, -np.inf, np.nan):
+        w[31, 31] = v
+        with pytest.raises(pkg.QtipError):
+            qz.nvfp4_quantize_prepared([w], 32)
+    w[31, 31] = -np.finfo(np.float32).max
+    assert qz.nvfp4_quantize_prepared([w], 32)[0].global_scale == np.finfo(np.float32).max / np.float32(448 * 6)
+
+
 @pytest.mark.parametrize("name", ["gauss", "heavy"])
 def test_group_meets_the_reference_test_criteria(qz, pkg, oracle, name):
     say("case: nvfp4 group %s" % name)
