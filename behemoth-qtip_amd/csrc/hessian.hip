@@ -243,6 +243,86 @@ __global__ __launch_bounds__(256, 1) void syrk_img_kernel(const uint16_t* __rest
   }
 }
 
+// The accumulating update for matrices whose 256 x 256 tiles leave most compute units idle: tiles of 128 x 128, four times
+// as many workgroups, from the same images (a half of a 16 KB slice, 128 columns, is contiguous as well).  Eight waves of
+// 64 x 32 outputs, two per SIMD, which cover each other's fragment reads and barriers (the kernel above spells an order
+// out for its lone wave instead), seven stages in flight: with few stages in all a launch is bound by the round trips
+// of its loads and by what a stage costs beside its MFMAs.  Same sums in the same order as the kernel above.
+constexpr int kSmallTile = 128, kHalfU16 = kSmallTile * IK, kSmallStages = 8;
+constexpr size_t kSmallLdsBytes = size_t(kSmallStages) * 2 * kHalfU16 * 2;  // 128 KB
+// this wave's loads have landed but for those of the last `stages` stages requested, two each (loads return in order)
+__device__ __forceinline__ void wait_all_but(int stages) {
+#define QTIP_WAIT(N) case N: __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * N)); break;
+  switch (stages) {
+    QTIP_WAIT(1) QTIP_WAIT(2) QTIP_WAIT(3) QTIP_WAIT(4) QTIP_WAIT(5) QTIP_WAIT(6)
+    default: __builtin_amdgcn_s_waitcnt(0x0F70);
+  }
+#undef QTIP_WAIT
+}
+__global__ __launch_bounds__(512, 1) void syrk_img_small_kernel(const uint16_t* __restrict__ I, int stages, long n,
+                                                                float* __restrict__ H, int tiles) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];  // [stage][operand][kHalfU16]
+  const int tile = blockIdx.x;
+  int ti = int((__builtin_sqrtf(8.0f * float(tile) + 1.0f) - 1.0f) * 0.5f);
+  while (ti * (ti + 1) / 2 > tile) --ti;
+  while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
+  const int tj = tile - ti * (ti + 1) / 2;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 2, wn = wave & 3;
+  // half ti & 1 of the slice of 256-column tile ti / 2; wave w brings its 1 KB of either operand's half
+  const size_t stage_stride = size_t(tiles) * kImgSliceU16;
+  const uint16_t* pa = I + size_t(ti >> 1) * kImgSliceU16 + (ti & 1) * kHalfU16 + wave * 512 + lane * 8;
+  const uint16_t* pb = I + size_t(tj >> 1) * kImgSliceU16 + (tj & 1) * kHalfU16 + wave * 512 + lane * 8;
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  auto request = [&](int st) {
+    uint16_t *a = lds + (st % kSmallStages) * 2 * kHalfU16 + wave * 512, *b = a + kHalfU16;
+    const uint16_t *ga = pa + size_t(st) * stage_stride, *gb = pb + size_t(st) * stage_stride;
+    __builtin_amdgcn_global_load_lds(ga, (lds_ptr)a, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(gb, (lds_ptr)b, 16, 0, 0);
+  };
+  floatx16 acc[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[a][v] = 0.f;
+  const int rl = lane & 31, hi = lane >> 5;
+  for (int p = 0; p < kSmallStages - 1 && p < stages; ++p) request(p);
+  for (int st = 0; st < stages; ++st) {
+    // this wave's loads of stage st have landed when only those of the later requested stages are outstanding; then
+    // everyone's have, and everyone is through with the stage whose place the next request takes
+    wait_all_but(stages - 1 - st < kSmallStages - 2 ? stages - 1 - st : kSmallStages - 2);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (st + kSmallStages - 1 < stages) request(st + kSmallStages - 1);
+    const uint16_t *A = lds + (st % kSmallStages) * 2 * kHalfU16, *B = A + kHalfU16;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      auto fragment = [&](const uint16_t* P, int c) {
+        return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(P + c * IK + (((2 * ks + hi) ^ ((c >> 2) & 3)) << 3)));
+      };
+      const bf16x8 fb = fragment(B, wn * 32 + rl), fa0 = fragment(A, wm * 64 + rl), fa1 = fragment(A, wm * 64 + 32 + rl);
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa0, fb, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa1, fb, acc[1], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int mi = 0; mi < 2; ++mi) {
+    float h[16];
+    const long gj = long(tj) * kSmallTile + wn * 32 + rl;
+      const long gi0 = long(ti) * kSmallTile + wm * 64 + mi * 32 + 4 * hi;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const long gi = gi0 + (v & 3) + 8 * (v >> 2);
+        h[v] = gi < n && gj < n ? H[gi * n + gj] : 0.f;
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const long gi = gi0 + (v & 3) + 8 * (v >> 2);
+        if (gi < n && gj < n) H[gi * n + gj] = h[v] + acc[mi][v];
+      }
+    }
+}
+
 // The batch of a Hessian accumulation (rows x n bf16, row-major) as the stage images of syrk_img_kernel: one workgroup
 // per stage of 32 rows and tile of 256 columns brings the 32 x 256 block in with 16-byte loads (zeros beyond the
 // matrix), turns it in LDS and writes each column's 32 values as the four swizzled 16-byte pieces of its image: 16 KB
@@ -371,6 +451,8 @@ struct SyrkGrid {
                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(kImgLdsBytes)));
         QTIP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(syrk_img_kernel<false>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(kImgLdsBytes)));
+        QTIP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(syrk_img_small_kernel),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(kSmallLdsBytes)));
         configured[size_t(dev)] = true;
       }
     }
@@ -398,8 +480,18 @@ void launch_hessian_accumulate(const uint16_t* X, long rows, long n, float* H, D
   image.ensure(size_t(stages) * size_t(g.tiles) * kImgSliceU16);
   batch_image_kernel<<<dim3(unsigned(g.tiles), unsigned(stages)), dim3(256), 0, s>>>(X, rows, n, g.tiles, image.p);
   QTIP_HIP(hipGetLastError());
-  syrk_img_kernel<false><<<dim3(g.grid), dim3(256), kImgLdsBytes, s>>>(image.p, image.p, int(stages), n, H, nullptr,
-                                                                      g.tiles, g.patch_cols);
+  // one tile per compute unit at a time, whatever its size: while the 128 x 128 tiles fit the chip at once (253 of them at
+  // n = 2816) a launch of them is over sooner than one of 256 x 256 tiles, which leaves three quarters of the chip idle;
+  // beyond that they come in two and more rounds and
+  // lose.  A call with 1000 / 4096 rows, image included: n = 512 20.7 / 54.5 us (big tiles 28.8 / 76.5), 2560 28.0 / 65.0
+  // (38.4 / 92.9), 2816 28.0 / 67.1 (37.9 / 93.3); with the small tiles at n = 3328 57 / 128 (38 / 95).
+  const long small = (n + kSmallTile - 1) / kSmallTile, small_tiles = small * (small + 1) / 2;
+  if (small_tiles <= 256) {
+    syrk_img_small_kernel<<<dim3(unsigned(small_tiles)), dim3(512), kSmallLdsBytes, s>>>(image.p, int(stages), n, H, g.tiles);
+  } else {
+    syrk_img_kernel<false><<<dim3(g.grid), dim3(256), kImgLdsBytes, s>>>(image.p, image.p, int(stages), n, H, nullptr,
+                                                                        g.tiles, g.patch_cols);
+  }
   QTIP_HIP(hipGetLastError());
 }
 
