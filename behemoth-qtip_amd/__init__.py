@@ -118,6 +118,7 @@ def lib():
     L.qtip_sign_vector.restype = None
     L.qtip_rotate_hessian.argtypes = [vp, vp, i, i, u64, d, vp, C.POINTER(d), vp]
     L.qtip_ldl_hessian.argtypes = [vp, i, i, vp]
+    L.qtip_selftest_pair_patience.argtypes = [vp, C.c_ulonglong]
     L.qtip_ldl_hessian_device_updates.argtypes = [vp, vp, i, i, vp]
     L.qtip_selftest_ldl_panel_handover.argtypes = [vp, i, i, vp]
     L.qtip_ldl_hessian_device_updates_dev.argtypes = [vp, vp, i, i, vp, vp]
@@ -304,6 +305,10 @@ class Quantizer:
     def stream_signal(self, stream=None):
         """`stream` waits for everything queued so far on the context's stream."""
         _check(lib().qtip_stream_signal(self._h, _stream_handle(stream)))
+
+    def selftest_pair_patience(self, ticks):
+        """Ticks of 10 ns for which the workgroups of a pair wait for each other (same results whatever it is)."""
+        _check(lib().qtip_selftest_pair_patience(self._h, ticks))
 
     def device_lut(self):
         """Device address of the 65536-entry fp16-pair table (device_lut(), src/quantizer.cpp:14-28)."""

@@ -441,6 +441,13 @@ int qtip_set_viterbi_mode(qtip_ctx* ctx, int mode, unsigned margin_units) {
   });
 }
 
+int qtip_selftest_pair_patience(qtip_ctx* ctx, unsigned long long ticks) {
+  return guarded([&] {
+    QTIP_REQUIRE(ctx != nullptr, "null context");
+    ctx->vit_pair_patience = ticks;
+  });
+}
+
 int qtip_ldlq_default_chains(qtip_ctx* ctx, int* chains) {
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr && chains != nullptr, "ldlq_default_chains: null argument");

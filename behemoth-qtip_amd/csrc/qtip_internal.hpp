@@ -259,8 +259,11 @@ struct TileJob {
   // 2^-26 is run again on fp64 metrics (same results as mode 1, bit for bit); 1: fp64 metrics only
   int mode = 0;
   // workgroups of 512 threads per tile instead of 256 (mode 0 only; same results): -1 = where the launch has at most
-  // a third as many tiles as the device has workgroup slots, 0 = never, 1 = always
+  // a third as many tiles as the device has workgroup slots, and two of them per tile where the device has a compute unit
+  // for each; 0 = never, 1 = always, one per tile
   int wide = -1;
+  // ticks of the 100 MHz clock a workgroup of a pair waits for the other before the first does the rest alone
+  unsigned long long pair_patience = 50000000ull;
   uint32_t margin = kViterbiMargin;
   unsigned* stats = nullptr;  // device counters (optional): [0], [1] += passes of the first / second kind run again
 };

@@ -22,11 +22,13 @@ struct qtip_ctx {
   int vit_mode = 0;
   int vit_wide = -1;  // TileJob::wide; a lane runs beside other lanes and keeps to the 256-thread workgroups
   uint32_t vit_margin = qtipmi::kViterbiMargin;
+  unsigned long long vit_pair_patience = qtipmi::TileJob{}.pair_patience;
   qtipmi::DBuf<unsigned> vit_stats;
   void viterbi_settings(qtipmi::TileJob& job) const {
     job.mode = vit_mode;
     job.wide = vit_slots_limit > 0 ? 0 : vit_wide;
     job.margin = vit_margin;
+    job.pair_patience = vit_pair_patience;
     job.stats = vit_stats.p;
   }
   int vit_slots_limit = 0;  // a lane (below) keeps slots for this many workgroups only; 0: all the device can hold

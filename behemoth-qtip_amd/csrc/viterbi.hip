@@ -51,6 +51,7 @@
 // threads per tile.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <mutex>
 #include <type_traits>
@@ -68,11 +69,25 @@ constexpr int kHistSteps = 63;                           // the metrics entering
 constexpr int kHistWordsPerTile = kHistSteps * kGroups;  // fp64 words
 enum StepKind { kPlain = 0, kStore = 1, kDigits = 2 };
 
+// What the two workgroups of a pair (viterbi_pair_kernel) exchange lies behind the kept metrics of their slots.
+struct PairArea {
+  uint32_t flag;      // how far the slot's workgroup has come in this launch (pair_reset_kernel clears it)
+  uint32_t alone;     // in the first workgroup's slot: one of the two gave up waiting for the other
+  uint32_t overlap;   // first workgroup: the overlap group and the winner of a free pass it had to repeat on fp64 metrics
+  uint32_t expected;
+  uint32_t doubt;     // second workgroup: its half of the path holds a decision that is too close
+  uint32_t states[64];     // second workgroup: the states of steps 64 .. 127
+  uint32_t x[kSeq];        // first workgroup: the block's targets (fp32 bits)
+  uint32_t mid[2][kGroups];  // the metrics at the middle of the two passes
+};
+constexpr int kPairWords = (sizeof(PairArea) + 255) / 256 * 32;  // in doubles
+constexpr int kSlotWords = kHistWordsPerTile + kPairWords;
+
 // Kept-metrics slots for callers that may not allocate (qtip_viterbi_tiles_dev_noalloc): part of the code object, so
-// every device that loads the library holds its own copy (63 MiB) until the process ends.  Host code must not use
+// every device that loads the library holds its own copy (64 MiB) until the process ends.  Host code must not use
 // this name as an address; the per-device address comes from hipGetSymbolAddress (static_scratch_of below).
 constexpr int kStaticSlots = 32;
-static __device__ __align__(256) double scratch[size_t(kStaticSlots) * kHistWordsPerTile];
+static __device__ __align__(256) double scratch[size_t(kStaticSlots) * kSlotWords];
 constexpr int kMaxDevices = 64;
 double* g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mutex;
@@ -113,6 +128,7 @@ struct Smem {
   alignas(16) uint32_t tr32[2][4][4];  // the same for the 32-bit passes: best, second best, d | d1 << 8, gap inside the best's row
   uint32_t red32[8][3];    // end of the free 32-bit pass: per wave the best group's metric, the second best, the group
   int overlap;
+  uint32_t heard;      // pair: what waiting for the other workgroup came to
   uint32_t final_state;
   float final_metric;  // the free fp64 pass's best final metric (what later 32-bit passes of the tile row may expect)
 };
@@ -597,7 +613,9 @@ __device__ __forceinline__ uint32_t err_units(double l0, double l1, double x0, d
 // a thread keeps its four codebook entries in registers.
 // kWide: 512 threads; the threads t and t + 256 share the eight groups of a column half, four each (slots 0..3 and
 // 4..7), and the table's 1024 entries two each instead of four.
-template <bool kSym, bool kWide>
+// kHalf: steps 0 .. 63 only; the metrics entering step 64 are left in metric buffer 0 (the other half of the sequence is
+// another workgroup's, viterbi_pair_kernel).
+template <bool kSym, bool kWide, bool kHalf = false>
 __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restrict__ entry_d, int roll, int ov,
                                                uint32_t* __restrict__ hist, int first_kept, const Unit unit) {
   constexpr int kT = kWide ? 2 * kThreads : kThreads, kSlotsOwn = kWide ? 4 : 8, kEnt = 1024 / kT;
@@ -809,11 +827,12 @@ __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restric
   static_assert((kSteps - 1) % 2 == 1, "steps 0 .. kSteps - 2 are pairs and one more even step");
   // two steps per turn, so that a step's parity is a constant (first_kept is even: the kept steps are even ones)
 #pragma nounroll
-  for (int it = 0; it < kSteps - 2; it += 2) {
+  for (int it = 0; it < (kHalf ? kSteps / 2 : kSteps - 2); it += 2) {
     if (it >= first_kept) step(it, Store{}, Even{});
     else step(it, Plain{}, Even{});
     step(it + 1, Plain{}, Odd{});
   }
+  if constexpr (kHalf) return;
   step(kSteps - 2, Store{}, Even{});
   if constexpr (kSym) {
     step(kSteps - 1, Last{}, Odd{});
@@ -875,11 +894,12 @@ __device__ __forceinline__ uint32_t row_min16_u32(uint32_t c) {
 // 2 KB table of fp16 pairs in LDS (tl), so that no other vector-memory load waits in line behind the streamed ones.
 // Beside other workgroups the streamed form loses more in their forward passes than it gains (measured), so the
 // 256-thread form fetches on demand.
+// last: the step the walk starts with (kSym: 127): j_last is the group entered after it.
 template <bool kSym, bool kStream>
 __device__ __forceinline__ uint32_t trace_back32(Smem& sm, const double* __restrict__ entry_d,
                                                  const uint32_t* __restrict__ hist, int roll, uint32_t j_last,
                                                  int it_min, bool record, uint32_t thr, uint32_t& flag,
-                                                 const uint32_t* tl, const Unit unit) {
+                                                 const uint32_t* tl, const Unit unit, int last = kSteps - 1) {
   const uint32_t tid = uint32_t(opaque_tid());
   const uint32_t lane = tid & 63u, wave = tid >> 6, dp = lane & 15u, d = 4u * wave + (lane >> 4);
   // streamed form: kept steps 63, 62, ..., it_min / 2 - 1 are the rows q = 0, 1, ... of a ring of kBufs buffers
@@ -888,12 +908,12 @@ __device__ __forceinline__ uint32_t trace_back32(Smem& sm, const double* __restr
   static_assert(sizeof(sm.E) + sizeof(sm.M) >= size_t(kBufs) * kRowWords * 4 && offsetof(Smem, M) == sizeof(sm.E));
   static_assert((kBufs - 2) * kLoads <= 15, "the count of outstanding loads must fit the low four bits of the wait");
   uint32_t* const rows = reinterpret_cast<uint32_t*>(sm.E);
-  const int count = 65 - it_min / 2;
+  const int top = last / 2, count = top + 2 - it_min / 2;
   int issued = 0, q = 0;  // rows requested so far; the row in use
   typedef __attribute__((address_space(3))) void* lds_ptr;
   auto issue = [&](int row) {
     const uint32_t wave8 = threadIdx.x >> 6;  // all eight waves bring a share
-    const uint32_t* g = hist + size_t(63 - row) * kGroups + 4u * lane;
+    const uint32_t* g = hist + size_t(top - row) * kGroups + 4u * lane;
     uint32_t* l = rows + (row % kBufs) * kRowWords;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
@@ -972,15 +992,15 @@ __device__ __forceinline__ uint32_t trace_back32(Smem& sm, const double* __restr
   };
   uint32_t s;
   if constexpr (!kSym) {  // step 127: the 16 states (digit << 12) | j_last, one per lane of a row; every row does the same
-    const int t = (2 * (kSteps - 1) + roll) & 255;
+    const int t = (2 * last + roll) & 255;
     const double x0 = double(sm.x[t]), x1 = double(sm.x[t + 1]);
     const uint32_t st = (dp << 12) | j_last;
-    const uint32_t c = sat_add(err_of(st, x0, x1), kept(63, st >> 4));
+    const uint32_t c = sat_add(err_of(st, x0, x1), kept(top, st >> 4));
     uint32_t k, gap;
     const uint32_t m = row_pick(c, k, gap);
     flag |= uint32_t(gap < thr) | uint32_t(m >= kWinnerMax);
     s = (k << 12) | j_last;
-    if (record && threadIdx.x == 0) sm.st[kSteps - 1] = uint16_t(s);
+    if (record && threadIdx.x == 0) sm.st[last] = uint16_t(s);
     if constexpr (kStream) round_barrier();
   } else {
     // Free pass: the final state is the best of all.  The forward pass has named the best group's column and
@@ -1031,7 +1051,7 @@ __device__ __forceinline__ uint32_t trace_back32(Smem& sm, const double* __restr
   }
   int set = 0;
 #pragma nounroll
-  for (int it = kSteps - 2; it >= it_min; it -= 2, set ^= 1) {
+  for (int it = last - 1; it >= it_min; it -= 2, set ^= 1) {
     const uint32_t j = s >> 4;
     const int ta = (2 * (it - 1) + roll) & 255, tb = (2 * it + roll) & 255;
     const double xa0 = double(sm.x[ta]), xa1 = double(sm.x[ta + 1]);
@@ -1107,42 +1127,23 @@ __device__ __forceinline__ uint32_t trace_back32(Smem& sm, const double* __restr
   return s;
 }
 
-// kWide: 512 threads per tile, one workgroup per compute unit, for launches that cannot fill the chip anyway (a lone
-// small group): a tile then takes about two thirds of the time.  Same results, bit for bit.
+// The passes first_pass .. passes_end - 1 (of two) of one block by one workgroup: targets in sm.x, states to sm.st (a
+// second pass by itself takes the overlap group from sm.overlap).  expected: the free pass's winner of this tile row's
+// previous column block (0: none yet), and of this one afterwards.  fp64_only: as job.mode 1.  Ends with a barrier.
 template <bool kWide>
-__global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) void viterbi_tiles_kernel(
-    TileJob job, const double* __restrict__ entry_d, const float* __restrict__ entry_f, double* __restrict__ hist_all) {
-  __shared__ Smem sm;
-  __shared__ uint32_t tl[kWide ? 512 : 1];  // wide form: the codebook's 512 value pairs as fp16 bits, for its trace-backs
+__device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const double* __restrict__ entry_d, double* hist,
+                                             const uint32_t* tl, float& expected, int first_pass, int passes_end,
+                                             bool fp64_only) {
   const int u = threadIdx.x & (kThreads - 1);
-  const bool first_half = threadIdx.x < kThreads;  // global results are written once
-  if constexpr (kWide) {  // the table's values are fp16 values (entry bit 9 is the sign of the first one)
-    const int i = threadIdx.x;
-    const uint32_t h0 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i]));
-    const uint32_t h1 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i + 1]));
-    tl[i] = h0 | (h1 << 16);
-    __syncthreads();
-  }
-  double* hist = hist_all + size_t(blockIdx.x) * kHistWordsPerTile;
-  for (long tile = blockIdx.x; tile < job.tiles; tile += gridDim.x) {
-  float expected = 0.f;  // the free pass's winner of this tile row's previous column block (0: none yet)
-  for (int blk = job.blocks - 1; blk >= 0; --blk) {
-    // the column block of this turn; the hatWT values the previous turn wrote for this tile row are visible after
-    // the barrier that ended it
-    const long col0 = job.col0 + 16 * blk;
-    if (job.X) sm.x[u] = job.X[tile * kSeq + u];
-    else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
-    else tile_targets<float>(sm, job, col0, tile, job.prod32);
-    __syncthreads();
     // pass 1 on the sequence rotated by half its length, free ends, traced back to step 64 for the overlap group;
     // pass 2 on the sequence itself, tail-biting through that group, traced back in full.  One loop, so that the
     // step bodies exist once in the instruction cache.
-    int ov = -1;
+    int ov = first_pass > 0 ? sm.overlap : -1;
 #pragma nounroll
-    for (int pass = 0; pass < 2; ++pass) {
+    for (int pass = first_pass; pass < passes_end; ++pass) {
       const int roll = pass == 0 ? kSeq / 2 : 0;
       bool done = false;
-      if (job.mode == 0) {
+      if (job.mode == 0 && !fp64_only) {
         uint32_t* const hist32 = reinterpret_cast<uint32_t*>(hist);
         uint32_t flag = 0;
         // (the same in every thread; said so, so that it lives in scalar registers)
@@ -1187,7 +1188,13 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
       __syncthreads();
       ov = sm.overlap;
     }
-    // ---- outputs
+}
+
+// States, packed words, decoded values and residual images of one block, from sm.st.
+__device__ __forceinline__ void block_outputs(const Smem& sm, const TileJob& job, const float* __restrict__ entry_f, long tile,
+                                              int blk, long col0) {
+  const int u = threadIdx.x & (kThreads - 1);
+  const bool first_half = threadIdx.x < kThreads;  // global results are written once
     if (job.states && first_half && u < kSteps) job.states[(tile * job.q_tile_stride + job.q_offset + blk) * kSteps + u] = sm.st[u];
     if (job.packed && first_half && u < kWords) {
       uint32_t v;
@@ -1213,8 +1220,463 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
         job.dimg_h[di] = uint16_t(hi), job.dimg_l[di] = uint16_t(lo);
       }
     }
+}
+
+// kWide: 512 threads per tile, one workgroup per compute unit, for launches that cannot fill the chip anyway (a lone
+// small group): a tile then takes about two thirds of the time.  Same results, bit for bit.
+template <bool kWide>
+__global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) void viterbi_tiles_kernel(
+    TileJob job, const double* __restrict__ entry_d, const float* __restrict__ entry_f, double* __restrict__ hist_all) {
+  __shared__ Smem sm;
+  __shared__ uint32_t tl[kWide ? 512 : 1];  // wide form: the codebook's 512 value pairs as fp16 bits, for its trace-backs
+  const int u = threadIdx.x & (kThreads - 1);
+  if constexpr (kWide) {  // the table's values are fp16 values (entry bit 9 is the sign of the first one)
+    const int i = threadIdx.x;
+    const uint32_t h0 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i]));
+    const uint32_t h1 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i + 1]));
+    tl[i] = h0 | (h1 << 16);
     __syncthreads();
   }
+  double* hist = hist_all + size_t(blockIdx.x) * kSlotWords;
+  for (long tile = blockIdx.x; tile < job.tiles; tile += gridDim.x) {
+  float expected = 0.f;  // the free pass's winner of this tile row's previous column block (0: none yet)
+  for (int blk = job.blocks - 1; blk >= 0; --blk) {
+    // the column block of this turn; the hatWT values the previous turn wrote for this tile row are visible after
+    // the barrier that ended it
+    const long col0 = job.col0 + 16 * blk;
+    if (job.X) sm.x[u] = job.X[tile * kSeq + u];
+    else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
+    else tile_targets<float>(sm, job, col0, tile, job.prod32);
+    __syncthreads();
+    block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
+    block_outputs(sm, job, entry_f, tile, blk, col0);
+    __syncthreads();
+  }
+  }
+}
+
+// ================================================================= a tile by two workgroups
+// A lone small layer is a chain of tiles: every column block of a tile row waits for the one before it, a tile by itself
+// takes 364 us on one compute unit, and with fewer tile rows than half the chip's compute units most of them idle.  The
+// two passes of a tile are then halved: the first workgroup of a pair runs the forward recursion over steps 0 .. 63 of a
+// pass while the second, on another compute unit, runs the recursion of the cheapest completions over steps 127 .. 64,
+//     B_i[g] = min_e ( E_i[entry(16 g + e)] + B_{i+1}[16 (g mod 256) + e] ),
+// and the best path is the group g with the smallest sum M_64[g] + B_64[g].  In the free pass that group is all that is
+// asked for: no trace-back.  In the tail-biting pass the first workgroup walks back from it to step 0 and the second
+// forward to step 127, at the same time.  The metrics are the 32-bit passes' (same units, same rounding: a sum of M and
+// B has 128 rounded terms), and so is the check: the group has to win by `margin` units against every other group and
+// every decision walked must be won by as many units as its candidates have rounded terms and more; then the path is
+// the fp64 recursion's.  Otherwise the first workgroup repeats the pass on fp64 metrics as before.
+// The free pass's mirror paths (see above): of two complementary paths the one with the smaller final state counts, which
+// is the one whose final state lies below 32768, so the completions start from those states alone and the second
+// workgroup computes all 4096 groups; the first still computes the lower half.
+// The pair talks through PairArea in device memory, with device-scope stores and loads that bypass the caches: the targets
+// (to the second), the metrics at the middle of either pass (both ways), the states of the second half (to the first,
+// which writes all results).  A wait is bounded: a workgroup whose partner does not answer for `patience` ticks (it is
+// not resident, say) marks the pair, the second workgroup ends, and the first does this block and the rest alone.
+// Measured: 24 tiles 374 -> 250 us; 64 tile rows through 64 blocks (a lone 1024 x 1024 group, everything included) 24.7 ->
+// 16.9 ms.
+template <bool kFree>
+__device__ __forceinline__ void backward_pass32(Smem& sm, const double* __restrict__ entry_d, int roll, uint32_t ov,
+                                                uint32_t* __restrict__ hist, const Unit unit) {
+  // A thread owns metric column c (the sixteen groups 16 c + e after the step; they continue the sixteen groups 256 h + c
+  // before it) with its mirror 255 - c, and the four h = 4 r + i: per j = 16 c + e the four table values of h serve group
+  // 256 h + c (with B[j]) and its mirror (with B[4095 - j]).  The table and the lanes' columns are the tail-biting
+  // forward pass's, so its reads are free of bank conflicts as there; metric j sits at m32_slot(j / 16, j mod 16), which
+  // makes the column reads conflict-free and leaves a four-way conflict in the eight writes per thread and step.
+  const int t = opaque_tid_wide();
+  const int p = t & 127, r = t >> 7;
+  const int colA = 4 * (p & 31) + (p >> 5), colB = 255 - colA;
+  uint32_t* const E32 = reinterpret_cast<uint32_t*>(sm.E);
+  uint32_t* const M32 = reinterpret_cast<uint32_t*>(sm.M);
+  double2 ent[2];
+  const double2* __restrict__ entries = reinterpret_cast<const double2*>(entry_d) + t;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) ent[q] = entries[512 * q], ent[q].x *= unit.pre, ent[q].y *= unit.pre;
+  int ebase[16], wslot[4];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const uint32_t j = 16u * colA + uint32_t(e), pj = j * (j + 1u);
+    ebase[e] = int((((pj >> 12) + uint32_t(4 * r * (2 * (e & 7) + 1))) & 15u) * 64u + ((pj >> 6) & 63u));
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int g = 256 * (4 * r + i) + colA;
+    wslot[i] = m32_slot(g >> 4, g & 15);
+  }
+  const int xA = m32_pos(colA) * 64 + m32_swz(colA) * 4, xB = m32_pos(colB) * 64 + m32_swz(colB) * 4;  // bytes
+  auto table = [&](int it, int par) __attribute__((always_inline)) {
+    const int at = (2 * it + roll) & 255;
+    const double x0 = double(sm.x[at]) * unit.pre, x1 = double(sm.x[at + 1]) * unit.pre;
+    uint32_t* const Ew = E32 + par * kESlots + t;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const uint32_t v = err_units(ent[q].x, ent[q].y, x0, x1);
+      Ew[512 * q] = v;
+      Ew[512 * q + 1024] = v;
+    }
+  };
+  for (int g = t; g < kGroups; g += 512) M32[m32_slot(g >> 4, g & 15)] = (kFree || uint32_t(g) == ov) ? 0u : kSat;
+  table(kSteps - 1, 0);
+  __syncthreads();
+  // step `it`: metrics and table of buffer par -> metrics of the other buffer, and the table of step it - 1
+  auto step = [&](int it, auto par_tag) __attribute__((always_inline)) {
+    constexpr int par = decltype(par_tag)::value;
+    const char* const Mb = reinterpret_cast<const char*>(M32 + par * kMSlots);
+    uint32_t* const Mw = M32 + (par ^ 1) * kMSlots;
+    const uint32_t* const Er = E32 + par * kESlots;
+    uint32_t MA[16], MB[16];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint4 a = *reinterpret_cast<const uint4*>(Mb + (xA ^ (16 * k)));
+      MA[4 * k] = a.x, MA[4 * k + 1] = a.y, MA[4 * k + 2] = a.z, MA[4 * k + 3] = a.w;
+      const uint4 b = *reinterpret_cast<const uint4*>(Mb + (xB ^ (16 * k)));
+      MB[4 * k] = b.x, MB[4 * k + 1] = b.y, MB[4 * k + 2] = b.z, MB[4 * k + 3] = b.w;
+    }
+    table(it - 1, par ^ 1);
+    uint32_t own[4] = {kSat, kSat, kSat, kSat}, mirror[4] = {kSat, kSat, kSat, kSat};
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+      uint32_t v0[4], v1[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v0[i] = Er[ebase[e] + ((i * (2 * (e & 7) + 1)) & 15) * 64];
+        v1[i] = Er[ebase[e + 1] + ((i * (2 * ((e + 1) & 7) + 1)) & 15) * 64];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        own[i] = min3u(own[i], sat_add(v0[i], MA[e]), sat_add(v1[i], MA[e + 1]));
+        mirror[i] = min3u(mirror[i], sat_add(v0[i], MB[15 - e]), sat_add(v1[i], MB[14 - e]));
+      }
+    }
+    if (kFree && it == kSteps - 1) {  // final states of 32768 and more do not count: groups of 2048 and more (r: the same in a wave)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        own[i] = r >= 2 ? kSat : own[i];
+        mirror[i] = r >= 2 ? mirror[i] : kSat;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      Mw[wslot[i]] = own[i];
+      Mw[wslot[i] ^ kMirror32] = mirror[i];
+    }
+    if (!kFree && par == 1 && it >= kSteps / 2 + 2) {
+      uint32_t* const hs = hist + size_t((it - kSteps / 2 - 2) >> 1) * kGroups + t;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) hs[512 * i] = own[i], hs[512 * (4 + i)] = mirror[i];
+    }
+    __syncthreads();
+  };
+#pragma nounroll
+  for (int it = kSteps - 1; it > kSteps / 2; it -= 2) {
+    step(it, std::integral_constant<int, 0>{});
+    step(it - 1, std::integral_constant<int, 1>{});
+  }
+}
+
+// place of group g in one kept step of the backward pass (the metrics B_66, B_68 .. B_126)
+__device__ __forceinline__ uint32_t back_index(uint32_t g) {
+  const bool m = (g & 255u) >= 128u;
+  const uint32_t q = m ? 4095u - g : g, c = q & 255u, h = q >> 8;
+  return ((m ? 4u : 0u) + (h & 3u)) * 512u + (h >> 2) * 128u + ((c >> 2) | ((c & 3u) << 5));
+}
+
+// From group g entering step 64 to the group ov after step 127, two steps a round, in the scheme of trace_back32's streamed
+// form with the directions exchanged; records the states of steps 64 .. 127.  A candidate of step t is a sum of 128 - t
+// rounded terms, and thr, which 128 terms need, shrinks by one unit per term less.
+__device__ __forceinline__ void trace_forward32(Smem& sm, const uint32_t* __restrict__ hist, uint32_t g, uint32_t ov,
+                                                uint32_t thr, uint32_t& flag, const uint32_t* tl, const Unit unit) {
+  const uint32_t tid = uint32_t(opaque_tid());
+  const uint32_t lane = tid & 63u, wave = tid >> 6, dp = lane & 15u, d = 4u * wave + (lane >> 4);
+  constexpr int kBufs = 3, kLoads = kGroups / (4 * 2 * kThreads), kRows = 31;
+  uint32_t* const rows = reinterpret_cast<uint32_t*>(sm.E);
+  int issued = 0, q = 0;
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  auto issue = [&](int row) {
+    const uint32_t wave8 = threadIdx.x >> 6;
+    const uint32_t* src = hist + size_t(row) * kGroups + 4u * lane;
+    uint32_t* l = rows + (row % kBufs) * kGroups;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const uint32_t w0 = (uint32_t(i) * 8u + wave8) * 256u;
+      __builtin_amdgcn_global_load_lds(src + w0, (lds_ptr)(l + w0), 16, 0, 0);
+    }
+  };
+  auto landed = [&](int later) {
+    if (later >= 1) __builtin_amdgcn_s_waitcnt(0x0F70 | kLoads);
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+  };
+  auto lds_barrier = [&] {  // orders LDS, not the loads in flight
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  for (; issued < kBufs; ++issued) issue(issued);
+  landed(issued - 1);
+  lds_barrier();
+  auto err_of = [&](uint32_t st, int at) -> uint32_t {
+    const uint32_t e = ((st * (st + 1u)) >> 6) & 1023u, w = tl[e & 511u];
+    const uint16_t h0 = uint16_t((w & 0xffffu) ^ ((e >> 9) << 15)), h1 = uint16_t(w >> 16);
+    const double l0 = double(float(__builtin_bit_cast(_Float16, h0))), l1 = double(float(__builtin_bit_cast(_Float16, h1)));
+    return err_units(l0 * unit.pre, l1 * unit.pre, double(sm.x[at]) * unit.pre, double(sm.x[at + 1]) * unit.pre);
+  };
+  int set = 0;
+#pragma nounroll
+  for (int t = kSteps / 2; t < kSteps; t += 2, set ^= 1) {
+    const uint32_t s1 = (g << 4) | d;                        // candidate state of step t
+    const uint32_t s2 = ((s1 & 0xfffu) << 4) | dp;           // and of step t + 1
+    const uint32_t g2 = s2 & 0xfffu;
+    const uint32_t kv = t < kSteps - 2 ? rows[(q % kBufs) * kGroups + back_index(g2)] : (g2 == ov ? 0u : kSat);
+    const uint32_t c1 = sat_add(err_of(s2, (2 * t + 2) & 255), kv);
+    // over the 16 lanes of a row: the smallest value, the first lane that holds it, the gap to the runner-up
+    const uint32_t low = row_min16_u32(c1);
+    const uint32_t bits = uint32_t(__builtin_amdgcn_ballot_w64(c1 == low) >> (lane & 48u)) & 0xffffu;
+    const uint32_t k1 = bits ? uint32_t(__builtin_ctz(bits)) : 0u;
+    const uint32_t gap1 = row_min16_u32(dp == k1 ? kSat : c1) - low;
+    const uint32_t c0 = sat_add(err_of(s1, (2 * t) & 255), low);
+    uint32_t bc = uint32_t(__builtin_amdgcn_readlane(int(c0), 0)), sc = kSat, bd = 4u * wave;
+    uint32_t bd1 = uint32_t(__builtin_amdgcn_readlane(int(k1), 0)), bg = uint32_t(__builtin_amdgcn_readlane(int(gap1), 0));
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+      const uint32_t oc = uint32_t(__builtin_amdgcn_readlane(int(c0), 16 * i));
+      const uint32_t od1 = uint32_t(__builtin_amdgcn_readlane(int(k1), 16 * i));
+      const uint32_t og = uint32_t(__builtin_amdgcn_readlane(int(gap1), 16 * i));
+      const bool take = oc < bc;
+      sc = take ? bc : min(sc, oc);
+      bd = take ? 4u * wave + uint32_t(i) : bd;
+      bd1 = take ? od1 : bd1;
+      bg = take ? og : bg;
+      bc = take ? oc : bc;
+    }
+    if (lane == 0) {
+      sm.tr32[set][wave][0] = bc;
+      sm.tr32[set][wave][1] = sc;
+      sm.tr32[set][wave][2] = bd | (bd1 << 8);
+      sm.tr32[set][wave][3] = bg;
+    }
+    // the next row has landed here, then everywhere; nobody reads the present one after the barrier
+    landed(issued - 2 - q > 0 ? issued - 2 - q : 0);
+    lds_barrier();
+    if (issued < kRows) issue(issued++);
+    ++q;
+    uint4 w4[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) w4[w] = *reinterpret_cast<const uint4*>(sm.tr32[set][w]);
+    bc = w4[0].x, sc = w4[0].y, bg = w4[0].w;
+    uint32_t bdd = w4[0].z;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      const bool take = w4[w].x < bc;
+      sc = take ? min(bc, w4[w].y) : min(sc, w4[w].x);
+      bdd = take ? w4[w].z : bdd;
+      bg = take ? w4[w].w : bg;
+      bc = take ? w4[w].x : bc;
+    }
+    const uint32_t fewer = uint32_t(t), thr_t = thr - (fewer < thr ? fewer : thr);
+    flag |= uint32_t(sc - bc < thr_t) | uint32_t(bg < thr_t) | uint32_t(bc >= kWinnerMax);
+    const uint32_t st1 = ((g << 4) | (bdd & 15u)) & 0xffffu, st2 = ((st1 << 4) | ((bdd >> 8) & 15u)) & 0xffffu;
+    if (threadIdx.x == 0) sm.st[t] = uint16_t(st1), sm.st[t + 1] = uint16_t(st2);
+    g = st2 & 0xfffu;
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void pair_put(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t pair_get(const uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void pair_reset_kernel(double* __restrict__ hist_all, int slots) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= slots) return;
+  PairArea* a = reinterpret_cast<PairArea*>(hist_all + size_t(i) * kSlotWords + kHistWordsPerTile);
+  pair_put(&a->flag, 0u);
+  pair_put(&a->alone, 0u);
+}
+
+// Workgroups b and b + 8 (bit 3 of the number) are a pair, 8 pairs per 16 workgroups: they are dealt to the XCDs in turn,
+// so that a pair shares one.  One tile row per pair.
+__global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob job, const double* __restrict__ entry_d,
+                                                                      const float* __restrict__ entry_f,
+                                                                      double* __restrict__ hist_all) {
+  __shared__ Smem sm;
+  __shared__ uint32_t tl[512];
+  const long tile = long(blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+  const bool second = (blockIdx.x >> 3) & 1;
+  if (tile >= job.tiles) return;
+  {
+    const int i = threadIdx.x;
+    const uint32_t h0 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i]));
+    const uint32_t h1 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i + 1]));
+    tl[i] = h0 | (h1 << 16);
+    __syncthreads();
+  }
+  const int tid = threadIdx.x;
+  double* const hist = hist_all + size_t(blockIdx.x) * kSlotWords;
+  uint32_t* const hist32 = reinterpret_cast<uint32_t*>(hist);
+  PairArea* const mine = reinterpret_cast<PairArea*>(hist + kHistWordsPerTile);
+  PairArea* const other = reinterpret_cast<PairArea*>(hist_all + size_t(blockIdx.x ^ 8u) * kSlotWords + kHistWordsPerTile);
+  uint32_t* const alone_word = second ? &other->alone : &mine->alone;
+  uint32_t* const M32 = reinterpret_cast<uint32_t*>(sm.M);
+  uint32_t* const Mc32 = reinterpret_cast<uint32_t*>(sm.E) + 2 * (2 * 16 * 64 * 2);  // the free pass's compact metrics
+  // everything this workgroup has put is where the other can get it before the flag says so
+  auto tell = [&](uint32_t v) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), every wave
+    asm volatile("" ::: "memory");
+    __syncthreads();
+    if (tid == 0) pair_put(&mine->flag, v);
+  };
+  // false: the pair is given up
+  auto hear = [&](uint32_t v) -> bool {
+    if (tid == 0) {
+      const unsigned long long t0 = wall_clock64();
+      uint32_t res = 0;
+      for (;;) {
+        if (pair_get(&other->flag) >= v) {
+          res = 1;
+          break;
+        }
+        if (pair_get(alone_word)) break;
+        if (wall_clock64() - t0 >= job.pair_patience) {
+          pair_put(alone_word, 1u);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      sm.heard = res;
+    }
+    __syncthreads();
+    const bool ok = __builtin_amdgcn_readfirstlane(int(sm.heard)) != 0;
+    __syncthreads();
+    return ok;
+  };
+  // best group and runner-up of M_64 + B_64; which: 0 free pass, 1 tail-biting pass
+  uint32_t b1 = 0, b2 = 0, bj = 0;
+  auto middle = [&](int which) {
+    b1 = kSat, b2 = kSat, bj = 0;
+#pragma unroll
+    for (int k = 0; k < kGroups / 512; ++k) {
+      const uint32_t g = uint32_t(tid) + 512u * uint32_t(k);
+      const uint32_t low = which == 0 && g >= 2048u ? 4095u - g : g;
+      uint32_t m;
+      if (second) m = M32[m32_slot(int(g >> 4), int(g & 15u))];
+      else m = which == 0 ? Mc32[m32c_slot(int(low & 255u), int(low >> 8))] : M32[m32_slot(int(g & 255u), int(g >> 8))];
+      const uint32_t v = sat_add(m, pair_get(&other->mid[which][second ? low : g]));
+      const bool take = v < b1;
+      b2 = take ? b1 : min(b2, v);
+      bj = take ? g : bj;
+      b1 = take ? v : b1;
+    }
+    auto merge = [&](uint32_t o1, uint32_t o2, uint32_t oj) {
+      const bool take = o1 < b1 || (o1 == b1 && oj < bj);
+      b2 = take ? min(o2, b1) : min(b2, o1);
+      bj = take ? oj : bj;
+      b1 = take ? o1 : b1;
+    };
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) merge(__shfl_xor(b1, off, 64), __shfl_xor(b2, off, 64), __shfl_xor(bj, off, 64));
+    if ((tid & 63) == 0) sm.red32[tid >> 6][0] = b1, sm.red32[tid >> 6][1] = b2, sm.red32[tid >> 6][2] = bj;
+    __syncthreads();
+    b1 = sm.red32[0][0], b2 = sm.red32[0][1], bj = sm.red32[0][2];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) merge(sm.red32[w][0], sm.red32[w][1], sm.red32[w][2]);
+    __syncthreads();
+  };
+  auto unit_log2 = [&](float expected, float room) { return __builtin_amdgcn_readfirstlane(unit_log2_for(expected, room)); };
+  float expected = 0.f;
+  uint32_t n = 0;
+  if (second) {
+    for (int blk = job.blocks - 1; blk >= 0; --blk, n += 8) {
+      if (!hear(n + 1)) return;
+      if (tid < kSeq) sm.x[tid] = __uint_as_float(pair_get(&other->x[tid]));
+      __syncthreads();
+      const int k1 = unit_log2(expected, 2.f);
+      backward_pass32<true>(sm, entry_d, kSeq / 2, 0u, nullptr, unit_of(k1));
+      for (int g = tid; g < kGroups; g += 512) pair_put(&mine->mid[0][g], M32[m32_slot(g >> 4, g & 15)]);
+      tell(n + 2);
+      if (!hear(n + 2)) return;
+      middle(0);
+      uint32_t ov = bj;
+      if (b2 - b1 < job.margin || b1 >= kWinnerMax) {
+        if (!hear(n + 3)) return;
+        ov = pair_get(&other->overlap);
+        expected = __uint_as_float(pair_get(&other->expected));
+      } else {
+        expected = __builtin_ldexpf(float(b1), -k1);
+      }
+      ov = uint32_t(__builtin_amdgcn_readfirstlane(int(ov)));
+      const Unit unit = unit_of(unit_log2(expected, 1.125f));
+      backward_pass32<false>(sm, entry_d, 0, ov, hist32, unit);
+      for (int g = tid; g < kGroups; g += 512) pair_put(&mine->mid[1][g], M32[m32_slot(g >> 4, g & 15)]);
+      tell(n + 4);
+      if (!hear(n + 4)) return;
+      middle(1);
+      uint32_t flag = 0;
+      trace_forward32(sm, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), ov, job.margin, flag, tl, unit);
+      if (tid < 64) pair_put(&mine->states[tid], sm.st[64 + tid]);
+      if (tid == 0) pair_put(&mine->doubt, flag);
+      tell(n + 5);
+    }
+    return;
+  }
+  bool alone = false;
+  for (int blk = job.blocks - 1; blk >= 0; --blk, n += 8) {
+    const long col0 = job.col0 + 16 * blk;
+    if (job.X) sm.x[tid & (kSeq - 1)] = job.X[tile * kSeq + (tid & (kSeq - 1))];
+    else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
+    else tile_targets<float>(sm, job, col0, tile, job.prod32);
+    __syncthreads();
+    // the block's two passes together; false if the second workgroup is not there
+    auto together = [&]() -> bool {
+      if (tid < kSeq) pair_put(&mine->x[tid], __float_as_uint(sm.x[tid]));
+      tell(n + 1);
+      const int k1 = unit_log2(expected, 2.f);
+      forward_pass32<true, true, true>(sm, entry_d, kSeq / 2, -1, hist32, kSteps, unit_of(k1));
+      for (int g = tid; g < kGroups / 2; g += 512) pair_put(&mine->mid[0][g], Mc32[m32c_slot(g & 255, g >> 8)]);
+      tell(n + 2);
+      if (!hear(n + 2)) return false;
+      middle(0);
+      if (b2 - b1 < job.margin || b1 >= kWinnerMax) {
+        if (tid == 0 && job.stats) atomicAdd(job.stats, 1u);
+        block_passes<true>(sm, job, entry_d, hist, tl, expected, 0, 1, true);
+        if (tid == 0) pair_put(&mine->overlap, uint32_t(sm.overlap)), pair_put(&mine->expected, __float_as_uint(expected));
+        tell(n + 3);
+      } else {
+        if (tid == 0) sm.overlap = int(bj);
+        expected = __builtin_ldexpf(float(b1), -k1);
+        __syncthreads();
+      }
+      const uint32_t ov = uint32_t(__builtin_amdgcn_readfirstlane(sm.overlap));
+      const Unit unit = unit_of(unit_log2(expected, 1.125f));
+      forward_pass32<false, true, true>(sm, entry_d, 0, int(ov), hist32, 0, unit);
+      for (int g = tid; g < kGroups; g += 512) pair_put(&mine->mid[1][g], M32[m32_slot(g & 255, g >> 8)]);
+      tell(n + 4);
+      if (!hear(n + 4)) return false;
+      middle(1);
+      uint32_t flag = uint32_t(b2 - b1 < job.margin) | uint32_t(b1 >= kWinnerMax);
+      const uint32_t s = trace_back32<false, true>(sm, entry_d, hist32, 0, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), 2,
+                                                  true, job.margin, flag, tl, unit, kSteps / 2 - 1);
+      // s is the state of step 1; at step 0 the one predecessor group with a finite initial metric is ov
+      if (tid == 0) sm.st[0] = uint16_t((s >> 4) | ((ov >> 8) << 12));
+      if (!hear(n + 5)) return false;
+      flag |= uint32_t(__builtin_amdgcn_readfirstlane(int(pair_get(&other->doubt))));
+      if (flag) {
+        if (tid == 0 && job.stats) atomicAdd(job.stats + 1, 1u);
+        block_passes<true>(sm, job, entry_d, hist, tl, expected, 1, 2, true);
+      } else if (tid < 64) {
+        sm.st[64 + tid] = uint16_t(pair_get(&other->states[tid]));
+      }
+      __syncthreads();
+      return true;
+    };
+    if (!alone && !together()) alone = true;
+    if (alone) block_passes<true>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
+    block_outputs(sm, job, entry_f, tile, blk, col0);
+    __syncthreads();
   }
 }
 
@@ -1236,7 +1698,7 @@ __global__ void decode_states_kernel(const uint16_t* __restrict__ st, long count
 
 }  // namespace
 
-size_t viterbi_workspace_bytes(int slots) { return size_t(slots) * kHistWordsPerTile * sizeof(double); }
+size_t viterbi_workspace_bytes(int slots) { return size_t(slots) * kSlotWords * sizeof(double); }
 
 // workgroup slots of the 256-thread kernel on `device`, which must be current (found once per device)
 int viterbi_max_slots(int device) {
@@ -1253,6 +1715,14 @@ int viterbi_max_slots(int device) {
   const int slots = per_cu * prop.multiProcessorCount;
   if (tracked) cached[device] = slots;
   return slots;
+}
+
+// compute units of the current device, at most what the reset kernel's one workgroup covers
+static long viterbi_device_cus() {
+  int dev = 0, cus = 0;
+  QTIP_HIP(hipGetDevice(&dev));
+  QTIP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return std::min(cus, 256);
 }
 
 static int viterbi_device_slots() {
@@ -1281,6 +1751,20 @@ void launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const flo
   // the wide form where the launch leaves two thirds of the chip's workgroup slots empty anyway (and the 32-bit
   // passes, which are what it shares out over its 512 threads, are in use)
   const bool wide = job.mode == 0 && (job.wide > 0 || (job.wide < 0 && 3 * job.tiles <= viterbi_device_slots()));
+  // two workgroups per tile where every one of them then still has a compute unit to itself
+  const long pair_grid = 16 * ((job.tiles + 7) / 8);
+  if (job.mode == 0 && job.wide < 0 && pair_grid <= slots && pair_grid <= viterbi_device_cus()) {
+    double* const ws = static_cast<double*>(workspace);
+    pair_reset_kernel<<<dim3(1), dim3(256), 0, s>>>(ws, int(pair_grid));
+    QTIP_HIP(hipGetLastError());
+    if (start || stop)
+      hipExtLaunchKernelGGL(viterbi_pair_kernel, dim3(unsigned(pair_grid)), dim3(2 * kThreads), 0, s, start, stop, 0, job,
+                            d_entry_d, d_entry_f, ws);
+    else
+      viterbi_pair_kernel<<<dim3(unsigned(pair_grid)), dim3(2 * kThreads), 0, s>>>(job, d_entry_d, d_entry_f, ws);
+    QTIP_HIP(hipGetLastError());
+    return;
+  }
   const auto kernel = wide ? viterbi_tiles_kernel<true> : viterbi_tiles_kernel<false>;
   const dim3 block(wide ? 2 * kThreads : kThreads);
   if (start || stop) {

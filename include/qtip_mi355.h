@@ -356,6 +356,10 @@ int qtip_trim(qtip_ctx* ctx, unsigned long long* bytes_released);
  * qtip_viterbi_tiles_dev_noalloc reads it before and after the call.  No counterpart in the reference. */
 long qtip_selftest_device_alloc_calls(void);
 
+/* Self test (no counterpart in the reference): how long, in ticks of 10 ns, one of the two workgroups that share a tile in
+ * a small launch waits for the other before the first does the rest alone (same results; default half a second). */
+int qtip_selftest_pair_patience(qtip_ctx* ctx, unsigned long long ticks);
+
 /* Host-only self test (no GPU needed, no counterpart in the reference): a device buffer of the context whose
  * allocation failed stays empty, so the next call allocates again instead of launching on a null pointer.  0 = ok. */
 int qtip_selftest_failed_alloc_is_retried(void);

@@ -242,6 +242,46 @@ def test_metric_unit_follows_the_scale_of_the_inputs(qz, oracle, hyb):
         qz.set_viterbi_mode(0)
 
 
+@pytest.mark.parametrize("B", [1, 7, 8, 9, 100, 128, 129])
+def test_two_workgroups_per_tile_give_the_same_states(qz, pkg, B):
+    """Launches of up to 128 tiles are shared by pairs of workgroups: states, packed words and repeats against the
+    256-thread form; every pass repeated on fp64 metrics; and a pair that does not wait for its second half at all (the
+    first workgroup does the tile alone).  129 tiles take the form with one workgroup per tile."""
+    import torch
+    say("case: pairs of workgroups, B = %d" % B)
+    qz.set_tlut(None)
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    x = torch.randn(B, 256, device="cuda", generator=gen)
+    x[::3] = (x[::3] * 0.87).half().float()
+    if B > 7:
+        x[5] = 0.0                 # every path of a tie
+        x[6] = 1e30                # metrics that do not fit 32 bits
+        x[7] *= 6
+    torch.cuda.synchronize()
+    got = {}
+    try:
+        for name, mode, margin, patience in (("256", 2, 0, None), ("pair", 0, 0, 50000000), ("repeated", 0, 0xffffffff, 50000000),
+                                             ("alone", 0, 0, 0)):
+            say("  " + name)
+            qz.set_viterbi_mode(mode, margin)
+            if patience is not None:
+                qz.selftest_pair_patience(patience)
+            st = torch.zeros(B, 128, dtype=torch.int16, device="cuda")
+            pk = torch.zeros(B, 32, dtype=torch.int16, device="cuda")
+            torch.cuda.synchronize()
+            for _ in range(2):
+                qz.viterbi_tiles_dev(x, B, st, pk)
+            qz.synchronize()
+            got[name] = (st.cpu(), pk.cpu())
+    finally:
+        qz.set_viterbi_mode(0)
+        qz.selftest_pair_patience(50000000)
+    for name in ("pair", "repeated", "alone"):
+        same = (got[name][0] == got["256"][0]).all(1)
+        assert same.all(), "%s: tiles %s" % (name, torch.nonzero(~same).flatten()[:10].tolist())
+        assert torch.equal(got[name][1], got["256"][1]), name
+
+
 def test_wide_workgroups_give_the_same_states(qz, oracle, hyb):
     """A launch that cannot fill the chip gives every tile 512 threads instead of 256 (the 32-bit forward passes
     share the groups out over all of them; everything else, the fp64 repeat of a pass included, is done by both
