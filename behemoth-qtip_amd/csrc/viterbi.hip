@@ -51,7 +51,6 @@
 // threads per tile.
 #include <hip/hip_ext.h>
 
-#include <algorithm>
 #include <cstddef>
 #include <mutex>
 #include <type_traits>
@@ -1274,34 +1273,35 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
 // (to the second), the metrics at the middle of either pass (both ways), the states of the second half (to the first,
 // which writes all results).  A wait is bounded: a workgroup whose partner does not answer for `patience` ticks (it is
 // not resident, say) marks the pair, the second workgroup ends, and the first does this block and the rest alone.
-// Measured: 24 tiles 374 -> 250 us; 64 tile rows through 64 blocks (a lone 1024 x 1024 group, everything included) 24.7 ->
-// 16.9 ms.
-template <bool kFree>
+// Measured: 24 tiles by themselves 334 -> 191 us and more; 64 tile rows through 64 blocks (a lone 1024 x 1024 group,
+// everything included) 24.7 -> 15.1 ms; 384 tile rows through 256 blocks (6144 x 4096) 146 -> 122 ms.
+template <bool kFree, bool kWide>
 __device__ __forceinline__ void backward_pass32(Smem& sm, const double* __restrict__ entry_d, int roll, uint32_t ov,
                                                 uint32_t* __restrict__ hist, const Unit unit) {
   // A thread owns metric column c (the sixteen groups 16 c + e after the step; they continue the sixteen groups 256 h + c
-  // before it) with its mirror 255 - c, and the four h = 4 r + i: per j = 16 c + e the four table values of h serve group
-  // 256 h + c (with B[j]) and its mirror (with B[4095 - j]).  The table and the lanes' columns are the tail-biting
+  // before it) with its mirror 255 - c, and the four (256 threads: eight) h = kH r + i: per j = 16 c + e the table values
+  // of these h serve group 256 h + c (with B[j]) and its mirror (with B[4095 - j]).  The table and the lanes' columns are the tail-biting
   // forward pass's, so its reads are free of bank conflicts as there; metric j sits at m32_slot(j / 16, j mod 16), which
-  // makes the column reads conflict-free and leaves a four-way conflict in the eight writes per thread and step.
-  const int t = opaque_tid_wide();
+  // makes the column reads conflict-free and leaves a four-way conflict in the writes.
+  constexpr int kT = kWide ? 2 * kThreads : kThreads, kEnt = 1024 / kT, kH = kWide ? 4 : 8;
+  const int t = kWide ? opaque_tid_wide() : opaque_tid();
   const int p = t & 127, r = t >> 7;
   const int colA = 4 * (p & 31) + (p >> 5), colB = 255 - colA;
   uint32_t* const E32 = reinterpret_cast<uint32_t*>(sm.E);
   uint32_t* const M32 = reinterpret_cast<uint32_t*>(sm.M);
-  double2 ent[2];
+  double2 ent[kEnt];
   const double2* __restrict__ entries = reinterpret_cast<const double2*>(entry_d) + t;
 #pragma unroll
-  for (int q = 0; q < 2; ++q) ent[q] = entries[512 * q], ent[q].x *= unit.pre, ent[q].y *= unit.pre;
-  int ebase[16], wslot[4];
+  for (int q = 0; q < kEnt; ++q) ent[q] = entries[kT * q], ent[q].x *= unit.pre, ent[q].y *= unit.pre;
+  int ebase[16], wslot[kH];
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const uint32_t j = 16u * colA + uint32_t(e), pj = j * (j + 1u);
-    ebase[e] = int((((pj >> 12) + uint32_t(4 * r * (2 * (e & 7) + 1))) & 15u) * 64u + ((pj >> 6) & 63u));
+    ebase[e] = int((((pj >> 12) + uint32_t(kH * r * (2 * (e & 7) + 1))) & 15u) * 64u + ((pj >> 6) & 63u));
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int g = 256 * (4 * r + i) + colA;
+  for (int i = 0; i < kH; ++i) {
+    const int g = 256 * (kH * r + i) + colA;
     wslot[i] = m32_slot(g >> 4, g & 15);
   }
   const int xA = m32_pos(colA) * 64 + m32_swz(colA) * 4, xB = m32_pos(colB) * 64 + m32_swz(colB) * 4;  // bytes
@@ -1310,13 +1310,13 @@ __device__ __forceinline__ void backward_pass32(Smem& sm, const double* __restri
     const double x0 = double(sm.x[at]) * unit.pre, x1 = double(sm.x[at + 1]) * unit.pre;
     uint32_t* const Ew = E32 + par * kESlots + t;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < kEnt; ++q) {
       const uint32_t v = err_units(ent[q].x, ent[q].y, x0, x1);
-      Ew[512 * q] = v;
-      Ew[512 * q + 1024] = v;
+      Ew[kT * q] = v;
+      Ew[kT * q + 1024] = v;
     }
   };
-  for (int g = t; g < kGroups; g += 512) M32[m32_slot(g >> 4, g & 15)] = (kFree || uint32_t(g) == ov) ? 0u : kSat;
+  for (int g = t; g < kGroups; g += kT) M32[m32_slot(g >> 4, g & 15)] = (kFree || uint32_t(g) == ov) ? 0u : kSat;
   table(kSteps - 1, 0);
   __syncthreads();
   // step `it`: metrics and table of buffer par -> metrics of the other buffer, and the table of step it - 1
@@ -1334,37 +1334,39 @@ __device__ __forceinline__ void backward_pass32(Smem& sm, const double* __restri
       MB[4 * k] = b.x, MB[4 * k + 1] = b.y, MB[4 * k + 2] = b.z, MB[4 * k + 3] = b.w;
     }
     table(it - 1, par ^ 1);
-    uint32_t own[4] = {kSat, kSat, kSat, kSat}, mirror[4] = {kSat, kSat, kSat, kSat};
+    uint32_t own[kH], mirror[kH];
+#pragma unroll
+    for (int i = 0; i < kH; ++i) own[i] = mirror[i] = kSat;
 #pragma unroll
     for (int e = 0; e < 16; e += 2) {
-      uint32_t v0[4], v1[4];
+      uint32_t v0[kH], v1[kH];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < kH; ++i) {
         v0[i] = Er[ebase[e] + ((i * (2 * (e & 7) + 1)) & 15) * 64];
         v1[i] = Er[ebase[e + 1] + ((i * (2 * ((e + 1) & 7) + 1)) & 15) * 64];
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < kH; ++i) {
         own[i] = min3u(own[i], sat_add(v0[i], MA[e]), sat_add(v1[i], MA[e + 1]));
         mirror[i] = min3u(mirror[i], sat_add(v0[i], MB[15 - e]), sat_add(v1[i], MB[14 - e]));
       }
     }
     if (kFree && it == kSteps - 1) {  // final states of 32768 and more do not count: groups of 2048 and more (r: the same in a wave)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        own[i] = r >= 2 ? kSat : own[i];
-        mirror[i] = r >= 2 ? mirror[i] : kSat;
+      for (int i = 0; i < kH; ++i) {
+        own[i] = kH * r >= 8 ? kSat : own[i];
+        mirror[i] = kH * r >= 8 ? mirror[i] : kSat;
       }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kH; ++i) {
       Mw[wslot[i]] = own[i];
       Mw[wslot[i] ^ kMirror32] = mirror[i];
     }
     if (!kFree && par == 1 && it >= kSteps / 2 + 2) {
       uint32_t* const hs = hist + size_t((it - kSteps / 2 - 2) >> 1) * kGroups + t;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) hs[512 * i] = own[i], hs[512 * (4 + i)] = mirror[i];
+      for (int i = 0; i < kH; ++i) hs[kT * i] = own[i], hs[kT * (kH + i)] = mirror[i];
     }
     __syncthreads();
   };
@@ -1376,17 +1378,21 @@ __device__ __forceinline__ void backward_pass32(Smem& sm, const double* __restri
 }
 
 // place of group g in one kept step of the backward pass (the metrics B_66, B_68 .. B_126)
+template <bool kWide>
 __device__ __forceinline__ uint32_t back_index(uint32_t g) {
+  constexpr uint32_t kT = kWide ? 2 * kThreads : kThreads, kH = kWide ? 4 : 8;
   const bool m = (g & 255u) >= 128u;
   const uint32_t q = m ? 4095u - g : g, c = q & 255u, h = q >> 8;
-  return ((m ? 4u : 0u) + (h & 3u)) * 512u + (h >> 2) * 128u + ((c >> 2) | ((c & 3u) << 5));
+  return ((m ? kH : 0u) + (h & (kH - 1))) * kT + (h / kH) * 128u + ((c >> 2) | ((c & 3u) << 5));
 }
 
-// From group g entering step 64 to the group ov after step 127, two steps a round, in the scheme of trace_back32's streamed
-// form with the directions exchanged; records the states of steps 64 .. 127.  A candidate of step t is a sum of 128 - t
+// From group g entering step 64 to the group ov after step 127, two steps a round, in the scheme of trace_back32 (kWide:
+// its streamed form) with the directions exchanged; records the states of steps 64 .. 127.  A candidate of step t is a sum of 128 - t
 // rounded terms, and thr, which 128 terms need, shrinks by one unit per term less.
-__device__ __forceinline__ void trace_forward32(Smem& sm, const uint32_t* __restrict__ hist, uint32_t g, uint32_t ov,
-                                                uint32_t thr, uint32_t& flag, const uint32_t* tl, const Unit unit) {
+template <bool kWide>
+__device__ __forceinline__ void trace_forward32(Smem& sm, const double* __restrict__ entry_d, const uint32_t* __restrict__ hist,
+                                                uint32_t g, uint32_t ov, uint32_t thr, uint32_t& flag, const uint32_t* tl,
+                                                const Unit unit) {
   const uint32_t tid = uint32_t(opaque_tid());
   const uint32_t lane = tid & 63u, wave = tid >> 6, dp = lane & 15u, d = 4u * wave + (lane >> 4);
   constexpr int kBufs = 3, kLoads = kGroups / (4 * 2 * kThreads), kRows = 31;
@@ -1413,13 +1419,22 @@ __device__ __forceinline__ void trace_forward32(Smem& sm, const uint32_t* __rest
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  for (; issued < kBufs; ++issued) issue(issued);
-  landed(issued - 1);
-  lds_barrier();
-  auto err_of = [&](uint32_t st, int at) -> uint32_t {
-    const uint32_t e = ((st * (st + 1u)) >> 6) & 1023u, w = tl[e & 511u];
-    const uint16_t h0 = uint16_t((w & 0xffffu) ^ ((e >> 9) << 15)), h1 = uint16_t(w >> 16);
-    const double l0 = double(float(__builtin_bit_cast(_Float16, h0))), l1 = double(float(__builtin_bit_cast(_Float16, h1)));
+  if constexpr (kWide) {
+    for (; issued < kBufs; ++issued) issue(issued);
+    landed(issued - 1);
+    lds_barrier();
+  }
+  auto entry_of = [&](uint32_t st, double& l0, double& l1) {
+    const uint32_t e = ((st * (st + 1u)) >> 6) & 1023u;
+    if constexpr (kWide) {
+      const uint32_t w = tl[e & 511u];
+      const uint16_t h0 = uint16_t((w & 0xffffu) ^ ((e >> 9) << 15)), h1 = uint16_t(w >> 16);
+      l0 = double(float(__builtin_bit_cast(_Float16, h0))), l1 = double(float(__builtin_bit_cast(_Float16, h1)));
+    } else {
+      l0 = entry_d[2 * e], l1 = entry_d[2 * e + 1];
+    }
+  };
+  auto err_at = [&](double l0, double l1, int at) -> uint32_t {
     return err_units(l0 * unit.pre, l1 * unit.pre, double(sm.x[at]) * unit.pre, double(sm.x[at + 1]) * unit.pre);
   };
   int set = 0;
@@ -1428,14 +1443,25 @@ __device__ __forceinline__ void trace_forward32(Smem& sm, const uint32_t* __rest
     const uint32_t s1 = (g << 4) | d;                        // candidate state of step t
     const uint32_t s2 = ((s1 & 0xfffu) << 4) | dp;           // and of step t + 1
     const uint32_t g2 = s2 & 0xfffu;
-    const uint32_t kv = t < kSteps - 2 ? rows[(q % kBufs) * kGroups + back_index(g2)] : (g2 == ov ? 0u : kSat);
-    const uint32_t c1 = sat_add(err_of(s2, (2 * t + 2) & 255), kv);
+    double la0, la1, lb0, lb1;  // (the entries are asked for before the kept metric: see trace_back32)
+    entry_of(s2, la0, la1);
+    entry_of(s1, lb0, lb1);
+    uint32_t kv;
+    if constexpr (kWide) {
+      kv = t < kSteps - 2 ? rows[(q % kBufs) * kGroups + back_index<true>(g2)] : (g2 == ov ? 0u : kSat);
+    } else {
+      kv = g2 == ov ? 0u : kSat;
+      if (t < kSteps - 2)
+        kv = __hip_atomic_load(hist + size_t((t - kSteps / 2) / 2) * kGroups + back_index<false>(g2), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    const uint32_t c1 = sat_add(err_at(la0, la1, (2 * t + 2) & 255), kv);
     // over the 16 lanes of a row: the smallest value, the first lane that holds it, the gap to the runner-up
     const uint32_t low = row_min16_u32(c1);
     const uint32_t bits = uint32_t(__builtin_amdgcn_ballot_w64(c1 == low) >> (lane & 48u)) & 0xffffu;
     const uint32_t k1 = bits ? uint32_t(__builtin_ctz(bits)) : 0u;
     const uint32_t gap1 = row_min16_u32(dp == k1 ? kSat : c1) - low;
-    const uint32_t c0 = sat_add(err_of(s1, (2 * t) & 255), low);
+    const uint32_t c0 = sat_add(err_at(lb0, lb1, (2 * t) & 255), low);
     uint32_t bc = uint32_t(__builtin_amdgcn_readlane(int(c0), 0)), sc = kSat, bd = 4u * wave;
     uint32_t bd1 = uint32_t(__builtin_amdgcn_readlane(int(k1), 0)), bg = uint32_t(__builtin_amdgcn_readlane(int(gap1), 0));
 #pragma unroll
@@ -1457,13 +1483,21 @@ __device__ __forceinline__ void trace_forward32(Smem& sm, const uint32_t* __rest
       sm.tr32[set][wave][3] = bg;
     }
     // the next row has landed here, then everywhere; nobody reads the present one after the barrier
-    landed(issued - 2 - q > 0 ? issued - 2 - q : 0);
-    lds_barrier();
-    if (issued < kRows) issue(issued++);
-    ++q;
+    if constexpr (kWide) {
+      landed(issued - 2 - q > 0 ? issued - 2 - q : 0);
+      lds_barrier();
+      if (issued < kRows) issue(issued++);
+      ++q;
+    } else {
+      __syncthreads();
+    }
     uint4 w4[4];
 #pragma unroll
     for (int w = 0; w < 4; ++w) w4[w] = *reinterpret_cast<const uint4*>(sm.tr32[set][w]);
+    // (all four read before the first is looked at: see trace_back32)
+    asm volatile("" : "+v"(w4[0].x), "+v"(w4[0].y), "+v"(w4[0].z), "+v"(w4[0].w), "+v"(w4[1].x), "+v"(w4[1].y),
+                 "+v"(w4[1].z), "+v"(w4[1].w), "+v"(w4[2].x), "+v"(w4[2].y), "+v"(w4[2].z), "+v"(w4[2].w), "+v"(w4[3].x),
+                 "+v"(w4[3].y), "+v"(w4[3].z), "+v"(w4[3].w));
     bc = w4[0].x, sc = w4[0].y, bg = w4[0].w;
     uint32_t bdd = w4[0].z;
 #pragma unroll
@@ -1500,15 +1534,16 @@ __global__ void pair_reset_kernel(double* __restrict__ hist_all, int slots) {
 
 // Workgroups b and b + 8 (bit 3 of the number) are a pair, 8 pairs per 16 workgroups: they are dealt to the XCDs in turn,
 // so that a pair shares one.  One tile row per pair.
-__global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob job, const double* __restrict__ entry_d,
-                                                                      const float* __restrict__ entry_f,
-                                                                      double* __restrict__ hist_all) {
+template <bool kWide>
+__global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) void viterbi_pair_kernel(
+    TileJob job, const double* __restrict__ entry_d, const float* __restrict__ entry_f, double* __restrict__ hist_all) {
+  constexpr int kT = kWide ? 2 * kThreads : kThreads;
   __shared__ Smem sm;
-  __shared__ uint32_t tl[512];
+  __shared__ uint32_t tl[kWide ? 512 : 1];
   const long tile = long(blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
   const bool second = (blockIdx.x >> 3) & 1;
   if (tile >= job.tiles) return;
-  {
+  if constexpr (kWide) {
     const int i = threadIdx.x;
     const uint32_t h0 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i]));
     const uint32_t h1 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i + 1]));
@@ -1516,6 +1551,12 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
     __syncthreads();
   }
   const int tid = threadIdx.x;
+  // the thread number anew wherever many addresses are made from it (see opaque_tid)
+  auto fresh = []() __attribute__((always_inline)) -> int {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+  };
   double* const hist = hist_all + size_t(blockIdx.x) * kSlotWords;
   uint32_t* const hist32 = reinterpret_cast<uint32_t*>(hist);
   PairArea* const mine = reinterpret_cast<PairArea*>(hist + kHistWordsPerTile);
@@ -1524,14 +1565,14 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
   uint32_t* const M32 = reinterpret_cast<uint32_t*>(sm.M);
   uint32_t* const Mc32 = reinterpret_cast<uint32_t*>(sm.E) + 2 * (2 * 16 * 64 * 2);  // the free pass's compact metrics
   // everything this workgroup has put is where the other can get it before the flag says so
-  auto tell = [&](uint32_t v) {
+  auto tell = [&](uint32_t v) __attribute__((always_inline)) {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), every wave
     asm volatile("" ::: "memory");
     __syncthreads();
     if (tid == 0) pair_put(&mine->flag, v);
   };
   // false: the pair is given up
-  auto hear = [&](uint32_t v) -> bool {
+  auto hear = [&](uint32_t v) __attribute__((always_inline)) -> bool {
     if (tid == 0) {
       const unsigned long long t0 = wall_clock64();
       uint32_t res = 0;
@@ -1556,11 +1597,12 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
   };
   // best group and runner-up of M_64 + B_64; which: 0 free pass, 1 tail-biting pass
   uint32_t b1 = 0, b2 = 0, bj = 0;
-  auto middle = [&](int which) {
+  auto middle = [&](int which) __attribute__((always_inline)) {
     b1 = kSat, b2 = kSat, bj = 0;
+    const int me = fresh();
 #pragma unroll
-    for (int k = 0; k < kGroups / 512; ++k) {
-      const uint32_t g = uint32_t(tid) + 512u * uint32_t(k);
+    for (int k = 0; k < kGroups / kT; ++k) {
+      const uint32_t g = uint32_t(me + kT * k);
       const uint32_t low = which == 0 && g >= 2048u ? 4095u - g : g;
       uint32_t m;
       if (second) m = M32[m32_slot(int(g >> 4), int(g & 15u))];
@@ -1583,7 +1625,7 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
     __syncthreads();
     b1 = sm.red32[0][0], b2 = sm.red32[0][1], bj = sm.red32[0][2];
 #pragma unroll
-    for (int w = 1; w < 8; ++w) merge(sm.red32[w][0], sm.red32[w][1], sm.red32[w][2]);
+    for (int w = 1; w < kT / 64; ++w) merge(sm.red32[w][0], sm.red32[w][1], sm.red32[w][2]);
     __syncthreads();
   };
   auto unit_log2 = [&](float expected, float room) { return __builtin_amdgcn_readfirstlane(unit_log2_for(expected, room)); };
@@ -1595,8 +1637,8 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
       if (tid < kSeq) sm.x[tid] = __uint_as_float(pair_get(&other->x[tid]));
       __syncthreads();
       const int k1 = unit_log2(expected, 2.f);
-      backward_pass32<true>(sm, entry_d, kSeq / 2, 0u, nullptr, unit_of(k1));
-      for (int g = tid; g < kGroups; g += 512) pair_put(&mine->mid[0][g], M32[m32_slot(g >> 4, g & 15)]);
+      backward_pass32<true, kWide>(sm, entry_d, kSeq / 2, 0u, nullptr, unit_of(k1));
+      for (int g = fresh(); g < kGroups; g += kT) pair_put(&mine->mid[0][g], M32[m32_slot(g >> 4, g & 15)]);
       tell(n + 2);
       if (!hear(n + 2)) return;
       middle(0);
@@ -1610,13 +1652,13 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
       }
       ov = uint32_t(__builtin_amdgcn_readfirstlane(int(ov)));
       const Unit unit = unit_of(unit_log2(expected, 1.125f));
-      backward_pass32<false>(sm, entry_d, 0, ov, hist32, unit);
-      for (int g = tid; g < kGroups; g += 512) pair_put(&mine->mid[1][g], M32[m32_slot(g >> 4, g & 15)]);
+      backward_pass32<false, kWide>(sm, entry_d, 0, ov, hist32, unit);
+      for (int g = fresh(); g < kGroups; g += kT) pair_put(&mine->mid[1][g], M32[m32_slot(g >> 4, g & 15)]);
       tell(n + 4);
       if (!hear(n + 4)) return;
       middle(1);
       uint32_t flag = 0;
-      trace_forward32(sm, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), ov, job.margin, flag, tl, unit);
+      trace_forward32<kWide>(sm, entry_d, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), ov, job.margin, flag, tl, unit);
       if (tid < 64) pair_put(&mine->states[tid], sm.st[64 + tid]);
       if (tid == 0) pair_put(&mine->doubt, flag);
       tell(n + 5);
@@ -1631,18 +1673,18 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
     else tile_targets<float>(sm, job, col0, tile, job.prod32);
     __syncthreads();
     // the block's two passes together; false if the second workgroup is not there
-    auto together = [&]() -> bool {
+    auto together = [&]() __attribute__((always_inline)) -> bool {
       if (tid < kSeq) pair_put(&mine->x[tid], __float_as_uint(sm.x[tid]));
       tell(n + 1);
       const int k1 = unit_log2(expected, 2.f);
-      forward_pass32<true, true, true>(sm, entry_d, kSeq / 2, -1, hist32, kSteps, unit_of(k1));
-      for (int g = tid; g < kGroups / 2; g += 512) pair_put(&mine->mid[0][g], Mc32[m32c_slot(g & 255, g >> 8)]);
+      forward_pass32<true, kWide, true>(sm, entry_d, kSeq / 2, -1, hist32, kSteps, unit_of(k1));
+      for (int g = fresh(); g < kGroups / 2; g += kT) pair_put(&mine->mid[0][g], Mc32[m32c_slot(g & 255, g >> 8)]);
       tell(n + 2);
       if (!hear(n + 2)) return false;
       middle(0);
       if (b2 - b1 < job.margin || b1 >= kWinnerMax) {
         if (tid == 0 && job.stats) atomicAdd(job.stats, 1u);
-        block_passes<true>(sm, job, entry_d, hist, tl, expected, 0, 1, true);
+        block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 1, true);
         if (tid == 0) pair_put(&mine->overlap, uint32_t(sm.overlap)), pair_put(&mine->expected, __float_as_uint(expected));
         tell(n + 3);
       } else {
@@ -1652,21 +1694,21 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
       }
       const uint32_t ov = uint32_t(__builtin_amdgcn_readfirstlane(sm.overlap));
       const Unit unit = unit_of(unit_log2(expected, 1.125f));
-      forward_pass32<false, true, true>(sm, entry_d, 0, int(ov), hist32, 0, unit);
-      for (int g = tid; g < kGroups; g += 512) pair_put(&mine->mid[1][g], M32[m32_slot(g & 255, g >> 8)]);
+      forward_pass32<false, kWide, true>(sm, entry_d, 0, int(ov), hist32, 0, unit);
+      for (int g = fresh(); g < kGroups; g += kT) pair_put(&mine->mid[1][g], M32[m32_slot(g & 255, g >> 8)]);
       tell(n + 4);
       if (!hear(n + 4)) return false;
       middle(1);
       uint32_t flag = uint32_t(b2 - b1 < job.margin) | uint32_t(b1 >= kWinnerMax);
-      const uint32_t s = trace_back32<false, true>(sm, entry_d, hist32, 0, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), 2,
-                                                  true, job.margin, flag, tl, unit, kSteps / 2 - 1);
+      const uint32_t s = trace_back32<false, kWide>(sm, entry_d, hist32, 0, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), 2,
+                                                   true, job.margin, flag, tl, unit, kSteps / 2 - 1);
       // s is the state of step 1; at step 0 the one predecessor group with a finite initial metric is ov
       if (tid == 0) sm.st[0] = uint16_t((s >> 4) | ((ov >> 8) << 12));
       if (!hear(n + 5)) return false;
       flag |= uint32_t(__builtin_amdgcn_readfirstlane(int(pair_get(&other->doubt))));
       if (flag) {
         if (tid == 0 && job.stats) atomicAdd(job.stats + 1, 1u);
-        block_passes<true>(sm, job, entry_d, hist, tl, expected, 1, 2, true);
+        block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 1, 2, true);
       } else if (tid < 64) {
         sm.st[64 + tid] = uint16_t(pair_get(&other->states[tid]));
       }
@@ -1674,7 +1716,7 @@ __global__ __launch_bounds__(2 * kThreads, 1) void viterbi_pair_kernel(TileJob j
       return true;
     };
     if (!alone && !together()) alone = true;
-    if (alone) block_passes<true>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
+    if (alone) block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
     block_outputs(sm, job, entry_f, tile, blk, col0);
     __syncthreads();
   }
@@ -1717,12 +1759,12 @@ int viterbi_max_slots(int device) {
   return slots;
 }
 
-// compute units of the current device, at most what the reset kernel's one workgroup covers
+// compute units of the current device
 static long viterbi_device_cus() {
   int dev = 0, cus = 0;
   QTIP_HIP(hipGetDevice(&dev));
   QTIP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  return std::min(cus, 256);
+  return cus;
 }
 
 static int viterbi_device_slots() {
@@ -1751,17 +1793,22 @@ void launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const flo
   // the wide form where the launch leaves two thirds of the chip's workgroup slots empty anyway (and the 32-bit
   // passes, which are what it shares out over its 512 threads, are in use)
   const bool wide = job.mode == 0 && (job.wide > 0 || (job.wide < 0 && 3 * job.tiles <= viterbi_device_slots()));
-  // two workgroups per tile where every one of them then still has a compute unit to itself
+  // Two workgroups per tile while all of them are resident at once: of 512 threads where every one of them has a compute
+  // unit to itself, of 256 threads up to three per compute unit.  Pairs against one workgroup per tile, us: 64 tiles
+  // 200 against 345, 128 210 / 350; then 192 336 / 349, 256 339 / 358, 264 439 / 514, 384 446 / 520 (at 1.5 tiles per
+  // compute unit a launch waits for those that have two; halves are dealt out evenly).
   const long pair_grid = 16 * ((job.tiles + 7) / 8);
-  if (job.mode == 0 && job.wide < 0 && pair_grid <= slots && pair_grid <= viterbi_device_cus()) {
+  if (job.mode == 0 && job.wide < 0 && pair_grid <= slots && pair_grid <= viterbi_device_slots()) {
     double* const ws = static_cast<double*>(workspace);
-    pair_reset_kernel<<<dim3(1), dim3(256), 0, s>>>(ws, int(pair_grid));
+    const bool lone = pair_grid <= viterbi_device_cus();
+    const auto pair = lone ? viterbi_pair_kernel<true> : viterbi_pair_kernel<false>;
+    const dim3 threads(lone ? 2 * kThreads : kThreads);
+    pair_reset_kernel<<<dim3(unsigned((pair_grid + 255) / 256)), dim3(256), 0, s>>>(ws, int(pair_grid));
     QTIP_HIP(hipGetLastError());
     if (start || stop)
-      hipExtLaunchKernelGGL(viterbi_pair_kernel, dim3(unsigned(pair_grid)), dim3(2 * kThreads), 0, s, start, stop, 0, job,
-                            d_entry_d, d_entry_f, ws);
+      hipExtLaunchKernelGGL(pair, dim3(unsigned(pair_grid)), threads, 0, s, start, stop, 0, job, d_entry_d, d_entry_f, ws);
     else
-      viterbi_pair_kernel<<<dim3(unsigned(pair_grid)), dim3(2 * kThreads), 0, s>>>(job, d_entry_d, d_entry_f, ws);
+      pair<<<dim3(unsigned(pair_grid)), threads, 0, s>>>(job, d_entry_d, d_entry_f, ws);
     QTIP_HIP(hipGetLastError());
     return;
   }

@@ -242,11 +242,11 @@ def test_metric_unit_follows_the_scale_of_the_inputs(qz, oracle, hyb):
         qz.set_viterbi_mode(0)
 
 
-@pytest.mark.parametrize("B", [1, 7, 8, 9, 100, 128, 129])
+@pytest.mark.parametrize("B", [1, 7, 8, 9, 100, 128, 129, 300, 384, 385])
 def test_two_workgroups_per_tile_give_the_same_states(qz, pkg, B):
-    """Launches of up to 128 tiles are shared by pairs of workgroups: states, packed words and repeats against the
+    """Launches of up to 384 tiles are shared by pairs of workgroups (of 512 threads up to 128, of 256 above): states, packed words and repeats against the
     256-thread form; every pass repeated on fp64 metrics; and a pair that does not wait for its second half at all (the
-    first workgroup does the tile alone).  129 tiles take the form with one workgroup per tile."""
+    first workgroup does the tile alone).  385 tiles take the form with one workgroup per tile."""
     import torch
     say("case: pairs of workgroups, B = %d" % B)
     qz.set_tlut(None)
