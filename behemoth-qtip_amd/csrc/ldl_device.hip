@@ -1,7 +1,8 @@
 // The fp64 block LDL of the group quantizer and the Cholesky factorization of the NVFP4 calibration on the device, in
 // the order of operations of the host factorization (host_ldl.cpp, host_ldl_diag.cpp; reference
 // src/qtip_core.cpp:321-487): the factor is the host's bit for bit.  Right-looking panels of 256 columns, three
-// launches per panel on one stream and nothing that goes through the host:
+// launches per panel on one stream (two where the trailing matrix is large: its update brings the next diagonal block with
+// it) and nothing that goes through the host:
 //   ldl_diag_kernel          the 256 x 256 diagonal block (one workgroup)
 //   ldl_solve_kernel         the rows below it, and the panel's columns of L
 //   rank_update_lower_kernel the trailing matrix
@@ -12,7 +13,7 @@
 //
 // The form it replaced kept the panels on the host (3.3 GB of panel columns down and up per factorization at n = 28672,
 // the diagonal blocks on one core) and only updated here.  n = 1024 / 4096 / 12288 / 28672, rotated Hessian on the
-// device, L on the device and in page-locked host memory: 1.4 / 6.7 / 36.6 / 229 ms against 2.9 / 16.4 / 81 / 361 ms.
+// device, L on the device and in page-locked host memory: 1.4 / 6.7 / 36.4 / 216 ms against 2.9 / 16.4 / 81 / 361 ms.
 // The copy of L down, which the group calls do not ask for, is 0.1 / 1.2 / 11 / 60 ms of that.  A panel's diagonal block
 // takes 0.20 ms, its solve 0.08 ms (4096 rows), its update runs at 57 TFLOP/s of the card's 71 (a large fp64 product).
 #include <algorithm>
@@ -80,16 +81,10 @@ __device__ __forceinline__ void subtract_tile(const double4_t (&acc)[4][4], doub
 // beyond the last row read); those columns only feed outputs that are never stored.
 constexpr int UT = 128;
 constexpr int VK = 8, VSTAGES = 3;
-__global__ __launch_bounds__(256, 3) void rank_update_lower_kernel(const double* __restrict__ Xt, long ldx, int nr,
-                                                                     int kb, double* __restrict__ C, long ldc) {
-  // tile index t -> row bi with bi (bi + 1) / 2 <= t: the square root in fp32, then one step either way
-  const int tile = blockIdx.x;
-  int bi = int((__builtin_sqrtf(8.0f * float(tile) + 1.0f) - 1.0f) * 0.5f);
-  while (bi * (bi + 1) / 2 > tile) --bi;
-  while ((bi + 1) * (bi + 2) / 2 <= tile) ++bi;
-  const int bj = tile - bi * (bi + 1) / 2;
+using UpdateLds = double[VSTAGES][2][VK][UT];  // [stage][Xi | Xj][k][column], 48 KB
+__device__ __forceinline__ void update_tile(UpdateLds& S, const double* __restrict__ Xt, long ldx, int nr, int kb,
+                                            double* __restrict__ C, long ldc, int bi, int bj) {
   const int i0 = bi * UT, j0 = bj * UT;
-  __shared__ __attribute__((aligned(16))) double S[VSTAGES][2][VK][UT];  // [stage][Xi | Xj][k][column]
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave >> 1, wn = wave & 1;
   double4_t acc[4][4];
 #pragma unroll
@@ -232,10 +227,9 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
   return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
 }
 
-__global__ __launch_bounds__(256, 3) void ldl_diag_kernel(double* __restrict__ A, long ld, int kb,
-                                                          double* __restrict__ rdiag, double* __restrict__ inv,
-                                                          int* __restrict__ bad) {
-  __shared__ __attribute__((aligned(16))) double P[kSub][kDiag];  // [column of the sub-panel][row of the block]
+using DiagLds = double[kSub][kDiag];  // [column of the sub-panel][row of the block], 32 KB
+__device__ __forceinline__ void factor_diag_block(DiagLds& P, double* __restrict__ A, long ld, int kb,
+                                                  double* __restrict__ rdiag, double* __restrict__ inv, int* __restrict__ bad) {
   const int t = threadIdx.x, lane = t & 63, l16 = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   bool ok = true;
@@ -371,6 +365,52 @@ __global__ __launch_bounds__(256, 3) void ldl_diag_kernel(double* __restrict__ A
       V[i] = s / row[i];
       inv[long(b0 + i) * 16 + cc] = V[i];
     }
+  }
+}
+
+__global__ __launch_bounds__(256, 3) void ldl_diag_kernel(double* __restrict__ A, long ld, int kb,
+                                                          double* __restrict__ rdiag, double* __restrict__ inv,
+                                                          int* __restrict__ bad) {
+  __shared__ __attribute__((aligned(16))) DiagLds P;
+  factor_diag_block(P, A, ld, kb, rdiag, inv, bad);
+}
+
+__device__ __forceinline__ void triangle_tile(int tile, int& bi, int& bj) {
+  // row bi with bi (bi + 1) / 2 <= tile: the square root in fp32, then one step either way
+  bi = int((__builtin_sqrtf(8.0f * float(tile) + 1.0f) - 1.0f) * 0.5f);
+  while (bi * (bi + 1) / 2 > tile) --bi;
+  while ((bi + 1) * (bi + 2) / 2 <= tile) ++bi;
+  bj = tile - bi * (bi + 1) / 2;
+}
+__global__ __launch_bounds__(256, 3) void rank_update_lower_kernel(const double* __restrict__ Xt, long ldx, int nr,
+                                                                     int kb, double* __restrict__ C, long ldc) {
+  __shared__ __attribute__((aligned(16))) UpdateLds S;
+  int bi, bj;
+  triangle_tile(blockIdx.x, bi, bj);
+  update_tile(S, Xt, ldx, nr, kb, C, ldc, bi, bj);
+}
+// The update of a large trailing matrix with the next panel's diagonal block: the first workgroup updates the three tiles
+// of the leading 256 x 256 block and factors it while the others update the rest.  Two launches a panel instead of three
+// with the diagonal block's 0.2 ms under the update - and, beside the quantization of another group, whose Viterbi
+// workgroups fill the chip, a launch waits some milliseconds for their places, so the launches are what the factorization
+// takes there (12288 x 28672 groups in a row: 1.34 -> 1.28 s a factorization; alone at n = 28672 229 -> 216 ms).
+__global__ __launch_bounds__(256, 3) void rank_update_next_diag_kernel(const double* __restrict__ Xt, long ldx, int nr, int kb,
+                                                                       double* __restrict__ C, long ldc,
+                                                                       double* __restrict__ rdiag, double* __restrict__ inv,
+                                                                       int* __restrict__ bad) {
+  __shared__ __attribute__((aligned(16))) UpdateLds S;
+  if (blockIdx.x == 0) {
+#pragma nounroll
+    for (int tile = 0; tile < 3; ++tile) {
+      update_tile(S, Xt, ldx, nr, kb, C, ldc, tile > 0, tile > 1);
+      __syncthreads();  // the next tile's operands take the place of this one's, and the block is whole after the last
+    }
+    static_assert(sizeof(DiagLds) <= sizeof(UpdateLds) && kDiag == 2 * UT);
+    factor_diag_block(*reinterpret_cast<DiagLds*>(&S), C, ldc, kDiag, rdiag, inv, bad);
+  } else {
+    int bi, bj;
+    triangle_tile(blockIdx.x + 2, bi, bj);
+    update_tile(S, Xt, ldx, nr, kb, C, ldc, bi, bj);
   }
 }
 
@@ -549,13 +589,18 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s) {
   int bad = 0;
   QTIP_HIP(hipMemcpyAsync(c->ldl_bad.p, &bad, sizeof bad, hipMemcpyHostToDevice, s));
   QTIP_HIP(hipMemsetAsync(L, 0, size_t(n) * n * sizeof(float), s));
-  for (long k = 0; k < n; k += kDiag) {
+  bool diag_done = false;  // this panel's diagonal block came with the update before it
+  int turn = 0;            // the reciprocals and inverses of a panel and of the one factored beside its update
+  for (long k = 0; k < n; k += kDiag, turn ^= 1) {
     const int kb = int(std::min<long>(kDiag, n - k));
     const long nr = n - k - kb;
     double* const D = c->ldl_A.p + k * n + k;
-    double *const rdiag = c->ldl_diag.p, *const inv = rdiag + kDiag;
-    ldl_diag_kernel<<<dim3(1), dim3(256), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_bad.p);
-    QTIP_HIP(hipGetLastError());
+    const size_t set = size_t(kDiag) * 17;
+    double *const rdiag = c->ldl_diag.p + turn * set, *const inv = rdiag + kDiag;
+    if (!diag_done) {
+      ldl_diag_kernel<<<dim3(1), dim3(256), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_bad.p);
+      QTIP_HIP(hipGetLastError());
+    }
     const dim3 grid(unsigned((kb + nr) / 16));
     if (dw)
       ldl_solve_kernel<true><<<grid, dim3(64), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_Xt.p, nr, L + k * n + k, n, dw + k, c->ldl_bad.p);
@@ -568,8 +613,17 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s) {
     // up to the end of the last tile row's 128 columns in every row of Xt
     QTIP_REQUIRE(kb % VK == 0 && nr % 4 == 0 && size_t(kb - 1) * nr + size_t(nt) * UT <= c->ldl_Xt.n,
                  "LDL update: operand shape the kernel does not cover (kb = %d, nr = %ld)", kb, nr);
-    rank_update_lower_kernel<<<dim3(unsigned(nt * (nt + 1) / 2)), dim3(256), 0, s>>>(
-        c->ldl_Xt.p, nr, int(nr), kb, c->ldl_A.p + (k + kb) * n + k + kb, n);
+    double* const C = c->ldl_A.p + (k + kb) * n + k + kb;
+    // three tiles in a row and a diagonal block take one workgroup 0.28 ms, a diagonal block by itself 0.20 ms after the
+    // update: even at about 6000 rows (1176 tiles, 0.1 ms), all of the 0.2 ms hidden from 12000 rows on
+    diag_done = nr >= 6144;
+    if (diag_done) {
+      double* const next = c->ldl_diag.p + (turn ^ 1) * set;
+      rank_update_next_diag_kernel<<<dim3(unsigned(nt * (nt + 1) / 2 - 2)), dim3(256), 0, s>>>(
+          c->ldl_Xt.p, nr, int(nr), kb, C, n, next, next + kDiag, c->ldl_bad.p);
+    } else {
+      rank_update_lower_kernel<<<dim3(unsigned(nt * (nt + 1) / 2)), dim3(256), 0, s>>>(c->ldl_Xt.p, nr, int(nr), kb, C, n);
+    }
     QTIP_HIP(hipGetLastError());
   }
   QTIP_HIP(hipMemcpyAsync(&bad, c->ldl_bad.p, sizeof bad, hipMemcpyDeviceToHost, s));
@@ -581,7 +635,7 @@ hipStream_t factor_stream(qtip_ctx* c, long n) {
   if (!c->ldl_stream) QTIP_HIP(hipStreamCreateWithFlags(&c->ldl_stream, hipStreamNonBlocking));
   c->ldl_A.ensure(size_t(n) * n);
   c->ldl_Xt.ensure(size_t(n) * kDiag);
-  c->ldl_diag.ensure(size_t(kDiag) + size_t(kDiag) * 16);
+  c->ldl_diag.ensure(2 * size_t(kDiag) * 17);
   return c->ldl_stream;
 }
 

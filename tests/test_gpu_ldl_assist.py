@@ -21,10 +21,11 @@ def spd(n, seed, rows=None):
     return H
 
 
-@pytest.mark.parametrize("n", [16, 496, 512, 1024, 1040, 1152, 2560])
+# 6656: trailing matrices on both sides of the 6144 rows from which an update brings the next diagonal block with it
+@pytest.mark.parametrize("n", [16, 496, 512, 1024, 1040, 1152, 2560, 6656])
 def test_factor_equals_host_factor(qz, pkg, n):
     say("case: LDL with device updates, n = %d" % n)
-    H = spd(n, 100 + n)
+    H = spd(n, 100 + n, rows=None if n < 4096 else n + 512)
     a = pkg.HessPrep(n=n, HRr=H.copy())
     b = pkg.HessPrep(n=n, HRr=H.copy())
     pkg.Quantizer.ldl_hessian(a, threads=16)
