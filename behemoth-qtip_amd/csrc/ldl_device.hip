@@ -13,10 +13,12 @@
 //
 // The form it replaced kept the panels on the host (3.3 GB of panel columns down and up per factorization at n = 28672,
 // the diagonal blocks on one core) and only updated here.  n = 1024 / 4096 / 12288 / 28672, rotated Hessian on the
-// device, L on the device and in page-locked host memory: 1.4 / 6.7 / 36.4 / 216 ms against 2.9 / 16.4 / 81 / 361 ms.
-// The copy of L down, which the group calls do not ask for, is 0.1 / 1.2 / 11 / 60 ms of that.  A panel's diagonal block
+// device, L on the device and in page-locked host memory: 1.5 / 5.8 / 26.2 / 161 ms against 2.9 / 16.4 / 81 / 361 ms.
+// The copy of L down, which the group calls do not ask for, runs beside it.  A panel's diagonal block
 // takes 0.20 ms, its solve 0.08 ms (4096 rows), its update runs at 57 TFLOP/s of the card's 71 (a large fp64 product).
 #include <algorithm>
+#include <utility>
+#include <vector>
 
 #include "quantizer_impl.hpp"
 
@@ -393,7 +395,7 @@ __global__ __launch_bounds__(256, 3) void rank_update_lower_kernel(const double*
 // of the leading 256 x 256 block and factors it while the others update the rest.  Two launches a panel instead of three
 // with the diagonal block's 0.2 ms under the update - and, beside the quantization of another group, whose Viterbi
 // workgroups fill the chip, a launch waits some milliseconds for their places, so the launches are what the factorization
-// takes there (12288 x 28672 groups in a row: 1.34 -> 1.28 s a factorization; alone at n = 28672 229 -> 216 ms).
+// takes there (12288 x 28672 groups in a row: 1.34 -> 1.28 s a factorization; alone at n = 28672 169 -> 156 ms).
 __global__ __launch_bounds__(256, 3) void rank_update_next_diag_kernel(const double* __restrict__ Xt, long ldx, int nr, int kb,
                                                                        double* __restrict__ C, long ldc,
                                                                        double* __restrict__ rdiag, double* __restrict__ inv,
@@ -583,8 +585,19 @@ __global__ void add_to_diagonal_kernel(double* __restrict__ A, long n, double v)
 namespace {
 // Factors the symmetric matrix whose lower triangle lies in c->ldl_A (n x n) on stream s.  L (n x n fp32, device)
 // receives the block LDL's factor, or with dw the scalar one's; everything outside its strict (block) lower triangle is
-// zero.  Waits for the stream; false if the matrix is not positive definite.
-bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s) {
+// zero.  host_L (optional) receives L as well: the rows of a panel's diagonal block are final once the panel is solved, and
+// go down from a stream of their own, 1024 at a time, while the factorization runs on (n = 28672 into pageable memory:
+// host buffers in and out 0.59 -> 0.44 s, page-locked L alone 216 -> 161 ms).  Waits for the stream; false if the matrix is not positive definite.
+bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s, float* host_L = nullptr) {
+  struct RowsDown {  // whatever ends the call, nothing of it is left behind
+    hipStream_t stream = nullptr;
+    std::vector<std::pair<long, hipEvent_t>> ready;  // (rows final, after this event)
+    ~RowsDown() {
+      if (stream) (void)hipStreamSynchronize(stream), (void)hipStreamDestroy(stream);
+      for (auto& r : ready) (void)hipEventDestroy(r.second);
+    }
+  } down;
+  if (host_L) QTIP_HIP(hipStreamCreateWithFlags(&down.stream, hipStreamNonBlocking));
   c->ldl_bad.ensure(1);
   int bad = 0;
   QTIP_HIP(hipMemcpyAsync(c->ldl_bad.p, &bad, sizeof bad, hipMemcpyHostToDevice, s));
@@ -607,6 +620,12 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s) {
     else
       ldl_solve_kernel<false><<<grid, dim3(64), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_Xt.p, nr, L + k * n + k, n, nullptr, c->ldl_bad.p);
     QTIP_HIP(hipGetLastError());
+    if (host_L && (nr <= 0 || (k + kb) % 1024 == 0)) {
+      hipEvent_t e;
+      QTIP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      down.ready.emplace_back(k + kb, e);
+      QTIP_HIP(hipEventRecord(e, s));
+    }
     if (nr <= 0) break;
     const long nt = (nr + UT - 1) / UT;
     // what the update kernel assumes: whole stages of 8 panel columns, 16-byte aligned rows of Xt, and readable memory
@@ -626,6 +645,14 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s) {
     }
     QTIP_HIP(hipGetLastError());
   }
+  long row = 0;
+  for (const auto& r : down.ready) {
+    QTIP_HIP(hipEventSynchronize(r.second));
+    QTIP_HIP(hipMemcpyAsync(host_L + size_t(row) * n, L + size_t(row) * n, size_t(r.first - row) * n * sizeof(float),
+                            hipMemcpyDeviceToHost, down.stream));
+    row = r.first;
+  }
+  if (host_L) QTIP_HIP(hipStreamSynchronize(down.stream));
   QTIP_HIP(hipMemcpyAsync(&bad, c->ldl_bad.p, sizeof bad, hipMemcpyDeviceToHost, s));
   QTIP_HIP(hipStreamSynchronize(s));
   return bad == 0;
@@ -647,8 +674,9 @@ struct Settle {
 }  // namespace
 
 // The Hessian preparation of the calibrated NVFP4 quantizer (nvfp4_prepare_host) on the device: the same chains, hence
-// the same L and dw bit for bit.  dev_L (n x n), dev_dw: device buffers of the caller.
-void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw) {
+// the same L and dw bit for bit.  dev_L (n x n), dev_dw: device buffers of the caller; host_L: optional.
+void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw,
+                               float* host_L) {
   QTIP_REQUIRE(c && host_H && dev_L && dev_dw && n > 0 && n % 16 == 0, "nvfp4_prepare (device): bad arguments (n = %d)", n);
   QTIP_REQUIRE(n <= 65535, "nvfp4_prepare (device): n = %d is beyond one grid dimension", n);
   double dsum = 0;
@@ -662,7 +690,7 @@ void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double s
   QTIP_HIP(hipGetLastError());
   add_to_diagonal_kernel<<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, s>>>(c->ldl_A.p, n, creg);
   QTIP_HIP(hipGetLastError());
-  if (!factor_on_device(c, n, dev_L, dev_dw, s)) throw Error(QTIP_E_NOT_PD, "NVFP4 calibration: Hessian not positive definite");
+  if (!factor_on_device(c, n, dev_L, dev_dw, s, host_L)) throw Error(QTIP_E_NOT_PD, "NVFP4 calibration: Hessian not positive definite");
 }
 
 // The block LDL of the rotated Hessian: dev_HRr, or host_HRr if that is null.  L goes to host_L, to dev_L (n x n device
@@ -683,11 +711,7 @@ void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* h
                                                                                               c->ldl_A.p);
   QTIP_HIP(hipGetLastError());
   float* const L = dev_L ? dev_L : own.p;
-  if (!factor_on_device(c, n, L, nullptr, s)) throw Error(QTIP_E_NOT_PD, "block LDL failed (H not PD)");
-  if (host_L) {
-    QTIP_HIP(hipMemcpyAsync(host_L, L, nn * 4, hipMemcpyDeviceToHost, s));
-    QTIP_HIP(hipStreamSynchronize(s));
-  }
+  if (!factor_on_device(c, n, L, nullptr, s, host_L)) throw Error(QTIP_E_NOT_PD, "block LDL failed (H not PD)");
 }
 
 }  // namespace qtipmi

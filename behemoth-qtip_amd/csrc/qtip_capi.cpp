@@ -653,8 +653,7 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
     QTIP_REQUIRE(host_H && host_L && host_dw && n > 0 && n % 16 == 0, "nvfp4_prepare (device): bad arguments (n = %d)", n);
     const size_t nn = size_t(n) * n;
     DBuf<float> L(nn), dw(static_cast<size_t>(n));
-    nvfp4_prepare_device_impl(ctx, host_H, n, sigma_reg, L.p, dw.p);
-    QTIP_HIP(hipMemcpyAsync(host_L, L.p, nn * 4, hipMemcpyDeviceToHost, ctx->stream));
+    nvfp4_prepare_device_impl(ctx, host_H, n, sigma_reg, L.p, dw.p, host_L);
     QTIP_HIP(hipMemcpyAsync(host_dw, dw.p, size_t(n) * 4, hipMemcpyDeviceToHost, ctx->stream));
     QTIP_HIP(hipStreamSynchronize(ctx->stream));
   });

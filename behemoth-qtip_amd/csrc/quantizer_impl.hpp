@@ -71,7 +71,8 @@ void rotate_hessian_impl(qtip_ctx* c, const float* H, bool on_device, int n, uin
                          float* host_su, double* creg, float* host_HRr, float* dev_HRr = nullptr);
 void ldl_hessian_impl(const float* host_HRr, int n, int threads, float* host_L);
 void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* host_L, const float* dev_HRr, float* dev_L);
-void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw);
+void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw,
+                               float* host_L = nullptr);
 void ldlq_impl(qtip_ctx* c, const float* dWT, const float* dL, long n, long m, float* d_hatWT, uint16_t* dQ,
                int feedback, double* vit_seconds, int chains);
 int ldlq_default_chains(qtip_ctx* c);  // what chains = 0 stands for in this context (decided on the first call)

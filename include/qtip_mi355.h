@@ -296,7 +296,8 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
 /* Several groups through one context with the overlap of run_qtip_groups, src/pipeline.cpp:229-312: Hessians are
  * rotated on the GPU ahead of use, a side thread runs the fp64 LDL of the groups in order, and group g is
  * quantized as soon as its factor is ready (the LDL of group g+1 overlaps the GPU work of group g).  HRr and L live
- * in page-locked staging buffers owned by the context (a ring of three pairs, 6 n^2 floats, kept between calls).
+ * on the device (a ring of three pairs, 6 n^2 floats, kept between calls), or with ldl_device_updates = 0 in page-locked
+ * staging buffers owned by the context, as many.
  * timings / ldl_wait_s (seconds the GPU side waited for each group's factor) may be NULL.  On an error the
  * groups before the failing one are complete.
  * Groups too small to fill the chip run side by side (qtip_opts.group_lanes: group g on lane g mod lanes, each lane
