@@ -119,6 +119,7 @@ def lib():
     L.qtip_rotate_hessian.argtypes = [vp, vp, i, i, u64, d, vp, C.POINTER(d), vp]
     L.qtip_ldl_hessian.argtypes = [vp, i, i, vp]
     L.qtip_selftest_pair_patience.argtypes = [vp, C.c_ulonglong]
+    L.qtip_selftest_upload_beside_factorization.argtypes = [vp, d, C.POINTER(d)]
     L.qtip_ldl_hessian_device_updates.argtypes = [vp, vp, i, i, vp]
     L.qtip_selftest_ldl_panel_handover.argtypes = [vp, i, i, vp]
     L.qtip_ldl_hessian_device_updates_dev.argtypes = [vp, vp, i, i, vp, vp]
@@ -309,6 +310,12 @@ class Quantizer:
     def selftest_pair_patience(self, ticks):
         """Ticks of 10 ns for which the workgroups of a pair wait for each other (same results whatever it is)."""
         _check(lib().qtip_selftest_pair_patience(self._h, ticks))
+
+    def selftest_upload_beside_factorization(self, busy_us):
+        """Microseconds 1 MB takes on the upload stream behind a wave that sleeps busy_us on the factorization's stream."""
+        us = C.c_double()
+        _check(lib().qtip_selftest_upload_beside_factorization(self._h, busy_us, C.byref(us)))
+        return us.value
 
     def device_lut(self):
         """Device address of the 65536-entry fp16-pair table (device_lut(), src/quantizer.cpp:14-28)."""

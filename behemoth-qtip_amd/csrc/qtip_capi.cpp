@@ -116,24 +116,24 @@ void find_side_streams(qtip_ctx* c) {
   std::vector<hipStream_t> kept, dropped;
   hipStream_t upload = nullptr;
   try {
-    // a delay on the context's stream, on the first `count` streams kept and on cand, all queued at once: microseconds
-    auto side_by_side_us = [&](size_t count, hipStream_t cand) {
+    // a delay on the context's stream, on `others` and on cand, all queued at once: microseconds
+    auto side_by_side_us = [&](const std::vector<hipStream_t>& others, hipStream_t cand) {
       auto wait_all = [&] {
         QTIP_HIP(hipStreamSynchronize(c->stream));
-        for (size_t i = 0; i < count; ++i) QTIP_HIP(hipStreamSynchronize(kept[i]));
+        for (hipStream_t o : others) QTIP_HIP(hipStreamSynchronize(o));
         QTIP_HIP(hipStreamSynchronize(cand));
       };
       wait_all();
       const auto t0 = std::chrono::steady_clock::now();
       launch_delay(kDelayUs, c->stream);
-      for (size_t i = 0; i < count; ++i) launch_delay(kDelayUs, kept[i]);
+      for (hipStream_t o : others) launch_delay(kDelayUs, o);
       launch_delay(kDelayUs, cand);
       wait_all();
       return std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
     };
-    auto beside = [&](size_t count, hipStream_t cand) {
+    auto beside = [&](const std::vector<hipStream_t>& others, hipStream_t cand) {
       for (int attempt = 0; attempt < 3; ++attempt)  // the first launch on a stream also sets its queue up
-        if (side_by_side_us(count, cand) < 1.5 * kDelayUs) return true;
+        if (side_by_side_us(others, cand) < 1.5 * kDelayUs) return true;
       return false;
     };
     launch_delay(1.0, c->stream);  // the kernel's code is on the device before anything is timed
@@ -142,17 +142,20 @@ void find_side_streams(qtip_ctx* c) {
       hipStream_t s = nullptr;
       QTIP_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
       dropped.push_back(s);  // until shown otherwise
-      if (beside(kept.size(), s)) {
+      if (beside(kept, s)) {
         dropped.pop_back();
         kept.push_back(s);
       }
     }
-    // The stream that brings host inputs up needs no queue of its own, but it had better share the factorization's,
-    // which has time to spare, than a chain's: a candidate that runs beside the context's stream and the two chain
-    // streams shares the third stream's queue or none of these four.
-    if (kept.size() == 3) {
+    // The stream that brings host inputs up needs no queue of its own, but it must not share the factorization's: a
+    // whole factorization is queued at once, and a copy waits for all of it.  A chain's queue is a few launches deep.
+    // Twelve 12288 x 28672 groups from host memory: an upload 1.62 s in the factorization's queue, more than a group
+    // takes, and 0.16 s in a chain's; 212 and 235 Mweights/s (237 from device memory).
+    if (kept.size() >= 2) {
+      std::vector<hipStream_t> others{kept.back()};  // the factorization's; of the chains one may share
+      if (kept.size() == 3) others.push_back(kept[0]);
       for (size_t i = 0; i < dropped.size() && !upload; ++i)
-        if (beside(2, dropped[i])) {
+        if (beside(others, dropped[i])) {
           upload = dropped[i];
           dropped.erase(dropped.begin() + long(i));
         }
@@ -160,7 +163,7 @@ void find_side_streams(qtip_ctx* c) {
         hipStream_t s = nullptr;
         QTIP_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
         dropped.push_back(s);  // until shown otherwise
-        if (beside(2, s)) {
+        if (beside(others, s)) {
           dropped.pop_back();
           upload = s;
         }
@@ -445,6 +448,27 @@ int qtip_selftest_pair_patience(qtip_ctx* ctx, unsigned long long ticks) {
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr, "null context");
     ctx->vit_pair_patience = ticks;
+  });
+}
+
+int qtip_selftest_upload_beside_factorization(qtip_ctx* ctx, double busy_us, double* upload_us) {
+  return guarded([&] {
+    QTIP_REQUIRE(ctx != nullptr && upload_us != nullptr && busy_us >= 0 && busy_us <= 1e6, "selftest: bad arguments");
+    DeviceGuard g(ctx);
+    QTIP_REQUIRE(ctx->ldl_stream && ctx->upload_stream, "this context found no streams that run beside each other");
+    const size_t bytes = size_t(1) << 20;
+    std::vector<uint8_t> host(bytes, 1);
+    DBuf<uint8_t> dev(bytes);
+    auto upload = [&] {
+      const auto t0 = std::chrono::steady_clock::now();
+      QTIP_HIP(hipMemcpyAsync(dev.p, host.data(), bytes, hipMemcpyHostToDevice, ctx->upload_stream));
+      QTIP_HIP(hipStreamSynchronize(ctx->upload_stream));
+      return std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
+    };
+    upload();  // the first copy also sets the stream up
+    launch_delay(busy_us, ctx->ldl_stream);
+    *upload_us = upload();
+    QTIP_HIP(hipStreamSynchronize(ctx->ldl_stream));
   });
 }
 

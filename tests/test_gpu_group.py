@@ -295,6 +295,15 @@ def test_default_chain_count(qz):
     assert n in (2, 3)
 
 
+def test_uploads_do_not_wait_for_a_factorization(qz):
+    """run_groups' host inputs come up while the next group's factorization is queued as a whole: the upload stream must
+    not share its hardware queue (a copy would take the 80 ms and more)."""
+    say("case: an upload beside the factorization's stream")
+    us = min(qz.selftest_upload_beside_factorization(80e3) for _ in range(3))
+    say("  1 MB in %.0f us" % us)
+    assert us < 20e3
+
+
 def test_ldlq_chains_give_the_same_codes(qz, oracle, pkg, hyb):
     """The tile rows of a group are dealt to 1, 2 or 3 independent chains of launches (streams of their own, feedback
     slabs of their own, ragged shares of rows with two linears of different height): every packed word, Wscale and
