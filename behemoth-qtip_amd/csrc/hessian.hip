@@ -250,12 +250,13 @@ __global__ __launch_bounds__(256, 1) void syrk_img_kernel(const uint16_t* __rest
 // of its loads and by what a stage costs beside its MFMAs.  Same sums in the same order as the kernel above.
 constexpr int kSmallTile = 128, kHalfU16 = kSmallTile * IK, kSmallStages = 8;
 constexpr size_t kSmallLdsBytes = size_t(kSmallStages) * 2 * kHalfU16 * 2;  // 128 KB
-// this wave's loads have landed but for those of the last `stages` stages requested, two each (loads return in order)
+// this wave's loads have landed but for those of the last `stages` stages requested, two each (loads return in order), and
+// its reads of the stage in use have returned: vmcnt(2 stages) lgkmcnt(0)
 __device__ __forceinline__ void wait_all_but(int stages) {
-#define QTIP_WAIT(N) case N: __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * N)); break;
+#define QTIP_WAIT(N) case N: __builtin_amdgcn_s_waitcnt(0x0070 | (2 * N)); break;
   switch (stages) {
     QTIP_WAIT(1) QTIP_WAIT(2) QTIP_WAIT(3) QTIP_WAIT(4) QTIP_WAIT(5) QTIP_WAIT(6)
-    default: __builtin_amdgcn_s_waitcnt(0x0F70);
+    default: __builtin_amdgcn_s_waitcnt(0x0070);
   }
 #undef QTIP_WAIT
 }
