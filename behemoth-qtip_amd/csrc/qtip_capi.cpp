@@ -579,13 +579,22 @@ int qtip_dequantize_linear(qtip_ctx* ctx, const uint16_t* host_trellis, const ui
     DeviceGuard g(ctx);
     hipStream_t s = ctx->stream;
     const size_t words = size_t(m / 16) * (n / 16) * 32;
+    // the result is formed in the caller's device buffer where that is this device's own memory; a peer's, or a host
+    // buffer the device can see, gets a copy of it (these kernels may not be able to reach it, or only over the bus)
+    hipPointerAttribute_t at{};
+    bool in_place = false;
+    if (hatW_on_device) {
+      const hipError_t known = hipPointerGetAttributes(&at, hatW);
+      if (known != hipSuccess) (void)hipGetLastError();
+      in_place = known == hipSuccess && at.type == hipMemoryTypeDevice && at.device == ctx->device;
+    }
     // the call's buffers stay in the context's arena: two hipMalloc and hipFree of 4 m n bytes per call (the frees wait
     // for the whole device) cost more than the kernels (12288 x 12288: 33 ms a call in a
     // row of calls, of which 4 were the kernels and the copy; now 2.4, of which the pageable copy of the words is 1.3)
     ArenaScope memory(&ctx->arena);
     DBuf<uint16_t> tr(words);
-    DBuf<float> a(size_t(n) * m), own(hatW_on_device ? 0 : size_t(m) * n), d_su(n), d_sv(m);
-    float* const b = hatW_on_device ? hatW : own.p;
+    DBuf<float> a(size_t(n) * m), own(in_place ? 0 : size_t(m) * n), d_su(n), d_sv(m);
+    float* const b = in_place ? hatW : own.p;
     std::vector<float> su(n);
     for (int i = 0; i < n; ++i) su[i] = bf16_to_f32(host_su_bf16[i]);
     QTIP_HIP(hipMemcpyAsync(tr, host_trellis, words * 2, hipMemcpyHostToDevice, s));
@@ -598,7 +607,8 @@ int qtip_dequantize_linear(qtip_ctx* ctx, const uint16_t* host_trellis, const ui
     ctx->rht.hadamard_rows(a, n, m, m, false);
     ctx->rht.transpose(a, n, m, m, b, n);
     ctx->rht.hadamard_rows(b, m, n, n, false, nullptr, nullptr, RowScale{wscale, d_sv.p, d_su.p});
-    if (!hatW_on_device) QTIP_HIP(hipMemcpyAsync(hatW, b, size_t(m) * n * 4, hipMemcpyDeviceToHost, s));
+    if (!in_place)
+      QTIP_HIP(hipMemcpyAsync(hatW, b, size_t(m) * n * 4, hatW_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
     QTIP_HIP(hipStreamSynchronize(s));
   });
 }

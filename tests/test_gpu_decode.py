@@ -150,6 +150,32 @@ def test_dequantize_equals_its_steps(qz, pkg, m, n):
         assert torch.equal(view, want)
 
 
+def test_dequantize_into_memory_that_is_not_the_devices_own(pkg):
+    """A buffer called device memory that is not this device's own (here: page-locked host memory the device can see; a peer's
+    memory is the same case) gets a copy of the result, which is formed in a buffer of the context."""
+    import torch
+    say("case: dequantize into the device's own memory and into page-locked host memory")
+    q = pkg.Quantizer(0)
+    m, n = 64, 256
+    rng = np.random.default_rng(5)
+    tr = rng.integers(0, 65536, (m // 16) * (n // 16) * 32, dtype=np.uint16)
+    su = np.where(rng.integers(0, 2, n), np.uint16(0xBF80), np.uint16(0x3F80))
+    sv = np.ones(m, np.float32)
+    lib = pkg.lib()
+
+    def run(t):
+        before = lib.qtip_selftest_device_alloc_calls()
+        torch.cuda.synchronize()
+        assert lib.qtip_dequantize_linear(q._h, tr.ctypes.data, su.ctypes.data, sv.ctypes.data, 0.0163, m, n, t.data_ptr(), 1) == 0
+        return lib.qtip_selftest_device_alloc_calls() - before
+    dev, pinned = torch.zeros(m, n, device="cuda"), torch.zeros(m, n, pin_memory=True)
+    run(dev)
+    assert run(dev) == 0                 # everything else is kept from the call before
+    assert run(pinned) == 1              # the result's buffer
+    assert torch.equal(dev.cpu(), pinned)
+    q.close()
+
+
 def test_decode_full_size_sample(qz, hyb):
     """Benchmark configuration 5 shape (12288 x 28672): random words decoded on the device, a sample of 32-row blocks
     compared with the CPU decoder, every value a codebook entry; prints the achieved HBM rate."""
