@@ -119,7 +119,7 @@ def lib():
     L.qtip_rotate_hessian.argtypes = [vp, vp, i, i, u64, d, vp, C.POINTER(d), vp]
     L.qtip_ldl_hessian.argtypes = [vp, i, i, vp]
     L.qtip_selftest_pair_patience.argtypes = [vp, C.c_ulonglong]
-    L.qtip_selftest_upload_beside_factorization.argtypes = [vp, d, C.POINTER(d)]
+    L.qtip_selftest_upload_beside_factorization.argtypes = [vp, C.c_size_t, d, C.POINTER(d)]
     L.qtip_ldl_hessian_device_updates.argtypes = [vp, vp, i, i, vp]
     L.qtip_selftest_ldl_panel_handover.argtypes = [vp, i, i, vp]
     L.qtip_ldl_hessian_device_updates_dev.argtypes = [vp, vp, i, i, vp, vp]
@@ -311,10 +311,10 @@ class Quantizer:
         """Ticks of 10 ns for which the workgroups of a pair wait for each other (same results whatever it is)."""
         _check(lib().qtip_selftest_pair_patience(self._h, ticks))
 
-    def selftest_upload_beside_factorization(self, busy_us):
-        """Microseconds 1 MB takes on the upload stream behind a wave that sleeps busy_us on the factorization's stream."""
+    def selftest_upload_beside_factorization(self, nbytes, busy_us):
+        """Microseconds `nbytes` take on the upload stream behind a wave that sleeps busy_us on the factorization's stream."""
         us = C.c_double()
-        _check(lib().qtip_selftest_upload_beside_factorization(self._h, busy_us, C.byref(us)))
+        _check(lib().qtip_selftest_upload_beside_factorization(self._h, nbytes, busy_us, C.byref(us)))
         return us.value
 
     def device_lut(self):

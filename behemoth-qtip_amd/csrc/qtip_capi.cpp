@@ -451,12 +451,11 @@ int qtip_selftest_pair_patience(qtip_ctx* ctx, unsigned long long ticks) {
   });
 }
 
-int qtip_selftest_upload_beside_factorization(qtip_ctx* ctx, double busy_us, double* upload_us) {
+int qtip_selftest_upload_beside_factorization(qtip_ctx* ctx, size_t bytes, double busy_us, double* upload_us) {
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr && upload_us != nullptr && busy_us >= 0 && busy_us <= 1e6, "selftest: bad arguments");
     DeviceGuard g(ctx);
     QTIP_REQUIRE(ctx->ldl_stream && ctx->upload_stream, "this context found no streams that run beside each other");
-    const size_t bytes = size_t(1) << 20;
     std::vector<uint8_t> host(bytes, 1);
     DBuf<uint8_t> dev(bytes);
     auto upload = [&] {

@@ -297,10 +297,10 @@ def test_default_chain_count(qz):
 
 def test_uploads_do_not_wait_for_a_factorization(qz):
     """run_groups' host inputs come up while the next group's factorization is queued as a whole: the upload stream must
-    not share its hardware queue (a copy would take the 80 ms and more)."""
+    not share its hardware queue (a copy of more than a megabyte or so would take the 80 ms and more)."""
     say("case: an upload beside the factorization's stream")
-    us = min(qz.selftest_upload_beside_factorization(80e3) for _ in range(3))
-    say("  1 MB in %.0f us" % us)
+    us = min(qz.selftest_upload_beside_factorization(16 << 20, 80e3) for _ in range(3))
+    say("  16 MB in %.0f us" % us)
     assert us < 20e3
 
 
