@@ -514,35 +514,50 @@ struct Settle {
 }  // namespace
 
 // The Hessian preparation of the calibrated NVFP4 quantizer (nvfp4_prepare_host) on the device: the same chains, hence
-// the same L and dw bit for bit.  dev_L (n x n), dev_dw: device buffers of the caller; host_L: optional.
+// the same L and dw bit for bit.  dev_L (n x n), dev_dw: device buffers of the caller, or null for the context's own;
+// host_L, host_dw: optional, or both with the context's own buffers.
 void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw,
-                               float* host_L) {
-  QTIP_REQUIRE(c && host_H && dev_L && dev_dw && n > 0 && n % 16 == 0, "nvfp4_prepare (device): bad arguments (n = %d)", n);
+                               float* host_L, float* host_dw) {
+  QTIP_REQUIRE(c && host_H && ((dev_L && dev_dw) || (host_L && host_dw)) && n > 0 && n % 16 == 0,
+               "nvfp4_prepare (device): bad arguments (n = %d)", n);
   QTIP_REQUIRE(n <= 65535, "nvfp4_prepare (device): n = %d is beyond one grid dimension", n);
   double dsum = 0;
   for (int i = 0; i < n; ++i) dsum += host_H[size_t(i) * n + i];
   const double creg = sigma_reg * dsum / n;
   hipStream_t s = factor_stream(c, n);
   Settle settle{s};
-  c->ldl_H.ensure(size_t(n) * n);
+  const size_t nn = size_t(n) * n;
+  if (!dev_L || !dev_dw) {
+    c->ldl_L.ensure(nn + size_t(n));
+    dev_L = c->ldl_L.p, dev_dw = dev_L + nn;
+  }
+  c->ldl_H.ensure(nn);
   QTIP_HIP(hipMemcpyAsync(c->ldl_H.p, host_H, size_t(n) * n * 4, hipMemcpyHostToDevice, s));
   symmetrize_lower_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n)), dim3(256), 0, s>>>(c->ldl_H.p, n, c->ldl_A.p);
   QTIP_HIP(hipGetLastError());
   add_to_diagonal_kernel<<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, s>>>(c->ldl_A.p, n, creg);
   QTIP_HIP(hipGetLastError());
   if (!factor_on_device(c, n, dev_L, dev_dw, s, host_L)) throw Error(QTIP_E_NOT_PD, "NVFP4 calibration: Hessian not positive definite");
+  if (host_dw) {
+    QTIP_HIP(hipMemcpyAsync(host_dw, dev_dw, size_t(n) * 4, hipMemcpyDeviceToHost, s));
+    QTIP_HIP(hipStreamSynchronize(s));
+  }
 }
 
 // The block LDL of the rotated Hessian: dev_HRr, or host_HRr if that is null.  L goes to host_L, to dev_L (n x n device
-// buffer), or to both.
+// buffer), or to both.  (Without dev_L it is formed in a buffer the context keeps: one made and freed here would have the
+// free wait for everything on the device, the quantization of another group included.)
 void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* host_L, const float* dev_HRr, float* dev_L) {
   QTIP_REQUIRE(c && n > 0 && n % 16 == 0 && (host_HRr || dev_HRr) && (host_L || dev_L),
                "ldl_hessian (device): bad arguments (n = %d)", n);
   QTIP_REQUIRE(n <= 65535, "ldl_hessian (device): n = %d is beyond one grid dimension", n);
   hipStream_t s = factor_stream(c, n);
   const size_t nn = size_t(n) * n;
-  DBuf<float> own(dev_L ? 0 : nn);
   Settle settle{s};
+  if (!dev_L) {
+    c->ldl_L.ensure(nn);
+    dev_L = c->ldl_L.p;
+  }
   if (!dev_HRr) {
     c->ldl_H.ensure(nn);
     QTIP_HIP(hipMemcpyAsync(c->ldl_H.p, host_HRr, nn * 4, hipMemcpyHostToDevice, s));
@@ -550,8 +565,7 @@ void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* h
   symmetrize_lower_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n)), dim3(256), 0, s>>>(dev_HRr ? dev_HRr : c->ldl_H.p, n,
                                                                                               c->ldl_A.p);
   QTIP_HIP(hipGetLastError());
-  float* const L = dev_L ? dev_L : own.p;
-  if (!factor_on_device(c, n, L, nullptr, s, host_L)) throw Error(QTIP_E_NOT_PD, "block LDL failed (H not PD)");
+  if (!factor_on_device(c, n, dev_L, nullptr, s, host_L)) throw Error(QTIP_E_NOT_PD, "block LDL failed (H not PD)");
 }
 
 }  // namespace qtipmi

@@ -684,11 +684,7 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
     QTIP_REQUIRE(ctx != nullptr, "nvfp4_prepare_device_updates: bad arguments");
     DeviceGuard g(ctx);
     QTIP_REQUIRE(host_H && host_L && host_dw && n > 0 && n % 16 == 0, "nvfp4_prepare (device): bad arguments (n = %d)", n);
-    const size_t nn = size_t(n) * n;
-    DBuf<float> L(nn), dw(static_cast<size_t>(n));
-    nvfp4_prepare_device_impl(ctx, host_H, n, sigma_reg, L.p, dw.p, host_L);
-    QTIP_HIP(hipMemcpyAsync(host_dw, dw.p, size_t(n) * 4, hipMemcpyDeviceToHost, ctx->stream));
-    QTIP_HIP(hipStreamSynchronize(ctx->stream));
+    nvfp4_prepare_device_impl(ctx, host_H, n, sigma_reg, nullptr, nullptr, host_L, host_dw);
   });
 }
 int qtip_nvfp4_quantize_prepared(qtip_ctx* ctx, int nmat, qtip_nvfp4_matrix* mats, int n, const float* host_L,

@@ -58,11 +58,12 @@ struct qtip_ctx {
   qtipmi::DBuf<uint8_t> up_W[kUploadSlots];
   qtipmi::DBuf<float> ring_dHRr[3], ring_dL[3];  // run_groups with device-updated LDL: rotated Hessians and factors stay here
   // LDL on the device (ldl_device.hip): own stream, fp64 work matrix, fp32 upload of HRr, a panel's solved rows
-  // transposed, the reciprocals and 16 x 16 inverses of its diagonal block, a flag; allocated on first use
+  // transposed, the reciprocals and 16 x 16 inverses of its diagonal block, a flag, the factor on its way to a caller's
+  // host memory; allocated on first use
   hipStream_t ldl_stream = nullptr;
   qtipmi::DBuf<double> ldl_A, ldl_Xt, ldl_diag;
   qtipmi::DBuf<int> ldl_bad;
-  qtipmi::DBuf<float> ldl_H;
+  qtipmi::DBuf<float> ldl_H, ldl_L;
 };
 
 namespace qtipmi {
@@ -72,7 +73,7 @@ void rotate_hessian_impl(qtip_ctx* c, const float* H, bool on_device, int n, uin
 void ldl_hessian_impl(const float* host_HRr, int n, int threads, float* host_L);
 void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* host_L, const float* dev_HRr, float* dev_L);
 void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw,
-                               float* host_L = nullptr);
+                               float* host_L = nullptr, float* host_dw = nullptr);
 void ldlq_impl(qtip_ctx* c, const float* dWT, const float* dL, long n, long m, float* d_hatWT, uint16_t* dQ,
                int feedback, double* vit_seconds, int chains);
 int ldlq_default_chains(qtip_ctx* c);  // what chains = 0 stands for in this context (decided on the first call)

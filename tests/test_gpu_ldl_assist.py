@@ -80,6 +80,21 @@ def test_factor_of_uneven_matrix_equals_host_factor(qz, pkg, n):
     assert np.array_equal(a.L.view(np.uint32), b.L.view(np.uint32))
 
 
+def test_a_second_factorization_allocates_nothing(pkg):
+    """The calls with host buffers keep what they need on the device: they run beside the quantization of other groups, and
+    a device free would wait for all of it."""
+    say("case: LDL on the device, second call of a size")
+    q = pkg.Quantizer(0)
+    n = 512
+    H = spd(n, 3)
+    for call in (lambda: q.ldl_hessian_device_updates(pkg.HessPrep(n=n, HRr=H.copy())), lambda: q.nvfp4_prepare_device_updates(H)):
+        call()
+        before = pkg.device_alloc_calls()
+        call()
+        assert pkg.device_alloc_calls() == before
+    q.close()
+
+
 def test_rank_deficient_matrix_is_refused(qz, pkg):
     say("case: LDL with device updates, matrix not positive definite")
     n = 1024
