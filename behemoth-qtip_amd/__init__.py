@@ -119,6 +119,7 @@ def lib():
     L.qtip_rotate_hessian.argtypes = [vp, vp, i, i, u64, d, vp, C.POINTER(d), vp]
     L.qtip_ldl_hessian.argtypes = [vp, i, i, vp]
     L.qtip_selftest_pair_patience.argtypes = [vp, C.c_ulonglong]
+    L.qtip_selftest_chain_tile_us.argtypes = [vp, C.POINTER(d)]
     L.qtip_selftest_upload_beside_factorization.argtypes = [vp, C.c_size_t, d, C.POINTER(d)]
     L.qtip_ldl_hessian_device_updates.argtypes = [vp, vp, i, i, vp]
     L.qtip_selftest_ldl_panel_handover.argtypes = [vp, i, i, vp]
@@ -310,6 +311,12 @@ class Quantizer:
     def selftest_pair_patience(self, ticks):
         """Ticks of 10 ns for which the workgroups of a pair wait for each other (same results whatever it is)."""
         _check(lib().qtip_selftest_pair_patience(self._h, ticks))
+
+    def selftest_chain_tile_us(self):
+        """The time per tile (us) that LDLQ's chains are offset by."""
+        us = C.c_double()
+        _check(lib().qtip_selftest_chain_tile_us(self._h, C.byref(us)))
+        return us.value
 
     def selftest_upload_beside_factorization(self, nbytes, busy_us):
         """Microseconds `nbytes` take on the upload stream behind a wave that sleeps busy_us on the factorization's stream."""

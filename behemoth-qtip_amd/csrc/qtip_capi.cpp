@@ -451,6 +451,13 @@ int qtip_selftest_pair_patience(qtip_ctx* ctx, unsigned long long ticks) {
   });
 }
 
+int qtip_selftest_chain_tile_us(qtip_ctx* ctx, double* tile_us) {
+  return guarded([&] {
+    QTIP_REQUIRE(ctx != nullptr && tile_us != nullptr, "selftest: null argument");
+    *tile_us = ctx->vit_tile_us;
+  });
+}
+
 int qtip_selftest_upload_beside_factorization(qtip_ctx* ctx, size_t bytes, double busy_us, double* upload_us) {
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr && upload_us != nullptr && busy_us >= 0 && busy_us <= 1e6, "selftest: bad arguments");

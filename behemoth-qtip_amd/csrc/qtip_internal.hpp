@@ -269,8 +269,9 @@ struct TileJob {
 };
 size_t viterbi_workspace_bytes(int slots);
 int viterbi_max_slots(int device);
-// start / stop (optional): events stamped at the kernel's own start and end
-void launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const float* d_entry_f, void* workspace,
+// start / stop (optional): events stamped at the kernel's own start and end.  Returns whether every tile has one workgroup of
+// 256 threads, the form of the launches that LDLQ's chains run side by side.
+bool launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const float* d_entry_f, void* workspace,
                           int slots, hipStream_t s, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 // Kept-metrics slots that are part of the code object (no allocation): viterbi_static_scratch_init looks up the
 // array's address on `device`, which must be current, once; viterbi_static_scratch returns it (null before that).

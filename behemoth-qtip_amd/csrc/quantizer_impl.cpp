@@ -173,6 +173,7 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
   hipEvent_t pace[qtip_ctx::kMaxChains][kAhead + 1];
   for (int k = 0; k < nch; ++k)
     for (auto& e : pace[k]) e = pacing.add(hipEventBlockingSync | hipEventDisableTiming);
+  bool one_workgroup_per_tile = false;  // of 256 threads (the same for all launches of a call)
   try {
     long nbuf_done = 0;
     for (long cur = nblk; cur > 0; cur -= 8, ++nbuf_done) {
@@ -222,8 +223,8 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
           if (nch > 1) job.wide = 0;  // the chains fill the chip between them: one launch is not the measure
           hipEvent_t t0 = nullptr, t1 = nullptr;
           if (vit_seconds) t0 = timed.add(hipEventDefault), t1 = timed.add(hipEventDefault);
-          launch_viterbi_tiles(job, c->d_entry_d, c->d_entry_f, c->vit_ws.p + viterbi_workspace_bytes(C.slot0), C.slots,
-                               C.s, t0, t1);
+          one_workgroup_per_tile = launch_viterbi_tiles(job, c->d_entry_d, c->d_entry_f,
+                                                        c->vit_ws.p + viterbi_workspace_bytes(C.slot0), C.slots, C.s, t0, t1);
         }
         QTIP_HIP(hipEventRecord(pace[k][nbuf_done % (kAhead + 1)], C.s));
       }
@@ -250,8 +251,9 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
     }
     *vit_seconds = t / nch;
     // per tile and resident workgroup: a launch takes its tile rows through 8 column blocks, tiles / slots rounds of them
+    // (of the chains' kind only: a tile that a small launch gives to more threads says nothing about theirs)
     const size_t launches = timed.ev.size() / 2;
-    if (launches > 0) {
+    if (launches > 0 && one_workgroup_per_tile) {
       const double rounds = double((ch[0].tiles + ch[0].slots - 1) / ch[0].slots);
       const double tile_us = t / double(launches) / (8.0 * rounds) * 1e6;
       if (tile_us > 50.0 && tile_us < 20000.0) c->vit_tile_us = tile_us;

@@ -46,7 +46,7 @@ struct qtip_ctx {
   int side_streams = 0;         // how many of chain_stream[0], chain_stream[1], ldl_stream (in this order) were found
                                 // to run beside the context's stream and beside each other when the context was made
   bool chains_checked = false;
-  double vit_tile_us = 800.0;   // a resident Viterbi workgroup's time per tile, from the last timed LDLQ call
+  double vit_tile_us = 800.0;   // a resident 256-thread Viterbi workgroup's time per tile, from the last timed LDLQ call of that kind
   qtipmi::Rht rht;
   qtipmi::DBuf<double> scratch;
   qtipmi::DBuf<uint16_t> hess_img;  // a batch of qtip_hessian_accumulate_dev as the stage images of its update kernel

@@ -1773,9 +1773,9 @@ static int viterbi_device_slots() {
   return viterbi_max_slots(dev);
 }
 
-void launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const float* d_entry_f, void* workspace,
+bool launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const float* d_entry_f, void* workspace,
                           int slots, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
-  if (job.tiles <= 0) return;
+  if (job.tiles <= 0) return true;
   QTIP_REQUIRE(slots > 0 && workspace != nullptr, "viterbi: missing workspace");
   if (!job.X) {  // LDLQ block: the targets come from the feedback operands
     QTIP_REQUIRE(job.WT && job.L && job.hatWT && ((job.prod64 != nullptr) != (job.prod32 != nullptr)),
@@ -1810,7 +1810,7 @@ void launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const flo
     else
       pair<<<dim3(unsigned(pair_grid)), threads, 0, s>>>(job, d_entry_d, d_entry_f, ws);
     QTIP_HIP(hipGetLastError());
-    return;
+    return false;
   }
   const auto kernel = wide ? viterbi_tiles_kernel<true> : viterbi_tiles_kernel<false>;
   const dim3 block(wide ? 2 * kThreads : kThreads);
@@ -1823,6 +1823,7 @@ void launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const flo
     kernel<<<dim3(grid), block, 0, s>>>(job, d_entry_d, d_entry_f, static_cast<double*>(workspace));
   }
   QTIP_HIP(hipGetLastError());
+  return !wide;
 }
 
 int viterbi_static_slots() { return kStaticSlots; }

@@ -361,6 +361,9 @@ long qtip_selftest_device_alloc_calls(void);
  * a small launch waits for the other before the first does the rest alone (same results; default half a second). */
 int qtip_selftest_pair_patience(qtip_ctx* ctx, unsigned long long ticks);
 
+/* Self test (no counterpart in the reference): the time per tile, in microseconds, that LDLQ's chains are offset by. */
+int qtip_selftest_chain_tile_us(qtip_ctx* ctx, double* tile_us);
+
 /* Self test (no counterpart in the reference): microseconds that `bytes` take from host memory on the stream that brings
  * qtip_run_groups' host inputs up, with a wave that sleeps for busy_us queued on the factorization's stream before it. */
 int qtip_selftest_upload_beside_factorization(qtip_ctx* ctx, size_t bytes, double busy_us, double* upload_us);

@@ -304,6 +304,23 @@ def test_uploads_do_not_wait_for_a_factorization(qz):
     assert us < 20e3
 
 
+def test_chain_offset_is_learned_from_the_chains_kind_of_launch(pkg, synth):
+    """What a tile takes in a small launch, whose tiles have two workgroups, is not what the chains of a large group are
+    offset by; a launch with one workgroup of 256 threads per tile (here 416 tile rows) is."""
+    say("case: the chains' time per tile after a small and after a larger group")
+    q = pkg.Quantizer(0)
+    try:
+        start = q.selftest_chain_tile_us()
+        for ms, learned in (((64, 32), False), ((4096, 2560), True)):
+            Ws, H = synth.small_group(seed=77, n=256, ms=ms)
+            q.quantize_group_h([pkg.LinearIn("w%d" % i, w.shape[0], w_f32=w) for i, w in enumerate(Ws)], 256, H, 3,
+                               pkg.QuantOpts(skip_proxy=True))
+            say("  %s: %.0f us" % (ms, q.selftest_chain_tile_us()))
+            assert (q.selftest_chain_tile_us() != start) == learned
+    finally:
+        q.close()
+
+
 def test_ldlq_chains_give_the_same_codes(qz, oracle, pkg, hyb):
     """The tile rows of a group are dealt to 1, 2 or 3 independent chains of launches (streams of their own, feedback
     slabs of their own, ragged shares of rows with two linears of different height): every packed word, Wscale and
