@@ -145,6 +145,7 @@ def lib():
     L.qtip_nvfp4_quantize_group.argtypes = [vp, i, vp, i, vp, C.POINTER(_Nvfp4OptsC), C.POINTER(i)]
     L.qtip_run_groups.argtypes = [vp, i, vp, C.POINTER(_OptsC), vp, vp]
     L.qtip_reserve_groups.argtypes = [vp, i]
+    L.qtip_reserve_groups_for.argtypes = [vp, i, vp]
     L.qtip_group_lanes.argtypes = [vp, i, vp, C.POINTER(_OptsC), C.POINTER(C.c_int)]
     L.qtip_selftest_group_lanes.argtypes = [i, i, i, i, i, C.POINTER(C.c_int)]
     L.qtip_st_create.argtypes = [C.POINTER(vp)]
@@ -573,11 +574,14 @@ class Quantizer:
             t.global_scale = mats[k].global_
         return outs
 
-    def reserve_groups(self, n):
-        _check(lib().qtip_reserve_groups(self._h, n))
+    def reserve_groups(self, n, opt: QuantOpts = None):
+        """Allocates what run_groups keeps of n x n Hessians with these options ahead of the first call."""
+        opt = opt or QuantOpts()
+        co = _OptsC(ldl_device_updates=1 if opt.ldl_device_updates else 0)
+        _check(lib().qtip_reserve_groups_for(self._h, n, C.byref(co)))
 
     def run_groups(self, groups, opt: QuantOpts = None):
-        """Several groups with the host LDL of group g+1 overlapping the GPU work of group g (run_qtip_groups,
+        """Several groups with the LDL of group g+1 overlapping the GPU work of group g (run_qtip_groups,
         src/pipeline.cpp:229-312).  groups: list of (lins, n, H, seed).  Returns a list of (outs, timing, ldl_wait)."""
         opt = opt or QuantOpts()
         G = (_GroupC * len(groups))()

@@ -1,9 +1,10 @@
 // Several Hessian groups through one context, scheduled like the reference's run_qtip_groups
 // (src/pipeline.cpp:229-312): Hessians are rotated on the GPU ahead of use, a side thread runs the fp64 LDL of
-// the groups in order (on the GPU by default, or on the host), and the calling thread quantizes group g as soon as its factor is there, so the LDL of group
-// g+1 overlaps the GPU work of group g.  The reference rotates all Hessians of a layer up front and keeps every HRr;
-// here rotation runs two groups ahead through a ring of three page-locked (HRr, L) pairs kept by the context, so
-// host memory stays at 6 n^2 floats however many groups are queued.
+// the groups in order (on the GPU by default, or on the host), and the calling thread quantizes group g as soon as its
+// factor is there, so the LDL of group g+1 overlaps the GPU work of group g.  The reference rotates all Hessians of a
+// layer up front and keeps every HRr; here rotation runs two groups ahead through a ring of three (HRr, L) pairs kept by
+// the context, on the device or, with the LDL on the host, in page-locked memory, so that it stays at 6 n^2 floats however
+// many groups are queued.
 #include <chrono>
 #include <condition_variable>
 #include <cstdlib>
@@ -20,10 +21,15 @@ namespace {
 double now_s() { return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
 }  // namespace
 
-void reserve_group_ring(qtip_ctx* c, int n, int depth) {
+void reserve_group_ring(qtip_ctx* c, int n, int depth, bool on_device) {
   QTIP_REQUIRE(n > 0 && depth >= 1 && depth <= 3, "reserve: bad arguments");
   const size_t need = size_t(n) * n;
   for (int b = 0; b < depth; ++b) {
+    if (on_device) {
+      c->ring_dHRr[b].ensure(need);
+      c->ring_dL[b].ensure(need);
+      continue;
+    }
     if (c->ring_HRr[b].n < need) {
       c->ring_HRr[b].alloc(need);
       std::memset(c->ring_HRr[b].p, 0, need * 4);
@@ -45,12 +51,7 @@ void run_groups_on(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opt
   // with the LDL on the device neither the rotated Hessian nor the factor leaves it: the factorization and the proxy read
   // the one, LDLQ the other, and the host ring is not used
   const bool keep_dev = opt.ldl_device_updates != 0;
-  if (!keep_dev) reserve_group_ring(c, nmax, R);
-  if (keep_dev)
-    for (int b = 0; b < R; ++b) {
-      c->ring_dHRr[b].ensure(size_t(nmax) * nmax);
-      c->ring_dL[b].ensure(size_t(nmax) * nmax);
-    }
+  reserve_group_ring(c, nmax, R, keep_dev);
   const size_t ngz = size_t(ng);
   std::vector<std::vector<float>> su;
   for (int b = 0; b < R; ++b) su.emplace_back(std::vector<float>(static_cast<size_t>(nmax), 0.0f));
@@ -275,11 +276,7 @@ void run_groups_in_line(qtip_ctx* c, int ng, const qtip_group* groups, const qti
   int nmax = 0;
   for (int g = 0; g < ng; ++g) nmax = std::max(nmax, groups[g].n);
   const bool keep_dev = opt.ldl_device_updates != 0;
-  if (!keep_dev) reserve_group_ring(c, nmax, 1);
-  if (keep_dev) {
-    c->ring_dHRr[0].ensure(size_t(nmax) * nmax);
-    c->ring_dL[0].ensure(size_t(nmax) * nmax);
-  }
+  reserve_group_ring(c, nmax, 1, keep_dev);
   std::vector<float> su(static_cast<size_t>(nmax), 0.0f);
   for (int g = 0; g < ng; ++g) {
     qtip_timing T{};

@@ -438,7 +438,6 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s, f
     }
   } down;
   if (host_L) QTIP_HIP(hipStreamCreateWithFlags(&down.stream, hipStreamNonBlocking));
-  c->ldl_bad.ensure(1);
   int bad = 0;
   QTIP_HIP(hipMemcpyAsync(c->ldl_bad.p, &bad, sizeof bad, hipMemcpyHostToDevice, s));
   QTIP_HIP(hipMemsetAsync(L, 0, size_t(n) * n * sizeof(float), s));
@@ -503,6 +502,7 @@ hipStream_t factor_stream(qtip_ctx* c, long n) {
   c->ldl_A.ensure(size_t(n) * n);
   c->ldl_Xt.ensure(size_t(n) * kDiag);
   c->ldl_diag.ensure(2 * size_t(kDiag) * 17);
+  c->ldl_bad.ensure(1);
   return c->ldl_stream;
 }
 
@@ -512,6 +512,8 @@ struct Settle {
   ~Settle() { (void)hipStreamSynchronize(s); }
 };
 }  // namespace
+
+void reserve_device_ldl(qtip_ctx* c, int n) { (void)factor_stream(c, n); }
 
 // The Hessian preparation of the calibrated NVFP4 quantizer (nvfp4_prepare_host) on the device: the same chains, hence
 // the same L and dw bit for bit.  dev_L (n x n), dev_dw: device buffers of the caller, or null for the context's own;

@@ -778,13 +778,16 @@ int qtip_selftest_group_lanes(int device_slots, int ngroups, int m, int n, int r
   });
 }
 
-int qtip_reserve_groups(qtip_ctx* ctx, int n) {
+int qtip_reserve_groups_for(qtip_ctx* ctx, int n, const qtip_opts* opts) {
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr && n > 0, "reserve_groups: bad arguments");
     DeviceGuard g(ctx);
-    reserve_group_ring(ctx, n, 3);
+    const bool on_device = !opts || opts->ldl_device_updates != 0;
+    reserve_group_ring(ctx, n, 3, on_device);
+    if (on_device) reserve_device_ldl(ctx, n);
   });
 }
+int qtip_reserve_groups(qtip_ctx* ctx, int n) { return qtip_reserve_groups_for(ctx, n, nullptr); }
 
 int qtip_selftest_failed_alloc_is_retried(void) {
   // host only: the next two device allocations are made to fail; a buffer whose allocation failed must stay empty,

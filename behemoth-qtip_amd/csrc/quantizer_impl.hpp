@@ -50,13 +50,13 @@ struct qtip_ctx {
   qtipmi::Rht rht;
   qtipmi::DBuf<double> scratch;
   qtipmi::DBuf<uint16_t> hess_img;  // a batch of qtip_hessian_accumulate_dev as the stage images of its update kernel
-  qtipmi::HBuf<float> ring_HRr[3], ring_L[3];  // page-locked staging of run_groups, kept between calls
+  qtipmi::HBuf<float> ring_HRr[3], ring_L[3];  // page-locked staging of run_groups with the LDL on the host, kept between calls
   // host inputs of qtip_run_groups on their way to the device: a stream and four staging slots (Hessian, weights)
   static constexpr int kUploadSlots = 4;
   hipStream_t upload_stream = nullptr;
   qtipmi::DBuf<float> up_H[kUploadSlots];
   qtipmi::DBuf<uint8_t> up_W[kUploadSlots];
-  qtipmi::DBuf<float> ring_dHRr[3], ring_dL[3];  // run_groups with device-updated LDL: rotated Hessians and factors stay here
+  qtipmi::DBuf<float> ring_dHRr[3], ring_dL[3];  // run_groups with the LDL on the device: rotated Hessians and factors stay here
   // LDL on the device (ldl_device.hip): own stream, fp64 work matrix, fp32 upload of HRr, a panel's solved rows
   // transposed, the reciprocals and 16 x 16 inverses of its diagonal block, a flag, the factor on its way to a caller's
   // host memory; allocated on first use
@@ -99,7 +99,10 @@ void quantize_group_impl(qtip_ctx* c, int nlin, const qtip_linear_in* lins, int 
                          double creg, const float* host_HRr, const float* host_L, const qtip_opts& opt,
                          qtip_linear_out* outs, qtip_timing* tm, const float* dev_HRr = nullptr,
                          const float* dev_L = nullptr);
-void reserve_group_ring(qtip_ctx* c, int n, int depth);
+// the ring of (HRr, L) pairs of run_groups, on the device or in page-locked host memory, and what the factorization of an
+// n x n matrix on the device keeps
+void reserve_group_ring(qtip_ctx* c, int n, int depth, bool on_device);
+void reserve_device_ldl(qtip_ctx* c, int n);
 // lane k of a context (made on first use with the parent's codebook), and the release of all of them
 qtip_ctx* lane_context(qtip_ctx* parent, int k);
 void release_lanes(qtip_ctx* parent);

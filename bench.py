@@ -186,7 +186,7 @@ def run_group(args, pkg):
                          wscale=float(res[-1][0][0].wscale), cmp_outs=res[min(K, 6) - 1][0],
                          cmp_outs3=res[min(K, 3) - 1][0])
 
-    q.reserve_groups(n)   # page-locked staging ring (3 x (HRr, L)); a worker keeps it for its lifetime
+    q.reserve_groups(n, opt)   # the ring of three (HRr, L) pairs and the LDL's work matrix; a worker keeps them for its lifetime
     q.set_viterbi_mode(1 if args.viterbi_fp64 else 0)
     if args.warmup > 0:
         run_steps(args.warmup, False)
@@ -244,6 +244,7 @@ def run_group(args, pkg):
         kh = min(args.steps, 6)
         hopt = pkg.QuantOpts(ldl_threads=args.ldl_threads, skip_proxy=False, feedback=args.feedback,
                              ldl_device_updates=False, ldlq_chains=args.chains, group_lanes=args.lanes)
+        q.reserve_groups(n, hopt)   # here the ring is page-locked host memory
         q.synchronize()
         th = time.time()
         hres = q.run_groups([(lins, n, H, 3 + k) for k in range(kh)], hopt)

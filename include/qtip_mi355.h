@@ -322,8 +322,11 @@ int qtip_group_lanes(qtip_ctx* ctx, int ngroups, const qtip_group* groups, const
 /* Host-only check of the lane rule: `ngroups` equal groups of one m x n linear on a device with `device_slots`
  * Viterbi workgroup slots, qtip_opts.group_lanes = requested. */
 int qtip_selftest_group_lanes(int device_slots, int ngroups, int m, int n, int requested, int* lanes);
-/* Allocates the staging ring of qtip_run_groups for Hessians up to n x n ahead of the first call (optional). */
+/* Allocates what qtip_run_groups keeps of Hessians up to n x n ahead of the first call (optional): its ring of three
+ * (HRr, L) pairs and the factorization's work matrix on the device, 32 n^2 bytes; with opts->ldl_device_updates = 0 the ring
+ * in page-locked host memory, 24 n^2 bytes.  qtip_reserve_groups: for the default options. */
 int qtip_reserve_groups(qtip_ctx* ctx, int n);
+int qtip_reserve_groups_for(qtip_ctx* ctx, int n, const qtip_opts* opts);
 
 /* Layer file writer: the safetensors container of SafeTensorsWriter, src/safetensors.cpp:93-137 (u64 header length,
  * JSON header with sorted keys padded to 8 bytes, tensors back to back in name order, written to path + ".tmp" and

@@ -295,6 +295,34 @@ def test_default_chain_count(qz):
     assert n in (2, 3)
 
 
+def test_reserve_groups_allocates_what_run_groups_keeps(pkg, synth):
+    """After reserve_groups the first run_groups of that width allocates neither its ring of three (HRr, L) pairs nor the
+    factorization's four buffers any more: ten device allocations fewer than without it."""
+    say("case: reserve_groups")
+    cases = []
+    for g in range(3):
+        Ws, H = synth.small_group(seed=90 + g, n=256, ms=(64,))
+        cases.append(([pkg.LinearIn("w", 64, w_f32=Ws[0])], 256, H, 5 + g))
+    opt = pkg.QuantOpts(group_lanes=1)
+    used, words = {}, {}
+    for reserve in (False, True):
+        q = pkg.Quantizer(0)
+        if reserve:
+            before = pkg.device_alloc_calls()
+            q.reserve_groups(256)
+            assert pkg.device_alloc_calls() - before == 10
+            q.reserve_groups(128)            # smaller: there already
+            assert pkg.device_alloc_calls() - before == 10
+            q.reserve_groups(128, pkg.QuantOpts(ldl_device_updates=False))      # page-locked host memory
+            assert pkg.device_alloc_calls() - before == 10
+        before = pkg.device_alloc_calls()
+        words[reserve] = [r[0][0].trellis for r in q.run_groups(cases, opt)]
+        used[reserve] = pkg.device_alloc_calls() - before
+        q.close()
+    assert used[False] - used[True] == 10
+    assert all(np.array_equal(a, b) for a, b in zip(words[False], words[True]))
+
+
 def test_uploads_do_not_wait_for_a_factorization(qz):
     """run_groups' host inputs come up while the next group's factorization is queued as a whole: the upload stream must
     not share its hardware queue (a copy of more than a megabyte or so would take the 80 ms and more)."""
