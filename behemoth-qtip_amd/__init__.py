@@ -122,7 +122,6 @@ def lib():
     L.qtip_selftest_chain_tile_us.argtypes = [vp, C.POINTER(d)]
     L.qtip_selftest_upload_beside_factorization.argtypes = [vp, C.c_size_t, d, C.POINTER(d)]
     L.qtip_ldl_hessian_device_updates.argtypes = [vp, vp, i, i, vp]
-    L.qtip_selftest_ldl_panel_handover.argtypes = [vp, i, i, vp]
     L.qtip_ldl_hessian_device_updates_dev.argtypes = [vp, vp, i, i, vp, vp]
     L.qtip_ldlq_dev.argtypes = [vp, vp, vp, l, l, vp, vp, i, C.POINTER(d)]
     L.qtip_prod_cache_bf16x3_dev.argtypes = [vp, i, l, vp, l, vp, vp, l, vp]

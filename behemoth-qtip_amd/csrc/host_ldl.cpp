@@ -220,12 +220,8 @@ static Kernels pick_kernels() {
 
 // Lower Cholesky of the n x n matrix at A (row stride ld) by right-looking panels of width NBT, shared out over the
 // team.
-// assist: the trailing matrix lives elsewhere.  Before a panel is factored its columns, rows k .. n-1, are fetched
-// into a buffer of row stride kb; after the solve the buffer holds the final columns of C and is handed back, and
-// whoever holds the trailing matrix applies the rank-kb update (every element one chain
-// acc = fma(x_ip, x_jp, acc), p ascending from zero, then c -= acc, as the micro-kernels here do).
 template <int NBT, int TILET>
-bool cholesky_panels(double* A, long ld, int n, HostTeam* team, PanelAssist* assist = nullptr) {
+bool cholesky_panels(double* A, long ld, int n, HostTeam* team) {
   const Kernels kn = pick_kernels();
   const int MR = kn.MR, NR = kn.NR;
   constexpr int LDT = (NBT + 31) / 32 * 32;
@@ -238,18 +234,12 @@ bool cholesky_panels(double* A, long ld, int n, HostTeam* team, PanelAssist* ass
   double* const packB = packA + capA;
   for (int k = 0; k < n; k += NBT) {
     const int kb = std::min(NBT, n - k);
-    // the panel: diagonal block at Ap, the rows below follow with stride ldp
-    double* Ap = assist ? assist->fetch(k, kb) : A + long(k) * ld + k;
-    const long ldp = assist ? kb : ld;
-    if (!kn.factor_diag(Ap, ldp, kb, diagT.data(), LDT)) return false;
-    if (assist) assist->factored(k, kb, Ap, ldp);
+    double* Ap = A + long(k) * ld + k;  // the panel: its diagonal block, the rows below follow
+    if (!kn.factor_diag(Ap, ld, kb, diagT.data(), LDT)) return false;
     const int r0 = k + kb, nr = n - r0;
-    if (nr <= 0) {
-      if (assist) assist->solved(k, kb, Ap);
-      break;
-    }
+    if (nr <= 0) break;
     for (int j = 0; j < kb; ++j) {
-      for (int p = 0; p < kb; ++p) L11[size_t(j) * kb + p] = p <= j ? Ap[long(j) * ldp + p] : 0.0;
+      for (int p = 0; p < kb; ++p) L11[size_t(j) * kb + p] = p <= j ? Ap[long(j) * ld + p] : 0.0;
       rdiag[j] = 1.0 / L11[size_t(j) * kb + j];
     }
     const int nPA = (nr + MR - 1) / MR, nPB = (nr + NR - 1) / NR;
@@ -264,17 +254,13 @@ bool cholesky_panels(double* A, long ld, int n, HostTeam* team, PanelAssist* ass
       const int rb = g * NR, rows = std::min(NR, nr - rb);
       double* x = packB + size_t(g) * NR * kb;  // [p][NR], rows beyond `rows` stay zero
       for (int r = 0; r < rows; ++r) {
-        const double* src = Ap + long(kb + rb + r) * ldp;
+        const double* src = Ap + long(kb + rb + r) * ld;
         for (int p = 0; p < kb; ++p) x[size_t(p) * NR + r] = src[p];
       }
       kn.tri_solve(kb, L11.data(), kb, rdiag.data(), x);
       for (int r = 0; r < rows; ++r) {
         const int i = rb + r;
-        double* dst = Ap + long(kb + i) * ldp;
-        if (assist) {  // the update runs elsewhere: no A-side pack
-          for (int p = 0; p < kb; ++p) dst[p] = x[size_t(p) * NR + r];
-          continue;
-        }
+        double* dst = Ap + long(kb + i) * ld;
         double* pa = packA + size_t(i / MR) * MR * kb + (i % MR);
         for (int p = 0; p < kb; ++p) {
           const double v = x[size_t(p) * NR + r];
@@ -283,19 +269,9 @@ bool cholesky_panels(double* A, long ld, int n, HostTeam* team, PanelAssist* ass
         }
       }
     };
-    auto solve_and_hand_over = [&](long gl) {
-      solve_chunk(gl);
-      const int rb = int(gl) * NR;
-      assist->rows_solved(k, kb, r0 + rb, std::min(NR, nr - rb), Ap + long(kb + rb) * ldp, ldp);
-    };
-    if (team && assist) team->parallel_for(nPB, 2, solve_and_hand_over);
-    else if (team) team->parallel_for(nPB, 2, solve_chunk);
+    if (team) team->parallel_for(nPB, 2, solve_chunk);
     else
-      for (long gl = 0; gl < nPB; ++gl) assist ? solve_and_hand_over(gl) : solve_chunk(gl);
-    if (assist) {
-      assist->solved(k, kb, Ap);
-      continue;
-    }
+      for (long gl = 0; gl < nPB; ++gl) solve_chunk(gl);
     // trailing update of the lower triangle, tiles (bi, bj <= bi) largest rows first
     const int nT = (nr + TILET - 1) / TILET;
     const long ntask = long(nT) * (nT + 1) / 2;
@@ -381,76 +357,6 @@ bool block_ldl_host(double* A, int n, float* L_out, int threads) {
   std::vector<double> inv(size_t(n / 16) * 256);
   invert_diag_blocks(A, n, n / 16, inv.data(), team);
   return assemble_L_columns(A, n, inv.data(), 0, n, n, n, L_out, team);
-}
-
-int ldl_panel_width() { return NB; }
-
-bool block_ldl_assisted(int n, float* L_out, int threads, PanelAssist& assist) {
-  if (n % 16 != 0) fail(QTIP_E_ARG, "block LDL needs n %% 16 == 0 (n = %d)", n);
-  HostTeam& team = team_of_this_thread(threads);
-  // L is assembled panel by panel from the solved columns as they pass through the host: the rows below a panel by
-  // the thread that solved them, while they are in its cache; the rows above (zeros) and those of the diagonal
-  // block after the update has been queued
-  struct Wrap : PanelAssist {
-    PanelAssist& inner;
-    int n;
-    float* L;
-    HostTeam& team;
-    const Kernels kn = pick_kernels();
-    std::vector<double> inv;
-    std::atomic<int> finite{1};
-    Wrap(PanelAssist& i, int n_, float* L_, HostTeam& t) : inner(i), n(n_), L(L_), team(t) {}
-    double* fetch(int k, int kb) override { return inner.fetch(k, kb); }
-    void factored(int k, int kb, const double* diag, long ld) override {
-      inv.resize(size_t(kb / 16) * 256);
-      invert_diag_blocks(diag, ld, kb / 16, inv.data(), team);
-    }
-    void rows_solved(int k, int kb, int row0, int count, const double* rows, long ld) override {
-      bool ok = true;
-      for (int i = 0; i < count; ++i)
-        ok = kn.assemble_row(rows + long(i) * ld, inv.data(), kb / 16, L + long(row0 + i) * n + k) && ok;
-      if (!ok) finite.store(0, std::memory_order_relaxed);
-    }
-    void solved(int k, int kb, const double* panel) override {
-      inner.solved(k, kb, panel);  // the update is queued first and runs while the rest of L's columns is written
-      if (!assemble_L_columns(panel, kb, inv.data(), k, kb, n, k + kb, L, team)) finite.store(0, std::memory_order_relaxed);
-      inner.assembled(k, kb);
-    }
-  } wrap(assist, n, L_out, team);
-  if (!cholesky_panels<NB, TILE>(nullptr, 0, n, &team, &wrap)) return false;
-  return wrap.finite.load() != 0;
-}
-
-// block_ldl_assisted with the trailing matrix held and updated by plain host code (one fma chain per element over the
-// panel, from zero, then one subtraction): exercises the panel hand-over without a device.  L must come out as
-// block_ldl_host's.
-bool block_ldl_assisted_on_host(const float* HRr, int n, float* L_out, int threads) {
-  struct HostTrailing final : PanelAssist {
-    long n;
-    std::vector<double> A, buf[2];
-    int turn = 0;
-    double* fetch(int k, int kb) override {
-      std::vector<double>& b = buf[turn ^= 1];  // alternate: a panel may be looked at while the next is fetched
-      b.resize(size_t(n - k) * kb);
-      for (long i = k; i < n; ++i)
-        for (int p = 0; p < kb; ++p) b[size_t(i - k) * kb + p] = A[size_t(i) * n + k + p];
-      return b.data();
-    }
-    void solved(int k, int kb, const double* panel) override {
-      const long r0 = k + kb;
-      const double* X = panel + size_t(kb) * kb;
-      for (long i = r0; i < n; ++i)
-        for (long j = r0; j <= i; ++j) {
-          double acc = 0;
-          for (int p = 0; p < kb; ++p) acc = __builtin_fma(X[size_t(i - r0) * kb + p], X[size_t(j - r0) * kb + p], acc);
-          A[size_t(i) * n + j] -= acc;
-        }
-    }
-  } host;
-  host.n = n;
-  host.A.assign(size_t(n) * n, 0.0);
-  symmetrize_lower_host(HRr, n, host.A.data(), threads);
-  return block_ldl_assisted(n, L_out, threads, host);
 }
 
 // A[i][j] = (HRr[i][j] + HRr[j][i]) / 2 in fp64, lower triangle (tiled so both reads stay in cache)

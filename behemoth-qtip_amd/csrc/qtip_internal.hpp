@@ -183,28 +183,6 @@ struct HostScratch {
 
 // fp64 block LDL on the host (host_ldl.cpp). A: n x n fp64, lower triangle used, destroyed. Returns false if not PD.
 bool block_ldl_host(double* A, int n, float* L_out, int threads);
-// The same factorization with the trailing matrix kept by someone else: the host factors and solves one
-// panel of ldl_panel_width() columns at a time.  fetch(k, kb) returns a buffer of row stride kb holding rows k .. n-1
-// of the columns k .. k+kb-1 as updated so far; solved(k, kb, panel) receives it back with the final columns of the
-// Cholesky factor: the rows kb .. n-k-1 of it are the operand of the rank-kb update of the trailing matrix, which
-// must form every element as one chain acc = fma(x_ip, x_jp, acc), p = 0 .. kb-1 from zero, then c -= acc, for L to
-// equal block_ldl_host's bit for bit.
-struct PanelAssist {
-  virtual double* fetch(int k, int kb) = 0;
-  virtual void solved(int k, int kb, const double* panel) = 0;
-  // optional: the kb x kb diagonal block of panel k is factored (lower triangle at diag, row stride ld); called before
-  // the rows below it are solved
-  virtual void factored(int k, int kb, const double* diag, long ld) {}
-  // optional: rows row0 .. row0 + count - 1 of the matrix (below the panel) are solved, `rows` holds their kb values
-  // (row stride ld).  Called from the team's threads, several at a time, while the rows are still in cache.
-  virtual void rows_solved(int k, int kb, int row0, int count, const double* rows, long ld) {}
-  // the columns k .. k+kb-1 of L_out are final (all n rows)
-  virtual void assembled(int k, int kb) {}
-  virtual ~PanelAssist() = default;
-};
-int ldl_panel_width();
-bool block_ldl_assisted(int n, float* L_out, int threads, PanelAssist& assist);
-bool block_ldl_assisted_on_host(const float* HRr, int n, float* L_out, int threads);
 // lower Cholesky in place (lower triangle of the n x n fp64 matrix A); false if not positive definite
 bool cholesky_lower_host(double* A, int n, int threads);
 // A[i][j] = (HRr[i][j] + HRr[j][i]) / 2 in fp64, lower triangle

@@ -375,11 +375,6 @@ int qtip_selftest_upload_beside_factorization(qtip_ctx* ctx, size_t bytes, doubl
  * allocation failed stays empty, so the next call allocates again instead of launching on a null pointer.  0 = ok. */
 int qtip_selftest_failed_alloc_is_retried(void);
 
-/* Host-only self test (no GPU needed, no counterpart in the reference): the block LDL through the panel hand-over
- * (a panel's columns fetched, factored and solved, the rows handed back, L assembled from them as they pass), with the
- * trailing matrix held and updated by plain host code.  host_L must come out as qtip_ldl_hessian's, bit for bit. */
-int qtip_selftest_ldl_panel_handover(const float* host_HRr, int n, int threads, float* host_L);
-
 /* Host packers (pack_trellis / unpack_trellis / swizzle_for_kernel / unswizzle_for_kernel,
  * src/qtip_core.cpp:194-253) */
 void qtip_pack_trellis(const uint16_t* states, long B, uint16_t* packed);
