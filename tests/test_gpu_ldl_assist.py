@@ -44,7 +44,7 @@ def test_factor_equals_host_factor(qz, pkg, n):
 @pytest.mark.parametrize("n", [272, 1040, 2560])
 def test_device_resident_form_equals_host_factor(qz, pkg, n):
     """qtip_ldl_hessian_device_updates_dev: the rotated Hessian stays on the device and is not written, L arrives in the
-    host buffer and, column block by column block, in the device buffer; both equal the host factorization's words."""
+    device buffer and from there, row block by row block, in the host buffer; both equal the host factorization's words."""
     import torch
     say("case: LDL with device updates, Hessian resident on the device, n = %d" % n)
     H = spd(n, 300 + n)
@@ -54,7 +54,7 @@ def test_device_resident_form_equals_host_factor(qz, pkg, n):
     L_pin = torch.full((n, n), -1.0, dtype=torch.float32).pin_memory()
     dL = torch.full((n, n), -1.0, dtype=torch.float32, device="cuda")
     torch.cuda.synchronize()
-    for _ in range(2):   # twice through the same context: the panel buffers alternate and are reused
+    for _ in range(2):   # twice through the same context: its buffers are reused
         qz.ldl_hessian_device_resident(dH, n, L_pin, dL, threads=16)
         assert np.array_equal(L_pin.numpy().view(np.uint32), a.L.view(np.uint32))
         assert torch.equal(dL.cpu(), L_pin)
@@ -63,6 +63,31 @@ def test_device_resident_form_equals_host_factor(qz, pkg, n):
     L2 = np.full((n, n), -1.0, np.float32)
     qz.ldl_hessian_device_resident(dH, n, L2, None, threads=16)
     assert np.array_equal(L2.view(np.uint32), a.L.view(np.uint32))
+
+
+def test_factor_of_a_large_matrix_equals_host_factor(qz, pkg):
+    """n = 12288: 24 panels whose diagonal block comes with the update before it, and 24 that have a launch of their own;
+    the form with host buffers, and the one that stays on the device with L in both places."""
+    import torch
+    n = 12288
+    say("case: LDL on the device, n = %d" % n)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    X = torch.randn(n + 1024, n, device="cuda", generator=gen) * torch.linspace(0.2, 3.0, n, device="cuda")
+    X[:, 1:] += 0.8 * X[:, :-1].clone()
+    dH = X.T @ X / X.shape[0]
+    del X
+    dH += 0.01 * dH.diagonal().mean() * torch.eye(n, device="cuda")
+    dH = dH.contiguous()
+    a = pkg.HessPrep(n=n, HRr=dH.cpu().numpy())
+    pkg.Quantizer.ldl_hessian(a, threads=16)
+    want = torch.from_numpy(a.L.view(np.int32))
+    b = pkg.HessPrep(n=n, HRr=a.HRr)
+    qz.ldl_hessian_device_updates(b, threads=16)
+    assert torch.equal(torch.from_numpy(b.L.view(np.int32)), want)
+    L, dL = torch.empty(n, n, pin_memory=True), torch.empty(n, n, device="cuda")
+    torch.cuda.synchronize()
+    qz.ldl_hessian_device_resident(dH, n, L, dL, threads=16)
+    assert torch.equal(L.view(torch.int32), want) and torch.equal(dL.cpu().view(torch.int32), want)
 
 
 @pytest.mark.parametrize("n", [32, 48, 256, 288])
