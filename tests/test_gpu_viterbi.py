@@ -282,6 +282,39 @@ def test_two_workgroups_per_tile_give_the_same_states(qz, pkg, B):
         assert torch.equal(got[name][1], got["256"][1]), name
 
 
+@pytest.mark.parametrize("ms,n,feedback", [((64, 32), 256, 0), ((1024,), 1024, 0), ((4096, 1024), 256, 1)])
+def test_pairs_in_a_group_give_the_same_words(qz, pkg, ms, n, feedback):
+    """LDLQ takes a pair through eight column blocks per launch (512 threads for 6 and 64 tile rows, 256 for 320): the words of
+    a group with pairs, with every pass repeated on fp64 metrics (the winner handed over each time), with a first
+    workgroup that goes on alone at some block of each launch or from the start, and with one workgroup per tile."""
+    say("case: pairs in a group, %s x %d, feedback %d" % (ms, n, feedback))
+    qz.set_tlut(None)
+    rng = np.random.default_rng(n + len(ms))
+    G = rng.standard_normal((n, 2 * n))
+    H = (G @ G.T / (2 * n)).astype(np.float32)
+    lins = [pkg.LinearIn("w%d" % i, m, w_f32=(rng.standard_normal((m, n)) * 0.02).astype(np.float32)) for i, m in enumerate(ms)]
+    opt = pkg.QuantOpts(feedback=feedback)
+    got = {}
+    try:
+        # ticks of 10 ns: a block takes about 20000 of them, so 0 gives up at once and 30, 300 and 3000 somewhere
+        for name, mode, margin, patience in (("256", 2, 0, 50000000), ("pairs", 0, 0, 50000000),
+                                             ("repeated", 0, 0xffffffff, 50000000), ("alone", 0, 0, 0),
+                                             ("alone, repeated", 0, 0xffffffff, 0), ("30", 0, 0, 30), ("300", 0, 0, 300),
+                                             ("3000", 0, 0, 3000)):
+            say("  " + name)
+            qz.set_viterbi_mode(mode, margin)
+            qz.selftest_pair_patience(patience)
+            outs, _ = qz.quantize_group_h(lins, n, H, 9, opt)
+            got[name] = [(o.trellis, o.wscale, o.proxy) for o in outs]
+    finally:
+        qz.set_viterbi_mode(0)
+        qz.selftest_pair_patience(50000000)
+    for name, outs in got.items():
+        for (tr, ws, px), (tr0, ws0, px0) in zip(outs, got["256"]):
+            assert np.array_equal(tr, tr0), "%s: %d words differ" % (name, np.count_nonzero(tr != tr0))
+            assert ws == ws0 and px == px0, name
+
+
 def test_wide_workgroups_give_the_same_states(qz, oracle, hyb):
     """A launch that cannot fill the chip gives every tile 512 threads instead of 256 (the 32-bit forward passes
     share the groups out over all of them; everything else, the fp64 repeat of a pass included, is done by both
