@@ -581,7 +581,10 @@ int qtip_dequantize_linear(qtip_ctx* ctx, const uint16_t* host_trellis, const ui
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr && host_trellis && host_su_bf16 && host_sv && hatW, "dequantize_linear: bad arguments");
     QTIP_REQUIRE(m > 0 && n > 0 && m % 32 == 0 && n % 32 == 0, "dequantize_linear: m, n must be multiples of 32 (m=%d n=%d)", m, n);
+    // (all that the transforms would refuse, before the caller's buffer is written)
     QTIP_REQUIRE(had_K(m) > 0 && had_K(n) > 0, "dequantize_linear: no Hadamard transform of size %d x %d", m, n);
+    QTIP_REQUIRE(m / had_K(m) <= 8192 && n / had_K(n) <= 8192,
+                 "dequantize_linear: hadamard pow2 part > 8192 unsupported (m=%d n=%d)", m, n);
     DeviceGuard g(ctx);
     hipStream_t s = ctx->stream;
     const size_t words = size_t(m / 16) * (n / 16) * 32;

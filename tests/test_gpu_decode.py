@@ -176,6 +176,22 @@ def test_dequantize_into_memory_that_is_not_the_devices_own(pkg):
     q.close()
 
 
+@pytest.mark.parametrize("m,n", [(32, 16384), (16384, 32), (32, 352)])
+def test_dequantize_refuses_before_it_writes(qz, pkg, m, n):
+    """Widths the transforms do not take (a power-of-two part above 8192, 11 x 32): an error, and the caller's device buffer as
+    it was."""
+    import torch
+    say("case: dequantize %dx%d is refused" % (m, n))
+    lo = pkg.LinearOut(name="w", m=m, n=n, wscale=0.0163, trellis=np.zeros((m // 16) * (n // 16) * 32, np.uint16),
+                       su_bf16=np.zeros(n, np.uint16), sv=np.ones(m, np.float32))
+    hat = torch.full((m, n), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    with pytest.raises(pkg.QtipError) as e:
+        qz.dequantize_linear(lo, hat)
+    assert e.value.code == pkg.QTIP_E_ARG
+    assert bool((hat == 7.0).all())
+
+
 def test_decode_full_size_sample(qz, hyb):
     """Benchmark configuration 5 shape (12288 x 28672): random words decoded on the device, a sample of 32-row blocks
     compared with the CPU decoder, every value a codebook entry; prints the achieved HBM rate."""
