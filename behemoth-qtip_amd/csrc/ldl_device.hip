@@ -260,8 +260,8 @@ __global__ __launch_bounds__(256, 3) void rank_update_next_diag_kernel(const dou
 // reciprocal), s_(p mod 4) a chain of fused multiply-adds over the full groups of four p < j, the p left over added to
 // s0's: the four sums of the 16 columns of a block over all earlier blocks are four chains on the matrix cores (k = the
 // four p of a block that share p mod 4), and only the 16 x 16 triangle of the block itself runs on the vector units.
-// One wave takes 16 rows; its solved values stay in LDS as the next blocks' operand (43 KB: four waves per compute
-// unit, or one in the place of a Viterbi workgroup).  It leaves them transposed for the update kernel (Xt, row
+// One wave takes 16 rows; its solved values stay in LDS as the next blocks' operand (45.6 KB in all: three waves per
+// compute unit, or one in the place of a Viterbi workgroup).  It leaves them transposed for the update kernel (Xt, row
 // stride ldx) and forms the panel's columns of the result from them:
 //   kScalar false: L = C blockdiag(C_bb^-1), a chain of 16 fused multiply-adds per value (again the matrix cores)
 //   kScalar true:  L_ij = C_ij / C_jj, and dw_j = C_jj^2

@@ -598,8 +598,8 @@ int qtip_dequantize_linear(qtip_ctx* ctx, const uint16_t* host_trellis, const ui
       in_place = known == hipSuccess && at.type == hipMemoryTypeDevice && at.device == ctx->device;
     }
     // the call's buffers stay in the context's arena: two hipMalloc and hipFree of 4 m n bytes per call (the frees wait
-    // for the whole device) cost more than the kernels (12288 x 12288: 33 ms a call in a
-    // row of calls, of which 4 were the kernels and the copy; now 2.4, of which the pageable copy of the words is 1.3)
+    // for the whole device) can cost more than the kernels (12288 x 12288, fifteen passes: 4.5 ms a call by itself, 12 to
+    // 33 in a row of calls; now 2.4 either way, of which the pageable copy of the words is 1.3)
     ArenaScope memory(&ctx->arena);
     DBuf<uint16_t> tr(words);
     DBuf<float> a(size_t(n) * m), own(in_place ? 0 : size_t(m) * n), d_su(n), d_sv(m);

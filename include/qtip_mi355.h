@@ -74,11 +74,12 @@ int qtip_viterbi_tiles_dev(qtip_ctx* ctx, const float* dev_X, long B, uint16_t* 
  * back-pointer buffer per call, src/quantizer.cpp:38); it is for callers that cannot allocate: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  The kept-metrics workspace, which
  * qtip_viterbi_tiles_dev allocates on its first call (2 MiB per resident workgroup, 768 of them), is here a fixed
- * array inside the library's code object: 32 slots, 63 MiB per device, held until the process ends; its address is
+ * array inside the library's code object: 32 slots, 64 MiB per device, held until the process ends; its address is
  * looked up once per device in qtip_create.  B <= QTIP_NOALLOC_MAX_TILES, else QTIP_E_ARG; 32 tiles run at a time.
  * Results equal qtip_viterbi_tiles_dev's bit for bit.  Asynchronous on the context's stream.  All calls on one device
  * share the array: calls that overlap on one device (two contexts, two streams) race.  Nothing in it needs clearing
- * between calls: a workgroup writes every kept metric before it reads it. */
+ * between calls: a workgroup writes every kept metric before it reads it, and the flags by which two workgroups share a
+ * tile (B <= 16) are cleared by the call, on its stream. */
 #define QTIP_NOALLOC_MAX_TILES 4096
 int qtip_viterbi_tiles_dev_noalloc(qtip_ctx* ctx, const float* dev_X, long B, uint16_t* dev_states,
                                    uint16_t* dev_packed);
@@ -92,9 +93,11 @@ int qtip_viterbi_tiles_dev_noalloc(qtip_ctx* ctx, const float* dev_X, long B, ui
  * than the rounding of 128 terms can move two candidates against each other; a pass that fails the check runs again on
  * fp64 metrics.  The states are those of mode 1 bit for bit.
  * mode 1: fp64 metrics only (viterbi_ref's own arithmetic, src/qtip_core.cpp:129-164).
- * In mode 0 a launch with at most a third as many tiles as the device has workgroup slots (a lone small group)
- * gives every tile a workgroup of 512 threads instead of 256, which shortens a tile's time by about a third; modes
- * 2 and 3 are mode 0 with the 256-thread and the 512-thread form whatever the size of the launch (tests).
+ * In mode 0 a launch that leaves room for it (a lone small group: up to 384 tiles on a device with 256 compute units)
+ * shares every tile between two workgroups, of 512 threads each while every workgroup has a compute unit to itself (up to
+ * 128 tiles), else of 256; a first workgroup whose partner does not answer for half a second goes on alone.  (The call
+ * without allocations has 32 workgroup slots: up to 16 tiles are shared, up to 256 get one workgroup of 512 threads.)
+ * Modes 2 and 3 are mode 0 with one workgroup per tile, of 256 and of 512 threads, whatever the size of the launch (tests).
  * margin_units: 0 = the default of 160; values below 129 give up the guarantee (tests only), UINT32_MAX sends every
  * pass to fp64. */
 int qtip_set_viterbi_mode(qtip_ctx* ctx, int mode, unsigned margin_units);
@@ -349,9 +352,10 @@ int qtip_st_write(qtip_st_writer* w, const char* path, const char* const* metada
 /* fp16 bits of the context's codebook table [512][2] (Codebook::tlut_h, src/qtip_core.hpp:24-31) */
 int qtip_get_tlut_f16(qtip_ctx* ctx, uint16_t* host_tlut_f16);
 
-/* Device memory the context keeps between calls for reuse (per-group buffers of qtip_run_groups and
- * qtip_quantize_group*, about 13 GB after 12288 x 28672 groups, and the same per lane) goes back to the runtime;
- * buffers in use are not touched.  No counterpart in the reference, whose buffers are freed on return
+/* Device memory the context keeps between calls for reuse goes back to the runtime: the per-call buffers of
+ * qtip_run_groups (11 GB after 12288 x 28672 groups, and the same per lane), qtip_quantize_group_h (18 GB),
+ * qtip_nvfp4_quantize_group (8 GB) and qtip_dequantize_linear (1.5 GB).  Another allocator of the process cannot ask for
+ * it: call this before a model's own large allocations.  Buffers in use are not touched.  No counterpart in the reference, whose buffers are freed on return
  * (RAII DBuf, src/gpu.hpp:139-160).  The library does the same by itself when an allocation finds the device out of
  * memory.  *bytes_released may be NULL.  Must not overlap another call on the same context. */
 int qtip_trim(qtip_ctx* ctx, unsigned long long* bytes_released);
