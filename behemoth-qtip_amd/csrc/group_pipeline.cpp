@@ -248,7 +248,8 @@ void run_groups_on(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opt
         T.rht = t_rot[size_t(g)];
         T.ldl_cpu = t_ldl[size_t(g)];
         quantize_group_impl(c, groups[g].nlin, dl[size_t(g)].data(), groups[g].n, groups[g].seed, su[size_t(b)].data(),
-                            creg[size_t(g)], keep_dev ? nullptr : c->ring_HRr[b].p, keep_dev ? nullptr : c->ring_L[b].p, opt, groups[g].outs, &T,
+                            creg[size_t(g)], keep_dev ? nullptr : c->ring_HRr[b].p,
+                            keep_dev ? nullptr : c->ring_L[b].p, opt, groups[g].outs, &T,
                             keep_dev ? c->ring_dHRr[b].p : nullptr, keep_dev ? c->ring_dL[b].p : nullptr);
         if (tms) tms[g] = T;
         {

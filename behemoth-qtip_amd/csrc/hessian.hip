@@ -310,18 +310,18 @@ __global__ __launch_bounds__(512, 1) void syrk_img_small_kernel(const uint16_t* 
   for (int mi = 0; mi < 2; ++mi) {
     float h[16];
     const long gj = long(tj) * kSmallTile + wn * 32 + rl;
-      const long gi0 = long(ti) * kSmallTile + wm * 64 + mi * 32 + 4 * hi;
+    const long gi0 = long(ti) * kSmallTile + wm * 64 + mi * 32 + 4 * hi;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const long gi = gi0 + (v & 3) + 8 * (v >> 2);
-        h[v] = gi < n && gj < n ? H[gi * n + gj] : 0.f;
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const long gi = gi0 + (v & 3) + 8 * (v >> 2);
-        if (gi < n && gj < n) H[gi * n + gj] = h[v] + acc[mi][v];
-      }
+    for (int v = 0; v < 16; ++v) {
+      const long gi = gi0 + (v & 3) + 8 * (v >> 2);
+      h[v] = gi < n && gj < n ? H[gi * n + gj] : 0.f;
     }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const long gi = gi0 + (v & 3) + 8 * (v >> 2);
+      if (gi < n && gj < n) H[gi * n + gj] = h[v] + acc[mi][v];
+    }
+  }
 }
 
 // The batch of a Hessian accumulation (rows x n bf16, row-major) as the stage images of syrk_img_kernel: one workgroup
@@ -483,12 +483,12 @@ void launch_hessian_accumulate(const uint16_t* X, long rows, long n, float* H, D
   QTIP_HIP(hipGetLastError());
   // one tile per compute unit at a time, whatever its size: while the 128 x 128 tiles fit the chip at once (253 of them at
   // n = 2816) a launch of them is over sooner than one of 256 x 256 tiles, which leaves three quarters of the chip idle;
-  // beyond that they come in two and more rounds and
-  // lose.  A call with 1000 / 4096 rows, image included: n = 512 20.7 / 54.5 us (big tiles 28.8 / 76.5), 2560 28.0 / 65.0
+  // beyond that they come in two and more rounds and lose.  A call with 1000 / 4096 rows, image included: n = 512 20.7 / 54.5 us (big tiles 28.8 / 76.5), 2560 28.0 / 65.0
   // (38.4 / 92.9), 2816 28.0 / 67.1 (37.9 / 93.3); with the small tiles at n = 3328 57 / 128 (38 / 95).
   const long small = (n + kSmallTile - 1) / kSmallTile, small_tiles = small * (small + 1) / 2;
   if (small_tiles <= 256) {
-    syrk_img_small_kernel<<<dim3(unsigned(small_tiles)), dim3(512), kSmallLdsBytes, s>>>(image.p, int(stages), n, H, g.tiles);
+    syrk_img_small_kernel<<<dim3(unsigned(small_tiles)), dim3(512), kSmallLdsBytes, s>>>(image.p, int(stages), n, H,
+                                                                                        g.tiles);
   } else {
     syrk_img_kernel<false><<<dim3(g.grid), dim3(256), kImgLdsBytes, s>>>(image.p, image.p, int(stages), n, H, nullptr,
                                                                         g.tiles, g.patch_cols);

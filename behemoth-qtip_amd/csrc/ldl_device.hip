@@ -236,8 +236,8 @@ __global__ __launch_bounds__(256, 3) void rank_update_lower_kernel(const double*
 // with the diagonal block's 0.2 ms under the update - and, beside the quantization of another group, whose Viterbi
 // workgroups fill the chip, a launch waits some milliseconds for their places, so the launches are what the factorization
 // takes there (12288 x 28672 groups in a row: 1.34 -> 1.28 s a factorization; alone at n = 28672 169 -> 156 ms).
-__global__ __launch_bounds__(256, 3) void rank_update_next_diag_kernel(const double* __restrict__ Xt, long ldx, int nr, int kb,
-                                                                       double* __restrict__ C, long ldc,
+__global__ __launch_bounds__(256, 3) void rank_update_next_diag_kernel(const double* __restrict__ Xt, long ldx, int nr,
+                                                                       int kb, double* __restrict__ C, long ldc,
                                                                        double* __restrict__ rdiag, double* __restrict__ inv,
                                                                        int* __restrict__ bad) {
   __shared__ __attribute__((aligned(16))) UpdateLds S;
@@ -403,7 +403,8 @@ __global__ __launch_bounds__(64) void ldl_solve_kernel(const double* __restrict_
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const int p = 4 * m + q;
-        o = __builtin_amdgcn_mfma_f64_16x16x4f64(X[(16 * b + p) * kXStride + r], inv[long(16 * b + p) * 16 + r], o, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f64_16x16x4f64(X[(16 * b + p) * kXStride + r], inv[long(16 * b + p) * 16 + r], o, 0, 0,
+                                                 0);
       }
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -427,7 +428,8 @@ namespace {
 // receives the block LDL's factor, or with dw the scalar one's; everything outside its strict (block) lower triangle is
 // zero.  host_L (optional) receives L as well: the rows of a panel's diagonal block are final once the panel is solved, and
 // go down from a stream of their own, 1024 at a time, while the factorization runs on (n = 28672 into pageable memory:
-// host buffers in and out 0.59 -> 0.44 s, page-locked L alone 216 -> 161 ms).  Waits for the stream; false if the matrix is not positive definite.
+// host buffers in and out 0.59 -> 0.44 s, page-locked L alone 216 -> 161 ms).  Waits for the stream; false if the matrix
+// is not positive definite.
 bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s, float* host_L = nullptr) {
   struct RowsDown {  // whatever ends the call, nothing of it is left behind
     hipStream_t stream = nullptr;
@@ -454,10 +456,9 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s, f
       QTIP_HIP(hipGetLastError());
     }
     const dim3 grid(unsigned((kb + nr) / 16));
-    if (dw)
-      ldl_solve_kernel<true><<<grid, dim3(64), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_Xt.p, nr, L + k * n + k, n, dw + k, c->ldl_bad.p);
-    else
-      ldl_solve_kernel<false><<<grid, dim3(64), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_Xt.p, nr, L + k * n + k, n, nullptr, c->ldl_bad.p);
+    const auto solve = dw ? ldl_solve_kernel<true> : ldl_solve_kernel<false>;
+    solve<<<grid, dim3(64), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_Xt.p, nr, L + k * n + k, n, dw ? dw + k : nullptr,
+                                    c->ldl_bad.p);
     QTIP_HIP(hipGetLastError());
     if (host_L && (nr <= 0 || (k + kb) % 1024 == 0)) {
       hipEvent_t e;
@@ -539,7 +540,8 @@ void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double s
   QTIP_HIP(hipGetLastError());
   add_to_diagonal_kernel<<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, s>>>(c->ldl_A.p, n, creg);
   QTIP_HIP(hipGetLastError());
-  if (!factor_on_device(c, n, dev_L, dev_dw, s, host_L)) throw Error(QTIP_E_NOT_PD, "NVFP4 calibration: Hessian not positive definite");
+  if (!factor_on_device(c, n, dev_L, dev_dw, s, host_L))
+    throw Error(QTIP_E_NOT_PD, "NVFP4 calibration: Hessian not positive definite");
   if (host_dw) {
     QTIP_HIP(hipMemcpyAsync(host_dw, dev_dw, size_t(n) * 4, hipMemcpyDeviceToHost, s));
     QTIP_HIP(hipStreamSynchronize(s));
@@ -564,8 +566,8 @@ void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* h
     c->ldl_H.ensure(nn);
     QTIP_HIP(hipMemcpyAsync(c->ldl_H.p, host_HRr, nn * 4, hipMemcpyHostToDevice, s));
   }
-  symmetrize_lower_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n)), dim3(256), 0, s>>>(dev_HRr ? dev_HRr : c->ldl_H.p, n,
-                                                                                              c->ldl_A.p);
+  symmetrize_lower_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n)), dim3(256), 0, s>>>(
+      dev_HRr ? dev_HRr : c->ldl_H.p, n, c->ldl_A.p);
   QTIP_HIP(hipGetLastError());
   if (!factor_on_device(c, n, dev_L, nullptr, s, host_L)) throw Error(QTIP_E_NOT_PD, "block LDL failed (H not PD)");
 }

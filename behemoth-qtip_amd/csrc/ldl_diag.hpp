@@ -28,7 +28,8 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
 
 using DiagLds = double[kSub][kDiag];  // [column of the sub-panel][row of the block], 32 KB
 __device__ __forceinline__ void factor_diag_block(DiagLds& P, double* __restrict__ A, long ld, int kb,
-                                                  double* __restrict__ rdiag, double* __restrict__ inv, int* __restrict__ bad) {
+                                                  double* __restrict__ rdiag, double* __restrict__ inv,
+                                                  int* __restrict__ bad) {
   const int t = threadIdx.x, lane = t & 63, l16 = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   bool ok = true;

@@ -87,7 +87,8 @@ __global__ __launch_bounds__(kBlockRows * kScaleTries) void nv_buffer_kernel(
     const int left = int(c0 - cb);  // columns of the buffer left of the block
     if (calibrate)
       for (int idx = threadIdx.x; idx < 16 * kBuffer; idx += blockDim.x)
-        if ((idx & (kBuffer - 1)) < left + 16) Lt[idx / kBuffer][idx & (kBuffer - 1)] = L[(c0 + idx / kBuffer) * n + cb + (idx & (kBuffer - 1))];
+        if ((idx & (kBuffer - 1)) < left + 16)
+          Lt[idx / kBuffer][idx & (kBuffer - 1)] = L[(c0 + idx / kBuffer) * n + cb + (idx & (kBuffer - 1))];
     float w[16], t0[16], err[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) w[k] = live ? WT[(c0 + k) * m + r] : 0.f;
@@ -144,7 +145,8 @@ __global__ __launch_bounds__(kBlockRows * kScaleTries) void nv_buffer_kernel(
         }
       }
     }
-    __syncthreads();  // (also before the costs of the next block, which has no other barrier in front of them when calibrate = 0)
+    // (also before the costs of the next block, which has no other barrier in front of them when calibrate = 0)
+    __syncthreads();
     if (calibrate && left) {
       float e[16];
 #pragma unroll
@@ -163,7 +165,8 @@ __global__ __launch_bounds__(kBlockRows * kScaleTries) void nv_buffer_kernel(
 // What the matrix's global scale is made from, and whether every value is finite: the largest bit pattern of |w| over the
 // matrix (the order of finite magnitudes is that of their bits, and those of infinities and NaNs lie above), one atomic
 // maximum per wave.  On one host core this was 9 ms of a 4096 x 4096 call; here 0.11 ms on the copy that is there anyway.
-__global__ __launch_bounds__(256) void nv_largest_kernel(const float* __restrict__ w, long count, unsigned* __restrict__ top) {
+__global__ __launch_bounds__(256) void nv_largest_kernel(const float* __restrict__ w, long count,
+                                                         unsigned* __restrict__ top) {
   unsigned most = 0;
   const long step = long(gridDim.x) * 256;
   for (long i = long(blockIdx.x) * 256 + threadIdx.x; i < count; i += step) {
@@ -186,9 +189,9 @@ __global__ __launch_bounds__(256) void nv_largest_kernel(const float* __restrict
 // so three of them find the error values in the vector L1.  The 16 x COLS piece of L of a block sits in COLS registers,
 // row j in lane j of every 16 lanes, and reaches the fused multiply-adds as their broadcast operand (DPP row_newbcast).
 // The scalar cache, which brought it before, serves a wave's 16 small pieces per block too slowly.  The values are
-// fetched DEPTH - 1 blocks ahead.  Bound by the vector pipes then, one wave per SIMD or a few: 88 us a
-// buffer of a 4096 x 4096 matrix on average, 144 before; 248 blocks behind the first buffer take 0.17 ms, 0.34 before.  COLS: 8, or 4 where 8
-// would not give every SIMD a wave (m < 4096).
+// fetched DEPTH - 1 blocks ahead.  Bound by the vector pipes then, one wave per SIMD or a few: 88 us a buffer of a
+// 4096 x 4096 matrix on average, 144 before; 248 blocks behind the first buffer take 0.17 ms, 0.34 before.  COLS: 8, or 4
+// where 8 would not give every SIMD a wave (m < 4096).
 template <int COLS, int DEPTH>
 __global__ __launch_bounds__(256) void nv_gather_kernel(float* __restrict__ FT, long m, long n, long cb,
                                                         const float* __restrict__ ET, const float* __restrict__ L) {
@@ -211,9 +214,10 @@ __global__ __launch_bounds__(256) void nv_gather_kernel(float* __restrict__ FT, 
     float acc[COLS];
 #pragma unroll
     for (int c = 0; c < COLS; ++c) acc[c] = 0.f;
-// four j at a time: v_fmac_f32 with the broadcast in its first operand (the compiler does not fold the broadcast into a
+    // four j at a time: v_fmac_f32 with the broadcast in its first operand (the compiler does not fold the broadcast into a
     // fused multiply-add by itself); s_nop 1: the wait a vector write of that operand, a copy say, would need before it
-#define QTIP_NV_1(ACC, LV, EV, J) "v_fmac_f32_dpp %" #ACC ", %" #LV ", %" #EV " row_newbcast:" #J " row_mask:0xf bank_mask:0xf\n\t"
+#define QTIP_NV_1(ACC, LV, EV, J) \
+  "v_fmac_f32_dpp %" #ACC ", %" #LV ", %" #EV " row_newbcast:" #J " row_mask:0xf bank_mask:0xf\n\t"
 #define QTIP_NV_4C(EV, J) QTIP_NV_1(0, 4, EV, J) QTIP_NV_1(1, 5, EV, J) QTIP_NV_1(2, 6, EV, J) QTIP_NV_1(3, 7, EV, J)
 #define QTIP_NV_4J(C, J0, J1, J2, J3)                                                                                 \
   asm("s_nop 1\n\t" QTIP_NV_4C(8, J0) QTIP_NV_4C(9, J1) QTIP_NV_4C(10, J2) QTIP_NV_4C(11, J3)                         \
@@ -282,8 +286,8 @@ void launch_nvfp4_buffer(const float* WT, const float* FT, long m, long n, long 
   QTIP_HIP(hipGetLastError());
 }
 void launch_nvfp4_gather(float* FT, long m, long n, long cb, const float* ET, const float* L, hipStream_t s) {
-  QTIP_REQUIRE(cb >= 0 && cb % 16 == 0 && cb + kBuffer < n && n % 16 == 0, "nvfp4 gather: buffer [%ld, %ld) outside [0, %ld)",
-               cb, cb + kBuffer, n);
+  QTIP_REQUIRE(cb >= 0 && cb % 16 == 0 && cb + kBuffer < n && n % 16 == 0,
+               "nvfp4 gather: buffer [%ld, %ld) outside [0, %ld)", cb, cb + kBuffer, n);
   const unsigned rows = unsigned((m + 63) / 64);
   if (m < 4096) nv_gather_kernel<4, 4><<<dim3(rows, kBuffer / 4 / 4), dim3(256), 0, s>>>(FT, m, n, cb, ET, L);
   else nv_gather_kernel<8, 3><<<dim3(rows, kBuffer / 8 / 4), dim3(256), 0, s>>>(FT, m, n, cb, ET, L);

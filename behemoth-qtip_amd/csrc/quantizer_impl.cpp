@@ -223,8 +223,9 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
           if (nch > 1) job.wide = 0;  // the chains fill the chip between them: one launch is not the measure
           hipEvent_t t0 = nullptr, t1 = nullptr;
           if (vit_seconds) t0 = timed.add(hipEventDefault), t1 = timed.add(hipEventDefault);
-          one_workgroup_per_tile = launch_viterbi_tiles(job, c->d_entry_d, c->d_entry_f,
-                                                        c->vit_ws.p + viterbi_workspace_bytes(C.slot0), C.slots, C.s, t0, t1);
+          one_workgroup_per_tile =
+              launch_viterbi_tiles(job, c->d_entry_d, c->d_entry_f, c->vit_ws.p + viterbi_workspace_bytes(C.slot0), C.slots,
+                                   C.s, t0, t1);
         }
         QTIP_HIP(hipEventRecord(pace[k][nbuf_done % (kAhead + 1)], C.s));
       }

@@ -46,17 +46,20 @@ struct qtip_ctx {
   int side_streams = 0;         // how many of chain_stream[0], chain_stream[1], ldl_stream (in this order) were found
                                 // to run beside the context's stream and beside each other when the context was made
   bool chains_checked = false;
-  double vit_tile_us = 800.0;   // a resident 256-thread Viterbi workgroup's time per tile, from the last timed LDLQ call of that kind
+  // a resident 256-thread Viterbi workgroup's time per tile, from the last timed LDLQ call with launches of that kind
+  double vit_tile_us = 800.0;
   qtipmi::Rht rht;
   qtipmi::DBuf<double> scratch;
   qtipmi::DBuf<uint16_t> hess_img;  // a batch of qtip_hessian_accumulate_dev as the stage images of its update kernel
-  qtipmi::HBuf<float> ring_HRr[3], ring_L[3];  // page-locked staging of run_groups with the LDL on the host, kept between calls
+  // page-locked staging of run_groups with the LDL on the host, kept between calls
+  qtipmi::HBuf<float> ring_HRr[3], ring_L[3];
   // host inputs of qtip_run_groups on their way to the device: a stream and four staging slots (Hessian, weights)
   static constexpr int kUploadSlots = 4;
   hipStream_t upload_stream = nullptr;
   qtipmi::DBuf<float> up_H[kUploadSlots];
   qtipmi::DBuf<uint8_t> up_W[kUploadSlots];
-  qtipmi::DBuf<float> ring_dHRr[3], ring_dL[3];  // run_groups with the LDL on the device: rotated Hessians and factors stay here
+  // run_groups with the LDL on the device: rotated Hessians and factors stay here
+  qtipmi::DBuf<float> ring_dHRr[3], ring_dL[3];
   // LDL on the device (ldl_device.hip): own stream, fp64 work matrix, fp32 upload of HRr, a panel's solved rows
   // transposed, the reciprocals and 16 x 16 inverses of its diagonal block, a flag, the factor on its way to a caller's
   // host memory; allocated on first use

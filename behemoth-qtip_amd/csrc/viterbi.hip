@@ -1134,39 +1134,41 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
                                              const uint32_t* tl, float& expected, int first_pass, int passes_end,
                                              bool fp64_only) {
   const int u = threadIdx.x & (kThreads - 1);
-    // pass 1 on the sequence rotated by half its length, free ends, traced back to step 64 for the overlap group;
-    // pass 2 on the sequence itself, tail-biting through that group, traced back in full.  One loop, so that the
-    // step bodies exist once in the instruction cache.
-    int ov = first_pass > 0 ? sm.overlap : -1;
+  // pass 1 on the sequence rotated by half its length, free ends, traced back to step 64 for the overlap group;
+  // pass 2 on the sequence itself, tail-biting through that group, traced back in full.  One loop, so that the
+  // step bodies exist once in the instruction cache.
+  int ov = first_pass > 0 ? sm.overlap : -1;
 #pragma nounroll
-    for (int pass = first_pass; pass < passes_end; ++pass) {
-      const int roll = pass == 0 ? kSeq / 2 : 0;
-      bool done = false;
-      if (job.mode == 0 && !fp64_only) {
-        uint32_t* const hist32 = reinterpret_cast<uint32_t*>(hist);
-        uint32_t flag = 0;
-        // (the same in every thread; said so, so that it lives in scalar registers)
-        const int unit_log2 = __builtin_amdgcn_readfirstlane(unit_log2_for(expected, pass == 0 ? 2.f : 1.125f));
-        const Unit unit = unit_of(unit_log2);
-        if (pass == 0) {
-          forward_pass32<true, kWide>(sm, entry_d, roll, -1, hist32, 62, unit);
-          const uint32_t winner = sm.red32[0][0];
-          flag |= uint32_t(sm.red32[0][1] < job.margin) | uint32_t(winner >= kWinnerMax);
-          const uint32_t s = trace_back32<true, kWide>(sm, entry_d, hist32, roll, sm.red32[0][2], 64, false, job.margin, flag, tl, unit);
-          if (!flag && u == 0) sm.overlap = int(s & 0xfffu);  // s is the state of step 63
-          // what the tail-biting pass of this block and the free pass of the next may expect (a winner that did
-          // not fit is replaced by the true one when the pass is repeated on fp64 metrics)
-          expected = __builtin_ldexpf(float(winner), -unit_log2);
-        } else {
-          forward_pass32<false, kWide>(sm, entry_d, roll, ov, hist32, 0, unit);
-          const uint32_t s = trace_back32<false, kWide>(sm, entry_d, hist32, roll, uint32_t(ov), 2, true, job.margin, flag, tl, unit);
-          // s is the state of step 1; at step 0 the one predecessor group with a finite initial metric is ov
-          if (!flag && u == 0) sm.st[0] = uint16_t((s >> 4) | ((uint32_t(ov) >> 8) << 12));
-        }
-        done = !flag;
-        if (flag && threadIdx.x == 0 && job.stats) atomicAdd(job.stats + pass, 1u);
+  for (int pass = first_pass; pass < passes_end; ++pass) {
+    const int roll = pass == 0 ? kSeq / 2 : 0;
+    bool done = false;
+    if (job.mode == 0 && !fp64_only) {
+      uint32_t* const hist32 = reinterpret_cast<uint32_t*>(hist);
+      uint32_t flag = 0;
+      // (the same in every thread; said so, so that it lives in scalar registers)
+      const int unit_log2 = __builtin_amdgcn_readfirstlane(unit_log2_for(expected, pass == 0 ? 2.f : 1.125f));
+      const Unit unit = unit_of(unit_log2);
+      if (pass == 0) {
+        forward_pass32<true, kWide>(sm, entry_d, roll, -1, hist32, 62, unit);
+        const uint32_t winner = sm.red32[0][0];
+        flag |= uint32_t(sm.red32[0][1] < job.margin) | uint32_t(winner >= kWinnerMax);
+        const uint32_t s = trace_back32<true, kWide>(sm, entry_d, hist32, roll, sm.red32[0][2], 64, false, job.margin, flag,
+                                                     tl, unit);
+        if (!flag && u == 0) sm.overlap = int(s & 0xfffu);  // s is the state of step 63
+        // what the tail-biting pass of this block and the free pass of the next may expect (a winner that did
+        // not fit is replaced by the true one when the pass is repeated on fp64 metrics)
+        expected = __builtin_ldexpf(float(winner), -unit_log2);
+      } else {
+        forward_pass32<false, kWide>(sm, entry_d, roll, ov, hist32, 0, unit);
+        const uint32_t s = trace_back32<false, kWide>(sm, entry_d, hist32, roll, uint32_t(ov), 2, true, job.margin, flag, tl,
+                                                      unit);
+        // s is the state of step 1; at step 0 the one predecessor group with a finite initial metric is ov
+        if (!flag && u == 0) sm.st[0] = uint16_t((s >> 4) | ((uint32_t(ov) >> 8) << 12));
       }
-      if (!done) {
+      done = !flag;
+      if (flag && threadIdx.x == 0 && job.stats) atomicAdd(job.stats + pass, 1u);
+    }
+    if (!done) {
       forward_pass(sm, entry_d, roll, ov, hist, pass == 0 ? 62 : 0);
       if (pass == 0) expected = sm.final_metric;  // the true winner, also where a 32-bit pass could not hold it
       {
@@ -1183,42 +1185,43 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
           }
         }
       }
-      }
-      __syncthreads();
-      ov = sm.overlap;
     }
+    __syncthreads();
+    ov = sm.overlap;
+  }
 }
 
 // States, packed words, decoded values and residual images of one block, from sm.st.
-__device__ __forceinline__ void block_outputs(const Smem& sm, const TileJob& job, const float* __restrict__ entry_f, long tile,
-                                              int blk, long col0) {
+__device__ __forceinline__ void block_outputs(const Smem& sm, const TileJob& job, const float* __restrict__ entry_f,
+                                              long tile, int blk, long col0) {
   const int u = threadIdx.x & (kThreads - 1);
   const bool first_half = threadIdx.x < kThreads;  // global results are written once
-    if (job.states && first_half && u < kSteps) job.states[(tile * job.q_tile_stride + job.q_offset + blk) * kSteps + u] = sm.st[u];
-    if (job.packed && first_half && u < kWords) {
-      uint32_t v;
-      if (u == 0) v = sm.st[0];
-      else {
-        v = 0;
+  if (job.states && first_half && u < kSteps)
+    job.states[(tile * job.q_tile_stride + job.q_offset + blk) * kSteps + u] = sm.st[u];
+  if (job.packed && first_half && u < kWords) {
+    uint32_t v;
+    if (u == 0) v = sm.st[0];
+    else {
+      v = 0;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v = (v << 4) | (sm.st[4 * u + k - 3] & 15u);
-      }
-      job.packed[tile * kWords + u] = uint16_t(v);
+      for (int k = 0; k < 4; ++k) v = (v << 4) | (sm.st[4 * u + k - 3] & 15u);
     }
-    if (job.hatWT && first_half) {
-      const uint32_t s = sm.st[u >> 1];
-      const uint32_t e = ((s * (s + 1u)) >> 6) & 1023u;
-      const int q = perm_fwd(u), r = q >> 4, c = q & 15;
-      const long wi = (col0 + c) * job.ldw + tile * 16 + r;
-      const float hv = entry_f[2 * e + (u & 1)];
-      job.hatWT[wi] = hv;
-      if (job.dimg_h) {
-        uint32_t hi, lo;
-        bf16_split_bits(job.WT[wi] - hv, hi, lo);
-        const long di = (tile * 16 + r) * job.ldd + col0 + c;
-        job.dimg_h[di] = uint16_t(hi), job.dimg_l[di] = uint16_t(lo);
-      }
+    job.packed[tile * kWords + u] = uint16_t(v);
+  }
+  if (job.hatWT && first_half) {
+    const uint32_t s = sm.st[u >> 1];
+    const uint32_t e = ((s * (s + 1u)) >> 6) & 1023u;
+    const int q = perm_fwd(u), r = q >> 4, c = q & 15;
+    const long wi = (col0 + c) * job.ldw + tile * 16 + r;
+    const float hv = entry_f[2 * e + (u & 1)];
+    job.hatWT[wi] = hv;
+    if (job.dimg_h) {
+      uint32_t hi, lo;
+      bf16_split_bits(job.WT[wi] - hv, hi, lo);
+      const long di = (tile * 16 + r) * job.ldd + col0 + c;
+      job.dimg_h[di] = uint16_t(hi), job.dimg_l[di] = uint16_t(lo);
     }
+  }
 }
 
 // kWide: 512 threads per tile, one workgroup per compute unit, for launches that cannot fill the chip anyway (a lone
@@ -1238,19 +1241,19 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
   }
   double* hist = hist_all + size_t(blockIdx.x) * kSlotWords;
   for (long tile = blockIdx.x; tile < job.tiles; tile += gridDim.x) {
-  float expected = 0.f;  // the free pass's winner of this tile row's previous column block (0: none yet)
-  for (int blk = job.blocks - 1; blk >= 0; --blk) {
-    // the column block of this turn; the hatWT values the previous turn wrote for this tile row are visible after
-    // the barrier that ended it
-    const long col0 = job.col0 + 16 * blk;
-    if (job.X) sm.x[u] = job.X[tile * kSeq + u];
-    else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
-    else tile_targets<float>(sm, job, col0, tile, job.prod32);
-    __syncthreads();
-    block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
-    block_outputs(sm, job, entry_f, tile, blk, col0);
-    __syncthreads();
-  }
+    float expected = 0.f;  // the free pass's winner of this tile row's previous column block (0: none yet)
+    for (int blk = job.blocks - 1; blk >= 0; --blk) {
+      // the column block of this turn; the hatWT values the previous turn wrote for this tile row are visible after
+      // the barrier that ended it
+      const long col0 = job.col0 + 16 * blk;
+      if (job.X) sm.x[u] = job.X[tile * kSeq + u];
+      else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
+      else tile_targets<float>(sm, job, col0, tile, job.prod32);
+      __syncthreads();
+      block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
+      block_outputs(sm, job, entry_f, tile, blk, col0);
+      __syncthreads();
+    }
   }
 }
 
@@ -1280,9 +1283,9 @@ __device__ __forceinline__ void backward_pass32(Smem& sm, const double* __restri
                                                 uint32_t* __restrict__ hist, const Unit unit) {
   // A thread owns metric column c (the sixteen groups 16 c + e after the step; they continue the sixteen groups 256 h + c
   // before it) with its mirror 255 - c, and the four (256 threads: eight) h = kH r + i: per j = 16 c + e the table values
-  // of these h serve group 256 h + c (with B[j]) and its mirror (with B[4095 - j]).  The table and the lanes' columns are the tail-biting
-  // forward pass's, so its reads are free of bank conflicts as there; metric j sits at m32_slot(j / 16, j mod 16), which
-  // makes the column reads conflict-free and leaves a four-way conflict in the writes.
+  // of these h serve group 256 h + c (with B[j]) and its mirror (with B[4095 - j]).  The table and the lanes' columns are
+  // the tail-biting forward pass's, so its reads are free of bank conflicts as there; metric j sits at m32_slot(j / 16,
+  // j mod 16), which makes the column reads conflict-free and leaves a four-way conflict in the writes.
   constexpr int kT = kWide ? 2 * kThreads : kThreads, kEnt = 1024 / kT, kH = kWide ? 4 : 8;
   const int t = kWide ? opaque_tid_wide() : opaque_tid();
   const int p = t & 127, r = t >> 7;
@@ -1351,7 +1354,8 @@ __device__ __forceinline__ void backward_pass32(Smem& sm, const double* __restri
         mirror[i] = min3u(mirror[i], sat_add(v0[i], MB[15 - e]), sat_add(v1[i], MB[14 - e]));
       }
     }
-    if (kFree && it == kSteps - 1) {  // final states of 32768 and more do not count: groups of 2048 and more (r: the same in a wave)
+    // final states of 32768 and more do not count: groups of 2048 and more (r: the same in a wave)
+    if (kFree && it == kSteps - 1) {
 #pragma unroll
       for (int i = 0; i < kH; ++i) {
         own[i] = kH * r >= 8 ? kSat : own[i];
@@ -1387,12 +1391,12 @@ __device__ __forceinline__ uint32_t back_index(uint32_t g) {
 }
 
 // From group g entering step 64 to the group ov after step 127, two steps a round, in the scheme of trace_back32 (kWide:
-// its streamed form) with the directions exchanged; records the states of steps 64 .. 127.  A candidate of step t is a sum of 128 - t
-// rounded terms, and thr, which 128 terms need, shrinks by one unit per term less.
+// its streamed form) with the directions exchanged; records the states of steps 64 .. 127.  A candidate of step t is a sum
+// of 128 - t rounded terms, and thr, which 128 terms need, shrinks by one unit per term less.
 template <bool kWide>
-__device__ __forceinline__ void trace_forward32(Smem& sm, const double* __restrict__ entry_d, const uint32_t* __restrict__ hist,
-                                                uint32_t g, uint32_t ov, uint32_t thr, uint32_t& flag, const uint32_t* tl,
-                                                const Unit unit) {
+__device__ __forceinline__ void trace_forward32(Smem& sm, const double* __restrict__ entry_d,
+                                                const uint32_t* __restrict__ hist, uint32_t g, uint32_t ov, uint32_t thr,
+                                                uint32_t& flag, const uint32_t* tl, const Unit unit) {
   const uint32_t tid = uint32_t(opaque_tid());
   const uint32_t lane = tid & 63u, wave = tid >> 6, dp = lane & 15u, d = 4u * wave + (lane >> 4);
   constexpr int kBufs = 3, kLoads = kGroups / (4 * 2 * kThreads), kRows = 31;
@@ -1658,7 +1662,8 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
       if (!hear(n + 4)) return;
       middle(1);
       uint32_t flag = 0;
-      trace_forward32<kWide>(sm, entry_d, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), ov, job.margin, flag, tl, unit);
+      trace_forward32<kWide>(sm, entry_d, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), ov, job.margin, flag, tl,
+                             unit);
       if (tid < 64) pair_put(&mine->states[tid], sm.st[64 + tid]);
       if (tid == 0) pair_put(&mine->doubt, flag);
       tell(n + 5);
@@ -1700,8 +1705,9 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
       if (!hear(n + 4)) return false;
       middle(1);
       uint32_t flag = uint32_t(b2 - b1 < job.margin) | uint32_t(b1 >= kWinnerMax);
-      const uint32_t s = trace_back32<false, kWide>(sm, entry_d, hist32, 0, uint32_t(__builtin_amdgcn_readfirstlane(int(bj))), 2,
-                                                   true, job.margin, flag, tl, unit, kSteps / 2 - 1);
+      const uint32_t middle_group = uint32_t(__builtin_amdgcn_readfirstlane(int(bj)));
+      const uint32_t s = trace_back32<false, kWide>(sm, entry_d, hist32, 0, middle_group, 2, true, job.margin, flag, tl, unit,
+                                                    kSteps / 2 - 1);
       // s is the state of step 1; at step 0 the one predecessor group with a finite initial metric is ov
       if (tid == 0) sm.st[0] = uint16_t((s >> 4) | ((ov >> 8) << 12));
       if (!hear(n + 5)) return false;
