@@ -28,9 +28,10 @@ namespace {
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
-// A[i][j] = (H[i][j] + H[j][i]) / 2 in fp64, lower triangle (symmetrize_lower_host)
-__global__ void symmetrize_lower_kernel(const float* __restrict__ H, long n, double* __restrict__ A) {
+// A[i][j] = (H[i][j] + H[j][i]) / 2 in fp64, lower triangle (symmetrize_lower_host); the factorization's flag is cleared
+__global__ void symmetrize_lower_kernel(const float* __restrict__ H, long n, double* __restrict__ A, int* __restrict__ bad) {
   const long j = long(blockIdx.x) * blockDim.x + threadIdx.x, i = blockIdx.y;
+  if (i == 0 && j == 0) *bad = 0;
   if (j > i || j >= n) return;
   A[i * n + j] = 0.5 * (double(H[i * n + j]) + double(H[j * n + i]));
 }
@@ -424,24 +425,26 @@ __global__ void add_to_diagonal_kernel(double* __restrict__ A, long n, double v)
 }  // namespace
 
 namespace {
-// Factors the symmetric matrix whose lower triangle lies in c->ldl_A (n x n) on stream s.  L (n x n fp32, device)
+// Factors the symmetric matrix whose lower triangle lies in c->ldl_A (n x n) on stream s, *c->ldl_bad cleared.  L (n x n fp32, device)
 // receives the block LDL's factor, or with dw the scalar one's; everything outside its strict (block) lower triangle is
 // zero.  host_L (optional) receives L as well: the rows of a panel's diagonal block are final once the panel is solved, and
 // go down from a stream of their own, 1024 at a time, while the factorization runs on (n = 28672 into pageable memory:
-// host buffers in and out 0.59 -> 0.44 s, page-locked L alone 216 -> 161 ms).  Waits for the stream; false if the matrix
-// is not positive definite.
+// host buffers in and out 0.59 -> 0.44 s, page-locked L alone 216 -> 161 ms; up to n = 1024 there is one such block, and it
+// follows on s).  Waits for the stream; false if the matrix is not positive definite.
 bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s, float* host_L = nullptr) {
   struct RowsDown {  // whatever ends the call, nothing of it is left behind
     hipStream_t stream = nullptr;
     std::vector<std::pair<long, hipEvent_t>> ready;  // (rows final, after this event)
     ~RowsDown() {
-      if (stream) (void)hipStreamSynchronize(stream), (void)hipStreamDestroy(stream);
+      if (stream) (void)hipStreamSynchronize(stream);
       for (auto& r : ready) (void)hipEventDestroy(r.second);
     }
   } down;
-  if (host_L) QTIP_HIP(hipStreamCreateWithFlags(&down.stream, hipStreamNonBlocking));
-  int bad = 0;
-  QTIP_HIP(hipMemcpyAsync(c->ldl_bad.p, &bad, sizeof bad, hipMemcpyHostToDevice, s));
+  constexpr long kRowsDown = 1024;
+  if (host_L && n > kRowsDown) {
+    if (!c->ldl_down_stream) QTIP_HIP(hipStreamCreateWithFlags(&c->ldl_down_stream, hipStreamNonBlocking));
+    down.stream = c->ldl_down_stream;
+  }
   QTIP_HIP(hipMemsetAsync(L, 0, size_t(n) * n * sizeof(float), s));
   bool diag_done = false;  // this panel's diagonal block came with the update before it
   int turn = 0;            // the reciprocals and inverses of a panel and of the one factored beside its update
@@ -460,7 +463,7 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s, f
     solve<<<grid, dim3(64), 0, s>>>(D, n, kb, rdiag, inv, c->ldl_Xt.p, nr, L + k * n + k, n, dw ? dw + k : nullptr,
                                     c->ldl_bad.p);
     QTIP_HIP(hipGetLastError());
-    if (host_L && (nr <= 0 || (k + kb) % 1024 == 0)) {
+    if (down.stream && (nr <= 0 || (k + kb) % kRowsDown == 0)) {
       hipEvent_t e;
       QTIP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       down.ready.emplace_back(k + kb, e);
@@ -492,7 +495,9 @@ bool factor_on_device(qtip_ctx* c, long n, float* L, float* dw, hipStream_t s, f
                             hipMemcpyDeviceToHost, down.stream));
     row = r.first;
   }
-  if (host_L) QTIP_HIP(hipStreamSynchronize(down.stream));
+  if (down.stream) QTIP_HIP(hipStreamSynchronize(down.stream));
+  else if (host_L) QTIP_HIP(hipMemcpyAsync(host_L, L, size_t(n) * n * sizeof(float), hipMemcpyDeviceToHost, s));
+  int bad = 0;
   QTIP_HIP(hipMemcpyAsync(&bad, c->ldl_bad.p, sizeof bad, hipMemcpyDeviceToHost, s));
   QTIP_HIP(hipStreamSynchronize(s));
   return bad == 0;
@@ -536,7 +541,8 @@ void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double s
   }
   c->ldl_H.ensure(nn);
   QTIP_HIP(hipMemcpyAsync(c->ldl_H.p, host_H, size_t(n) * n * 4, hipMemcpyHostToDevice, s));
-  symmetrize_lower_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n)), dim3(256), 0, s>>>(c->ldl_H.p, n, c->ldl_A.p);
+  symmetrize_lower_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n)), dim3(256), 0, s>>>(c->ldl_H.p, n, c->ldl_A.p,
+                                                                                           c->ldl_bad.p);
   QTIP_HIP(hipGetLastError());
   add_to_diagonal_kernel<<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, s>>>(c->ldl_A.p, n, creg);
   QTIP_HIP(hipGetLastError());
@@ -567,7 +573,7 @@ void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* h
     QTIP_HIP(hipMemcpyAsync(c->ldl_H.p, host_HRr, nn * 4, hipMemcpyHostToDevice, s));
   }
   symmetrize_lower_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n)), dim3(256), 0, s>>>(
-      dev_HRr ? dev_HRr : c->ldl_H.p, n, c->ldl_A.p);
+      dev_HRr ? dev_HRr : c->ldl_H.p, n, c->ldl_A.p, c->ldl_bad.p);
   QTIP_HIP(hipGetLastError());
   if (!factor_on_device(c, n, dev_L, nullptr, s, host_L)) throw Error(QTIP_E_NOT_PD, "block LDL failed (H not PD)");
 }

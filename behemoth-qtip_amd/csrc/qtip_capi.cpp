@@ -198,6 +198,11 @@ void destroy_context(qtip_ctx* ctx) {
     (void)hipStreamDestroy(ctx->ldl_stream);
   }
   ctx->ldl_stream = nullptr;
+  if (ctx->ldl_down_stream) {
+    (void)hipStreamSynchronize(ctx->ldl_down_stream);
+    (void)hipStreamDestroy(ctx->ldl_down_stream);
+    ctx->ldl_down_stream = nullptr;
+  }
   if (ctx->upload_stream) {
     (void)hipStreamSynchronize(ctx->upload_stream);
     (void)hipStreamDestroy(ctx->upload_stream);
@@ -694,7 +699,8 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
     QTIP_REQUIRE(ctx != nullptr, "nvfp4_prepare_device_updates: bad arguments");
     DeviceGuard g(ctx);
     QTIP_REQUIRE(host_H && host_L && host_dw && n > 0 && n % 16 == 0, "nvfp4_prepare (device): bad arguments (n = %d)", n);
-    nvfp4_prepare_device_impl(ctx, host_H, n, sigma_reg, nullptr, nullptr, host_L, host_dw);
+    if (n <= kSmallFactor) nvfp4_prepare_host(host_H, n, sigma_reg, true, 1, host_L, host_dw);
+    else nvfp4_prepare_device_impl(ctx, host_H, n, sigma_reg, nullptr, nullptr, host_L, host_dw);
   });
 }
 int qtip_nvfp4_quantize_prepared(qtip_ctx* ctx, int nmat, qtip_nvfp4_matrix* mats, int n, const float* host_L,
@@ -908,7 +914,8 @@ int qtip_ldl_hessian_device_updates(qtip_ctx* ctx, const float* host_HRr, int n,
     QTIP_REQUIRE(ctx != nullptr, "null context");
     DeviceGuard g(ctx);
     QTIP_REQUIRE(host_HRr != nullptr && host_L != nullptr, "ldl_hessian (device): bad arguments (n = %d)", n);
-    ldl_hessian_device_impl(ctx, host_HRr, n, host_L, nullptr, nullptr);
+    if (n <= kSmallFactor) ldl_hessian_impl(host_HRr, n, 1, host_L);
+    else ldl_hessian_device_impl(ctx, host_HRr, n, host_L, nullptr, nullptr);
   });
 }
 

@@ -150,7 +150,7 @@ int qtip_cholesky_inplace(double* host_A, int n, int threads);
 /* The same factorization on the GPU.  No counterpart in the reference (its ldl_hessian is host only,
  * src/quantizer.cpp:154-165): the device factors the diagonal blocks, solves the panels and applies the rank-256
  * updates in fp64 in the host's own order of operations, so host_L is qtip_ldl_hessian's bit for bit; threads is not
- * used.  Works on a stream of its own inside ctx; may run on a side thread while another thread quantizes through the
+ * used.  (Up to n = 160 the calling thread factors: from host memory to host memory that is sooner done.)  Works on a stream of its own inside ctx; may run on a side thread while another thread quantizes through the
  * same ctx. */
 int qtip_ldl_hessian_device_updates(qtip_ctx* ctx, const float* host_HRr, int n, int threads, float* host_L);
 
@@ -292,7 +292,8 @@ int qtip_nvfp4_prepare(const float* host_H, int n, double sigma_reg, int calibra
 int qtip_nvfp4_quantize_prepared(qtip_ctx* ctx, int nmat, qtip_nvfp4_matrix* mats, int n, const float* host_L,
                                  const float* host_dw, int scale_search);
 /* qtip_nvfp4_prepare with calibration, its fp64 Cholesky factorization on the GPU: the same L and dw bit for bit;
- * threads is not used.  No counterpart in the reference, which factors on the host (src/nvfp4_gpu.hip:181-207). */
+ * threads is not used; up to n = 160 the calling thread factors.  No counterpart in the reference, which factors on the
+ * host (src/nvfp4_gpu.hip:181-207). */
 int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n, double sigma_reg, int threads,
                                       float* host_L, float* host_dw);
 

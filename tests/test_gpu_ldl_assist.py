@@ -22,7 +22,9 @@ def spd(n, seed, rows=None):
 
 
 # 6656: trailing matrices on both sides of the 6144 rows from which an update brings the next diagonal block with it
-@pytest.mark.parametrize("n", [16, 496, 512, 1024, 1040, 1152, 2560, 6656])
+# 160, 176: the most that the form with host buffers leaves to the host, and the next; 1024, 1040: L goes down at the end, or
+# in blocks of 1024 rows on the way
+@pytest.mark.parametrize("n", [16, 160, 176, 496, 512, 1024, 1040, 1152, 2560, 6656])
 def test_factor_equals_host_factor(qz, pkg, n):
     say("case: LDL with device updates, n = %d" % n)
     H = spd(n, 100 + n, rows=None if n < 4096 else n + 512)
@@ -41,7 +43,7 @@ def test_factor_equals_host_factor(qz, pkg, n):
         assert np.array_equal(a2.L.view(np.uint32), b2.L.view(np.uint32))
 
 
-@pytest.mark.parametrize("n", [272, 1040, 2560])
+@pytest.mark.parametrize("n", [16, 48, 160, 272, 1024, 1040, 2560])
 def test_device_resident_form_equals_host_factor(qz, pkg, n):
     """qtip_ldl_hessian_device_updates_dev: the rotated Hessian stays on the device and is not written, L arrives in the
     device buffer and from there, row block by row block, in the host buffer; both equal the host factorization's words."""
@@ -103,6 +105,29 @@ def test_factor_of_uneven_matrix_equals_host_factor(qz, pkg, n):
     pkg.Quantizer.ldl_hessian(a, threads=4)
     qz.ldl_hessian_device_updates(b)
     assert np.array_equal(a.L.view(np.uint32), b.L.view(np.uint32))
+    import torch
+    dH, L = torch.from_numpy(H).cuda(), np.full((n, n), -1.0, np.float32)
+    torch.cuda.synchronize()
+    qz.ldl_hessian_device_resident(dH, n, L)
+    assert np.array_equal(a.L.view(np.uint32), L.view(np.uint32))
+
+
+def test_small_matrices_are_factored_where_they_are(pkg):
+    """From host memory to host memory up to 160 columns: no launch, and nothing kept on the device."""
+    say("case: LDL from host to host, 160 and 176 columns")
+    q = pkg.Quantizer(0)
+    for n, on_device in ((160, False), (176, True)):
+        H = spd(n, 40 + n)
+        before = pkg.device_alloc_calls()
+        a, b = pkg.HessPrep(n=n, HRr=H.copy()), pkg.HessPrep(n=n, HRr=H.copy())
+        q.ldl_hessian_device_updates(a)
+        L, dw = q.nvfp4_prepare_device_updates(H)
+        assert (pkg.device_alloc_calls() > before) == on_device
+        pkg.Quantizer.ldl_hessian(b, threads=4)
+        L0, dw0 = pkg.nvfp4_prepare(H, 1e-2, True, 4)
+        assert np.array_equal(a.L.view(np.uint32), b.L.view(np.uint32))
+        assert np.array_equal(L.view(np.uint32), L0.view(np.uint32)) and np.array_equal(dw, dw0)
+    q.close()
 
 
 def test_a_second_factorization_allocates_nothing(pkg):
