@@ -21,6 +21,9 @@ float global_scale_of(uint32_t top_bits) {
   QTIP_REQUIRE(g > 0 && g <= 3.4028234663852886e38f, "NVFP4: global scale %g is not a positive finite float", double(g));
   return g;
 }
+// Up to this many weights the host looks for the largest itself: 0.5 ns a weight against 15 us for the launch, the copy
+// back and the wait.
+constexpr size_t kHostScan = 16384;
 float global_scale(const float* w, size_t numel) {
   uint32_t top = 0;
   for (size_t i = 0; i < numel; ++i) {
@@ -176,15 +179,22 @@ void nvfp4_quantize_prepared_impl(qtip_ctx* c, int nmat, const qtip_nvfp4_matrix
     const long m = M.m;
     // E: the residuals W - q of the finished columns, transposed like W, for the feedback
     DBuf<float> W(size_t(m) * n), WT(size_t(m) * n), FT, E(cal ? size_t(m) * n : 0);
-    DBuf<unsigned> top(1);
+    const bool scan_here = size_t(m) * n <= kHostScan;
+    DBuf<unsigned> top(scan_here ? 0 : 1);
     DBuf<uint8_t> pT(size_t(m) * n / 2), sT(size_t(m) * n / 16), pk(size_t(m) * n / 2), sc(size_t(m) * n / 16);
     unsigned top_bits = 0;
     QTIP_HIP(hipMemcpyAsync(W, M.w, W.bytes(), hipMemcpyHostToDevice, s));
-    QTIP_HIP(hipMemcpyAsync(top, &top_bits, sizeof top_bits, hipMemcpyHostToDevice, s));
-    launch_nvfp4_largest(W, m * n, top, s);
-    QTIP_HIP(hipMemcpyAsync(&top_bits, top, sizeof top_bits, hipMemcpyDeviceToHost, s));
-    QTIP_HIP(hipStreamSynchronize(s));
-    const float g = global_scale_of(top_bits);  // refuses a matrix that is not finite before anything is quantized
+    // (refuses a matrix that is not finite before anything is quantized)
+    float g;
+    if (scan_here) {
+      g = global_scale(M.w, size_t(m) * n);
+    } else {
+      QTIP_HIP(hipMemcpyAsync(top, &top_bits, sizeof top_bits, hipMemcpyHostToDevice, s));
+      launch_nvfp4_largest(W, m * n, top, s);
+      QTIP_HIP(hipMemcpyAsync(&top_bits, top, sizeof top_bits, hipMemcpyDeviceToHost, s));
+      QTIP_HIP(hipStreamSynchronize(s));
+      g = global_scale_of(top_bits);
+    }
     const_cast<qtip_nvfp4_matrix&>(M).global = g;
     c->rht.transpose(W, m, n, n, WT, m);
     // Columns go in buffers of 128 from the last to the first.  A buffer first gathers the feedback of every block

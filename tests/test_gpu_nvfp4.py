@@ -52,16 +52,17 @@ def test_buffers_with_remainders_equal_the_cpu_restatement(qz, oracle, m, n):
         assert np.array_equal(t.packed, want[0]) and np.array_equal(t.scales, want[1]), (Lx is not None, search)
 
 
-def test_values_that_are_not_finite_are_refused(qz, pkg):
-    say("case: nvfp4, infinities and NaN are refused, zeros and the largest value are not")
-    w = np.zeros((32, 32), np.float32)
-    assert qz.nvfp4_quantize_prepared([w], 32)[0].global_scale == 1.0
+@pytest.mark.parametrize("m,n", [(32, 32), (128, 128), (129, 128)])   # the host looks for the largest up to 16384 weights
+def test_values_that_are_not_finite_are_refused(qz, pkg, m, n):
+    say("case: nvfp4 %dx%d, infinities and NaN are refused, zeros and the largest value are not" % (m, n))
+    w = np.zeros((m, n), np.float32)
+    assert qz.nvfp4_quantize_prepared([w], n)[0].global_scale == 1.0
     for v in (np.inf, -np.inf, np.nan):
-        w[31, 31] = v
+        w[m - 1, n - 1] = v
         with pytest.raises(pkg.QtipError):
-            qz.nvfp4_quantize_prepared([w], 32)
-    w[31, 31] = -np.finfo(np.float32).max
-    assert qz.nvfp4_quantize_prepared([w], 32)[0].global_scale == np.finfo(np.float32).max / np.float32(448 * 6)
+            qz.nvfp4_quantize_prepared([w], n)
+    w[m - 1, n - 1] = -np.finfo(np.float32).max
+    assert qz.nvfp4_quantize_prepared([w], n)[0].global_scale == np.finfo(np.float32).max / np.float32(448 * 6)
 
 
 @pytest.mark.parametrize("name", ["gauss", "heavy"])
