@@ -70,7 +70,8 @@ enum StepKind { kPlain = 0, kStore = 1, kDigits = 2 };
 
 // What the two workgroups of a pair (viterbi_pair_kernel) exchange lies behind the kept metrics of their slots.
 struct PairArea {
-  uint32_t flag;      // how far the slot's workgroup has come in this launch (pair_reset_kernel clears it)
+  uint32_t flag;      // how far the slot's workgroup has come in this launch (pair_reset_kernel clears it); in the first
+                      // slot of a launch with one workgroup per tile: the tiles handed out beyond the first of each
   uint32_t alone;     // in the first workgroup's slot: one of the two gave up waiting for the other
   uint32_t overlap;   // first workgroup: the overlap group and the winner of a free pass it had to repeat on fp64 metrics
   uint32_t expected;
@@ -126,7 +127,11 @@ struct Smem {
   uint32_t tr_d[2][4];
   alignas(16) uint32_t tr32[2][4][4];  // the same for the 32-bit passes: best, second best, d | d1 << 8, gap inside the best's row
   uint32_t red32[8][3];    // end of the free 32-bit pass: per wave the best group's metric, the second best, the group
+  uint32_t grown[8];       // end of a free pass's second round: per wave the least growth of a metric
+  uint32_t close_count[2];   // search for the closed path: partial paths found, by turn
+  uint32_t close_least[2];   // the smallest bound among them off the free path and on it
   int overlap;
+  uint32_t next_tile;  // tiles kernel: what this workgroup takes on next
   uint32_t heard;      // pair: what waiting for the other workgroup came to
   uint32_t final_state;
   float final_metric;  // the free fp64 pass's best final metric (what later 32-bit passes of the tile row may expect)
@@ -557,6 +562,17 @@ struct Unit {
 __device__ __forceinline__ Unit unit_of(int k) { return Unit{__builtin_bit_cast(double, uint64_t(1023 + k / 2) << 52)}; }
 constexpr int kMirror32 = 0xfeb;
 static_assert(64 * kGroups <= 2 * kHistWordsPerTile, "the 32-bit kept metrics (64 steps) must fit the fp64 slot");
+// What the search for the closed path needs of a free pass (close_path below) lies behind the 32-bit kept metrics: the
+// upper halves of the metrics entering the steps 1 .. 128 + kTurn (kBoundRow values each).
+constexpr int kTurn = 40;              // steps the free pass runs on into the sequence's second round
+constexpr int kBoundRow = kGroups / 2;
+constexpr int kCloseList = 256;        // partial paths of a step
+constexpr int kCloseSlots = 512;       // hash slots in which partial paths of one group meet
+constexpr int kClosePaths = 3520;      // partial paths of all steps together
+constexpr int kCloseRing = 4;          // rows of bounds in LDS
+constexpr size_t kBoundsAt = size_t(64) * kGroups * sizeof(uint32_t);                       // bytes into the slot
+static_assert(kTurn % 2 == 0 && kTurn < kSteps / 2);
+static_assert(kBoundsAt + size_t(kSteps + kTurn + 1) * kBoundRow * sizeof(uint16_t) <= size_t(kHistWordsPerTile) * sizeof(double));
 
 __device__ __forceinline__ int m32_pos(int col) {  // bits 7..0: b7 b6 b5 b4 b1 b0 b3 (b2 ^ b6)
   return (col & 0xf0) | ((col & 3) << 2) | (((col >> 3) & 1) << 1) | (((col >> 2) ^ (col >> 6)) & 1);
@@ -614,9 +630,14 @@ __device__ __forceinline__ uint32_t err_units(double l0, double l1, double x0, d
 // 4..7), and the table's 1024 entries two each instead of four.
 // kHalf: steps 0 .. 63 only; the metrics entering step 64 are left in metric buffer 0 (the other half of the sequence is
 // another workgroup's, viterbi_pair_kernel).
+// bounds (a whole free pass): the upper halves of the metrics entering step i go to row i, and after its end the pass runs
+// on for kTurn steps, whose metrics are kept as bounds only; returns the least by which a metric has grown over the last
+// round, that is from entering step kTurn to entering step 128 + kTurn, rounded down.
 template <bool kSym, bool kWide, bool kHalf = false>
-__device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restrict__ entry_d, int roll, int ov,
-                                               uint32_t* __restrict__ hist, int first_kept, const Unit unit) {
+__device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __restrict__ entry_d, int roll, int ov,
+                                                   uint32_t* __restrict__ hist, int first_kept, const Unit unit,
+                                                   uint16_t* __restrict__ bounds = nullptr) {
+  constexpr bool kBounds = kSym && !kHalf;
   constexpr int kT = kWide ? 2 * kThreads : kThreads, kSlotsOwn = kWide ? 4 : 8, kEnt = 1024 / kT;
   const int tfull = kWide ? opaque_tid_wide() : opaque_tid();
   const int tid = tfull & (kThreads - 1), upper = kWide ? tfull >> 8 : 0;
@@ -703,9 +724,10 @@ __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restric
   __syncthreads();
 
   uint32_t fin[kSlotsOwn];
+  uint32_t packed[kSlotsOwn / 2];  // the upper halves of this thread's new metrics, two to a word
   // step `it`: metrics of buffer it & 1 and table buffer it & 1 -> metrics of buffer (it + 1) & 1; par = it & 1
   auto step = [&](int it, auto kind_tag, auto par_tag) __attribute__((always_inline)) {
-    constexpr int kind = decltype(kind_tag)::value;  // kDigits: the free pass's last step, results to fin only
+    constexpr int kind = decltype(kind_tag)::value;  // kDigits: the free pass's last step, results to fin as well
     constexpr int par = decltype(par_tag)::value;
     uint32_t* hs = nullptr;
     if constexpr (kind == kStore) hs = hist + size_t(it >> 1) * kGroups + tid;
@@ -733,7 +755,7 @@ __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restric
         MB[4 * k] = b.x, MB[4 * k + 1] = b.y, MB[4 * k + 2] = b.z, MB[4 * k + 3] = b.w;
       }
     }
-    if constexpr (kind != kDigits) table(it + 1, std::integral_constant<int, par ^ 1>{});
+    table(it + 1, std::integral_constant<int, par ^ 1>{});
     // The 16 table values of a slot are fetched while the slot before it is worked on; the value of digit k of slot
     // m lies (k (2 m + 1)) % 16 positions after the slot's first.  m0: the first slot of this thread, a constant in
     // each of the two copies of the loop that the wide form needs.  Tail-biting pass: evb[.][k] is the value of digit
@@ -798,11 +820,12 @@ __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restric
         for (int k = 0; k < 8; ++k)
           bb = min3u(bb, sat_add(ev[2 * k], MB[15 - 2 * k]), sat_add(ev[2 * k + 1], MB[14 - 2 * k]));
       }
-      if constexpr (kind == kDigits) {
-        fin[m] = ba;
-      } else {
-        Mw[wslot[m]] = ba;
-        if constexpr (!kSym) Mw[wslot[m] ^ kMirror32] = bb;
+      if constexpr (kind == kDigits) fin[m] = ba;
+      Mw[wslot[m]] = ba;
+      if constexpr (!kSym) Mw[wslot[m] ^ kMirror32] = bb;
+      if constexpr (kBounds) {
+        if (m & 1) packed[m >> 1] = __builtin_amdgcn_perm(ba, packed[m >> 1], 0x07060302u);
+        else packed[m >> 1] = ba;
       }
       if constexpr (kind == kStore) {
         hs[(m0 + m) * kThreads] = ba;
@@ -815,6 +838,11 @@ __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restric
     } else {
       if (upper) slots(std::integral_constant<int, 4>{});
       else slots(std::integral_constant<int, 0>{});
+    }
+    if constexpr (kBounds) {
+      uint16_t* const b = bounds + size_t(it + 1) * kBoundRow + 8 * tid + 4 * upper;
+      if constexpr (kWide) *reinterpret_cast<uint2*>(b) = uint2{packed[0], packed[1]};
+      else *reinterpret_cast<uint4*>(b) = uint4{packed[0], packed[1], packed[2], packed[3]};
     }
     __syncthreads();
   };
@@ -831,7 +859,7 @@ __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restric
     else step(it, Plain{}, Even{});
     step(it + 1, Plain{}, Odd{});
   }
-  if constexpr (kHalf) return;
+  if constexpr (kHalf) return 0;
   step(kSteps - 2, Store{}, Even{});
   if constexpr (kSym) {
     step(kSteps - 1, Last{}, Odd{});
@@ -866,7 +894,30 @@ __device__ __forceinline__ void forward_pass32(Smem& sm, const double* __restric
     __syncthreads();
     if (tfull == 0) sm.red32[0][0] = b1, sm.red32[0][1] = b2 - b1, sm.red32[0][2] = bj;
     __syncthreads();
+#pragma nounroll
+    for (int it = kSteps; it < kSteps + kTurn; it += 2) {
+      step(it, Plain{}, Even{});
+      step(it + 1, Plain{}, Odd{});
+    }
+    // each thread compares the values it has kept itself
+    const uint16_t* const b0 = bounds + size_t(kTurn) * kBoundRow + 8 * tid + 4 * upper;
+    uint32_t grown = 0xffffu;
+#pragma unroll
+    for (int i = 0; i < kSlotsOwn; ++i) {
+      const uint32_t now = (i & 1) ? packed[i >> 1] >> 16 : packed[i >> 1] & 0xffffu;
+      const uint32_t before = __hip_atomic_load(b0 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      grown = min(grown, now > before ? now - before - 1u : 0u);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) grown = min(grown, uint32_t(__shfl_xor(int(grown), off, 64)));
+    if ((tfull & 63) == 0) sm.grown[tfull >> 6] = grown;
+    __syncthreads();
+    grown = sm.grown[0];
+#pragma unroll
+    for (int w = 1; w < kT / 64; ++w) grown = min(grown, sm.grown[w]);
+    return uint32_t(__builtin_amdgcn_readfirstlane(int(grown))) << 16;
   }
+  return 0;
 }
 
 __device__ __forceinline__ uint32_t row_min16_u32(uint32_t c) {
@@ -1126,10 +1177,279 @@ __device__ __forceinline__ uint32_t trace_back32(Smem& sm, const double* __restr
   return s;
 }
 
+// The tail-biting pass without its forward recursion.  The cheapest path from group ov before step 0 back to ov after step
+// 127 is searched for from its end, step 127 down to step 0: of the partial paths (a group entering a step and the
+// cheapest completion from there to ov) only those are followed that can still belong to a closed path under a limit, and
+// the free pass of the same block says which.  It ran on the same values rotated by half the sequence and then kTurn steps
+// into its second round, so with M_i its metrics entering its step i, a path from ov at the sequence's start to group h
+// entering step p costs at least
+//     M_{64 + p}[h] - M_64[ov]              for p <= 64 + kTurn  (M_{64 + p}[h] is at most M_64[ov] + that cost), and
+//     M_{p - 64}[h] + grown - M_64[ov]      beyond, `grown` being the least growth of a metric over one round
+// (the recursion is monotone and commutes with adding a constant).  The free path itself goes through ov, and a closed path
+// differs from it around the join only, by 0.2 to 1.2 of a cost of 14 (normalized weights), most of which lies in the
+// kTurn steps behind the join that the bounds have seen: the search follows 1 to 20 partial paths a step where the
+// forward recursion updates 4096 groups from 65536 candidates.
+// What is left to pay is often the mirror: free paths come in complementary pairs, the metrics do not say which of the two
+// a group belongs to, and the closed path through ov must not arrive at its complement.  Half of the tiles have to
+// change over somewhere, at a cost of up to 0.25.  The others are done as soon as the free path's own group is the only
+// one left near the limit: the rest of the free path leads from it to ov, at the least cost there is.
+// Costs are the 32-bit passes' integers in the free pass's unit, summed exactly; bounds are kept as the upper halves of
+// the metrics, which makes them weaker by less than 65536 units and never too large.  A result counts if it is under the
+// limit the search ended with (a path left out then costs more) and no two paths that met in a group were closer than
+// `margin`: the winner then beats every other closed path by that much, and the fp64 recursion takes it.  Otherwise
+// the limit is raised twice, then false is returned and the caller runs the pass (0.6 % of the tiles).
+// What bounds it: latency.  A step is a chain of five LDS round trips and some 150 instructions, 0.85 us by itself and
+// 1.1 us beside two other workgroups, 120 steps a tile; the pipes it leaves idle are the other workgroups' forward passes'.
+// Per tile with three workgroups on a compute unit 140 us instead of 294 + 75 for the forward recursion and its
+// trace-back, with 60 us more in the free pass for its longer way (kTurn 32 / 40 / 48: 76.5 / 72.5 / 72.4 ms for 768 tile
+// rows of 128 blocks; a forward pass: 89.5).
+// LDS operations of the search.  Written out: rows of bounds are on their way into LDS meanwhile (direct-to-LDS loads), and
+// before an LDS write or atomic of its own the compiler would wait for all of them.
+__device__ __forceinline__ uint32_t lds_at(const void* p) { return uint32_t(reinterpret_cast<size_t>(p)); }
+__device__ __forceinline__ unsigned long long lds_min(uint32_t at, unsigned long long v) {
+  unsigned long long old;
+  asm volatile("ds_min_rtn_u64 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=&v"(old) : "v"(at), "v"(v) : "memory");
+  return old;
+}
+__device__ __forceinline__ uint32_t lds_add(uint32_t at, uint32_t v) {
+  uint32_t old;
+  asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=&v"(old) : "v"(at), "v"(v) : "memory");
+  return old;
+}
+__device__ __forceinline__ void lds_min(uint32_t at, uint32_t v) {
+  asm volatile("ds_min_u32 %0, %1" : : "v"(at), "v"(v) : "memory");
+}
+__device__ __forceinline__ void lds_put32(uint32_t at, uint32_t v) {
+  asm volatile("ds_write_b32 %0, %1" : : "v"(at), "v"(v) : "memory");
+}
+__device__ __forceinline__ void lds_put64(uint32_t at, unsigned long long v) {
+  asm volatile("ds_write_b64 %0, %1" : : "v"(at), "v"(v) : "memory");
+}
+template <bool kWide>
+__device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const uint32_t* __restrict__ hist32, uint32_t ov,
+                                           uint32_t winner, uint32_t grown, uint32_t margin, const Unit unit) {
+  constexpr uint32_t kT = kWide ? 2 * kThreads : kThreads;
+  typedef unsigned long long u64;
+  const uint32_t tid = uint32_t(kWide ? opaque_tid_wide() : opaque_tid()), lane = tid & 63u, d = tid & 15u;
+  const int wave = __builtin_amdgcn_readfirstlane(int(tid) >> 6);
+  const char* const bounds = reinterpret_cast<const char*>(hist32) + kBoundsAt;
+  // LDS: a ring of rows of bounds in sm.E; in sm.M the codebook's 512 entries and the inputs as pairs of fp64 values times
+  // Unit::pre, the meeting places, two lists of partial paths (cost << 32 | place bits << 20 | position of the path
+  // continued in its step's list << 12 | group) and the lower words of all of them in the order found
+  char* const area = reinterpret_cast<char*>(sm.M);
+  double2* const book = reinterpret_cast<double2*>(area);
+  double2* const input = book + 512;
+  u64* const meet = reinterpret_cast<u64*>(input + kSteps);
+  u64* const lists = meet + kCloseSlots;
+  uint32_t* const paths = reinterpret_cast<uint32_t*>(lists + 2 * kCloseList);
+  uint16_t* const list0 = reinterpret_cast<uint16_t*>(paths + kClosePaths);  // where the paths of a step begin there
+  static_assert(kCloseRing * kBoundRow * 2 <= sizeof(sm.E) &&
+                (512 + kSteps) * 16 + (kCloseSlots + 2 * kCloseList) * 8 + kClosePaths * 4 + kSteps * 2 <= sizeof(sm.M));
+  // Byte offset of group h in a row: bits 4..11 of h and 0..3 of its digit d apart.  Group h = (d << 8) | (j >> 4) of a
+  // partial path to group j lies at the place of h or, from 2048 up, of 4095 - h = ~h, so bits and digit contribute by XOR.
+  auto place = [](uint32_t jj) -> uint32_t { return (owner32(jj) * 8u + (jj & 7u)) * 2u; };
+  const uint32_t d_place = d < 8u ? place(d << 8) : place(((15u - d) << 8) | 0xffu);
+  const uint32_t d_meet = lds_at(meet);
+  const uint32_t d_slot = ((d & 1u) << 8 | (d >> 1) << 5) * 8u;
+  const uint32_t d_next = place(d << 4) << 20;  // what the digit adds to the place bits of the group it leads to
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  auto issue = [&](int p) {  // the bounds of step p, 1 KB per wave of the first four
+    const int r = p <= kSteps / 2 + kTurn ? p + kSteps / 2 : p - kSteps / 2;
+    if (wave < 4)
+      __builtin_amdgcn_global_load_lds(bounds + size_t(r) * (kBoundRow * 2) + wave * 1024 + 16 * lane,
+                                       (lds_ptr)(reinterpret_cast<char*>(sm.E) + uint32_t(p) % kCloseRing * (kBoundRow * 2) + wave * 1024),
+                                       16, 0, 0);
+  };
+  auto lds_barrier = [] {  // orders LDS, not the loads in flight
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  const uint32_t ov_low = ov < 2048u ? ov : 4095u - ov;
+  // M_64[ov], rounded down: what every bound above starts from
+  const uint32_t start = uint32_t(__builtin_amdgcn_readfirstlane(int(__hip_atomic_load(
+      reinterpret_cast<const uint16_t*>(bounds + size_t(kSteps / 2) * (kBoundRow * 2) + place(ov_low)), __ATOMIC_RELAXED,
+      __HIP_MEMORY_SCOPE_WORKGROUP)))) << 16;
+  const uint32_t least = uint32_t(__builtin_amdgcn_readfirstlane(int(sat_add(start, grown))));
+  __syncthreads();
+  for (uint32_t g = tid; g < kCloseSlots; g += kT) meet[g] = ~0ull;
+  for (uint32_t g = tid; g < 512u; g += kT) {
+    const uint32_t w = tl[g];
+    book[g].x = double(float(__builtin_bit_cast(_Float16, uint16_t(w)))) * unit.pre;
+    book[g].y = double(float(__builtin_bit_cast(_Float16, uint16_t(w >> 16)))) * unit.pre;
+  }
+  if (tid < kSteps) input[tid].x = double(sm.x[2 * tid]) * unit.pre, input[tid].y = double(sm.x[2 * tid + 1]) * unit.pre;
+  const u64 root = (place(ov >> 4) << 20) | ov;
+  if (tid < 2) sm.close_count[tid] = 0, sm.close_least[tid] = kSat;
+  // turn: one round of the loop below, a step or another try at it with a lower limit; the stamp, counted downwards in the
+  // keys, tells the meeting places' entries of different turns apart.  Two counters, used in turn, run on; `seen` is what
+  // the one in use stood at.
+  uint32_t stamp = 0xfffff000u, counter = lds_at(sm.close_count), seen = 0, seen_other = 0;
+  bool ok = false;
+#pragma nounroll
+  for (int attempt = 0; attempt < 3 && !ok; ++attempt) {
+    uint32_t limit = least + 131072u + winner / (attempt == 0 ? 32u : attempt == 1 ? 20u : 12u);
+    if (limit >= kWinnerMax || limit < least) return false;
+    issue(kSteps - 1);
+    issue(kSteps - 2);
+    issue(kSteps - 3);
+    issue(kSteps - 4);
+    __builtin_amdgcn_s_waitcnt(0x0F73);  // vmcnt(3)
+    lds_barrier();
+    uint32_t n = 1, total = 0, found = 0;  // the present list's length; all paths so far
+    int p = kSteps - 1;
+    double2 x = input[p];
+    u64 first = root;
+#pragma nounroll
+    for (;;) {
+      const u64* const list = lists + (p & 1 ? 0 : kCloseList);
+      const uint32_t next = lds_at(lists + (p & 1 ? kCloseList : 0));
+      const uint32_t row = lds_at(sm.E) + uint32_t(p) % kCloseRing * (kBoundRow * 2);
+      const uint32_t most = limit - (p > kSteps / 2 + kTurn ? grown : 0u);
+      // every fourth step of the first half the free path's group is looked at by itself, and at the end of the second
+      // round's steps the smallest bound
+      const bool on_free = p < kSteps / 2 && (p & 3) == 0, watched = on_free || p == kSteps / 2 + kTurn;
+      uint32_t on_path = kSat;
+      if (on_free) on_path = uint32_t(__builtin_amdgcn_readfirstlane(int(sm.st[kSteps / 2 + p]))) >> 4;
+      u64 path = first;
+      for (uint32_t k = tid >> 4; k < n; k += kT / 16) {
+        if (k >= kT / 16) path = list[k];
+        const uint32_t lo = uint32_t(path), s = (d << 12) | (lo & 0xfffu), h = s >> 4;
+        const uint32_t v = __umul24(s, s) + s;
+        const double2 l = book[(v >> 6) & 511u];
+        const uint32_t bound = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t*>(row + ((lo >> 20) ^ d_place));
+        const double lx = __hiloint2double(__double2hiint(l.x) ^ int((v << 16) & 0x80000000u), __double2loint(l.x));
+        const double a0 = lx - x.x, a1 = l.y - x.y;
+        const double q = __builtin_fma(a0, a0, __builtin_fma(a1, a1, 0.5));
+        uint32_t err;  // stops at 2^32 - 1 by itself
+        asm("v_cvt_u32_f64 %0, %1" : "=v"(err) : "v"(q));
+        const uint32_t c = sat_add(uint32_t(path >> 32), err), f = sat_add(bound << 16, c);
+        if (f <= most) {
+          bool keep = true;
+          uint32_t doubt = 0;
+          if (n > 1) {  // (the sixteen continuations of one path lead to sixteen groups)
+            const u64 old = lds_min(d_meet + (((lo >> 1) & 0x7f8u) ^ d_slot), (u64(stamp | (c >> 20)) << 32) | ((c << 12) | h));
+            if (uint32_t(old >> 32) < stamp + 4096u && (uint32_t(old) & 0xfffu) == h) {  // another path to h
+              const uint32_t o = uint32_t(old >> 12);
+              keep = c < o;
+              doubt = min(o - c, c - o) < margin ? 0x10000u : 0u;  // counted as more than any list holds
+            }
+          }
+          if (watched) lds_min(lds_at(sm.close_least) + (h == on_path ? 4u : 0u), f);
+          if (doubt) (void)lds_add(counter, doubt);
+          if (keep) {
+            const u64 mask = __builtin_amdgcn_ballot_w64(true);
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0u));
+            uint32_t at = 0;
+            if (rank == 0) at = lds_add(counter, uint32_t(__builtin_popcountll(mask)));
+            at = uint32_t(__builtin_amdgcn_readfirstlane(int(at))) - seen + rank;
+            if (at < kCloseList) {
+              const uint32_t word = d_next | (lo & 0x700u) << 13 | (lo & 0x800u) << 20 | k << 12 | h;
+              lds_put64(next + 8u * at, (u64(c) << 32) | word);
+              lds_put32(lds_at(paths + total) + 4u * at, word);
+            }
+          }
+        }
+      }
+      // the next step's inputs and bounds (the two rows after them may be under way)
+      const double2 x_next = input[p > 0 ? p - 1 : 0];
+      if (p >= 3) __builtin_amdgcn_s_waitcnt(0x0F72);
+      else __builtin_amdgcn_s_waitcnt(0x0F70);
+      lds_barrier();
+      uint32_t count;
+      u64 path_next;
+      asm volatile("ds_read_b32 %0, %2\n\tds_read_b64 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(count), "=&v"(path_next)
+                   : "v"(counter), "v"(next + 8u * (tid >> 4))
+                   : "memory");
+      count = uint32_t(__builtin_amdgcn_readfirstlane(int(count)));
+      const uint32_t m = count - seen;
+      seen = seen_other, seen_other = count, counter ^= lds_at(sm.close_count) ^ lds_at(sm.close_count + 1), stamp -= 4096u;
+      if (m - 1u >= uint32_t(kCloseList)) {
+        // none left, or two too close together, or too many: those once more with a lower limit
+        if (m == 0 || m >= 0x10000u || limit - least < 4096u || stamp < 0x10000000u) break;
+        limit -= (limit - least) / 4;
+        if (watched) {
+          lds_barrier();
+          if (tid < 2) lds_put32(lds_at(sm.close_least + tid), kSat);
+          lds_barrier();
+        }
+        continue;
+      }
+      if (tid == 0) asm volatile("ds_write_b16 %0, %1" : : "v"(lds_at(list0 + p)), "v"(total) : "memory");
+      if (watched) {
+        const uint32_t off = uint32_t(__builtin_amdgcn_readfirstlane(int(sm.close_least[0])));
+        const uint32_t on = uint32_t(__builtin_amdgcn_readfirstlane(int(sm.close_least[1])));
+        if (on_free && on < kWinnerMax && on + 131072u + margin <= off && on + 65536u + margin <= limit) {
+          found = m;
+          break;
+        }
+        // a path that has come to the free path's group is closed by it, at a cost below on + 131072 - M_64[ov]
+        if (on < kWinnerMax) limit = min(limit, on + 131072u + 2u * min(margin, 1u << 20));
+        if (!on_free && attempt < 2) limit = min(limit, off + min(kSat - off, 131072u + winner / (attempt ? 32u : 56u)));
+        lds_barrier();
+        if (tid < 2) lds_put32(lds_at(sm.close_least + tid), kSat);
+      }
+      if (p == 0) {
+        found = m;
+        break;
+      }
+      total += m;
+      if (total + kCloseList > kClosePaths) break;
+      n = m;
+      --p;
+      if (p >= 3) issue(p - 3);  // into the buffer of step p + 1
+      first = path_next, x = x_next;
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if (tid < 2) sm.close_least[tid] = kSat;
+    if (found) {
+      // the cheapest of the paths to the group in question, and how far behind the next one is (every wave alike)
+      const uint32_t target = p == 0 ? ov : uint32_t(sm.st[kSteps / 2 + p]) >> 4;
+      u64 best = ~0ull, second = ~0ull;
+      for (uint32_t i = lane; i < found; i += 64) {
+        const u64 path = lists[(p & 1 ? kCloseList : 0) + i], key = (path & 0xffffffff00000000ull) | i;
+        if ((uint32_t(path) & 0xfffu) != target) continue;
+        second = min(second, max(best, key));
+        best = min(best, key);
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const u64 ob = __shfl_xor(best, o, 64), os = __shfl_xor(second, o, 64);
+        second = min(min(second, os), max(best, ob));
+        best = min(best, ob);
+      }
+      const uint32_t c = uint32_t(best >> 32), c2 = uint32_t(second >> 32);
+      const uint32_t sum = p == 0 ? sat_add(start + 65536u, sat_add(c, margin)) : 0u;
+      ok = __builtin_amdgcn_readfirstlane(int(sum <= limit && best != ~0ull && (second == ~0ull || c2 - c >= margin))) != 0;
+      if (ok && wave == 0) {
+        // steps 0 .. p - 1 as the free path has them, then from path to path continued
+        const uint16_t v = sm.st[kSteps / 2 + lane];
+        if (int(lane) < p) sm.st[lane] = v;
+        const uint32_t begin_lo = list0[lane], begin_hi = list0[lane + 64];
+        uint32_t at = total + uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(best))));
+        uint32_t lo = uint32_t(__builtin_amdgcn_readfirstlane(int(paths[at])));
+#pragma nounroll
+        for (int q = p; q < kSteps; ++q) {
+          const uint32_t g = lo & 0xfffu, k = (lo >> 12) & 0xffu;
+          const uint32_t begin = uint32_t(__builtin_amdgcn_readlane(int(q + 1 < 64 ? begin_lo : begin_hi), (q + 1) & 63));
+          at = q == kSteps - 1 ? 0u : begin + k;
+          lo = q == kSteps - 1 ? ov : uint32_t(__builtin_amdgcn_readfirstlane(int(paths[at])));
+          if (lane == 0) sm.st[q] = uint16_t((g << 4) | (lo & 15u));
+        }
+      }
+    }
+    __syncthreads();
+  }
+  return ok;
+}
+
 // The passes first_pass .. passes_end - 1 (of two) of one block by one workgroup: targets in sm.x, states to sm.st (a
 // second pass by itself takes the overlap group from sm.overlap).  expected: the free pass's winner of this tile row's
 // previous column block (0: none yet), and of this one afterwards.  fp64_only: as job.mode 1.  Ends with a barrier.
-template <bool kWide>
+template <bool kWide, bool kClose>
 __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const double* __restrict__ entry_d, double* hist,
                                              const uint32_t* tl, float& expected, int first_pass, int passes_end,
                                              bool fp64_only) {
@@ -1138,8 +1458,9 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
   // pass 2 on the sequence itself, tail-biting through that group, traced back in full.  One loop, so that the
   // step bodies exist once in the instruction cache.
   int ov = first_pass > 0 ? sm.overlap : -1;
+  bool closed = false;
 #pragma nounroll
-  for (int pass = first_pass; pass < passes_end; ++pass) {
+  for (int pass = first_pass; pass < passes_end && !closed; ++pass) {
     const int roll = pass == 0 ? kSeq / 2 : 0;
     bool done = false;
     if (job.mode == 0 && !fp64_only) {
@@ -1149,15 +1470,21 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
       const int unit_log2 = __builtin_amdgcn_readfirstlane(unit_log2_for(expected, pass == 0 ? 2.f : 1.125f));
       const Unit unit = unit_of(unit_log2);
       if (pass == 0) {
-        forward_pass32<true, kWide>(sm, entry_d, roll, -1, hist32, 62, unit);
+        const uint32_t grown = forward_pass32<true, kWide>(
+            sm, entry_d, roll, -1, hist32, 62, unit, reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(hist32) + kBoundsAt));
         const uint32_t winner = sm.red32[0][0];
         flag |= uint32_t(sm.red32[0][1] < job.margin) | uint32_t(winner >= kWinnerMax);
-        const uint32_t s = trace_back32<true, kWide>(sm, entry_d, hist32, roll, sm.red32[0][2], 64, false, job.margin, flag,
-                                                     tl, unit);
+        const uint32_t s = trace_back32<true, kWide>(sm, entry_d, hist32, roll, sm.red32[0][2], 64, kClose, job.margin,
+                                                     flag, tl, unit);
         if (!flag && u == 0) sm.overlap = int(s & 0xfffu);  // s is the state of step 63
         // what the tail-biting pass of this block and the free pass of the next may expect (a winner that did
         // not fit is replaced by the true one when the pass is repeated on fp64 metrics)
         expected = __builtin_ldexpf(float(winner), -unit_log2);
+        if constexpr (kClose) {
+          if (!flag && passes_end > 1)
+            closed = close_path<kWide>(sm, tl, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(s & 0xfffu))),
+                                       uint32_t(__builtin_amdgcn_readfirstlane(int(winner))), grown, job.margin, unit);
+        }
       } else {
         forward_pass32<false, kWide>(sm, entry_d, roll, ov, hist32, 0, unit);
         const uint32_t s = trace_back32<false, kWide>(sm, entry_d, hist32, roll, uint32_t(ov), 2, true, job.margin, flag, tl,
@@ -1230,17 +1557,20 @@ template <bool kWide>
 __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) void viterbi_tiles_kernel(
     TileJob job, const double* __restrict__ entry_d, const float* __restrict__ entry_f, double* __restrict__ hist_all) {
   __shared__ Smem sm;
-  __shared__ uint32_t tl[kWide ? 512 : 1];  // wide form: the codebook's 512 value pairs as fp16 bits, for its trace-backs
+  __shared__ uint32_t tl[512];  // the codebook's 512 value pairs as fp16 bits, for the searches and the wide form's trace-backs
   const int u = threadIdx.x & (kThreads - 1);
-  if constexpr (kWide) {  // the table's values are fp16 values (entry bit 9 is the sign of the first one)
-    const int i = threadIdx.x;
+  // the table's values are fp16 values (entry bit 9 is the sign of the first one)
+  for (int i = threadIdx.x; i < 512; i += kWide ? 2 * kThreads : kThreads) {
     const uint32_t h0 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i]));
     const uint32_t h1 = __builtin_bit_cast(uint16_t, _Float16(entry_f[2 * i + 1]));
     tl[i] = h0 | (h1 << 16);
-    __syncthreads();
   }
+  __syncthreads();
   double* hist = hist_all + size_t(blockIdx.x) * kSlotWords;
-  for (long tile = blockIdx.x; tile < job.tiles; tile += gridDim.x) {
+  // More tiles than workgroups: whoever is done takes the next one (a tile's time depends on its search: 4096 tiles
+  // 3.31 ms dealt out beforehand, 2.7 ms this way)
+  uint32_t* const handed_out = &reinterpret_cast<PairArea*>(hist_all + kHistWordsPerTile)->flag;
+  for (long tile = blockIdx.x; tile < job.tiles;) {
     float expected = 0.f;  // the free pass's winner of this tile row's previous column block (0: none yet)
     for (int blk = job.blocks - 1; blk >= 0; --blk) {
       // the column block of this turn; the hatWT values the previous turn wrote for this tile row are visible after
@@ -1250,10 +1580,14 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
       else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
       else tile_targets<float>(sm, job, col0, tile, job.prod32);
       __syncthreads();
-      block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
+      block_passes<kWide, true>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
       block_outputs(sm, job, entry_f, tile, blk, col0);
       __syncthreads();
     }
+    if (job.tiles <= long(gridDim.x)) break;
+    if (threadIdx.x == 0) sm.next_tile = __hip_atomic_fetch_add(handed_out, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    tile = long(gridDim.x) + __builtin_amdgcn_readfirstlane(int(sm.next_tile));
   }
 }
 
@@ -1689,7 +2023,7 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
       middle(0);
       if (b2 - b1 < job.margin || b1 >= kWinnerMax) {
         if (tid == 0 && job.stats) atomicAdd(job.stats, 1u);
-        block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 1, true);
+        block_passes<kWide, false>(sm, job, entry_d, hist, tl, expected, 0, 1, true);
         if (tid == 0) pair_put(&mine->overlap, uint32_t(sm.overlap)), pair_put(&mine->expected, __float_as_uint(expected));
         tell(n + 3);
       } else {
@@ -1714,7 +2048,7 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
       flag |= uint32_t(__builtin_amdgcn_readfirstlane(int(pair_get(&other->doubt))));
       if (flag) {
         if (tid == 0 && job.stats) atomicAdd(job.stats + 1, 1u);
-        block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 1, 2, true);
+        block_passes<kWide, false>(sm, job, entry_d, hist, tl, expected, 1, 2, true);
       } else if (tid < 64) {
         sm.st[64 + tid] = uint16_t(pair_get(&other->states[tid]));
       }
@@ -1722,7 +2056,7 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
       return true;
     };
     if (!alone && !together()) alone = true;
-    if (alone) block_passes<kWide>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
+    if (alone) block_passes<kWide, false>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
     block_outputs(sm, job, entry_f, tile, blk, col0);
     __syncthreads();
   }
@@ -1817,6 +2151,10 @@ bool launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const flo
       pair<<<dim3(unsigned(pair_grid)), threads, 0, s>>>(job, d_entry_d, d_entry_f, ws);
     QTIP_HIP(hipGetLastError());
     return false;
+  }
+  if (job.tiles > long(grid)) {
+    pair_reset_kernel<<<dim3(1), dim3(64), 0, s>>>(static_cast<double*>(workspace), 1);
+    QTIP_HIP(hipGetLastError());
   }
   const auto kernel = wide ? viterbi_tiles_kernel<true> : viterbi_tiles_kernel<false>;
   const dim3 block(wide ? 2 * kThreads : kThreads);

@@ -347,3 +347,54 @@ def test_wide_workgroups_give_the_same_states(qz, oracle, hyb):
     finally:
         qz.set_viterbi_mode(0)
         qz.set_tlut(None)
+
+
+def _closing_inputs(kind, B, l0, l1):
+    """Inputs whose closed path is easy, hard or impossible to tell from the free one's metrics."""
+    rng = np.random.default_rng(B + len(kind))
+    X = rng.standard_normal((B, 256))
+    if kind == "scales":
+        X *= np.exp(rng.uniform(np.log(0.02), np.log(8.0), (B, 1)))
+    elif kind == "join":          # the free path's ends meet where the inputs allow no detour: large values around step 64
+        X[:, 96:160] *= 6.0
+    elif kind == "flat":          # many paths of nearly the same cost
+        X = np.round(X * 4) / 4 * 0.25
+    elif kind == "zeros":
+        X[:, 20:230] = 0.0
+    elif kind == "mirror":
+        # decoded values of a path that arrives at the complement of the state it started from: the free path costs next to
+        # nothing and the closed one has to change over to its mirror path somewhere
+        nib = rng.integers(0, 16, (B, 128))
+        st = np.zeros((B, 128), np.uint32)
+        for t in range(128):
+            for k in range(4):
+                v = nib[:, (t - k) % 128] ^ (15 if t - k < 0 else 0)
+                st[:, t] |= (v << (4 * k)).astype(np.uint32)
+        X = np.stack([l0[st], l1[st]], axis=-1).reshape(B, 256) + 0.02 * X
+    return X.astype(np.float16).astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["scales", "join", "flat", "zeros", "mirror"])
+@pytest.mark.parametrize("B", [1, 767, 769])
+def test_closed_path_search_gives_the_fp64_states(qz, oracle, hyb, kind, B):
+    """The tail-biting pass is searched for between bounds from the free pass and run in full only where the search does not
+    settle it: the states of the 256- and 512-thread forms against fp64 metrics, and a few tiles against the CPU
+    algorithm.  767 and 769 tiles are one fewer and one more than the workgroups of a launch."""
+    say("case: closed paths, %s, B = %d" % (kind, B))
+    qz.set_tlut(None)
+    l0, l1 = qz.lut()
+    X = _closing_inputs(kind, B, np.asarray(l0), np.asarray(l1))
+    got = {}
+    try:
+        for mode in (1, 2, 3):
+            say("  mode %d" % mode)
+            qz.set_viterbi_mode(mode)
+            got[mode] = qz.viterbi_tiles(X)
+    finally:
+        qz.set_viterbi_mode(0)
+    for mode in (2, 3):
+        same = np.all(got[mode][0] == got[1][0], axis=1)
+        assert same.all(), "mode %d: tiles %s" % (mode, np.nonzero(~same)[0][:10])
+        assert np.array_equal(got[mode][1], got[1][1])
+    some = list(range(0, B, 97))
+    assert np.array_equal(got[1][0][some], oracle.quantize_tiles(hyb, X[some], fast=True))
