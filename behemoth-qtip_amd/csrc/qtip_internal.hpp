@@ -243,6 +243,7 @@ struct TileJob {
   // ticks of the 100 MHz clock a workgroup of a pair waits for the other before the first does the rest alone
   unsigned long long pair_patience = 50000000ull;
   uint32_t margin = kViterbiMargin;
+  bool search = true;  // mode 0: the second pass as a search between bounds from the first (set by launch_viterbi_tiles; same results)
   unsigned* stats = nullptr;  // device counters (optional): [0], [1] += passes of the first / second kind run again
 };
 size_t viterbi_workspace_bytes(int slots);

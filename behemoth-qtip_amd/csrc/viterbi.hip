@@ -564,9 +564,9 @@ constexpr int kMirror32 = 0xfeb;
 static_assert(64 * kGroups <= 2 * kHistWordsPerTile, "the 32-bit kept metrics (64 steps) must fit the fp64 slot");
 // What the search for the closed path needs of a free pass (close_path below) lies behind the 32-bit kept metrics: the
 // upper halves of the metrics entering the steps 1 .. 128 + kTurn (kBoundRow values each).
-constexpr int kTurn = 40;              // steps the free pass runs on into the sequence's second round
+constexpr int kTurn = 48;              // steps the free pass runs on into the sequence's second round
 constexpr int kBoundRow = kGroups / 2;
-constexpr int kCloseList = 256;        // partial paths of a step
+constexpr int kCloseList = 256;        // room for the partial paths of a step
 constexpr int kCloseSlots = 512;       // hash slots in which partial paths of one group meet
 constexpr int kClosePaths = 3520;      // partial paths of all steps together
 constexpr int kCloseRing = 4;          // rows of bounds in LDS
@@ -630,13 +630,13 @@ __device__ __forceinline__ uint32_t err_units(double l0, double l1, double x0, d
 // 4..7), and the table's 1024 entries two each instead of four.
 // kHalf: steps 0 .. 63 only; the metrics entering step 64 are left in metric buffer 0 (the other half of the sequence is
 // another workgroup's, viterbi_pair_kernel).
-// bounds (a whole free pass): the upper halves of the metrics entering step i go to row i, and after its end the pass runs
-// on for kTurn steps, whose metrics are kept as bounds only; returns the least by which a metric has grown over the last
+// bounds (a whole free pass): the upper halves of the metrics entering step i go to row i; run_on: they are
+// wanted, and after its end the pass runs on for kTurn steps, whose metrics are kept as bounds only; returns the least by which a metric has grown over the last
 // round, that is from entering step kTurn to entering step 128 + kTurn, rounded down.
 template <bool kSym, bool kWide, bool kHalf = false>
 __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __restrict__ entry_d, int roll, int ov,
                                                    uint32_t* __restrict__ hist, int first_kept, const Unit unit,
-                                                   uint16_t* __restrict__ bounds = nullptr) {
+                                                   uint16_t* __restrict__ bounds = nullptr, bool run_on = false) {
   constexpr bool kBounds = kSym && !kHalf;
   constexpr int kT = kWide ? 2 * kThreads : kThreads, kSlotsOwn = kWide ? 4 : 8, kEnt = 1024 / kT;
   const int tfull = kWide ? opaque_tid_wide() : opaque_tid();
@@ -839,7 +839,7 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
       if (upper) slots(std::integral_constant<int, 4>{});
       else slots(std::integral_constant<int, 0>{});
     }
-    if constexpr (kBounds) {
+    if (kBounds && run_on) {
       uint16_t* const b = bounds + size_t(it + 1) * kBoundRow + 8 * tid + 4 * upper;
       if constexpr (kWide) *reinterpret_cast<uint2*>(b) = uint2{packed[0], packed[1]};
       else *reinterpret_cast<uint4*>(b) = uint4{packed[0], packed[1], packed[2], packed[3]};
@@ -894,6 +894,7 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
     __syncthreads();
     if (tfull == 0) sm.red32[0][0] = b1, sm.red32[0][1] = b2 - b1, sm.red32[0][2] = bj;
     __syncthreads();
+    if (!run_on) return 0;
 #pragma nounroll
     for (int it = kSteps; it < kSteps + kTurn; it += 2) {
       step(it, Plain{}, Even{});
@@ -1197,12 +1198,13 @@ __device__ __forceinline__ uint32_t trace_back32(Smem& sm, const double* __restr
 // the metrics, which makes them weaker by less than 65536 units and never too large.  A result counts if it is under the
 // limit the search ended with (a path left out then costs more) and no two paths that met in a group were closer than
 // `margin`: the winner then beats every other closed path by that much, and the fp64 recursion takes it.  Otherwise
-// the limit is raised twice, then false is returned and the caller runs the pass (0.6 % of the tiles).
+// the search is tried once more with a higher limit, then false is returned and the caller runs the pass.
 // What bounds it: latency.  A step is a chain of five LDS round trips and some 150 instructions, 0.85 us by itself and
 // 1.1 us beside two other workgroups, 120 steps a tile; the pipes it leaves idle are the other workgroups' forward passes'.
 // Per tile with three workgroups on a compute unit 140 us instead of 294 + 75 for the forward recursion and its
-// trace-back, with 60 us more in the free pass for its longer way (kTurn 32 / 40 / 48: 76.5 / 72.5 / 72.4 ms for 768 tile
-// rows of 128 blocks; a forward pass: 89.5).
+// trace-back, with 60 us more in the free pass for its longer way (768 tile rows through 128 blocks 89.3 -> 69.9 ms; kTurn
+// 40 / 48 / 56: 70.0 / 69.9 / 71.3; at most 48 / 64 / 128 partial paths in the first attempt: 70.6 / 70.0 / 70.7, three
+// attempts with up to 256: 73.3, one: 73.8).
 // LDS operations of the search.  Written out: rows of bounds are on their way into LDS meanwhile (direct-to-LDS loads), and
 // before an LDS write or atomic of its own the compiler would wait for all of them.
 __device__ __forceinline__ uint32_t lds_at(const void* p) { return uint32_t(reinterpret_cast<size_t>(p)); }
@@ -1288,8 +1290,9 @@ __device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const u
   uint32_t stamp = 0xfffff000u, counter = lds_at(sm.close_count), seen = 0, seen_other = 0;
   bool ok = false;
 #pragma nounroll
-  for (int attempt = 0; attempt < 3 && !ok; ++attempt) {
-    uint32_t limit = least + 131072u + winner / (attempt == 0 ? 32u : attempt == 1 ? 20u : 12u);
+  for (int attempt = 0; attempt < 2 && !ok; ++attempt) {
+    uint32_t limit = least + 131072u + winner / (attempt ? 20u : 32u);
+    const uint32_t cap = attempt ? 128u : 64u;  // partial paths of a step
     if (limit >= kWinnerMax || limit < least) return false;
     issue(kSteps - 1);
     issue(kSteps - 2);
@@ -1366,7 +1369,7 @@ __device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const u
       count = uint32_t(__builtin_amdgcn_readfirstlane(int(count)));
       const uint32_t m = count - seen;
       seen = seen_other, seen_other = count, counter ^= lds_at(sm.close_count) ^ lds_at(sm.close_count + 1), stamp -= 4096u;
-      if (m - 1u >= uint32_t(kCloseList)) {
+      if (m - 1u >= cap) {
         // none left, or two too close together, or too many: those once more with a lower limit
         if (m == 0 || m >= 0x10000u || limit - least < 4096u || stamp < 0x10000000u) break;
         limit -= (limit - least) / 4;
@@ -1387,7 +1390,7 @@ __device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const u
         }
         // a path that has come to the free path's group is closed by it, at a cost below on + 131072 - M_64[ov]
         if (on < kWinnerMax) limit = min(limit, on + 131072u + 2u * min(margin, 1u << 20));
-        if (!on_free && attempt < 2) limit = min(limit, off + min(kSat - off, 131072u + winner / (attempt ? 32u : 56u)));
+        if (!on_free) limit = min(limit, off + min(kSat - off, 131072u + winner / (attempt ? 32u : 56u)));
         lds_barrier();
         if (tid < 2) lds_put32(lds_at(sm.close_least + tid), kSat);
       }
@@ -1471,7 +1474,8 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
       const Unit unit = unit_of(unit_log2);
       if (pass == 0) {
         const uint32_t grown = forward_pass32<true, kWide>(
-            sm, entry_d, roll, -1, hist32, 62, unit, reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(hist32) + kBoundsAt));
+            sm, entry_d, roll, -1, hist32, 62, unit, reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(hist32) + kBoundsAt),
+            kClose && job.search);
         const uint32_t winner = sm.red32[0][0];
         flag |= uint32_t(sm.red32[0][1] < job.margin) | uint32_t(winner >= kWinnerMax);
         const uint32_t s = trace_back32<true, kWide>(sm, entry_d, hist32, roll, sm.red32[0][2], 64, kClose, job.margin,
@@ -1481,7 +1485,7 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
         // not fit is replaced by the true one when the pass is repeated on fp64 metrics)
         expected = __builtin_ldexpf(float(winner), -unit_log2);
         if constexpr (kClose) {
-          if (!flag && passes_end > 1)
+          if (!flag && passes_end > 1 && job.search)
             closed = close_path<kWide>(sm, tl, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(s & 0xfffu))),
                                        uint32_t(__builtin_amdgcn_readfirstlane(int(winner))), grown, job.margin, unit);
         }
@@ -1568,7 +1572,7 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
   __syncthreads();
   double* hist = hist_all + size_t(blockIdx.x) * kSlotWords;
   // More tiles than workgroups: whoever is done takes the next one (a tile's time depends on its search: 4096 tiles
-  // 3.31 ms dealt out beforehand, 2.7 ms this way)
+  // 3.31 ms dealt out beforehand, 2.66 ms this way)
   uint32_t* const handed_out = &reinterpret_cast<PairArea*>(hist_all + kHistWordsPerTile)->flag;
   for (long tile = blockIdx.x; tile < job.tiles;) {
     float expected = 0.f;  // the free pass's winner of this tile row's previous column block (0: none yet)
@@ -2113,8 +2117,9 @@ static int viterbi_device_slots() {
   return viterbi_max_slots(dev);
 }
 
-bool launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const float* d_entry_f, void* workspace,
+bool launch_viterbi_tiles(const TileJob& tile_job, const double* d_entry_d, const float* d_entry_f, void* workspace,
                           int slots, hipStream_t s, hipEvent_t start, hipEvent_t stop) {
+  TileJob job = tile_job;
   if (job.tiles <= 0) return true;
   QTIP_REQUIRE(slots > 0 && workspace != nullptr, "viterbi: missing workspace");
   if (!job.X) {  // LDLQ block: the targets come from the feedback operands
@@ -2130,6 +2135,10 @@ bool launch_viterbi_tiles(const TileJob& job, const double* d_entry_d, const flo
   }
   QTIP_REQUIRE(job.blocks == 1 || (!job.X && !job.packed), "viterbi: several blocks per tile row only for LDLQ launches");
   const unsigned grid = unsigned(job.tiles < slots ? job.tiles : slots);
+  // A search takes a third of the pass's time on average and longer than the pass where it has to give up, and a launch
+  // lasts as long as its slowest workgroup: one tile each, 768 tiles 732 us with searches and 695 without; 1100 tiles
+  // 1005 / 1063, 1600 1364 / 1491, 4096 2660 / 3700, 768 tile rows of 8 blocks each 4.2 / 5.1 ms.
+  job.search = job.blocks > 1 || job.tiles > long(grid);
   // the wide form where the launch leaves two thirds of the chip's workgroup slots empty anyway (and the 32-bit
   // passes, which are what it shares out over its 512 threads, are in use)
   const bool wide = job.mode == 0 && (job.wide > 0 || (job.wide < 0 && 3 * job.tiles <= viterbi_device_slots()));

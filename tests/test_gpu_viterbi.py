@@ -375,11 +375,11 @@ def _closing_inputs(kind, B, l0, l1):
 
 
 @pytest.mark.parametrize("kind", ["scales", "join", "flat", "zeros", "mirror"])
-@pytest.mark.parametrize("B", [1, 767, 769])
+@pytest.mark.parametrize("B", [1, 769, 1100])
 def test_closed_path_search_gives_the_fp64_states(qz, oracle, hyb, kind, B):
     """The tail-biting pass is searched for between bounds from the free pass and run in full only where the search does not
     settle it: the states of the 256- and 512-thread forms against fp64 metrics, and a few tiles against the CPU
-    algorithm.  767 and 769 tiles are one fewer and one more than the workgroups of a launch."""
+    algorithm.  A launch searches when it has more tiles than workgroups (768); one tile runs both passes in full."""
     say("case: closed paths, %s, B = %d" % (kind, B))
     qz.set_tlut(None)
     l0, l1 = qz.lut()
