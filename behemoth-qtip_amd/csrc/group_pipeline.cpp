@@ -336,6 +336,129 @@ int group_lanes_for(int ng, const qtip_group* groups, const qtip_opts& opt, int 
   return lanes < 2 ? 1 : int(lanes);
 }
 
+// Small groups of one shape, together.  On lanes, LDLQ is a launch per buffer and lane, and the lanes share what hardware
+// queues the process has: six groups of 128 tile rows ran two or three at a time.  Here the lanes prepare their groups
+// (rotation, factor, weights), one call walks the tile rows of all of them (ldlq_impl with parts: a launch takes rows of
+// several groups, each with its own factor), and the lanes finish them.  Same results: every tile sees the operands it sees
+// alone.  Six 2048 x 2560 groups from host memory: 166 -> 95 ms.
+// A group that cannot be prepared (its H is not positive definite, say) does not keep the others from their results; the
+// first such error is thrown at the end.
+int together_batch(int ng, long rows, int n, int device_slots) {
+  // groups per call: the fewest rounds of workgroups in all, then the fewest calls; its buffers stay under 32 GiB
+  const long bytes = 24L * n * n + 10L * n * 16 * rows;
+  const long most = std::min<long>({long(ng), long(qtip_ctx::kMaxLanes), std::max<long>(1, (32L << 30) / bytes)});
+  long best = 1, best_cost = -1;
+  for (long b = 1; b <= most; ++b) {
+    long cost = 0;
+    for (long g = 0; g < ng; g += b) cost += (std::min<long>(b, ng - g) * rows + device_slots - 1) / device_slots;
+    if (best_cost < 0 || cost <= best_cost) best = b, best_cost = cost;
+  }
+  return int(best);
+}
+
+static void run_groups_together(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opts& opt, qtip_timing* tms,
+                                double* ldl_wait) {
+  const int n = groups[0].n;
+  const long mt = 16 * tile_rows_of(groups[0]);
+  const int batch = together_batch(ng, mt / 16, n, viterbi_max_slots(c->device));
+  const size_t nm = size_t(n) * mt, nn = size_t(n) * n, states = size_t(mt / 16) * (n / 16) * 128;
+  ArenaScope memory(&c->arena);
+  DBuf<float> WT(nm * batch), hat(nm * batch), L(nn * batch);
+  DBuf<uint16_t> Q(states * batch);
+  qtip_opts gopt = opt;
+  const int team = opt.ldl_threads > 0 ? opt.ldl_threads : std::max(1, int(std::thread::hardware_concurrency()));
+  gopt.ldl_threads = std::max(1, team / batch);
+  struct Lane {
+    qtip_ctx* c = nullptr;
+    GroupWork w;
+    std::vector<float> su;
+    double creg = 0;
+    std::exception_ptr err;
+  };
+  std::exception_ptr first_err;
+  for (int g0 = 0; g0 < ng; g0 += batch) {
+    const int count = std::min(batch, ng - g0);
+    std::vector<Lane> lanes(static_cast<size_t>(count));
+    for (int k = 0; k < count; ++k) {
+      lanes[size_t(k)].c = lane_context(c, k);
+      order_streams(c->stream, lanes[size_t(k)].c->stream);  // inputs the caller ordered before the context's stream
+    }
+    // `work` for every group of the batch, each on its lane's thread (the calling thread takes the first)
+    auto on_lanes = [&](auto work) {
+      auto run = [&](int k) {
+        Lane& l = lanes[size_t(k)];
+        if (l.err) return;
+        try {
+          QTIP_HIP(hipSetDevice(c->device));  // this thread's own current device
+          ArenaScope lane_memory(&l.c->arena);
+          work(k, l, groups[g0 + k]);
+        } catch (...) {
+          l.err = std::current_exception();
+          // nothing queued for the group may outlive its buffers
+          (void)hipStreamSynchronize(l.c->stream);
+        }
+      };
+      std::vector<std::thread> th;
+      std::vector<int> deferred;
+      for (int k = 1; k < count; ++k) {
+        try {
+          th.emplace_back(run, k);
+        } catch (...) {
+          deferred.push_back(k);  // no thread could be started for it
+        }
+      }
+      run(0);
+      for (int k : deferred) run(k);
+      for (std::thread& t : th) t.join();
+    };
+    on_lanes([&](int k, Lane& l, const qtip_group& g) {
+      qtip_timing T{};
+      l.su.assign(size_t(n), 0.0f);
+      reserve_group_ring(l.c, n, 1, true);
+      double t0 = now_s();
+      rotate_hessian_impl(l.c, g.H, g.h_on_device != 0, n, g.seed, opt.sigma_reg, l.su.data(), &l.creg, nullptr,
+                          l.c->ring_dHRr[0].p);
+      T.rht = now_s() - t0;
+      t0 = now_s();
+      ldl_hessian_device_impl(l.c, nullptr, n, nullptr, l.c->ring_dHRr[0].p, L.p + nn * k);
+      T.ldl_cpu = now_s() - t0;
+      if (ldl_wait) ldl_wait[g0 + k] = T.ldl_cpu;
+      l.w.wt = WT.p + nm * k, l.w.hat = hat.p + nm * k, l.w.states = Q.p + states * k;
+      group_prepare(l.c, l.w, g.nlin, g.lins, n, g.seed, l.su.data(), gopt, g.outs, &T);
+    });
+    // the groups that are ready, as runs of neighbours in the buffers (all of them, unless one failed)
+    const double t0 = now_s();
+    double vit = 0;
+    int ready = 0;
+    for (int k = 0; k < count;) {
+      if (lanes[size_t(k)].err) {
+        ++k;
+        continue;
+      }
+      int end = k;
+      while (end < count && !lanes[size_t(end)].err) ++end;
+      double v = 0;
+      ldlq_impl(c, WT.p + nm * k, L.p + nn * k, n, mt, hat.p + nm * k, Q.p + states * k, opt.feedback, &v, opt.ldlq_chains,
+                end - k);
+      vit += v;
+      ready += end - k;
+      k = end;
+    }
+    const double ldlq_s = now_s() - t0;
+    on_lanes([&](int k, Lane& l, const qtip_group& g) {
+      qtip_timing T{};
+      l.w.T.ldlq += ldlq_s / ready, l.w.T.viterbi += vit / ready;  // a group's share of the call
+      group_finish(l.c, l.w, g.nlin, g.lins, n, l.creg, nullptr, l.c->ring_dHRr[0].p, gopt, g.outs, &T);
+      if (tms) tms[g0 + k] = T;
+    });
+    for (Lane& l : lanes) {
+      order_streams(l.c->stream, c->stream);
+      if (l.err && !first_err) first_err = l.err;
+    }
+  }
+  if (first_err) std::rethrow_exception(first_err);
+}
+
 void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opts& opt, qtip_timing* tms,
                      double* ldl_wait) {
   QTIP_REQUIRE(ng >= 0 && (ng == 0 || groups), "run_groups: bad arguments");
@@ -344,15 +467,36 @@ void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_o
     QTIP_REQUIRE(groups[g].n > 0 && groups[g].H && groups[g].nlin > 0 && groups[g].lins && groups[g].outs,
                  "run_groups: group %d is incomplete", g);
   // Mixed sizes (a layer's gate/up group beside its o-proj group): the groups that fill the chip on their own go
-  // through the overlapped schedule first, in their order, the others then share the chip on lanes.
+  // through the overlapped schedule first, in their order, then those of one shape together, and what is left shares the
+  // chip on lanes.
+  const int slots = viterbi_max_slots(c->device);
+  const bool may_group = opt.group_lanes == 0 && opt.ldl_device_updates != 0;
+  auto alike = [&](int a, int b) { return groups[a].n == groups[b].n && tile_rows_of(groups[a]) == tile_rows_of(groups[b]); };
   if (opt.group_lanes == 0 && ng >= 3) {
-    const long slots = viterbi_max_slots(c->device);
-    std::vector<int> large, small;
-    for (int g = 0; g < ng; ++g) (tile_rows_of(groups[g]) >= slots ? large : small).push_back(g);
-    if (!large.empty() && small.size() >= 2) {
-      for (const std::vector<int>* part : {&large, &small}) {
+    std::vector<std::vector<int>> parts(1), shapes;  // parts[0]: the large ones
+    std::vector<int> left;
+    for (int g = 0; g < ng; ++g) {
+      if (tile_rows_of(groups[g]) >= slots) {
+        parts[0].push_back(g);
+        continue;
+      }
+      size_t k = 0;
+      while (k < shapes.size() && !(may_group && alike(shapes[k][0], g))) ++k;
+      if (k == shapes.size()) shapes.emplace_back();
+      shapes[k].push_back(g);
+    }
+    for (std::vector<int>& shape : shapes)
+      if (shape.size() >= 2) parts.push_back(shape);
+      else left.push_back(shape[0]);
+    if (!left.empty()) parts.push_back(left);
+    if (parts[0].empty()) parts.erase(parts.begin());
+    // (a large group or two beside one small one: in their order, as one schedule)
+    const bool one_schedule = parts.size() == 1 || (parts.size() == 2 && left.size() == 1 && parts[1].size() == 1 &&
+                                                    tile_rows_of(groups[parts[0][0]]) >= slots);
+    if (!one_schedule) {
+      for (const std::vector<int>& part : parts) {
         std::vector<qtip_group> sub;
-        for (int g : *part) sub.push_back(groups[g]);
+        for (int g : part) sub.push_back(groups[g]);
         std::vector<qtip_timing> st(sub.size());
         std::vector<double> sw(sub.size(), 0.0);
         std::exception_ptr err;
@@ -361,16 +505,22 @@ void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_o
         } catch (...) {
           err = std::current_exception();
         }
-        for (size_t i = 0; i < part->size(); ++i) {
-          if (tms) tms[(*part)[i]] = st[i];
-          if (ldl_wait) ldl_wait[(*part)[i]] = sw[i];
+        for (size_t i = 0; i < part.size(); ++i) {
+          if (tms) tms[part[i]] = st[i];
+          if (ldl_wait) ldl_wait[part[i]] = sw[i];
         }
         if (err) std::rethrow_exception(err);
       }
       return;
     }
   }
-  const int lanes = group_lanes_for(ng, groups, opt, viterbi_max_slots(c->device));
+  bool one_shape = may_group && ng >= 2 && tile_rows_of(groups[0]) < slots && groups[0].n % 128 == 0;
+  for (int g = 1; g < ng; ++g) one_shape = one_shape && alike(0, g);
+  if (one_shape) {
+    run_groups_together(c, ng, groups, opt, tms, ldl_wait);
+    return;
+  }
+  const int lanes = group_lanes_for(ng, groups, opt, slots);
   if (lanes == 1) {
     // the per-group device buffers of the quantizing thread come from the context's arena and stay there between
     // groups and calls: a hipFree waits for the whole device, the factorization's queued updates included (a dozen

@@ -37,7 +37,8 @@ constexpr int GVK = 8, GST = 4;
 __global__ __launch_bounds__(256, 3) void gemm_tn_f64_splitk_kernel(int N, long K, const float* __restrict__ A, long lda,
                                                                     const float* __restrict__ B1,
                                                                     const float* __restrict__ B2, long ldb,
-                                                                    double* __restrict__ out, long ldo) {
+                                                                    double* __restrict__ out, long ldo, PartStrides part) {
+  A += blockIdx.z * part.a, B1 += blockIdx.z * part.b, B2 += blockIdx.z * part.b, out += blockIdx.z * part.out;
   __shared__ __attribute__((aligned(16))) float S[GST][3][GVK][BM];  // [stage][A | B1 | B2][k][column]
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -182,7 +183,9 @@ __global__ __launch_bounds__(256, 3) void gather_img_kernel(int N, long K, const
                                                             const uint16_t* __restrict__ Al, long lda,
                                                             const uint16_t* __restrict__ Bh,
                                                             const uint16_t* __restrict__ Bl, long ldb,
-                                                            float* __restrict__ out, long ldo) {
+                                                            float* __restrict__ out, long ldo, PartStrides part) {
+  Ah += blockIdx.z * part.a, Al += blockIdx.z * part.a, Bh += blockIdx.z * part.b, Bl += blockIdx.z * part.b;
+  out += blockIdx.z * part.out;
   __shared__ __attribute__((aligned(16))) uint16_t S[IST][4][SB][IK];  // [stage][Ah | Al | Bh | Bl][row][k]
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave >> 1, wn = wave & 1;
   const long j0 = long(blockIdx.x) * SB;
@@ -293,12 +296,15 @@ int gemm_splitk_splits(long K, int N, int slots) {
 }
 
 int launch_gemm_tn_f64_gather(int N, long K, const float* A, long lda, const float* B1, const float* B2, long ldb,
-                              double* P, double* partials, int slots, hipStream_t s, bool reduce) {
+                              double* P, double* partials, int slots, hipStream_t s, bool reduce, int parts,
+                              PartStrides strides) {
   QTIP_REQUIRE(N >= 4 && K > 0 && K % KC == 0 && N % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && B2 != nullptr,
                "fp64 gather GEMM needs 16-byte aligned fp32 rows and K %% 16 == 0");
-  const int S = gemm_splitk_splits(K, N, slots);
-  dim3 grid(unsigned((N + BN - 1) / BN), unsigned(S));
-  gemm_tn_f64_splitk_kernel<<<grid, dim3(256), 0, s>>>(N, K, A, lda, B1, B2, ldb, S == 1 ? P : partials, N);
+  QTIP_REQUIRE(parts == 1 || (parts > 1 && !reduce), "products side by side leave the sum to the reader");
+  const int S = gemm_splitk_splits(K, N * parts, slots);
+  dim3 grid(unsigned((N + BN - 1) / BN), unsigned(S), unsigned(parts));
+  if (S == 1) strides.out = long(BM) * N;
+  gemm_tn_f64_splitk_kernel<<<grid, dim3(256), 0, s>>>(N, K, A, lda, B1, B2, ldb, S == 1 ? P : partials, N, strides);
   QTIP_HIP(hipGetLastError());
   if (S > 1 && reduce) {
     const long count = long(BM) * N;
@@ -319,12 +325,14 @@ void launch_split_transpose_bf16(const float* X, const float* X2, long ldx, long
 
 int launch_gemm_img_gather(int N, long K, const uint16_t* Ah, const uint16_t* Al, long lda, const uint16_t* Bh,
                            const uint16_t* Bl, long ldb, float* P, float* partials, int slots, hipStream_t s,
-                           bool reduce) {
+                           bool reduce, int parts, PartStrides strides) {
   QTIP_REQUIRE(N > 0 && K > 0 && K % IK == 0 && lda % 8 == 0 && ldb % 8 == 0 && Ah && Al && Bh && Bl,
                "split-bf16 gather GEMM needs K %% 16 == 0 and 16-byte aligned image rows");
-  const int S = gemm_splitk_splits(K, N, slots);
-  dim3 grid(unsigned((N + SB - 1) / SB), unsigned(S));
-  gather_img_kernel<<<grid, dim3(256), 0, s>>>(N, K, Ah, Al, lda, Bh, Bl, ldb, S == 1 ? P : partials, N);
+  QTIP_REQUIRE(parts == 1 || (parts > 1 && !reduce), "products side by side leave the sum to the reader");
+  const int S = gemm_splitk_splits(K, N * parts, slots);
+  dim3 grid(unsigned((N + SB - 1) / SB), unsigned(S), unsigned(parts));
+  if (S == 1) strides.out = long(SB) * N;
+  gather_img_kernel<<<grid, dim3(256), 0, s>>>(N, K, Ah, Al, lda, Bh, Bl, ldb, S == 1 ? P : partials, N, strides);
   QTIP_HIP(hipGetLastError());
   if (S > 1 && reduce) {
     const long count = long(SB) * N;

@@ -233,6 +233,10 @@ struct TileJob {
   // col0 + 16 (blocks - 1) ..) down to the first (col0 ..), state words at q_offset + block: the blocks of a tile row
   // depend on each other only through that row's own hatWT values, so nothing has to wait for another workgroup
   int blocks = 1;
+  // LDLQ of several groups of one shape in one launch (0: one group): tiles part_tiles p .. part_tiles (p + 1) - 1 belong to
+  // group p, whose operands lie p times these many elements behind the pointers above
+  long part_tiles = 0;
+  long part_w = 0, part_l = 0, part_prod = 0, part_states = 0, part_dimg = 0;  // WT and hatWT, L, prod, states, dimg
   // 0: both passes run on 32-bit metrics first and a pass whose traced decisions are not all won by `margin` units of
   // 2^-26 is run again on fp64 metrics (same results as mode 1, bit for bit); 1: fp64 metrics only
   int mode = 0;

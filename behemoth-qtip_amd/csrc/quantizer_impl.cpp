@@ -102,15 +102,18 @@ int ldlq_default_chains(qtip_ctx* c) {
   return c->default_chains;
 }
 
+// parts > 1: that many groups of one shape, whose WT, L, hatWT and Q follow each other; a chain takes whole groups.  Every tile
+// sees the operands it sees in a call of its own group.
 void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, float* hatWT, uint16_t* Q, int feedback,
-               double* vit_seconds, int chains) {
+               double* vit_seconds, int chains, int parts) {
   QTIP_REQUIRE(n % 128 == 0, "LDLQ needs n %% 128 == 0 (n = %ld)", n);
   QTIP_REQUIRE(chains >= 0 && chains <= qtip_ctx::kMaxChains, "LDLQ runs as 1 to %d chains (0: default), not %d", qtip_ctx::kMaxChains, chains);
   QTIP_REQUIRE(m % 16 == 0 && m > 0, "LDLQ needs m %% 16 == 0 (m = %ld)", m);
   QTIP_REQUIRE(feedback == 0 || feedback == 1, "unknown feedback mode %d", feedback);
   hipStream_t s = c->stream;
   ensure_viterbi_workspace(c);
-  const long ntr = m / 16, nblk = n / 16;
+  QTIP_REQUIRE(parts >= 1, "LDLQ of %d groups", parts);
+  const long ptr = m / 16, ntr = ptr * parts, nblk = n / 16;  // tile rows of a group and of all
   // chains: only where every chain still fills its share of the chip.  Default: three where the context found its two
   // chain streams and the LDL's stream running beside its own stream and beside each other when it was made (each on
   // a hardware queue of its own), or where the environment says the process was given six queues or more; else two.
@@ -118,14 +121,19 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
   // time stamps and the context goes back to two for good when the first launches of the chains ran one after the
   // other.
   int nch = chains == 0 ? ldlq_default_chains(c) : chains;
-  while (nch > 1 && ntr < long(nch) * (c->vit_slots / nch)) --nch;
+  // (groups side by side: whole groups to a chain, and from half of the chip on, below which pairs of workgroups are faster)
+  if (parts > 1)
+    while (nch > 1 && (parts % nch != 0 || 2 * ntr <= c->vit_slots)) --nch;
+  else
+    while (nch > 1 && ntr < long(nch) * (c->vit_slots / nch)) --nch;
   struct Chain {
     hipStream_t s;
     long tile0, tiles;   // tile rows tile0 .. tile0 + tiles - 1
-    long r0, rows;       // weight rows (columns of WT) 16 tile0 .., 16 tiles of them
+    long r0, rows;       // weight rows (columns of WT) 16 tile0 .., 16 tiles of them (of all groups; one group: its own)
+    int part0, parts;    // groups
     int slot0, slots;    // share of the kept-metrics workspace
-    double *prod, *parts;     // feedback 0: 128 x rows slab and the split-K partial slabs
-    float *prod32, *parts32;  // feedback 1: the same in fp32
+    double *prod, *slabs;     // feedback 0: 128 x rows slab and the split-K partial slabs
+    float *prod32, *slabs32;  // feedback 1: the same in fp32
   } ch[qtip_ctx::kMaxChains];
   for (int k = 0; k < nch; ++k) {
     if (k > 0 && !c->chain_stream[k - 1]) QTIP_HIP(hipStreamCreateWithFlags(&c->chain_stream[k - 1], hipStreamNonBlocking));
@@ -134,25 +142,31 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
     ch[k].tiles = ntr * (k + 1) / nch - ch[k].tile0;
     ch[k].r0 = 16 * ch[k].tile0;
     ch[k].rows = 16 * ch[k].tiles;
+    ch[k].part0 = parts > 1 ? parts * k / nch : 0;
+    ch[k].parts = parts > 1 ? parts / nch : 1;
     ch[k].slot0 = c->vit_slots * k / nch;
     ch[k].slots = c->vit_slots * (k + 1) / nch - ch[k].slot0;
   }
   // The feedback of the rows quantized in earlier buffers is gathered per buffer into a 128 x rows slab per chain:
   // feedback 0 in fp64 (fp64 MFMA), feedback 1 in fp32 from bf16 hi/lo split operands (the reference GPU's arithmetic)
   const int max_splits = kMaxGatherSplits;
-  DBuf<double> prod(feedback == 0 ? size_t(128) * m : 0), parts(feedback == 0 ? size_t(max_splits) * 128 * m : 0);
-  DBuf<float> prod32(feedback == 1 ? size_t(128) * m : 0), parts32(feedback == 1 ? size_t(max_splits) * 128 * m : 0);
+  const size_t mall = size_t(m) * parts, nm = size_t(n) * m, nn = size_t(n) * n;
+  DBuf<double> prod(feedback == 0 ? 128 * mall : 0), slabs(feedback == 0 ? max_splits * 128 * mall : 0);
+  DBuf<float> prod32(feedback == 1 ? 128 * mall : 0), slabs32(feedback == 1 ? max_splits * 128 * mall : 0);
   for (int k = 0; k < nch; ++k) {
     ch[k].prod = feedback == 0 ? prod.p + size_t(128) * ch[k].r0 : nullptr;
-    ch[k].parts = feedback == 0 ? parts.p + size_t(max_splits) * 128 * ch[k].r0 : nullptr;
+    ch[k].slabs = feedback == 0 ? slabs.p + size_t(max_splits) * 128 * ch[k].r0 : nullptr;
     ch[k].prod32 = feedback == 1 ? prod32.p + size_t(128) * ch[k].r0 : nullptr;
-    ch[k].parts32 = feedback == 1 ? parts32.p + size_t(max_splits) * 128 * ch[k].r0 : nullptr;
+    ch[k].slabs32 = feedback == 1 ? slabs32.p + size_t(max_splits) * 128 * ch[k].r0 : nullptr;
   }
   // feedback 1: the operands of the gathered product as bf16 hi / lo images with k contiguous: L transposed, made
   // here once; the residual WT - hatWT, weight row major, written by the Viterbi launches as they decode
-  DBuf<uint16_t> limg(feedback == 1 ? size_t(2) * n * n : 0), dimg(feedback == 1 ? size_t(2) * m * n : 0);
-  if (feedback == 1) launch_split_transpose_bf16(L, nullptr, n, n, n, limg.p, limg.p + size_t(n) * n, n, true, s);
-  QTIP_HIP(hipMemsetAsync(hatWT, 0, size_t(n) * m * 4, s));
+  // (hi and lo of a group follow each other)
+  DBuf<uint16_t> limg(feedback == 1 ? 2 * nn * parts : 0), dimg(feedback == 1 ? 2 * nm * parts : 0);
+  if (feedback == 1)
+    for (int p = 0; p < parts; ++p)
+      launch_split_transpose_bf16(L + nn * p, nullptr, n, n, n, limg.p + 2 * nn * p, limg.p + 2 * nn * p + nn, n, true, s);
+  QTIP_HIP(hipMemsetAsync(hatWT, 0, nm * parts * 4, s));
   Events timed, pacing, joins;  // timed: a (start, stop) pair per Viterbi launch, stamped by the launch itself
   // the other chains start once the caller's inputs and the cleared outputs are there, a third (two thirds) of a
   // tile's time later; a launch walks tiles / slots of them
@@ -182,8 +196,10 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
         const Chain& C = ch[k];
         if (nbuf_done >= kAhead) QTIP_HIP(hipEventSynchronize(pace[k][(nbuf_done - kAhead) % (kAhead + 1)]));
         // prod[r][:] = sum_{k >= bufend} L[k][c0 + r] (WT - hatWT)[k][:], r < 128
-        const float* Lp = L + long(bufend) * n + c0;
-        const float *Wp = WT + long(bufend) * m + C.r0, *Hp = hatWT + long(bufend) * m + C.r0;
+        const size_t r0 = parts > 1 ? nm * C.part0 : size_t(C.r0);  // the chain's first operand in WT and hatWT
+        const long crows = parts > 1 ? m : C.rows;                  // its weight rows of a group
+        const float* Lp = L + nn * C.part0 + long(bufend) * n + c0;
+        const float *Wp = WT + long(bufend) * m + r0, *Hp = hatWT + long(bufend) * m + r0;
         // (the split-K partial slabs are summed by the Viterbi launch as it forms its targets, in the order the
         // product's own reduction kernel would add them)
         int splits = 1;
@@ -191,32 +207,42 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
           if (feedback == 0) QTIP_HIP(hipMemsetAsync(C.prod, 0, size_t(128) * C.rows * sizeof(double), C.s));
           else QTIP_HIP(hipMemsetAsync(C.prod32, 0, size_t(128) * C.rows * sizeof(float), C.s));
         } else if (feedback == 0) {
-          splits = launch_gemm_tn_f64_gather(int(C.rows), n - bufend, Lp, n, Wp, Hp, m, C.prod, C.parts, C.slots, C.s, false);
+          splits = launch_gemm_tn_f64_gather(int(crows), n - bufend, Lp, n, Wp, Hp, m, C.prod, C.slabs, C.slots, C.s, false,
+                                             C.parts, {long(nn), long(nm), long(max_splits) * 128 * m});
         } else {
-          const uint16_t* la = limg.p + size_t(c0) * n + bufend;
-          const uint16_t* da = dimg.p + size_t(C.r0) * n + bufend;
-          splits = launch_gemm_img_gather(int(C.rows), n - bufend, la, la + size_t(n) * n, n, da, da + size_t(m) * n, n,
-                                          C.prod32, C.parts32, C.slots, C.s, false);
+          const uint16_t* la = limg.p + 2 * nn * C.part0 + size_t(c0) * n + bufend;
+          const uint16_t* da = dimg.p + (parts > 1 ? 2 * nm * C.part0 : size_t(C.r0) * n) + bufend;
+          splits = launch_gemm_img_gather(int(crows), n - bufend, la, la + nn, n, da, da + nm, n, C.prod32, C.slabs32, C.slots,
+                                          C.s, false, C.parts, {long(2 * nn), long(2 * nm), long(max_splits) * 128 * m});
         }
         {
           // one launch per buffer: a workgroup takes its tile row through the 8 column blocks, last to first, and
           // forms each block's targets (in-buffer feedback) itself; no workgroup waits for another between blocks
           TileJob job;
           job.tiles = C.tiles;
-          job.WT = WT + C.r0;
-          job.L = L;
+          job.WT = WT + r0;
+          job.L = L + nn * C.part0;
+          if (parts > 1) {
+            job.part_tiles = ptr;
+            job.part_w = long(nm), job.part_l = long(nn), job.part_dimg = long(2 * nm);
+            job.part_states = ptr * nblk * 128;
+            job.part_prod = (splits > 1 ? long(max_splits) : 1L) * 128 * m;
+          }
           job.ldl = n;
           job.bufend = bufend;
-          if (feedback == 0) job.prod64 = splits > 1 ? C.parts : C.prod;
-          else job.prod32 = splits > 1 ? C.parts32 : C.prod32;
-          job.prod_row0 = c0, job.ldp = C.rows;
-          job.prod_splits = splits, job.prod_split_stride = long(128) * C.rows;
+          if (feedback == 0) job.prod64 = splits > 1 ? C.slabs : C.prod;
+          else job.prod32 = splits > 1 ? C.slabs32 : C.prod32;
+          job.prod_row0 = c0, job.ldp = crows;
+          job.prod_splits = splits, job.prod_split_stride = long(128) * crows;
           job.states = Q + size_t(C.tile0) * nblk * 128;
           job.q_tile_stride = nblk;
           job.q_offset = c0 / 16;
-          job.hatWT = hatWT + C.r0;
+          job.hatWT = hatWT + r0;
           job.ldw = m;
-          if (feedback == 1) job.dimg_h = dimg.p + size_t(C.r0) * n, job.dimg_l = job.dimg_h + size_t(m) * n, job.ldd = n;
+          if (feedback == 1) {
+            job.dimg_h = dimg.p + (parts > 1 ? 2 * nm * C.part0 : size_t(C.r0) * n);
+            job.dimg_l = job.dimg_h + nm, job.ldd = n;
+          }
           job.col0 = c0;
           job.blocks = 8;
           c->viterbi_settings(job);
@@ -313,8 +339,8 @@ void group_prepare(qtip_ctx* c, GroupWork& w, int nlin, const qtip_linear_in* li
   QTIP_HIP(hipMemcpyAsync(d_su, host_su, size_t(n) * 4, hipMemcpyHostToDevice, s));
 
   // ---- weights -> Wr^T (n x mt), each linear's column block scaled by 1/Wscale (src/quantizer.cpp:195-249)
-  w.WT.alloc(size_t(n) * mt);
-  DBuf<float>& WT = w.WT;
+  if (!w.wt) w.WT.alloc(size_t(n) * mt), w.wt = w.WT.p;
+  float* const WT = w.wt;
   {
     DBuf<float> Wt(size_t(maxm) * n);
     DBuf<uint8_t> raw;
@@ -373,10 +399,10 @@ void group_ldlq(qtip_ctx* c, GroupWork& w, int n, const float* host_L, const flo
   QTIP_HIP(hipStreamSynchronize(s));
   T.load += now_s() - t0;
   t0 = now_s();
-  w.hatWT.alloc(size_t(n) * mt);
-  w.Q.alloc(size_t(mt / 16) * (n / 16) * 128);
+  w.hatWT.alloc(size_t(n) * mt), w.hat = w.hatWT.p;
+  w.Q.alloc(size_t(mt / 16) * (n / 16) * 128), w.states = w.Q.p;
   double vit = 0;
-  ldlq_impl(c, w.WT, dev_L ? dev_L : Ld.p, n, mt, w.hatWT, w.Q, opt.feedback, &vit, opt.ldlq_chains);
+  ldlq_impl(c, w.wt, dev_L ? dev_L : Ld.p, n, mt, w.hat, w.states, opt.feedback, &vit, opt.ldlq_chains);
   T.ldlq += now_s() - t0;
   T.viterbi += vit;
 }
@@ -389,8 +415,9 @@ void group_finish(qtip_ctx* c, GroupWork& w, int nlin, const qtip_linear_in* lin
   qtip_timing& T = w.T;
   const long mt = w.mt;
   const std::vector<long>& off = w.off;
-  DBuf<float>&WT = w.WT, &hatWT = w.hatWT, &d_su = w.d_su, &d_sv = w.d_sv;
-  DBuf<uint16_t>& Q = w.Q;
+  float *const WT = w.wt, *const hatWT = w.hat;
+  uint16_t* const Q = w.states;
+  DBuf<float>&d_su = w.d_su, &d_sv = w.d_sv;
   double t0 = now_s();
   // ---- states -> packed trellis in kernel layout, src/quantizer.cpp:305-320 (packed on the device).  The packing
   // kernel is small and the copy to the caller's (pageable) memory is the copy engines' and a host thread's work:

@@ -82,7 +82,7 @@ void ldl_hessian_device_impl(qtip_ctx* c, const float* host_HRr, int n, float* h
 void nvfp4_prepare_device_impl(qtip_ctx* c, const float* host_H, int n, double sigma_reg, float* dev_L, float* dev_dw,
                                float* host_L = nullptr, float* host_dw = nullptr);
 void ldlq_impl(qtip_ctx* c, const float* dWT, const float* dL, long n, long m, float* d_hatWT, uint16_t* dQ,
-               int feedback, double* vit_seconds, int chains);
+               int feedback, double* vit_seconds, int chains, int parts = 1);
 int ldlq_default_chains(qtip_ctx* c);  // what chains = 0 stands for in this context (decided on the first call)
 // what a group carries from one phase of its quantization to the next (device buffers, offsets of its linears, times)
 struct GroupWork {
@@ -90,10 +90,14 @@ struct GroupWork {
   std::vector<long> off;
   DBuf<float> d_su, d_sv, WT, hatWT;
   DBuf<uint16_t> Q;
+  // where Wr^T, its reconstruction and the states are: in the buffers above, or in the caller's (wt set before group_prepare)
+  float *wt = nullptr, *hat = nullptr;
+  uint16_t* states = nullptr;
   qtip_timing T{};
   double t_start = 0, carried = 0;
   void release() {
     d_su.release(), d_sv.release(), WT.release(), hatWT.release(), Q.release();
+    wt = hat = nullptr, states = nullptr;
   }
 };
 void group_prepare(qtip_ctx* c, GroupWork& w, int nlin, const qtip_linear_in* lins, int n, uint64_t seed,

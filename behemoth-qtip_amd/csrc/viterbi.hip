@@ -379,10 +379,20 @@ __device__ __forceinline__ void forward_pass(Smem& sm, const double* __restrict_
 // at TileJob), which the reference computes in a kernel of its own (ldlq_prep_kernel, src/viterbi.hip:241-267; CPU
 // form tests/test_gpu.cpp:196-207).  The (<= 112) x 16 blocks of L, WT and hatWT the tile needs are staged in the
 // metric array, which is idle between tiles; thread u then owns the sequence position u.
+// part: the group the tile belongs to, of which it is tile `tile` (TileJob::part_tiles).
+__device__ __forceinline__ long part_of(const TileJob& job, long& tile) {
+  if (!job.part_tiles) return 0;
+  const uint32_t part = uint32_t(tile) / uint32_t(job.part_tiles);
+  tile -= long(part) * job.part_tiles;
+  return part;
+}
 template <typename Acc>
-__device__ __forceinline__ void tile_targets(Smem& sm, const TileJob& job, long col0, long tile,
-                                             const Acc* __restrict__ prod) {
+__device__ __forceinline__ void tile_targets(Smem& sm, const TileJob& job, long col0, long tile, long part,
+                                             const Acc* __restrict__ prod0) {
   const int u = opaque_tid();
+  const float *const L = job.L + part * job.part_l, *const WT = job.WT + part * job.part_w;
+  const float* const hatWT = job.hatWT + part * job.part_w;
+  const Acc* const prod = prod0 + part * job.part_prod;
   const int k0 = int(col0) + 16, nk = job.bufend - k0;
   float* Ls = reinterpret_cast<float*>(sm.M);
   float* Ws = Ls + 112 * 16;
@@ -391,9 +401,9 @@ __device__ __forceinline__ void tile_targets(Smem& sm, const TileJob& job, long 
   for (int idx = u; idx < nk * 16; idx += kThreads) {
     const long k = k0 + (idx >> 4);
     const int e = idx & 15;
-    Ls[idx] = job.L[k * job.ldl + col0 + e];
-    Ws[idx] = job.WT[k * job.ldw + row0 + e];
-    Hs[idx] = job.hatWT[k * job.ldw + row0 + e];
+    Ls[idx] = L[k * job.ldl + col0 + e];
+    Ws[idx] = WT[k * job.ldw + row0 + e];
+    Hs[idx] = hatWT[k * job.ldw + row0 + e];
   }
   __syncthreads();
   const int q = perm_fwd(u), r = q >> 4, c = q & 15;
@@ -401,7 +411,7 @@ __device__ __forceinline__ void tile_targets(Smem& sm, const TileJob& job, long 
   const Acc* pp = prod + (col - job.prod_row0) * (job.ldp ? job.ldp : job.ldw) + row0 + r;
   Acc gathered = pp[0];
   for (int sp = 1; sp < job.prod_splits; ++sp) gathered += pp[long(sp) * job.prod_split_stride];
-  Acc acc = Acc(job.WT[col * job.ldw + row0 + r]) + gathered;
+  Acc acc = Acc(WT[col * job.ldw + row0 + r]) + gathered;
   for (int kk = 0; kk < nk; ++kk) acc += Acc(Ls[kk * 16 + c]) * (Acc(Ws[kk * 16 + r]) - Acc(Hs[kk * 16 + r]));
   sm.x[u] = float(_Float16(float(acc)));
 }
@@ -1524,11 +1534,11 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
 
 // States, packed words, decoded values and residual images of one block, from sm.st.
 __device__ __forceinline__ void block_outputs(const Smem& sm, const TileJob& job, const float* __restrict__ entry_f,
-                                              long tile, int blk, long col0) {
+                                              long tile, long part, int blk, long col0) {
   const int u = threadIdx.x & (kThreads - 1);
   const bool first_half = threadIdx.x < kThreads;  // global results are written once
   if (job.states && first_half && u < kSteps)
-    job.states[(tile * job.q_tile_stride + job.q_offset + blk) * kSteps + u] = sm.st[u];
+    job.states[part * job.part_states + (tile * job.q_tile_stride + job.q_offset + blk) * kSteps + u] = sm.st[u];
   if (job.packed && first_half && u < kWords) {
     uint32_t v;
     if (u == 0) v = sm.st[0];
@@ -1543,13 +1553,13 @@ __device__ __forceinline__ void block_outputs(const Smem& sm, const TileJob& job
     const uint32_t s = sm.st[u >> 1];
     const uint32_t e = ((s * (s + 1u)) >> 6) & 1023u;
     const int q = perm_fwd(u), r = q >> 4, c = q & 15;
-    const long wi = (col0 + c) * job.ldw + tile * 16 + r;
+    const long wi = part * job.part_w + (col0 + c) * job.ldw + tile * 16 + r;
     const float hv = entry_f[2 * e + (u & 1)];
     job.hatWT[wi] = hv;
     if (job.dimg_h) {
       uint32_t hi, lo;
       bf16_split_bits(job.WT[wi] - hv, hi, lo);
-      const long di = (tile * 16 + r) * job.ldd + col0 + c;
+      const long di = part * job.part_dimg + (tile * 16 + r) * job.ldd + col0 + c;
       job.dimg_h[di] = uint16_t(hi), job.dimg_l[di] = uint16_t(lo);
     }
   }
@@ -1576,16 +1586,18 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
   uint32_t* const handed_out = &reinterpret_cast<PairArea*>(hist_all + kHistWordsPerTile)->flag;
   for (long tile = blockIdx.x; tile < job.tiles;) {
     float expected = 0.f;  // the free pass's winner of this tile row's previous column block (0: none yet)
+    long own = tile;
+    const long part = part_of(job, own);
     for (int blk = job.blocks - 1; blk >= 0; --blk) {
       // the column block of this turn; the hatWT values the previous turn wrote for this tile row are visible after
       // the barrier that ended it
       const long col0 = job.col0 + 16 * blk;
       if (job.X) sm.x[u] = job.X[tile * kSeq + u];
-      else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
-      else tile_targets<float>(sm, job, col0, tile, job.prod32);
+      else if (job.prod64) tile_targets<double>(sm, job, col0, own, part, job.prod64);
+      else tile_targets<float>(sm, job, col0, own, part, job.prod32);
       __syncthreads();
       block_passes<kWide, true>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
-      block_outputs(sm, job, entry_f, tile, blk, col0);
+      block_outputs(sm, job, entry_f, own, part, blk, col0);
       __syncthreads();
     }
     if (job.tiles <= long(gridDim.x)) break;
@@ -2009,11 +2021,13 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
     return;
   }
   bool alone = false;
+  long own = tile;
+  const long part = part_of(job, own);
   for (int blk = job.blocks - 1; blk >= 0; --blk, n += 8) {
     const long col0 = job.col0 + 16 * blk;
     if (job.X) sm.x[tid & (kSeq - 1)] = job.X[tile * kSeq + (tid & (kSeq - 1))];
-    else if (job.prod64) tile_targets<double>(sm, job, col0, tile, job.prod64);
-    else tile_targets<float>(sm, job, col0, tile, job.prod32);
+    else if (job.prod64) tile_targets<double>(sm, job, col0, own, part, job.prod64);
+    else tile_targets<float>(sm, job, col0, own, part, job.prod32);
     __syncthreads();
     // the block's two passes together; false if the second workgroup is not there
     auto together = [&]() __attribute__((always_inline)) -> bool {
@@ -2061,7 +2075,7 @@ __global__ __launch_bounds__(kWide ? 2 * kThreads : kThreads, kWide ? 1 : 3) voi
     };
     if (!alone && !together()) alone = true;
     if (alone) block_passes<kWide, false>(sm, job, entry_d, hist, tl, expected, 0, 2, false);
-    block_outputs(sm, job, entry_f, tile, blk, col0);
+    block_outputs(sm, job, entry_f, own, part, blk, col0);
     __syncthreads();
   }
 }
@@ -2130,9 +2144,11 @@ bool launch_viterbi_tiles(const TileJob& tile_job, const double* d_entry_d, cons
     const long nk = job.bufend - job.col0 - 16;
     QTIP_REQUIRE(job.col0 >= 0 && nk >= 0 && nk <= 112 && job.blocks >= 1 && job.col0 + 16 * job.blocks <= job.bufend,
                  "viterbi: column blocks outside their 128-column buffer");
-    QTIP_REQUIRE(job.col0 >= job.prod_row0 && job.ldw >= 16 * job.tiles && job.ldl >= job.bufend,
+    QTIP_REQUIRE(job.col0 >= job.prod_row0 && job.ldw >= 16 * (job.part_tiles ? job.part_tiles : job.tiles) && job.ldl >= job.bufend,
                  "viterbi: LDLQ operand geometry");
   }
+  QTIP_REQUIRE(job.part_tiles >= 0 && (!job.part_tiles || (!job.X && !job.packed && job.tiles <= 0x7fffffffL)),
+               "viterbi: groups side by side only for LDLQ launches");
   QTIP_REQUIRE(job.blocks == 1 || (!job.X && !job.packed), "viterbi: several blocks per tile row only for LDLQ launches");
   const unsigned grid = unsigned(job.tiles < slots ? job.tiles : slots);
   // A search takes a third of the pass's time on average and longer than the pass where it has to give up, and a launch

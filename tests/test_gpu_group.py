@@ -567,3 +567,36 @@ def test_run_groups_equals_group_by_group(qz, oracle, pkg, synth):
     # the context is still usable
     again = qz.run_groups(cases[:1], opt)
     assert np.array_equal(again[0][0][0].trellis, res[0][0][0].trellis)
+
+
+@pytest.mark.parametrize("count,ms,n,feedback", [(3, (64, 32), 256, 0), (6, (1024,), 1280, 0), (6, (2048,), 1280, 0),
+                                                 (6, (1024, 1024), 1280, 1), (5, (2048,), 256, 1), (13, (32,), 128, 0)])
+def test_groups_of_one_shape_run_together(qz, pkg, count, ms, n, feedback):
+    """Small groups of one shape go through LDLQ together, a launch taking tile rows of several groups with a factor each
+    (pairs of workgroups, one chain, three chains of two groups; products with one and several splits; more groups than a
+    call takes): words, scales and proxies of each group by itself.  A group whose Hessian is not positive definite is
+    reported and does not keep the others from their results."""
+    say("case: %d groups of %s x %d together, feedback %d" % (count, ms, n, feedback))
+    qz.set_tlut(None)
+    rng = np.random.default_rng(n + count)
+    cases = []
+    for g in range(count):
+        G = rng.standard_normal((n, n + 64)).astype(np.float32)
+        H = (G @ G.T / n).astype(np.float32)
+        lins = [pkg.LinearIn("w%d_%d" % (g, i), m, w_f32=(rng.standard_normal((m, n)) * 0.02 * (g + 1)).astype(np.float32))
+                for i, m in enumerate(ms)]
+        cases.append((lins, n, ((H + H.T) * 0.5).astype(np.float32), 50 + g))
+    got = qz.run_groups(cases, pkg.QuantOpts(feedback=feedback))
+    for case, (outs, t, _) in zip(cases, got):
+        alone, _ = qz.quantize_group_h(*case, pkg.QuantOpts(feedback=feedback))
+        for a, b in zip(outs, alone):
+            assert np.array_equal(a.trellis, b.trellis), "%d words differ" % np.count_nonzero(a.trellis != b.trellis)
+            assert np.array_equal(a.sv, b.sv) and np.array_equal(a.su_bf16, b.su_bf16)
+            assert a.wscale == b.wscale and a.proxy == b.proxy and a.proxy_rot_reg == b.proxy_rot_reg
+        assert t.total > 0 and t.ldl_cpu > 0
+    if count == 3:
+        bad = [cases[0], (cases[1][0], n, np.full((n, n), -1.0, np.float32), 3), cases[2]]
+        with pytest.raises(pkg.QtipError):
+            qz.run_groups(bad, pkg.QuantOpts(feedback=feedback))
+        again = qz.run_groups(cases, pkg.QuantOpts(feedback=feedback))
+        assert np.array_equal(again[2][0][0].trellis, got[2][0][0].trellis)
