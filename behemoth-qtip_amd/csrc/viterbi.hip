@@ -47,8 +47,9 @@
 // one barrier per step; the free pass computes the groups below 2048 only, since complementary states decode alike),
 // its trace-back checks that every decision it takes was won by more than the rounding can move two candidates
 // against each other, and a pass that fails the check is run again through the fp64 form in the same launch: the
-// states are the fp64 form's, bit for bit.  A launch that cannot fill the chip uses the kernel's wide form, 512
-// threads per tile.
+// states are the fp64 form's, bit for bit.  The tail-biting pass itself is replaced by a search of the few paths that
+// can still win where the free pass has left lower bounds (close_path).  A launch that cannot fill the chip uses the
+// kernel's wide form, 512 threads per tile.
 #include <hip/hip_ext.h>
 
 #include <cstddef>
@@ -630,9 +631,9 @@ __device__ __forceinline__ uint32_t err_units(double l0, double l1, double x0, d
 }
 
 // One forward pass on 32-bit metrics.  kSym: free ends, the groups below 2048 only (a mirror group's metric is read
-// from the group it mirrors), all 128 steps, and the best final group, its metric and the gap to the runner-up are left in sm.red32[0]; otherwise:
-// start in group ov, steps 0 .. 126 (the last step's decision is taken by the trace-back from the metrics entering
-// it).  The results of the even steps first_kept .. 126 (the metrics entering the next, odd step) go to hist.
+// from the group it mirrors), all 128 steps, and the best final group, its metric and the gap to the runner-up are left
+// in sm.red32[0]; otherwise: start in group ov, steps 0 .. 126 (the last step's decision is taken by the trace-back from
+// the metrics entering it).  The results of the even steps first_kept .. 126 (the metrics entering the next, odd step) go to hist.
 // Metrics and error table are double-buffered in LDS (2 x 16 KB, 2 x 8 KB: the footprint of the fp64 arrays): a step
 // reads the present buffers and writes the next metrics and the next step's table, so one barrier per step suffices;
 // a thread keeps its four codebook entries in registers.
@@ -640,9 +641,10 @@ __device__ __forceinline__ uint32_t err_units(double l0, double l1, double x0, d
 // 4..7), and the table's 1024 entries two each instead of four.
 // kHalf: steps 0 .. 63 only; the metrics entering step 64 are left in metric buffer 0 (the other half of the sequence is
 // another workgroup's, viterbi_pair_kernel).
-// bounds (a whole free pass): the upper halves of the metrics entering step i go to row i; run_on: they are
-// wanted, and after its end the pass runs on for kTurn steps, whose metrics are kept as bounds only; returns the least by which a metric has grown over the last
-// round, that is from entering step kTurn to entering step 128 + kTurn, rounded down.
+// bounds (a whole free pass): the upper halves of the metrics entering step i go to row i; run_on: they are wanted,
+// and after its end the pass runs on for kTurn steps, whose metrics are kept as bounds only.  Returns the least by
+// which a metric has grown over the last round, that is from entering step kTurn to entering step 128 + kTurn,
+// rounded down.
 template <bool kSym, bool kWide, bool kHalf = false>
 __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __restrict__ entry_d, int roll, int ov,
                                                    uint32_t* __restrict__ hist, int first_kept, const Unit unit,
@@ -692,37 +694,26 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
   // bytes
   int xA = kSym ? m32c_pos(colA) * 32 + m32c_swz(colA) * 4 : m32_pos(colA) * 64 + m32_swz(colA) * 4;
   int xB = kSym ? m32c_pos(colB) * 32 + m32c_swz(colB) * 4 : m32_pos(colB) * 64 + m32_swz(colB) * 4;
-  // the error table of step `it` into table buffer it & 1 (given as a constant: the buffers' offsets then are part
-  // of the instructions)
-  auto table = [&](int it, auto par_tag) __attribute__((always_inline)) {
+  // Entry q of this thread in the error table of a step (x0, x1: the step's targets) into table buffer tpar (given as
+  // a constant: the buffers' offsets then are part of the instructions).
+  auto table_entry = [&](int q, double x0, double x1, auto par_tag) __attribute__((always_inline)) {
     constexpr int tpar = decltype(par_tag)::value;
-    const int t = (2 * it + roll) & 255;
-    const double x0 = double(sm.x[t]) * unit.pre, x1 = double(sm.x[t + 1]) * unit.pre;
-
+    const double2 l = ent[q];
+    const uint32_t v = err_units(l.x, l.y, x0, x1);
     if constexpr (kSym) {
       // Parity 0: pair position / 2, half position % 2; parity 1: pair floor((position - 1) / 2), the other half;
       // pair -1, which position 0 asks for, is pair 15 of parity 0, which like itself nobody reads.  Every pair a
       // second time 8 further on.  Both addresses advance by kT words per q (kT / 128 pairs).
       uint32_t* const Ew0 = E32 + tpar * kEPairWords + e_wr0;
       uint32_t* const Ew1 = E32 + tpar * kEPairWords + e_wr1;
-#pragma unroll
-      for (int q = 0; q < kEnt; ++q) {
-        const double2 l = ent[q];
-        const uint32_t v = err_units(l.x, l.y, x0, x1);
-        Ew0[kT * q] = v;
-        Ew0[kT * q + 8 * 128] = v;
-        Ew1[kT * q] = v;
-        Ew1[kT * q + 8 * 128] = v;
-      }
+      Ew0[kT * q] = v;
+      Ew0[kT * q + 8 * 128] = v;
+      Ew1[kT * q] = v;
+      Ew1[kT * q + 8 * 128] = v;
     } else {
       uint32_t* const Ew = E32 + tpar * kESlots + e_wr;
-#pragma unroll
-      for (int q = 0; q < kEnt; ++q) {
-        const double2 l = ent[q];
-        const uint32_t v = err_units(l.x, l.y, x0, x1);
-        Ew[kT * q] = v;
-        Ew[kT * q + 1024] = v;
-      }
+      Ew[kT * q] = v;
+      Ew[kT * q + 1024] = v;
     }
   };
   if constexpr (kSym) {
@@ -730,7 +721,12 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
   } else {
     for (int g = tfull; g < kGroups; g += kT) M32[m32_slot(g & 255, g >> 8)] = (ov < 0 || g == ov) ? 0u : kSat;
   }
-  table(0, std::integral_constant<int, 0>{});
+  {
+    const int t = roll & 255;
+    const double x0 = double(sm.x[t]) * unit.pre, x1 = double(sm.x[t + 1]) * unit.pre;
+#pragma unroll
+    for (int q = 0; q < kEnt; ++q) table_entry(q, x0, x1, std::integral_constant<int, 0>{});
+  }
   __syncthreads();
 
   uint32_t fin[kSlotsOwn];
@@ -765,7 +761,18 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
         MB[4 * k] = b.x, MB[4 * k + 1] = b.y, MB[4 * k + 2] = b.z, MB[4 * k + 3] = b.w;
       }
     }
-    table(it + 1, std::integral_constant<int, par ^ 1>{});
+    // The next step's table.  The free pass of the 256-thread form fills it behind its last kEnt slots, one entry
+    // after each: in front of the slots it is 600 cycles of a step of 3300 in which the slots' reads wait, and three
+    // workgroups to a compute unit do not cover them (4096 tiles 2665 -> 2640 us, 768 tiles 708 -> 688; an entry after
+    // every other slot 2660, all of them at the end 2665).  The 512-thread form has a compute unit to itself and is
+    // faster with the table first (256 tiles 379 against 384 us).
+    constexpr bool kTableLate = kSym && !kWide;
+    const int tn = (2 * (it + 1) + roll) & 255;
+    const double xn0 = double(sm.x[tn]) * unit.pre, xn1 = double(sm.x[tn + 1]) * unit.pre;
+    if constexpr (!kTableLate) {
+#pragma unroll
+      for (int q = 0; q < kEnt; ++q) table_entry(q, xn0, xn1, std::integral_constant<int, par ^ 1>{});
+    }
     // The 16 table values of a slot are fetched while the slot before it is worked on; the value of digit k of slot
     // m lies (k (2 m + 1)) % 16 positions after the slot's first.  m0: the first slot of this thread, a constant in
     // each of the two copies of the loop that the wide form needs.  Tail-biting pass: evb[.][k] is the value of digit
@@ -820,9 +827,14 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
         }
       };
       // the table value of digit k is the candidate of digit k of the group and of digit 15 - k of its mirror
-      uint32_t ba = kSat;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) ba = min3u(ba, sat_add(at(2 * k), MA[2 * k]), sat_add(at(2 * k + 1), MA[2 * k + 1]));
+      // (two chains of minima: one alone waits for itself; 4096 tiles 2725 -> 2690 us)
+      auto pair_min = [&](auto value) __attribute__((always_inline)) -> uint32_t {
+        uint32_t c0 = min3u(value(0), value(1), value(2)), c1 = min3u(value(3), value(4), value(5));
+        c0 = min3u(c0, value(6), value(7)), c1 = min3u(c1, value(8), value(9));
+        c0 = min3u(c0, value(10), value(11)), c1 = min3u(c1, value(12), value(13));
+        return min(min3u(c0, value(14), value(15)), c1);
+      };
+      const uint32_t ba = pair_min([&](int k) __attribute__((always_inline)) { return sat_add(at(k), MA[k]); });
       uint32_t bb = ba;
       if constexpr (!kSym) {
         bb = kSat;
@@ -840,6 +852,9 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
       if constexpr (kind == kStore) {
         hs[(m0 + m) * kThreads] = ba;
         if constexpr (!kSym) hs[(8 + m0 + m) * kThreads] = bb;
+      }
+      if constexpr (kTableLate) {
+        if (i >= kSlotsOwn - kEnt) table_entry(i - (kSlotsOwn - kEnt), xn0, xn1, std::integral_constant<int, par ^ 1>{});
       }
     }
     };
