@@ -212,7 +212,9 @@ typedef struct { /* QuantOpts, src/quantizer.hpp:11-19 */
                             the number.  At most 12.  1: one group after the other, as the reference schedules them.
                             0 (default): as many as it takes for the largest group's 16-row tile rows to fill the
                             chip's 768 Viterbi workgroup slots (a 1024-row group fills a twelfth of them), 1 for
-                            groups of 12288 rows and more.
+                            groups of 12288 rows and more; groups of one shape (same n, a multiple of 128, and as many
+                            tile rows) then go through LDLQ in one call, a lane preparing and finishing each, unless
+                            the LDL is the host's (ldl_device_updates = 0).
                             Lanes whose streams share a hardware queue run one after the other: small groups gain
                             most where the process has a queue per lane (GPU_MAX_HW_QUEUES=16 in the environment
                             when the HIP runtime starts; HIP's default is 4) */
@@ -308,7 +310,9 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
  * takes its groups one after the other on a stream of its own; same results); then an error leaves the groups before the
  * failing one on its lane complete, the other lanes finish their groups, and the first failing lane's error is
  * reported.  With group_lanes = 0 and groups of mixed sizes, the groups of 12288 rows and more run first, in their
- * order, one after the other, and the smaller ones then share the chip on lanes. */
+ * order, one after the other, then those of one shape together, and the rest share the chip on lanes.  Groups that run
+ * together (group_lanes = 0, one shape): a failing group leaves the others' results complete, and the first error is
+ * reported at the end. */
 typedef struct {
   int nlin;
   const qtip_linear_in* lins;
@@ -320,7 +324,8 @@ typedef struct {
 } qtip_group;
 int qtip_run_groups(qtip_ctx* ctx, int ngroups, const qtip_group* groups, const qtip_opts* opts, qtip_timing* timings,
                     double* ldl_wait_s);
-/* The number of lanes qtip_run_groups would use for these groups and options (1: one group after the other).  Reads
+/* The number of lanes qtip_run_groups would use for these groups and options (1: one group after the other; groups of
+ * one shape run in one LDLQ call instead, group_lanes above).  Reads
  * only nlin, lins[].m and n of each group.  No counterpart in the reference, which runs one group at a time. */
 int qtip_group_lanes(qtip_ctx* ctx, int ngroups, const qtip_group* groups, const qtip_opts* opts, int* lanes);
 /* Host-only check of the lane rule: `ngroups` equal groups of one m x n linear on a device with `device_slots`
