@@ -1,0 +1,38 @@
+"""The search for the closed path on the CPU (tests/cpp/close_path_emulation.cpp): where it settles a tile, the states are those of
+the cheapest closed path by the plain recursion; each way in which a search can end is taken by some kind of inputs."""
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+
+@pytest.fixture(scope="module")
+def emulation(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("emulation") / "close_path_emulation")
+    subprocess.check_call(["g++", "-O2", "-std=c++20", "-ffp-contract=off", "-mfma", "-mf16c", "-Wno-unknown-pragmas",
+                           os.path.join(ROOT, "tests", "cpp", "close_path_emulation.cpp"), "-o", exe])
+    return exe
+
+
+def _run(exe, kind, threads, order, tiles):
+    run = subprocess.run([exe, kind, str(threads), order, str(tiles)], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0, run.stdout
+    words = run.stdout.split()
+    return dict(zip(words[0::2], map(int, words[1::2])))
+
+
+@pytest.mark.parametrize("kind,ends", [("gauss", {"early": 6, "step0": 6, "second": 1, "lowered": 1}),
+                                       ("join", {"early": 6, "step0": 6, "lowered": 6}),
+                                       ("flat", {"early": 3, "step0": 6}),
+                                       ("alike", {"early": 3, "full": 1, "gave_up": 3}),
+                                       ("mirror", {"gave_up": 6})])
+def test_search_finds_the_cheapest_closed_path(emulation, kind, ends):
+    got = _run(emulation, kind, 256, "3210", 24)
+    assert all(got[end] >= least for end, least in ends.items()), got
+
+
+def test_search_by_512_threads(emulation):
+    got = _run(emulation, "gauss", 512, "76543210", 12)
+    assert got["early"] + got["step0"] == 12, got
