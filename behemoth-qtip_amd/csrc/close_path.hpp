@@ -217,8 +217,10 @@ __device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const u
     wait_loads<0>();
     __syncthreads();
     if (tid < 2) sm.close_least[tid] = kSat;
-    if (found) {
-      // the cheapest of the paths to the group in question, and how far behind the next one is (every wave alike)
+    // The verdict is the first wave's, and the others hear it behind the barrier: a search that ends on the free path writes
+    // the states over that path's own, which only that wave may read by then, and the waves must not part over it.
+    if (found && wave == 0) {
+      // the cheapest of the paths to the group in question, and how far behind the next one is
       const uint32_t target = p == 0 ? ov : uint32_t(sm.st[kSteps / 2 + p]) >> 4;
       u64 best = ~0ull, second = ~0ull;
       for (uint32_t i = lane; i < found; i += 64) {
@@ -235,8 +237,9 @@ __device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const u
       }
       const uint32_t c = uint32_t(best >> 32), c2 = uint32_t(second >> 32);
       const uint32_t sum = p == 0 ? sat_add(start + 65536u, sat_add(c, margin)) : 0u;
-      ok = __builtin_amdgcn_readfirstlane(int(sum <= limit && best != ~0ull && (second == ~0ull || c2 - c >= margin))) != 0;
-      if (ok && wave == 0) {
+      const bool good = __builtin_amdgcn_readfirstlane(int(sum <= limit && best != ~0ull && (second == ~0ull || c2 - c >= margin))) != 0;
+      if (lane == 0) sm.close_ok = good;
+      if (good) {
         // steps 0 .. p - 1 as the free path has them, then from path to path continued
         const uint16_t v = sm.st[kSteps / 2 + lane];
         if (int(lane) < p) sm.st[lane] = v;
@@ -254,6 +257,7 @@ __device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const u
       }
     }
     __syncthreads();
+    if (found) ok = __builtin_amdgcn_readfirstlane(int(sm.close_ok)) != 0;
   }
   return ok;
 }

@@ -131,6 +131,7 @@ struct Smem {
   uint32_t grown[8];       // end of a free pass's second round: per wave the least growth of a metric
   uint32_t close_count[2];   // search for the closed path: partial paths found, by turn
   uint32_t close_least[2];   // the smallest bound among them off the free path and on it
+  uint32_t close_ok;         // the first wave's verdict on what was found
   int overlap;
   uint32_t next_tile;  // tiles kernel: what this workgroup takes on next
   uint32_t heard;      // pair: what waiting for the other workgroup came to

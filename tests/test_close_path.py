@@ -1,5 +1,6 @@
 """The search for the closed path on the CPU (tests/cpp/close_path_emulation.cpp): where it settles a tile, the states are those of
-the cheapest closed path by the plain recursion; each way in which a search can end is taken by some kind of inputs."""
+the cheapest closed path by the plain recursion, whichever wave comes first; each way in which a search can end is taken by some kind
+of inputs."""
 import os
 import subprocess
 
@@ -33,6 +34,14 @@ def test_search_finds_the_cheapest_closed_path(emulation, kind, ends):
     assert all(got[end] >= least for end, least in ends.items()), got
 
 
-def test_search_by_512_threads(emulation):
-    got = _run(emulation, "gauss", 512, "76543210", 12)
+@pytest.mark.parametrize("kind", ["gauss", "alike"])
+@pytest.mark.parametrize("order", ["0123", "1032", "2301"])
+def test_search_does_not_depend_on_the_order_of_the_waves(emulation, kind, order):
+    """The first wave writes the states that the search has found; the others are still to come."""
+    assert _run(emulation, kind, 256, order, 24)["early"] >= 3
+
+
+@pytest.mark.parametrize("order", ["01234567", "76543210"])
+def test_search_by_512_threads(emulation, order):
+    got = _run(emulation, "gauss", 512, order, 12)
     assert got["early"] + got["step0"] == 12, got
