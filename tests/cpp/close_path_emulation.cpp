@@ -2,7 +2,7 @@
 // closed path by the plain recursion.  The lanes of a wave that have come to the same wave operation take it together, the
 // earliest one in the source first; between two barriers the waves run one after the other, each as far as the barrier, in the
 // order given: what a wave reads must not depend on how far the others have come.  A row on its way into LDS is rubbish until it
-// is waited for, and a thread that returns false writes to LDS at once, as the pass that follows does.
+// is waited for.  (Whoever has left the search meets the others at a barrier before anything else: block_passes.)
 //   close_path_emulation KIND THREADS ORDER TILES [SEED]    e.g. gauss 256 3210 8    exit code 0: no fault
 // Prints how the searches ended: early settled at the free path's group, step0 settled at step 0, (second: in the second attempt,
 // lowered: with a step done again under a lower limit,) refused before the first attempt, full and gave_up unsettled.
@@ -310,9 +310,6 @@ void thread_main() {
   answers[me] = threads == kThreads
                     ? close_path<false>(sm_all, book, hist, tile.ov, tile.winner, tile.grown, kMargin, tile.unit)
                     : close_path<true>(sm_all, book, hist, tile.ov, tile.winner, tile.grown, kMargin, tile.unit);
-  if (!answers[me])
-    for (size_t at = 4 * size_t(me); at < sizeof sm_all.E + sizeof sm_all.M; at += 4 * size_t(threads))
-      put(uint32_t(at), uint32_t(0xbeef0000u + at));
   pause_at(kBarrier, 0);
   pause_at(kEnd, 0);
 }
@@ -414,11 +411,6 @@ int main(int argc, char** argv) {
       else ++step0;
       second += attempts > 1;
     } else {
-      for (size_t at = 0; at < sizeof sm_all.E + sizeof sm_all.M; at += 4)
-        if (get<uint32_t>(uint32_t(at)) != uint32_t(0xbeef0000u + at)) {
-          std::printf("tile %d: the search writes to LDS (at %zu) after one of its threads has left it\n", n, at), ++faults;
-          break;
-        }
       if (attempts == 0 && rounds == 0) ++refused;
       else if (rounds == steps_done) ++full;  // every step fitted, the room for all of them ended
       else ++gave_up;

@@ -28,7 +28,9 @@ def _run(exe, kind, threads, order, tiles):
                                        ("join", {"early": 6, "step0": 6, "lowered": 6}),
                                        ("flat", {"early": 3, "step0": 6}),
                                        ("alike", {"early": 3, "full": 1, "gave_up": 3}),
-                                       ("mirror", {"gave_up": 6})])
+                                       ("mirror", {"gave_up": 6}),
+                                       # costs that leave no room for a limit
+                                       ("coarse", {"early": 3, "step0": 3, "refused": 3})])
 def test_search_finds_the_cheapest_closed_path(emulation, kind, ends):
     got = _run(emulation, kind, 256, "3210", 24)
     assert all(got[end] >= least for end, least in ends.items()), got
