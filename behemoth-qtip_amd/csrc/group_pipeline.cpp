@@ -340,7 +340,7 @@ int group_lanes_for(int ng, const qtip_group* groups, const qtip_opts& opt, int 
 // queues the process has: six groups of 128 tile rows ran two or three at a time.  Here the lanes prepare their groups
 // (rotation, factor, weights), one call walks the tile rows of all of them (ldlq_impl with parts: a launch takes rows of
 // several groups, each with its own factor), and the lanes finish them.  Same results: every tile sees the operands it sees
-// alone.  Six 2048 x 2560 groups from host memory: 166 -> 95 ms.
+// alone (fp32 sums of products are cut as alone, gemm_splitk_splits).  Six 2048 x 2560 groups from host memory: 166 -> 95 ms.
 // A group that cannot be prepared (its H is not positive definite, say) does not keep the others from their results; the
 // first such error is thrown at the end.
 int together_batch(int ng, long rows, int n, int device_slots) {

@@ -283,6 +283,9 @@ int gemm_splitk_splits(long K, int N, int slots) {
   // of them, half of the chip with two chains), so the number of splits is chosen to fill whole rounds of those
   // slots: the smallest count that fills at least 95 % of the rounds it needs, else the best there is; a split has
   // at least 512 rows of K.  m = 12288 in two chains: 48 column tiles x 8 splits = 384 workgroups on 384 slots.
+  // Another number of splits is another order of the sums.  On fp64 that is out of reach of a target's fp16 rounding; on fp32
+  // (split-bf16 products) it moves targets and from there words, so these are cut as for the group by itself, whoever
+  // else is in the launch and whatever share of the chip the call has.
   const long tiles = (N + BN - 1) / BN, most = std::min<long>(kMaxGatherSplits, std::max<long>(1, K / 512));
   long best = 1;
   double best_fill = 0;
@@ -329,7 +332,7 @@ int launch_gemm_img_gather(int N, long K, const uint16_t* Ah, const uint16_t* Al
   QTIP_REQUIRE(N > 0 && K > 0 && K % IK == 0 && lda % 8 == 0 && ldb % 8 == 0 && Ah && Al && Bh && Bl,
                "split-bf16 gather GEMM needs K %% 16 == 0 and 16-byte aligned image rows");
   QTIP_REQUIRE(parts == 1 || (parts > 1 && !reduce), "products side by side leave the sum to the reader");
-  const int S = gemm_splitk_splits(K, N * parts, slots);
+  const int S = gemm_splitk_splits(K, N, slots);  // (not N * parts: see gemm_splitk_splits)
   dim3 grid(unsigned((N + SB - 1) / SB), unsigned(S), unsigned(parts));
   if (S == 1) strides.out = long(SB) * N;
   gather_img_kernel<<<grid, dim3(256), 0, s>>>(N, K, Ah, Al, lda, Bh, Bl, ldb, S == 1 ? P : partials, N, strides);

@@ -17,7 +17,8 @@ int launch_gemm_tn_f64_gather(int N, long K, const float* A, long lda, const flo
                               double* P, double* partials, int slots, hipStream_t s, bool reduce = true, int parts = 1,
                               PartStrides strides = {});
 // The gathered product in the reference GPU path's arithmetic: operands as bf16 hi + lo images with k contiguous,
-// three MFMA terms, fp32 accumulate; P and the partials (up to kMaxGatherSplits x 128 x N) in fp32.
+// three MFMA terms, fp32 accumulate; P and the partials (up to kMaxGatherSplits x 128 x N) in fp32.  slots: those that the
+// group by itself would have, and the number of splits comes from N alone: the fp32 sums do not depend on the other parts.
 //   a: Ah / Al[i * lda + k], i < 128   (launch_split_transpose_bf16 of L, offset to the buffer's columns and rows)
 //   b: Bh / Bl[j * ldb + k], j < N     (written by the Viterbi kernel, TileJob::dimg_h / dimg_l)
 int launch_gemm_img_gather(int N, long K, const uint16_t* Ah, const uint16_t* Al, long lda, const uint16_t* Bh,

@@ -103,7 +103,7 @@ int ldlq_default_chains(qtip_ctx* c) {
 }
 
 // parts > 1: that many groups of one shape, whose WT, L, hatWT and Q follow each other; a chain takes whole groups.  Every tile
-// sees the operands it sees in a call of its own group.
+// sees the operands it sees in a call of its own group (feedback 0: up to the order of the gathered products' fp64 sums).
 void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, float* hatWT, uint16_t* Q, int feedback,
                double* vit_seconds, int chains, int parts) {
   QTIP_REQUIRE(n % 128 == 0, "LDLQ needs n %% 128 == 0 (n = %ld)", n);
@@ -212,7 +212,9 @@ void ldlq_impl(qtip_ctx* c, const float* WT, const float* L, long n, long m, flo
         } else {
           const uint16_t* la = limg.p + 2 * nn * C.part0 + size_t(c0) * n + bufend;
           const uint16_t* da = dimg.p + (parts > 1 ? 2 * nm * C.part0 : size_t(C.r0) * n) + bufend;
-          splits = launch_gemm_img_gather(int(crows), n - bufend, la, la + nn, n, da, da + nm, n, C.prod32, C.slabs32, C.slots,
+          // (a chain that holds whole groups: by itself a group of this size has the chip to itself, on a lane as well)
+          const int slots = nch == 1 || parts > 1 ? viterbi_max_slots(c->device) : C.slots;
+          splits = launch_gemm_img_gather(int(crows), n - bufend, la, la + nn, n, da, da + nm, n, C.prod32, C.slabs32, slots,
                                           C.s, false, C.parts, {long(2 * nn), long(2 * nm), long(max_splits) * 128 * m});
         }
         {

@@ -600,3 +600,35 @@ def test_groups_of_one_shape_run_together(qz, pkg, count, ms, n, feedback):
             qz.run_groups(bad, pkg.QuantOpts(feedback=feedback))
         again = qz.run_groups(cases, pkg.QuantOpts(feedback=feedback))
         assert np.array_equal(again[2][0][0].trellis, got[2][0][0].trellis)
+
+
+def _device_group(pkg, torch, seed, ms, n, H):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    lins = [pkg.LinearIn("w%d" % i, m, w_f32=torch.randn(m, n, device="cuda", generator=g) * 0.02) for i, m in enumerate(ms)]
+    return lins, n, H, seed
+
+
+def _device_hessian(torch, n):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(n + 64, n, device="cuda", generator=g)
+    h = x.T @ x / n
+    return ((h + h.T) * 0.5).contiguous()
+
+
+@pytest.mark.parametrize("count,m,n,lanes", [(6, 4096, 4096, 0), (4, 4096, 4096, 0), (2, 1024, 5120, 2)])
+def test_feedback_1_words_do_not_depend_on_the_other_groups(qz, pkg, count, m, n, lanes):
+    """fp32 feedback: the gathered products are summed in as many splits as for the group by itself, whoever else is in the
+    launch and on a lane as well.  (4096 x 4096: 7 splits at the last buffers; 6 and 4 if they were taken for the four or six
+    groups of a launch.  5120 on a lane: 9, and 8 if they were taken for the lane's slots.)"""
+    import torch
+    say("case: feedback 1, %d groups of %d x %d, lanes %d" % (count, m, n, lanes))
+    qz.set_tlut(None)
+    H = _device_hessian(torch, n)
+    cases = [_device_group(pkg, torch, 70 + k, (m,), n, H) for k in range(count)]
+    got = qz.run_groups(cases, pkg.QuantOpts(feedback=1, group_lanes=lanes))
+    for k, (case, (outs, _, _)) in enumerate(zip(cases, got)):
+        say("  group %d by itself" % k)
+        alone, _ = qz.quantize_group_h(*case, pkg.QuantOpts(feedback=1))
+        differ = np.count_nonzero(outs[0].trellis != alone[0].trellis)
+        assert differ == 0, "group %d: %d of %d words differ" % (k, differ, alone[0].trellis.size)
+        assert outs[0].wscale == alone[0].wscale and outs[0].proxy == alone[0].proxy
