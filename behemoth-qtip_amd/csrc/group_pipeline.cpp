@@ -494,23 +494,26 @@ void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_o
     const bool one_schedule = parts.size() == 1 || (parts.size() == 2 && left.size() == 1 && parts[1].size() == 1 &&
                                                     tile_rows_of(groups[parts[0][0]]) >= slots);
     if (!one_schedule) {
+      // an error among the large groups ends the call, as it ends their schedule; one among the others does not keep the
+      // other parts from their results and is reported at the end
+      std::exception_ptr first_err;
       for (const std::vector<int>& part : parts) {
         std::vector<qtip_group> sub;
         for (int g : part) sub.push_back(groups[g]);
         std::vector<qtip_timing> st(sub.size());
         std::vector<double> sw(sub.size(), 0.0);
-        std::exception_ptr err;
         try {
           run_groups_impl(c, int(sub.size()), sub.data(), opt, st.data(), sw.data());
         } catch (...) {
-          err = std::current_exception();
+          if (!first_err) first_err = std::current_exception();
         }
         for (size_t i = 0; i < part.size(); ++i) {
           if (tms) tms[part[i]] = st[i];
           if (ldl_wait) ldl_wait[part[i]] = sw[i];
         }
-        if (err) std::rethrow_exception(err);
+        if (first_err && tile_rows_of(groups[part[0]]) >= slots) break;
       }
+      if (first_err) std::rethrow_exception(first_err);
       return;
     }
   }

@@ -310,7 +310,8 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
  * takes its groups one after the other on a stream of its own; same results); then an error leaves the groups before the
  * failing one on its lane complete, the other lanes finish their groups, and the first failing lane's error is
  * reported.  With group_lanes = 0 and groups of mixed sizes, the groups of 12288 rows and more run first, in their
- * order, one after the other, then those of one shape together, and the rest share the chip on lanes.  Groups that run
+ * order, one after the other, then those of one shape together, and the rest share the chip on lanes: an error among the
+ * large ones ends the call, one among the others leaves the groups of the other shapes complete.  Groups that run
  * together (group_lanes = 0, one shape): a failing group leaves the others' results complete, and the first error is
  * reported at the end. */
 typedef struct {

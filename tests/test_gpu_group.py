@@ -632,3 +632,31 @@ def test_feedback_1_words_do_not_depend_on_the_other_groups(qz, pkg, count, m, n
         differ = np.count_nonzero(outs[0].trellis != alone[0].trellis)
         assert differ == 0, "group %d: %d of %d words differ" % (k, differ, alone[0].trellis.size)
         assert outs[0].wscale == alone[0].wscale and outs[0].proxy == alone[0].proxy
+
+
+@pytest.mark.parametrize("bad", [0, 2, 4])
+def test_a_failing_small_group_leaves_the_other_shapes_complete(qz, pkg, monkeypatch, bad):
+    """Two groups of one shape, two of another and one of a third: whichever fails, the four others are quantized (those on its own
+    lane before it, all of the other parts of the call) and its error is reported."""
+    import torch
+    say("case: shapes A, A, B, B, C with group %d not positive definite" % bad)
+    qz.set_tlut(None)
+    shapes = [((64,), 256), ((64,), 256), ((32, 32), 512), ((32, 32), 512), ((32,), 256)]
+    cases = [_device_group(pkg, torch, 80 + k, ms, n, _device_hessian(torch, n)) for k, (ms, n) in enumerate(shapes)]
+    want = [qz.quantize_group_h(*case, pkg.QuantOpts())[0] for case in cases]
+    lins, n, H, seed = cases[bad]
+    cases[bad] = (lins, n, torch.full_like(H, -1.0), seed)
+    outs, marshal = [], qz._marshal
+
+    def kept(*args):  # the output buffers of the call, which run_groups does not return when it raises
+        r = marshal(*args)
+        outs.append(r[2])
+        return r
+
+    monkeypatch.setattr(qz, "_marshal", kept)
+    with pytest.raises(pkg.QtipError) as e:
+        qz.run_groups(cases, pkg.QuantOpts())
+    assert e.value.code == pkg.QTIP_E_NOT_PD
+    for k in range(len(cases)):
+        if k != bad:
+            assert all(np.array_equal(a.trellis, b.trellis) for a, b in zip(outs[k], want[k])), "group %d" % k
