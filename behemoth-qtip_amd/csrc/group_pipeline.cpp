@@ -459,79 +459,8 @@ static void run_groups_together(qtip_ctx* c, int ng, const qtip_group* groups, c
   if (first_err) std::rethrow_exception(first_err);
 }
 
-void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opts& opt, qtip_timing* tms,
-                     double* ldl_wait) {
-  QTIP_REQUIRE(ng >= 0 && (ng == 0 || groups), "run_groups: bad arguments");
-  if (ng == 0) return;
-  for (int g = 0; g < ng; ++g)
-    QTIP_REQUIRE(groups[g].n > 0 && groups[g].H && groups[g].nlin > 0 && groups[g].lins && groups[g].outs,
-                 "run_groups: group %d is incomplete", g);
-  // Mixed sizes (a layer's gate/up group beside its o-proj group): the groups that fill the chip on their own go
-  // through the overlapped schedule first, in their order, then those of one shape together, and what is left shares the
-  // chip on lanes.
-  const int slots = viterbi_max_slots(c->device);
-  const bool may_group = opt.group_lanes == 0 && opt.ldl_device_updates != 0;
-  auto alike = [&](int a, int b) { return groups[a].n == groups[b].n && tile_rows_of(groups[a]) == tile_rows_of(groups[b]); };
-  if (opt.group_lanes == 0 && ng >= 3) {
-    std::vector<std::vector<int>> parts(1), shapes;  // parts[0]: the large ones
-    std::vector<int> left;
-    for (int g = 0; g < ng; ++g) {
-      if (tile_rows_of(groups[g]) >= slots) {
-        parts[0].push_back(g);
-        continue;
-      }
-      size_t k = 0;
-      while (k < shapes.size() && !(may_group && alike(shapes[k][0], g))) ++k;
-      if (k == shapes.size()) shapes.emplace_back();
-      shapes[k].push_back(g);
-    }
-    for (std::vector<int>& shape : shapes)
-      if (shape.size() >= 2) parts.push_back(shape);
-      else left.push_back(shape[0]);
-    if (!left.empty()) parts.push_back(left);
-    if (parts[0].empty()) parts.erase(parts.begin());
-    // (a large group or two beside one small one: in their order, as one schedule)
-    const bool one_schedule = parts.size() == 1 || (parts.size() == 2 && left.size() == 1 && parts[1].size() == 1 &&
-                                                    tile_rows_of(groups[parts[0][0]]) >= slots);
-    if (!one_schedule) {
-      // an error among the large groups ends the call, as it ends their schedule; one among the others does not keep the
-      // other parts from their results and is reported at the end
-      std::exception_ptr first_err;
-      for (const std::vector<int>& part : parts) {
-        std::vector<qtip_group> sub;
-        for (int g : part) sub.push_back(groups[g]);
-        std::vector<qtip_timing> st(sub.size());
-        std::vector<double> sw(sub.size(), 0.0);
-        try {
-          run_groups_impl(c, int(sub.size()), sub.data(), opt, st.data(), sw.data());
-        } catch (...) {
-          if (!first_err) first_err = std::current_exception();
-        }
-        for (size_t i = 0; i < part.size(); ++i) {
-          if (tms) tms[part[i]] = st[i];
-          if (ldl_wait) ldl_wait[part[i]] = sw[i];
-        }
-        if (first_err && tile_rows_of(groups[part[0]]) >= slots) break;
-      }
-      if (first_err) std::rethrow_exception(first_err);
-      return;
-    }
-  }
-  bool one_shape = may_group && ng >= 2 && tile_rows_of(groups[0]) < slots && groups[0].n % 128 == 0;
-  for (int g = 1; g < ng; ++g) one_shape = one_shape && alike(0, g);
-  if (one_shape) {
-    run_groups_together(c, ng, groups, opt, tms, ldl_wait);
-    return;
-  }
-  const int lanes = group_lanes_for(ng, groups, opt, slots);
-  if (lanes == 1) {
-    // the per-group device buffers of the quantizing thread come from the context's arena and stay there between
-    // groups and calls: a hipFree waits for the whole device, the factorization's queued updates included (a dozen
-    // of them per group cost 10 ms of a 2.5 s config-5 group)
-    ArenaScope memory(&c->arena);
-    run_groups_on(c, ng, groups, opt, tms, ldl_wait);
-    return;
-  }
+static void run_groups_on_lanes(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opts& opt, int lanes,
+                                qtip_timing* tms, double* ldl_wait) {
   // group g goes to lane g % lanes; a lane's context keeps kept-metrics slots for its largest group only, and the
   // host threads of the factorizations are shared out
   struct Lane {
@@ -596,6 +525,92 @@ void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_o
   }
   for (Lane& l : L)
     if (l.err) std::rethrow_exception(l.err);
+}
+
+// How a call's groups are run, in this order.  Mixed sizes (a layer's gate/up group beside its o-proj group): the groups that
+// fill the chip on their own go through the overlapped schedule first, in their order, then those of one shape together, and
+// what is left shares the chip on lanes.
+std::vector<GroupPart> plan_groups(int ng, const qtip_group* groups, const qtip_opts& opt, int device_slots) {
+  auto by_lanes = [&](std::vector<int> some) {
+    std::vector<qtip_group> sub;
+    for (int g : some) sub.push_back(groups[g]);
+    const int lanes = group_lanes_for(int(sub.size()), sub.data(), opt, device_slots);
+    return GroupPart{lanes == 1 ? GroupRoute::kSchedule : GroupRoute::kLanes, lanes, std::move(some)};
+  };
+  std::vector<int> all;
+  for (int g = 0; g < ng; ++g) all.push_back(g);
+  if (opt.group_lanes != 0 || ng < 2) return {by_lanes(all)};
+  // groups that may go together, if there are several of their shape
+  auto shaped = [&](int g) { return opt.ldl_device_updates != 0 && groups[g].n % 128 == 0; };
+  auto alike = [&](int a, int b) {
+    return shaped(a) && groups[a].n == groups[b].n && tile_rows_of(groups[a]) == tile_rows_of(groups[b]);
+  };
+  std::vector<int> large, left;
+  std::vector<std::vector<int>> shapes;
+  for (int g = 0; g < ng; ++g) {
+    if (tile_rows_of(groups[g]) >= device_slots) {
+      large.push_back(g);
+      continue;
+    }
+    size_t k = 0;
+    while (k < shapes.size() && !alike(shapes[k][0], g)) ++k;
+    if (k == shapes.size()) shapes.emplace_back();
+    shapes[k].push_back(g);
+  }
+  std::vector<GroupPart> parts;
+  for (std::vector<int>& shape : shapes)
+    if (shape.size() >= 2) parts.push_back({GroupRoute::kTogether, 1, shape});
+    else left.push_back(shape[0]);
+  // (large groups beside one small one: in their order, as one schedule)
+  if (!large.empty() && parts.empty() && left.size() <= 1) return {by_lanes(all)};
+  if (!large.empty()) parts.insert(parts.begin(), by_lanes(large));
+  if (!left.empty()) parts.push_back(by_lanes(left));
+  return parts;
+}
+
+void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_opts& opt, qtip_timing* tms,
+                     double* ldl_wait) {
+  QTIP_REQUIRE(ng >= 0 && (ng == 0 || groups), "run_groups: bad arguments");
+  if (ng == 0) return;
+  for (int g = 0; g < ng; ++g)
+    QTIP_REQUIRE(groups[g].n > 0 && groups[g].H && groups[g].nlin > 0 && groups[g].lins && groups[g].outs,
+                 "run_groups: group %d is incomplete", g);
+  const int slots = viterbi_max_slots(c->device);
+  // an error among the large groups ends the call, as it ends their schedule; one among the others does not keep the other
+  // parts from their results and is reported at the end
+  std::exception_ptr first_err;
+  for (const GroupPart& part : plan_groups(ng, groups, opt, slots)) {
+    const size_t count = part.groups.size();
+    std::vector<qtip_group> sub;
+    for (int g : part.groups) sub.push_back(groups[g]);
+    std::vector<qtip_timing> st(count);
+    std::vector<double> sw(count, 0.0);
+    for (size_t i = 0; i < count; ++i) {  // (a group that is not reached keeps the caller's values)
+      if (tms) st[i] = tms[part.groups[i]];
+      if (ldl_wait) sw[i] = ldl_wait[part.groups[i]];
+    }
+    try {
+      if (part.route == GroupRoute::kTogether) {
+        run_groups_together(c, int(count), sub.data(), opt, st.data(), sw.data());
+      } else if (part.route == GroupRoute::kLanes) {
+        run_groups_on_lanes(c, int(count), sub.data(), opt, part.lanes, st.data(), sw.data());
+      } else {
+        // the per-group device buffers of the quantizing thread come from the context's arena and stay there between
+        // groups and calls: a hipFree waits for the whole device, the factorization's queued updates included (a dozen
+        // of them per group cost 10 ms of a 2.5 s config-5 group)
+        ArenaScope memory(&c->arena);
+        run_groups_on(c, int(count), sub.data(), opt, st.data(), sw.data());
+      }
+    } catch (...) {
+      if (!first_err) first_err = std::current_exception();
+    }
+    for (size_t i = 0; i < count; ++i) {
+      if (tms) tms[part.groups[i]] = st[i];
+      if (ldl_wait) ldl_wait[part.groups[i]] = sw[i];
+    }
+    if (first_err && tile_rows_of(sub[0]) >= slots) break;
+  }
+  if (first_err) std::rethrow_exception(first_err);
 }
 
 }  // namespace qtipmi

@@ -787,6 +787,29 @@ int qtip_selftest_group_lanes(int device_slots, int ngroups, int m, int n, int r
   });
 }
 
+int qtip_selftest_group_plan(int device_slots, int ngroups, const int* m, const int* n, const qtip_opts* opts, int* part, int* route) {
+  // host only: the parts that qtip_run_groups makes of groups of one m x n linear each
+  return guarded([&] {
+    QTIP_REQUIRE(device_slots > 0 && ngroups >= 0 && ngroups <= 4096 && (ngroups == 0 || (m && n && part && route)),
+                 "selftest: bad arguments");
+    std::vector<qtip_linear_in> lins(static_cast<size_t>(ngroups));
+    std::vector<qtip_group> groups(static_cast<size_t>(ngroups));
+    for (int g = 0; g < ngroups; ++g) {
+      lins[size_t(g)] = qtip_linear_in{}, groups[size_t(g)] = qtip_group{};
+      lins[size_t(g)].m = m[g];
+      groups[size_t(g)].nlin = 1, groups[size_t(g)].lins = &lins[size_t(g)], groups[size_t(g)].n = n[g];
+    }
+    qtip_opts o;
+    qtip_default_opts(&o);
+    if (opts) o = *opts;
+    int at = 0;
+    for (const GroupPart& p : plan_groups(ngroups, groups.data(), o, device_slots)) {
+      for (int g : p.groups) part[g] = at, route[g] = p.route == GroupRoute::kTogether ? 0 : p.lanes;
+      ++at;
+    }
+  });
+}
+
 int qtip_reserve_groups_for(qtip_ctx* ctx, int n, const qtip_opts* opts) {
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr && n > 0, "reserve_groups: bad arguments");

@@ -121,6 +121,15 @@ void release_lanes(qtip_ctx* parent);
 void order_streams(hipStream_t first, hipStream_t then);
 // how many groups qtip_run_groups runs side by side (1: one after the other on the context itself)
 int group_lanes_for(int ngroups, const qtip_group* groups, const qtip_opts& opt, int device_slots);
+// how qtip_run_groups runs its groups: as parts, one after the other - groups one after the other on the context itself
+// (kSchedule), on that many lanes, or through LDLQ in one call (kTogether).  Host only.
+enum class GroupRoute { kSchedule, kLanes, kTogether };
+struct GroupPart {
+  GroupRoute route;
+  int lanes;
+  std::vector<int> groups;
+};
+std::vector<GroupPart> plan_groups(int ngroups, const qtip_group* groups, const qtip_opts& opt, int device_slots);
 void run_groups_impl(qtip_ctx* c, int ngroups, const qtip_group* groups, const qtip_opts& opt, qtip_timing* timings,
                      double* ldl_wait);
 uint8_t f32_to_fp8e4m3(float x);

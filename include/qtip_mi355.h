@@ -332,6 +332,10 @@ int qtip_group_lanes(qtip_ctx* ctx, int ngroups, const qtip_group* groups, const
 /* Host-only check of the lane rule: `ngroups` equal groups of one m x n linear on a device with `device_slots`
  * Viterbi workgroup slots, qtip_opts.group_lanes = requested. */
 int qtip_selftest_group_lanes(int device_slots, int ngroups, int m, int n, int requested, int* lanes);
+/* Host-only check of the order and manner in which qtip_run_groups runs groups of one m[g] x n[g] linear each: group g belongs
+ * to part[g] (0, 1, ...: one after the other) and runs there on route[g] lanes (1: one group after the other; 0: together
+ * with the part's others through one LDLQ call). */
+int qtip_selftest_group_plan(int device_slots, int ngroups, const int* m, const int* n, const qtip_opts* opts, int* part, int* route);
 /* Allocates what qtip_run_groups keeps of Hessians up to n x n ahead of the first call (optional): its ring of three
  * (HRr, L) pairs and the factorization's work matrix on the device, 32 n^2 bytes; with opts->ldl_device_updates = 0 the ring
  * in page-locked host memory, 24 n^2 bytes.  qtip_reserve_groups: for the default options. */

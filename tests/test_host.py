@@ -138,6 +138,41 @@ def test_group_lane_rule(pkg):
     assert rc != 0
 
 
+def _plan(pkg, shapes, slots=768, **opt):
+    """[(part, route)] of groups (m, n): route 0 together, else the number of lanes."""
+    import ctypes as C
+    k = len(shapes)
+    ints = C.c_int * k
+    part, route = ints(), ints()
+    q = pkg.QuantOpts(**opt)
+    co = pkg._OptsC(q.sigma_reg, q.scale_override, q.ldl_threads, q.feedback, 0, 1 if q.ldl_device_updates else 0, q.ldlq_chains,
+                    q.group_lanes)
+    rc = pkg.lib().qtip_selftest_group_plan(slots, k, ints(*[m for m, _ in shapes]), ints(*[n for _, n in shapes]), C.byref(co),
+                                            part, route)
+    assert rc == 0, pkg.lib().qtip_last_error()
+    return list(zip(part, route))
+
+
+def test_group_plan(pkg):
+    """What qtip_run_groups makes of a call: groups that fill the chip one after the other, small ones of one shape together,
+    the rest on lanes; an explicit number of lanes, or the LDL on the host, keeps everything on lanes."""
+    A, B, big = (1024, 1024), (2048, 1024), (12288, 1024)
+    assert _plan(pkg, []) == []
+    assert _plan(pkg, [A]) == [(0, 1)]
+    assert _plan(pkg, [A] * 3) == [(0, 0)] * 3
+    assert _plan(pkg, [A, B]) == [(0, 2)] * 2
+    assert _plan(pkg, [big] * 3) == [(0, 1)] * 3
+    assert _plan(pkg, [big, A]) == [(0, 1)] * 2                     # in their order, as one schedule
+    assert _plan(pkg, [A, big, big]) == [(0, 1)] * 3
+    assert _plan(pkg, [big, A, big, A]) == [(0, 1), (1, 0), (0, 1), (1, 0)]
+    assert _plan(pkg, [A, big, B]) == [(1, 2), (0, 1), (1, 2)]
+    assert _plan(pkg, [A] * 3, group_lanes=2) == [(0, 2)] * 3
+    assert _plan(pkg, [A] * 3, group_lanes=1) == [(0, 1)] * 3
+    assert _plan(pkg, [A] * 3, ldl_device_updates=False) == [(0, 3)] * 3
+    assert _plan(pkg, [(1024, 1040)] * 2) == [(0, 2)] * 2           # refused there
+
+
+
 def test_cholesky_inplace_fp64_bits(pkg, oracle):
     """qtip_cholesky_inplace: every bit of the fp64 factor equals the compiled reference's committed rows (n = 528) and
     the oracle's factor of a matrix with correlated, badly scaled channels (n = 784)."""
