@@ -343,9 +343,12 @@ int group_lanes_for(int ng, const qtip_group* groups, const qtip_opts& opt, int 
 // alone (fp32 sums of products are cut as alone, gemm_splitk_splits).  Six 2048 x 2560 groups from host memory: 166 -> 95 ms.
 // A group that cannot be prepared (its H is not positive definite, say) does not keep the others from their results; the
 // first such error is thrown at the end.
-int together_batch(int ng, long rows, int n, int device_slots) {
-  // groups per call: the fewest rounds of workgroups in all, then the fewest calls; its buffers stay under 32 GiB
-  const long bytes = 24L * n * n + 10L * n * 16 * rows;
+static int together_batch(int ng, long rows, int n, int feedback, int device_slots) {
+  // groups per call: the fewest rounds of workgroups in all, then the fewest calls; its buffers stay under 32 GiB.  Of each
+  // group: the rotated Hessian, what it is rotated from and its factor in fp32, the fp64 work matrix (20 n^2); the weights as
+  // they come, in fp32 and rotated, their reconstruction and states, the proxy's images (29 n m); the gathered products and
+  // their splits (17 KB a row).  fp32 feedback: the images of the factor and of the residuals.
+  const long m = 16 * rows, bytes = (20L + 4 * feedback) * n * n + (29L + 4 * feedback) * n * m + 17408L * m;
   const long most = std::min<long>({long(ng), long(qtip_ctx::kMaxLanes), std::max<long>(1, (32L << 30) / bytes)});
   long best = 1, best_cost = -1;
   for (long b = 1; b <= most; ++b) {
@@ -360,7 +363,7 @@ static void run_groups_together(qtip_ctx* c, int ng, const qtip_group* groups, c
                                 double* ldl_wait) {
   const int n = groups[0].n;
   const long mt = 16 * tile_rows_of(groups[0]);
-  const int batch = together_batch(ng, mt / 16, n, viterbi_max_slots(c->device));
+  const int batch = together_batch(ng, mt / 16, n, opt.feedback, viterbi_max_slots(c->device));
   const size_t nm = size_t(n) * mt, nn = size_t(n) * n, states = size_t(mt / 16) * (n / 16) * 128;
   ArenaScope memory(&c->arena);
   DBuf<float> WT(nm * batch), hat(nm * batch), L(nn * batch);
@@ -414,7 +417,7 @@ static void run_groups_together(qtip_ctx* c, int ng, const qtip_group* groups, c
     on_lanes([&](int k, Lane& l, const qtip_group& g) {
       qtip_timing T{};
       l.su.assign(size_t(n), 0.0f);
-      reserve_group_ring(l.c, n, 1, true);
+      l.c->ring_dHRr[0].ensure(nn);  // (the factor goes to the call's buffer)
       double t0 = now_s();
       rotate_hessian_impl(l.c, g.H, g.h_on_device != 0, n, g.seed, opt.sigma_reg, l.su.data(), &l.creg, nullptr,
                           l.c->ring_dHRr[0].p);
@@ -540,8 +543,12 @@ std::vector<GroupPart> plan_groups(int ng, const qtip_group* groups, const qtip_
   std::vector<int> all;
   for (int g = 0; g < ng; ++g) all.push_back(g);
   if (opt.group_lanes != 0 || ng < 2) return {by_lanes(all)};
-  // groups that may go together, if there are several of their shape
-  auto shaped = [&](int g) { return opt.ldl_device_updates != 0 && groups[g].n % 128 == 0; };
+  // groups that may go together, if there are several of their shape.  (Not where there is room for one at a time only: two
+  // lanes have a group's factorization under the other's LDLQ.  Two 4096 x 28672 groups 1213 ms on lanes, 1666 one by one.)
+  auto shaped = [&](int g) {
+    return opt.ldl_device_updates != 0 && groups[g].n % 128 == 0 &&
+           together_batch(2, tile_rows_of(groups[g]), groups[g].n, opt.feedback, device_slots) >= 2;
+  };
   auto alike = [&](int a, int b) {
     return shaped(a) && groups[a].n == groups[b].n && tile_rows_of(groups[a]) == tile_rows_of(groups[b]);
   };
