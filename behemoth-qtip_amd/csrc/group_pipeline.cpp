@@ -545,7 +545,10 @@ std::vector<GroupPart> plan_groups(int ng, const qtip_group* groups, const qtip_
   if (opt.group_lanes != 0 || ng < 2) return {by_lanes(all)};
   // groups that may go together, if there are several of their shape.  (Not where there is room for one at a time only: two
   // lanes have a group's factorization under the other's LDLQ.  Two 4096 x 28672 groups 1213 ms on lanes, 1666 one by one.)
+  // A group that will be refused for its sizes must not size the call's buffers.
   auto shaped = [&](int g) {
+    for (int i = 0; i < groups[g].nlin; ++i)
+      if (groups[g].lins[i].m <= 0 || groups[g].lins[i].m % 32 != 0) return false;
     return opt.ldl_device_updates != 0 && groups[g].n % 128 == 0 &&
            together_batch(2, tile_rows_of(groups[g]), groups[g].n, opt.feedback, device_slots) >= 2;
   };

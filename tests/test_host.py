@@ -170,6 +170,7 @@ def test_group_plan(pkg):
     assert _plan(pkg, [A] * 3, group_lanes=1) == [(0, 1)] * 3
     assert _plan(pkg, [A] * 3, ldl_device_updates=False) == [(0, 3)] * 3
     assert _plan(pkg, [(1024, 1040)] * 2) == [(0, 2)] * 2           # refused there
+    assert _plan(pkg, [(-32, 1024)] * 2) == _plan(pkg, [(48, 1024)] * 2) == [(0, 2)] * 2
     # 32 GiB hold one such group of a call, so they keep to lanes
     assert _plan(pkg, [(4096, 28672)] * 2) == [(0, 2)] * 2
     assert _plan(pkg, [(4096, 20480)] * 2) == [(0, 0)] * 2
