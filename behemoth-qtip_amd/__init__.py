@@ -147,7 +147,7 @@ def lib():
     L.qtip_reserve_groups_for.argtypes = [vp, i, vp]
     L.qtip_group_lanes.argtypes = [vp, i, vp, C.POINTER(_OptsC), C.POINTER(C.c_int)]
     L.qtip_selftest_group_lanes.argtypes = [i, i, i, i, i, C.POINTER(C.c_int)]
-    L.qtip_selftest_group_plan.argtypes = [i, i, vp, vp, vp, vp, vp]
+    L.qtip_selftest_group_plan.argtypes = [i, i, i, vp, vp, vp, vp, vp]
     L.qtip_st_create.argtypes = [C.POINTER(vp)]
     L.qtip_st_destroy.argtypes = [vp]
     L.qtip_st_destroy.restype = None

@@ -5,11 +5,13 @@
 // layer up front and keeps every HRr; here rotation runs two groups ahead through a ring of three (HRr, L) pairs kept by
 // the context, on the device or, with the LDL on the host, in page-locked memory, so that it stays at 6 n^2 floats however
 // many groups are queued.
+#include <algorithm>
 #include <chrono>
 #include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <exception>
+#include <functional>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -533,7 +535,14 @@ static void run_groups_on_lanes(qtip_ctx* c, int ng, const qtip_group* groups, c
 // How a call's groups are run, in this order.  Mixed sizes (a layer's gate/up group beside its o-proj group): the groups that
 // fill the chip on their own go through the overlapped schedule first, in their order, then those of one shape together, and
 // what is left shares the chip on lanes.
-std::vector<GroupPart> plan_groups(int ng, const qtip_group* groups, const qtip_opts& opt, int device_slots) {
+// Several shapes that fill less than half of the slots each may be better off side by side than one shape after the other.
+// A call of a shape is a chain of tiles by pairs of workgroups, as long as its n, and the shapes' chains add up; a lane's tiles
+// take twice as long, but the lanes' chains run at the same time, if each lane has a hardware queue, which the process may
+// not have: beside(k) says whether k lanes do.  Twelve groups of 64 tile rows in six shapes of n = 640 .. 1280: 88 ms shape by
+// shape, on lanes 47 ms with 16 queues and 104 with HIP's default of 4; in two shapes of n = 1024 and 1280 35 and 38 ms.  From
+// half of the slots on there is little between the two (two shapes of 2 x 384 rows 110 and 107 ms).
+std::vector<GroupPart> plan_groups(int ng, const qtip_group* groups, const qtip_opts& opt, int device_slots,
+                                   const std::function<bool(int)>& beside) {
   auto by_lanes = [&](std::vector<int> some) {
     std::vector<qtip_group> sub;
     for (int g : some) sub.push_back(groups[g]);
@@ -568,9 +577,28 @@ std::vector<GroupPart> plan_groups(int ng, const qtip_group* groups, const qtip_
     shapes[k].push_back(g);
   }
   std::vector<GroupPart> parts;
-  for (std::vector<int>& shape : shapes)
-    if (shape.size() >= 2) parts.push_back({GroupRoute::kTogether, 1, shape});
-    else left.push_back(shape[0]);
+  std::vector<std::vector<int>> few;  // several groups of a shape, which fill less than half of the slots
+  for (std::vector<int>& shape : shapes) {
+    if (shape.size() < 2) left.push_back(shape[0]);
+    else if (2 * long(shape.size()) * tile_rows_of(groups[shape[0]]) < device_slots) few.push_back(shape);
+    else parts.push_back({GroupRoute::kTogether, 1, shape});
+  }
+  std::vector<int> side = left;
+  for (const std::vector<int>& shape : few) side.insert(side.end(), shape.begin(), shape.end());
+  std::sort(side.begin(), side.end());
+  auto longest = [&](const std::vector<int>& some) {
+    long n = 0;
+    for (int g : some) n = std::max<long>(n, groups[g].n);
+    return n;
+  };
+  long by_shape = longest(left) * (left.size() >= 2 ? 2 : 1);
+  for (const std::vector<int>& shape : few) by_shape += groups[shape[0]].n;
+  GroupPart lanes;
+  if (!few.empty() && few.size() + left.size() >= 2) lanes = by_lanes(side);
+  const long rounds = lanes.lanes > 1 ? (long(side.size()) + lanes.lanes - 1) / lanes.lanes : 1;
+  if (lanes.lanes > 1 && 2 * longest(side) * rounds < by_shape && beside(lanes.lanes)) left = side;
+  else
+    for (const std::vector<int>& shape : few) parts.push_back({GroupRoute::kTogether, 1, shape});
   // (large groups beside one small one: in their order, as one schedule)
   if (!large.empty() && parts.empty() && left.size() <= 1) return {by_lanes(all)};
   if (!large.empty()) parts.insert(parts.begin(), by_lanes(large));
@@ -589,7 +617,11 @@ void run_groups_impl(qtip_ctx* c, int ng, const qtip_group* groups, const qtip_o
   // an error among the large groups ends the call, as it ends their schedule; one among the others does not keep the other
   // parts from their results and is reported at the end
   std::exception_ptr first_err;
-  for (const GroupPart& part : plan_groups(ng, groups, opt, slots)) {
+  auto beside = [&](int lanes) {
+    for (int k = 0; k < lanes; ++k) (void)lane_context(c, k);
+    return c->lanes_beside >= lanes;
+  };
+  for (const GroupPart& part : plan_groups(ng, groups, opt, slots, beside)) {
     const size_t count = part.groups.size();
     std::vector<qtip_group> sub;
     for (int g : part.groups) sub.push_back(groups[g]);

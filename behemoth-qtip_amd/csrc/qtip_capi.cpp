@@ -286,6 +286,7 @@ qtip_ctx* lane_context(qtip_ctx* parent, int k) {
       if (own) (void)hipStreamDestroy(own);
       throw;
     }
+    if (parent->lanes_beside == k && (k == 0 || own)) parent->lanes_beside = k + 1;
     // one stream per lane, the factorization's work included: a stream only runs beside the others if it has a
     // hardware queue to itself, and a process has few of them (GPU_MAX_HW_QUEUES, 4 unless the environment says
     // more); with a stream more per lane for the factorization 1024 x 1024 groups ran at 59 instead of 134 Mweights/s
@@ -301,6 +302,7 @@ qtip_ctx* lane_context(qtip_ctx* parent, int k) {
 void release_lanes(qtip_ctx* parent) {
   parent->arena.children.clear();
   parent->lane_streams_exhausted = false;
+  parent->lanes_beside = 0;
   for (qtip_ctx*& l : parent->lane)
     if (l) {
       destroy_context(l);
@@ -787,7 +789,8 @@ int qtip_selftest_group_lanes(int device_slots, int ngroups, int m, int n, int r
   });
 }
 
-int qtip_selftest_group_plan(int device_slots, int ngroups, const int* m, const int* n, const qtip_opts* opts, int* part, int* route) {
+int qtip_selftest_group_plan(int device_slots, int lanes_beside, int ngroups, const int* m, const int* n, const qtip_opts* opts,
+                             int* part, int* route) {
   // host only: the parts that qtip_run_groups makes of groups of one m x n linear each
   return guarded([&] {
     QTIP_REQUIRE(device_slots > 0 && ngroups >= 0 && ngroups <= 4096 && (ngroups == 0 || (m && n && part && route)),
@@ -803,7 +806,7 @@ int qtip_selftest_group_plan(int device_slots, int ngroups, const int* m, const 
     qtip_default_opts(&o);
     if (opts) o = *opts;
     int at = 0;
-    for (const GroupPart& p : plan_groups(ngroups, groups.data(), o, device_slots)) {
+    for (const GroupPart& p : plan_groups(ngroups, groups.data(), o, device_slots, [&](int k) { return k <= lanes_beside; })) {
       for (int g : p.groups) part[g] = at, route[g] = p.route == GroupRoute::kTogether ? 0 : p.lanes;
       ++at;
     }

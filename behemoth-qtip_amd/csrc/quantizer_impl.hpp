@@ -1,5 +1,7 @@
 // The context behind the C ABI and the group-quantizer entry points implemented in quantizer_impl.cpp.
 #pragma once
+#include <functional>
+
 #include "ldlq.hpp"
 #include "misc.hpp"
 #include "qtip_internal.hpp"
@@ -36,6 +38,7 @@ struct qtip_ctx {
   // (streams, workspaces, rings) made on first use, kept here and released with this context
   static constexpr int kMaxLanes = 12;
   qtip_ctx* lane[kMaxLanes] = {};
+  int lanes_beside = 0;                 // the lanes up to here were found to run beside each other when they were made
   bool lane_streams_exhausted = false;  // a lane found no stream that runs beside the earlier lanes': no search for the later ones
 
   // LDLQ runs its tile rows as up to kMaxChains independent chains of launches, on the context's stream and these,
@@ -122,14 +125,15 @@ void order_streams(hipStream_t first, hipStream_t then);
 // how many groups qtip_run_groups runs side by side (1: one after the other on the context itself)
 int group_lanes_for(int ngroups, const qtip_group* groups, const qtip_opts& opt, int device_slots);
 // how qtip_run_groups runs its groups: as parts, one after the other - groups one after the other on the context itself
-// (kSchedule), on that many lanes, or through LDLQ in one call (kTogether).  Host only.
+// (kSchedule), on that many lanes, or through LDLQ in one call (kTogether).  beside(k): whether k lanes run beside each other.
 enum class GroupRoute { kSchedule, kLanes, kTogether };
 struct GroupPart {
-  GroupRoute route;
-  int lanes;
+  GroupRoute route = GroupRoute::kLanes;
+  int lanes = 0;
   std::vector<int> groups;
 };
-std::vector<GroupPart> plan_groups(int ngroups, const qtip_group* groups, const qtip_opts& opt, int device_slots);
+std::vector<GroupPart> plan_groups(int ngroups, const qtip_group* groups, const qtip_opts& opt, int device_slots,
+                                   const std::function<bool(int)>& beside);
 void run_groups_impl(qtip_ctx* c, int ngroups, const qtip_group* groups, const qtip_opts& opt, qtip_timing* timings,
                      double* ldl_wait);
 uint8_t f32_to_fp8e4m3(float x);

@@ -310,8 +310,9 @@ int qtip_nvfp4_prepare_device_updates(qtip_ctx* ctx, const float* host_H, int n,
  * takes its groups one after the other on a stream of its own; same results); then an error leaves the groups before the
  * failing one on its lane complete, the other lanes finish their groups, and the first failing lane's error is
  * reported.  With group_lanes = 0 and groups of mixed sizes, the groups of 12288 rows and more run first, in their
- * order, one after the other, then those of one shape together, and the rest share the chip on lanes: an error among the
- * large ones ends the call, one among the others leaves the groups of the other shapes complete.  Groups that run
+ * order, one after the other, then those of one shape together, and the rest share the chip on lanes.  (Shapes that fill less than
+ * half of the chip's slots also go to lanes where that is shorter than one shape after the other and the process has a hardware
+ * queue for each lane.)  An error among the large ones ends the call, one among the others leaves the groups of the other shapes complete.  Groups that run
  * together (group_lanes = 0, one shape): a failing group leaves the others' results complete, and the first error is
  * reported at the end. */
 typedef struct {
@@ -332,10 +333,11 @@ int qtip_group_lanes(qtip_ctx* ctx, int ngroups, const qtip_group* groups, const
 /* Host-only check of the lane rule: `ngroups` equal groups of one m x n linear on a device with `device_slots`
  * Viterbi workgroup slots, qtip_opts.group_lanes = requested. */
 int qtip_selftest_group_lanes(int device_slots, int ngroups, int m, int n, int requested, int* lanes);
-/* Host-only check of the order and manner in which qtip_run_groups runs groups of one m[g] x n[g] linear each: group g belongs
- * to part[g] (0, 1, ...: one after the other) and runs there on route[g] lanes (1: one group after the other; 0: together
- * with the part's others through one LDLQ call). */
-int qtip_selftest_group_plan(int device_slots, int ngroups, const int* m, const int* n, const qtip_opts* opts, int* part, int* route);
+/* Host-only check of the order and manner in which qtip_run_groups runs groups of one m[g] x n[g] linear each, where lanes_beside
+ * lanes run beside each other: group g belongs to part[g] (0, 1, ...: one after the other) and runs there on route[g] lanes
+ * (1: one group after the other; 0: together with the part's others through one LDLQ call). */
+int qtip_selftest_group_plan(int device_slots, int lanes_beside, int ngroups, const int* m, const int* n, const qtip_opts* opts,
+                             int* part, int* route);
 /* Allocates what qtip_run_groups keeps of Hessians up to n x n ahead of the first call (optional): its ring of three
  * (HRr, L) pairs and the factorization's work matrix on the device, 32 n^2 bytes; with opts->ldl_device_updates = 0 the ring
  * in page-locked host memory, 24 n^2 bytes.  qtip_reserve_groups: for the default options. */

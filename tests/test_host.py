@@ -138,7 +138,7 @@ def test_group_lane_rule(pkg):
     assert rc != 0
 
 
-def _plan(pkg, shapes, slots=768, **opt):
+def _plan(pkg, shapes, beside=4, slots=768, **opt):
     """[(part, route)] of groups (m, n): route 0 together, else the number of lanes."""
     import ctypes as C
     k = len(shapes)
@@ -147,7 +147,7 @@ def _plan(pkg, shapes, slots=768, **opt):
     q = pkg.QuantOpts(**opt)
     co = pkg._OptsC(q.sigma_reg, q.scale_override, q.ldl_threads, q.feedback, 0, 1 if q.ldl_device_updates else 0, q.ldlq_chains,
                     q.group_lanes)
-    rc = pkg.lib().qtip_selftest_group_plan(slots, k, ints(*[m for m, _ in shapes]), ints(*[n for _, n in shapes]), C.byref(co),
+    rc = pkg.lib().qtip_selftest_group_plan(slots, beside, k, ints(*[m for m, _ in shapes]), ints(*[n for _, n in shapes]), C.byref(co),
                                             part, route)
     assert rc == 0, pkg.lib().qtip_last_error()
     return list(zip(part, route))
@@ -171,6 +171,18 @@ def test_group_plan(pkg):
     assert _plan(pkg, [A] * 3, ldl_device_updates=False) == [(0, 3)] * 3
     assert _plan(pkg, [(1024, 1040)] * 2) == [(0, 2)] * 2           # refused there
     assert _plan(pkg, [(-32, 1024)] * 2) == _plan(pkg, [(48, 1024)] * 2) == [(0, 2)] * 2
+    # several shapes that fill less than half of the slots each: on lanes where the shapes' chains add up to more than twice the
+    # longest and every lane has a queue, else shape by shape
+    C, six = (1024, 512), [(1024, 128 * k) for k in range(3, 9)]
+    assert _plan(pkg, [A, C, A, C], beside=12) == [(0, 0), (1, 0), (0, 0), (1, 0)]
+    assert _plan(pkg, six * 2, beside=12) == [(0, 12)] * 12
+    assert _plan(pkg, six * 2, beside=4) == [(k, 0) for k in range(6)] * 2
+    assert _plan(pkg, six[3:] * 4, beside=12) == [(0, 12)] * 12
+    assert _plan(pkg, six[3:] * 5, beside=12) == [(k, 0) for k in range(3)] * 5  # two rounds of lanes
+    assert _plan(pkg, six[:5] * 2 + six[5:], beside=12) == [(0, 11)] * 11       # and one alone in its shape
+    assert _plan(pkg, [A, A, C], beside=12) == [(0, 0), (0, 0), (1, 1)]
+    assert _plan(pkg, [A, A, big]) == [(1, 0), (1, 0), (0, 1)]
+    assert _plan(pkg, [(6144, 512)] * 2 + six * 2, beside=12) == [(0, 0)] * 2 + [(1, 12)] * 12
     # 32 GiB hold one such group of a call, so they keep to lanes
     assert _plan(pkg, [(4096, 28672)] * 2) == [(0, 2)] * 2
     assert _plan(pkg, [(4096, 20480)] * 2) == [(0, 0)] * 2
