@@ -105,6 +105,7 @@ def lib():
     L.qtip_selftest_device_alloc_calls.restype = l
     L.qtip_set_viterbi_mode.argtypes = [vp, i, C.c_uint]
     L.qtip_viterbi_stats.argtypes = [vp, C.POINTER(C.c_ulonglong), C.POINTER(C.c_ulonglong), i]
+    L.qtip_selftest_viterbi_searches.argtypes = [vp, C.POINTER(C.c_ulonglong), C.POINTER(C.c_ulonglong)]
     L.qtip_ldlq_default_chains.argtypes = [vp, C.POINTER(C.c_int)]
     L.qtip_stream_wait.argtypes = [vp, vp]
     L.qtip_stream_signal.argtypes = [vp, vp]
@@ -377,6 +378,12 @@ class Quantizer:
         """(first passes, second passes) that mode 0 ran again on fp64 metrics."""
         a, b = C.c_ulonglong(0), C.c_ulonglong(0)
         _check(lib().qtip_viterbi_stats(self._h, C.byref(a), C.byref(b), 1 if reset else 0))
+        return int(a.value), int(b.value)
+
+    def viterbi_searches(self):
+        """(searches that settled their tile's second pass, searches that gave up) since viterbi_stats(reset=True)."""
+        a, b = C.c_ulonglong(0), C.c_ulonglong(0)
+        _check(lib().qtip_selftest_viterbi_searches(self._h, C.byref(a), C.byref(b)))
         return int(a.value), int(b.value)
 
     def viterbi_tiles_dev(self, dX, B, d_states=None, d_packed=None):

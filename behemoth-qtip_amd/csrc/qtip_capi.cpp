@@ -299,6 +299,21 @@ qtip_ctx* lane_context(qtip_ctx* parent, int k) {
   return parent->lane[k];
 }
 
+// the Viterbi counters of a context and its lanes (TileJob::stats), once the device is idle
+static void take_viterbi_stats(qtip_ctx* ctx, unsigned long long (&sum)[4], bool reset) {
+  for (auto& v : sum) v = 0;
+  auto take = [&](qtip_ctx* c) {
+    QTIP_HIP(hipDeviceSynchronize());
+    unsigned v[4];
+    QTIP_HIP(hipMemcpy(v, c->vit_stats.p, sizeof v, hipMemcpyDeviceToHost));
+    for (int i = 0; i < 4; ++i) sum[i] += v[i];
+    if (reset) QTIP_HIP(hipMemset(c->vit_stats.p, 0, sizeof v));
+  };
+  take(ctx);
+  for (qtip_ctx* l : ctx->lane)
+    if (l) take(l);
+}
+
 void release_lanes(qtip_ctx* parent) {
   parent->arena.children.clear();
   parent->lane_streams_exhausted = false;
@@ -496,19 +511,20 @@ int qtip_viterbi_stats(qtip_ctx* ctx, unsigned long long* redone_first, unsigned
   return guarded([&] {
     QTIP_REQUIRE(ctx != nullptr, "null context");
     DeviceGuard g(ctx);
-    unsigned long long sum[2] = {0, 0};
-    auto take = [&](qtip_ctx* c) {
-      QTIP_HIP(hipDeviceSynchronize());
-      unsigned v[4];
-      QTIP_HIP(hipMemcpy(v, c->vit_stats.p, sizeof v, hipMemcpyDeviceToHost));
-      sum[0] += v[0], sum[1] += v[1];
-      if (reset) QTIP_HIP(hipMemset(c->vit_stats.p, 0, sizeof v));
-    };
-    take(ctx);
-    for (qtip_ctx* l : ctx->lane)
-      if (l) take(l);
+    unsigned long long sum[4];
+    take_viterbi_stats(ctx, sum, reset != 0);
     if (redone_first) *redone_first = sum[0];
     if (redone_second) *redone_second = sum[1];
+  });
+}
+
+int qtip_selftest_viterbi_searches(qtip_ctx* ctx, unsigned long long* settled, unsigned long long* gave_up) {
+  return guarded([&] {
+    QTIP_REQUIRE(ctx != nullptr && settled != nullptr && gave_up != nullptr, "selftest: null argument");
+    DeviceGuard g(ctx);
+    unsigned long long sum[4];
+    take_viterbi_stats(ctx, sum, false);
+    *settled = sum[2], *gave_up = sum[3];
   });
 }
 

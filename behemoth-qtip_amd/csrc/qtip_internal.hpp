@@ -248,7 +248,9 @@ struct TileJob {
   unsigned long long pair_patience = 50000000ull;
   uint32_t margin = kViterbiMargin;
   bool search = true;  // mode 0: the second pass as a search between bounds from the first (set by launch_viterbi_tiles; same results)
-  unsigned* stats = nullptr;  // device counters (optional): [0], [1] += passes of the first / second kind run again
+  // device counters (optional): [0], [1] += passes of the first / second kind run again; [2], [3] += searches that settled
+  // their tile / gave up
+  unsigned* stats = nullptr;
 };
 size_t viterbi_workspace_bytes(int slots);
 int viterbi_max_slots(int device);

@@ -20,7 +20,7 @@ struct qtip_ctx {
   qtipmi::DBuf<unsigned char> vit_ws;  // kept-metrics slots of the resident Viterbi workgroups
   int vit_slots = 0;
   // Viterbi passes: 0 = 32-bit metrics first, fp64 again where a traced decision is too close (same results);
-  // 1 = fp64 only.  vit_stats: two device counters, passes of the first / second kind that were run again.
+  // 1 = fp64 only.  vit_stats: four device counters (TileJob::stats).
   int vit_mode = 0;
   int vit_wide = -1;  // TileJob::wide; a lane runs beside other lanes and keeps to the 256-thread workgroups
   uint32_t vit_margin = qtipmi::kViterbiMargin;

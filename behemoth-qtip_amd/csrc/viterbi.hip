@@ -1290,9 +1290,11 @@ __device__ __forceinline__ void block_passes(Smem& sm, const TileJob& job, const
         // not fit is replaced by the true one when the pass is repeated on fp64 metrics)
         expected = __builtin_ldexpf(float(winner), -unit_log2);
         if constexpr (kClose) {
-          if (!flag && passes_end > 1 && job.search)
+          if (!flag && passes_end > 1 && job.search) {
             closed = close_path<kWide>(sm, tl, hist32, uint32_t(__builtin_amdgcn_readfirstlane(int(s & 0xfffu))),
                                        uint32_t(__builtin_amdgcn_readfirstlane(int(winner))), grown, job.margin, unit);
+            if (threadIdx.x == 0 && job.stats) atomicAdd(job.stats + (closed ? 2 : 3), 1u);
+          }
         }
       } else {
         forward_pass32<false, kWide>(sm, entry_d, roll, ov, hist32, 0, unit);
@@ -1948,7 +1950,9 @@ bool launch_viterbi_tiles(const TileJob& tile_job, const double* d_entry_d, cons
   const unsigned grid = unsigned(job.tiles < slots ? job.tiles : slots);
   // A search takes a third of the pass's time on average and longer than the pass where it has to give up, and a launch
   // lasts as long as its slowest workgroup: one tile each, 768 tiles 732 us with searches and 695 without; 1100 tiles
-  // 1005 / 1063, 1600 1364 / 1491, 4096 2660 / 3700, 768 tile rows of 8 blocks each 4.2 / 5.1 ms.
+  // 1005 / 1063, 1600 1364 / 1491, 4096 2660 / 3700.  A workgroup that takes several tiles, or a tile row through several
+  // blocks, evens that out, however full the chip is: LDLQ of one group with n = 1024, 392 tile rows 29.3 ms with searches
+  // and 34.3 without, 512 30.0 / 35.6, 640 36.3 / 47.9, 760 38.8 / 50.2; on twelve lanes of 64 rows 46.7 / 61.1.
   job.search = job.blocks > 1 || job.tiles > long(grid);
   // the wide form where the launch leaves two thirds of the chip's workgroup slots empty anyway (and the 32-bit
   // passes, which are what it shares out over its 512 threads, are in use)

@@ -105,6 +105,9 @@ int qtip_set_viterbi_mode(qtip_ctx* ctx, int mode, unsigned margin_units);
  * first passes (free ends, on the rotated sequence) and second passes (tail-biting).  Waits for the device.
  * Either pointer may be NULL. */
 int qtip_viterbi_stats(qtip_ctx* ctx, unsigned long long* redone_first, unsigned long long* redone_second, int reset);
+/* Second passes of mode 0 that a search between the first pass's bounds has settled, and those that were run in full after a search
+ * gave up, since the last reset of qtip_viterbi_stats.  Waits for the device. */
+int qtip_selftest_viterbi_searches(qtip_ctx* ctx, unsigned long long* settled, unsigned long long* gave_up);
 /* What qtip_opts.ldlq_chains = 0 stands for in this context: 2 or 3 (see there).  No counterpart in the reference,
  * whose LDLQ is one sequence of launches (src/quantizer.cpp:42-108). */
 int qtip_ldlq_default_chains(qtip_ctx* ctx, int* chains);

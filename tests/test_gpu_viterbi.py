@@ -356,7 +356,12 @@ def _closing_inputs(kind, B, l0, l1):
     if kind == "scales":
         X *= np.exp(rng.uniform(np.log(0.02), np.log(8.0), (B, 1)))
     elif kind == "join":          # the free path's ends meet where the inputs allow no detour: large values around step 64
-        X[:, 96:160] *= 6.0
+        X *= 0.6
+        X[:, 96:160] *= 3.0
+    elif kind == "turn":          # the same where the closed path's ends meet
+        X *= 0.6
+        X[:, :32] *= 3.0
+        X[:, 224:] *= 3.0
     elif kind == "flat":          # many paths of nearly the same cost
         X = np.round(X * 4) / 4 * 0.25
     elif kind == "zeros":
@@ -374,7 +379,7 @@ def _closing_inputs(kind, B, l0, l1):
     return X.astype(np.float16).astype(np.float32)
 
 
-@pytest.mark.parametrize("kind", ["scales", "join", "flat", "zeros", "mirror"])
+@pytest.mark.parametrize("kind", ["scales", "join", "turn", "flat", "zeros", "mirror"])
 @pytest.mark.parametrize("B", [1, 769, 1100])
 def test_closed_path_search_gives_the_fp64_states(qz, oracle, hyb, kind, B):
     """The tail-biting pass is searched for between bounds from the free pass and run in full only where the search does not
@@ -398,3 +403,31 @@ def test_closed_path_search_gives_the_fp64_states(qz, oracle, hyb, kind, B):
         assert np.array_equal(got[mode][1], got[1][1])
     some = list(range(0, B, 97))
     assert np.array_equal(got[1][0][some], oracle.quantize_tiles(hyb, X[some], fast=True))
+
+
+@pytest.mark.parametrize("kind,searched,settled", [("gauss", 1000, 0.97), ("scales", 600, 0.9), ("join", 1000, 0.5),
+                                                   ("turn", 1000, 0.5), ("flat", 1000, 0.9), ("zeros", 0, 0), ("mirror", 1000, 0)])
+def test_searches_settle_ordinary_tiles(qz, oracle, hyb, kind, searched, settled):
+    """A launch with more tiles than workgroups searches every tile whose first pass is clear: nearly all ordinary ones are settled
+    that way, those whose free path arrives at the complement of its start are not.  (How many are searched and the share settled of
+    them, at least; what these inputs give, settled of searched: 1099 of 1100, 762 of 798, 855 of 1095, 891 of 1089, 1095 of 1100, 97 of
+    1079, 0 of 1100.)  One tile per workgroup is not searched."""
+    B = 1100
+    say("case: searches, %s" % kind)
+    qz.set_tlut(None)
+    qz.set_viterbi_mode(0)
+    l0, l1 = qz.lut()
+    X = _closing_inputs(kind, B, np.asarray(l0), np.asarray(l1))
+    if kind == "gauss":
+        X = (X * (0.9 * qz.lut_rms)).astype(np.float16).astype(np.float32)
+    qz.viterbi_stats(reset=True)
+    qz.viterbi_tiles(X)
+    found, without = qz.viterbi_searches()
+    first, _ = qz.viterbi_stats(reset=True)
+    say("  settled %d, gave up %d, first passes again %d" % (found, without, first))
+    assert found + without == B - first
+    assert found + without >= searched and found >= settled * (found + without)
+    if kind == "mirror":
+        assert without >= 1000
+    qz.viterbi_tiles(X[:700])
+    assert qz.viterbi_searches() == (0, 0)
