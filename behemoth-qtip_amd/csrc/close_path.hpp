@@ -39,10 +39,10 @@ static_assert(kTurn % 2 == 0 && kTurn < kSteps / 2);
 // the search is tried once more with a higher limit, then false is returned and the caller runs the pass.
 // What bounds it: latency.  A step is a chain of five LDS round trips and some 150 instructions, 0.85 us by itself and
 // 1.1 us beside two other workgroups, 120 steps a tile; the pipes it leaves idle are the other workgroups' forward passes'.
-// Per tile with three workgroups on a compute unit 140 us instead of 294 + 75 for the forward recursion and its
-// trace-back, with 60 us more in the free pass for its longer way (768 tile rows through 128 blocks 89.3 -> 69.9 ms; kTurn
-// 40 / 48 / 56: 70.0 / 69.9 / 71.3; at most 48 / 64 / 128 partial paths in the first attempt: 70.6 / 70.0 / 70.7, three
-// attempts with up to 256: 73.3, one: 73.8).
+// Per block with three workgroups on a compute unit (LDLQ of 768 tile rows) 134 us instead of 268 + 76 for the forward
+// recursion and its trace-back, with 20 us more in the free pass and its trace-back; 99.7 % of the searches settle their block.
+// (768 tile rows through 128 blocks 89.3 -> 69.9 ms; kTurn 40 / 48 / 56: 70.0 / 69.9 / 71.3; at most 48 / 64 / 128 partial
+// paths in the first attempt: 70.6 / 70.0 / 70.7, three attempts with up to 256: 73.3, one: 73.8.)
 template <bool kWide>
 __device__ __forceinline__ bool close_path(Smem& sm, const uint32_t* tl, const uint32_t* __restrict__ hist32, uint32_t ov,
                                            uint32_t winner, uint32_t grown, uint32_t margin, const Unit unit) {

@@ -806,8 +806,8 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
     }
     // The next step's table.  The free pass of the 256-thread form fills it behind its last kEnt slots, one entry
     // after each: in front of the slots it is 600 cycles of a step of 3300 in which the slots' reads wait, and three
-    // workgroups to a compute unit do not cover them (4096 tiles 2665 -> 2640 us, 768 tiles 708 -> 688; an entry after
-    // every other slot 2660, all of them at the end 2665).  The 512-thread form has a compute unit to itself and is
+    // workgroups to a compute unit do not cover them (4096 tiles 2665 -> 2640 us, 768 tiles 708 -> 690; an entry after
+    // every other slot 2660, all of them at the end 2667).  The 512-thread form has a compute unit to itself and is
     // faster with the table first (256 tiles 379 against 384 us).
     constexpr bool kTableLate = kSym && !kWide;
     const int tn = (2 * (it + 1) + roll) & 255;
@@ -870,7 +870,7 @@ __device__ __forceinline__ uint32_t forward_pass32(Smem& sm, const double* __res
         }
       };
       // the table value of digit k is the candidate of digit k of the group and of digit 15 - k of its mirror
-      // (256 threads: two chains of minima, one alone waits for itself; 4096 tiles 2725 -> 2690 us.  512 threads: one chain,
+      // (256 threads: two chains of minima, one alone waits for itself; 4096 tiles 2724 -> 2665 us.  512 threads: one chain,
       // which is 0.5 to 1 % faster where a workgroup has a compute unit to itself.)
       auto pair_min = [&](auto value) __attribute__((always_inline)) -> uint32_t {
         if constexpr (kWide) {
