@@ -309,16 +309,23 @@ def run_group(args, pkg):
     nch = args.chains or q.ldlq_default_chains()
     while nch > 1 and ntr < 768:
         nch -= 1
-    # groups too small to fill the chip run side by side (qtip_opts.group_lanes): that many times as many launches
-    # share the chip
+    # groups too small to fill the chip: twelve go through LDLQ together, a chain of launches taking whole groups (a group's
+    # viterbi_s is its share of the call's), or, on lanes (qtip_opts.group_lanes, the LDL on the host), side by side, and that
+    # many times as many launches share the chip
     lanes = q.group_lanes([(ms, n)] * args.steps, opt)
+    together = min(args.steps, 12) if lanes > 1 and args.lanes == 0 and not args.host_ldl else 0
+    if together:
+        lanes = 1
+        nch = args.chains or q.ldlq_default_chains()
+        while nch > 1 and (together % nch or 2 * together * ntr <= 768):
+            nch -= 1
     gpu_s = stats["rht_s"] + stats["load_s"] + stats["ldlq_s"] + stats["proxy_s"] + stats["pack_s"]
     extra = dict(stats)
     extra.update(gpu_only_Mweights_s=weights_per_step / gpu_s / 1e6,
                  serial_Mweights_s=weights_per_step / (gpu_s + stats["ldl_s"]) / 1e6,
                  viterbi_only_Mweights_s=weights_per_step / stats["viterbi_s"] / 1e6,
                  proxy_in_timed_region=True, ldl_threads=args.ldl_threads, feedback=args.feedback,
-                 hw_queues=int(os.environ.get("GPU_MAX_HW_QUEUES", "4")), ldlq_chains=nch, group_lanes=lanes,
+                 hw_queues=int(os.environ.get("GPU_MAX_HW_QUEUES", "4")), ldlq_chains=nch, group_lanes=lanes, groups_together=together,
                  ldl_device_updates=not args.host_ldl)
     extra.update(vit)
     extra.update(legs)
@@ -327,8 +334,8 @@ def run_group(args, pkg):
     extra.update(fb1)
     names = {2: "config2: 1024x1024 group", 3: "config3: 12288x12288 q-proj group",
              4: "config4: gate+up 2x(28672x12288) group", 5: "config5: 12288x28672 down-proj group"}
-    return dict(weights=weights_per_step * args.steps, wall=wall, vit_launch_s=stats["viterbi_s"] / launches,
-                vit_launch_weights=ntr * 256 * 8 * lanes, blocks_per_launch=8, workload=names[cfg] + (" (RHT + host fp64 LDL + LDLQ + 2-pass Viterbi + pack)" if args.host_ldl else
+    return dict(weights=weights_per_step * args.steps, wall=wall, vit_launch_s=stats["viterbi_s"] * max(together, 1) / launches,
+                vit_launch_weights=ntr * 256 * 8 * lanes * max(together, 1), blocks_per_launch=8, workload=names[cfg] + (" (RHT + host fp64 LDL + LDLQ + 2-pass Viterbi + pack)" if args.host_ldl else
                                        " (RHT + fp64 LDL + LDLQ + 2-pass Viterbi + pack)"),
                 extra=extra, cpu_group=cpu_group, concurrent=nch * lanes,
                 ldlq_s=stats["ldlq_s"], weights_per_step=weights_per_step)
